@@ -169,9 +169,9 @@ def _attention_program(mask, window, cap, groups, dynamic):
 
 
 @functools.lru_cache(maxsize=None)
-def _masked_program(groups):
+def _masked_program(grouped):
     def attn(q, k, v, mask):
-        return F.scaled_dot_product_attention(q, k, v, attn_mask=mask, enable_gqa=groups > 1)
+        return F.scaled_dot_product_attention(q, k, v, attn_mask=mask, enable_gqa=grouped)
 
     return torch.compile(attn, backend=_backend, dynamic=True)
 
@@ -216,7 +216,7 @@ def prepare(case, seed):
         lengths = torch.tensor(_lengths(case), device=dev)[order]
         pos = torch.arange(S, device=dev)
         mask = (pos[None, :] <= pos[:, None])[None, None] & (pos[None, :] < lengths[:, None])[:, None, None, :]
-        return {"kind": "masked", "fn": _masked_program(group), "args": (q, k, v, mask)}
+        return {"kind": "masked", "fn": _masked_program(group > 1), "args": (q, k, v, mask)}
     # a serving program sees every prompt length (dynamic shapes), a training step is traced for its own
     train = case["kind"] == "train"
     fn = _attention_program(case["mask"], case["window"], case["softcap"], group, not train)
