@@ -224,15 +224,10 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   const int g = lane >> 5;
 
   const int nkt = (p.Sk + 127) / 128;
-  // Workgroup ids with equal id % 8 run on one XCD.  All key blocks of a (batch, kv head) go to one
-  // XCD, so the Q / dO tiles they all walk are fetched into one L2, once; within an XCD the ids come
-  // in groups of LF_BW_GROUP (batch, kv head) pairs and, inside a group, by key block, the ones with
-  // the most steps under a causal mask first.  The grid is padded to whole groups.
-  const int slot = blockIdx.x / 8;
-  const int in_grp = slot % (LF_BW_GROUP * nkt);
-  const int kt = in_grp / LF_BW_GROUP;
-  const int bhkv = (slot / (LF_BW_GROUP * nkt) * LF_BW_GROUP + in_grp % LF_BW_GROUP) * 8 + (int)(blockIdx.x % 8);
-  if (bhkv >= p.B * p.Hkv) return;
+  // All key blocks of a (batch, kv head) share the Q / dO tiles they walk in one XCD's L2; the first key
+  // block has the most steps under a causal mask.
+  int bhkv, kt;
+  if (!lf_slot_of_block(blockIdx.x, p.B * p.Hkv, nkt, LF_BW_GROUP, bhkv, kt)) return;
   const int hkv = bhkv % p.Hkv;
   const int b = bhkv / p.Hkv;
   const int group = p.Hq / p.Hkv;
@@ -501,14 +496,11 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
 
   constexpr int kBM = LF_BW_DQ_NT / 2;                    // query rows of a workgroup
   const int nqt = (p.Sq + kBM - 1) / kBM;
-  // As in lf_attn_bwd_dkdv: the q tiles of all query heads of a (batch, kv head) run on one XCD
-  // and share its K / V tiles there; inside a group of LF_BW_GROUP pairs the long q tiles come first.
+  // As in lf_attn_bwd_dkdv: the q tiles of all query heads of a (batch, kv head) share its K / V tiles in one
+  // XCD's L2, the long q tiles first.
   const int nrow = (p.Hq / p.Hkv) * nqt;                  // (query head of the group, q tile) per pair
-  const int slot = blockIdx.x / 8;
-  const int in_grp = slot % (LF_BW_GROUP * nrow);
-  const int row = in_grp / LF_BW_GROUP;
-  const int bhkv = (slot / (LF_BW_GROUP * nrow) * LF_BW_GROUP + in_grp % LF_BW_GROUP) * 8 + (int)(blockIdx.x % 8);
-  if (bhkv >= p.B * p.Hkv) return;
+  int bhkv, row;
+  if (!lf_slot_of_block(blockIdx.x, p.B * p.Hkv, nrow, LF_BW_GROUP, bhkv, row)) return;
   const int qt = nqt - 1 - row / (p.Hq / p.Hkv);
   const int hkv = bhkv % p.Hkv;
   const int b = bhkv / p.Hkv;

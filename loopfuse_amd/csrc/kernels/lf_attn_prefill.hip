@@ -112,23 +112,14 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_OCC) lf_attn_prefill(cons
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
-  // ---- workgroup -> (batch*head, q tile).  Workgroup ids are dealt round-robin
-  // to the 8 XCDs, so ids with equal id%8 share an L2: keep all q tiles of one
-  // (batch, head) on one XCD, heaviest (latest) q tile first.
+  // ---- workgroup -> (batch*head, pair of q tiles): lf_slot_of_block, groups of 4 (batch, head) pairs (their K/V
+  // fit an XCD's 4 MB L2 together); a workgroup takes q tile nqt-1-i and then q tile i of its (batch, head), so that
+  // under a causal mask every workgroup walks the same number of KV tiles (2(i+1) + 2(nqt-i) of them) and the
+  // grid has no long tail
   const int nqt = (p.Sq + LF_BM - 1) / LF_BM;
   const int npair = (nqt + 1) / 2;
-  const int nbh = p.B * p.Hq;
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  // within an XCD: groups of 4 (batch, head) pairs (their K/V fit the 4 MB L2
-  // together); a workgroup takes q tile nqt-1-i and then q tile i of its (batch,
-  // head), so that under a causal mask every workgroup walks the same number of
-  // KV tiles (2(i+1) + 2(nqt-i) of them) and the grid has no long tail
-  const int grp = slot / (4 * npair);
-  const int in_grp = slot % (4 * npair);
-  const int bh = (grp * 4 + (in_grp & 3)) * 8 + xcd;
-  if (bh >= nbh) return;
-  const int pair = in_grp >> 2;
+  int bh, pair;
+  if (!lf_slot_of_block(blockIdx.x, p.B * p.Hq, npair, 4, bh, pair)) return;
   const int b = bh / p.Hq;
   const int h = bh % p.Hq;
   const int hkv = h / (p.Hq / p.Hkv);

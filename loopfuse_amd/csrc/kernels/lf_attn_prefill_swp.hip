@@ -102,23 +102,12 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
-  // ---- workgroup -> (batch*head, q tile).  blockIdx.x % 8 is the XCD (workgroups go to the
-  // XCDs round-robin), so all q tiles of a (batch, head) run on one XCD and share its L2.
-  // Within an XCD class the slots come in groups of LF_QGROUP (batch, head) pairs -- so many
-  // that the resident workgroups of an XCD walk the K/V of few heads at a time -- and within
-  // a group by q tile, the one with the most kv tiles first: workgroups are dispatched in
-  // blockIdx order, so under a causal mask the long tiles start early and the short ones
-  // fill the end of the launch (longest-first list scheduling).
+  // ---- workgroup -> (batch*head, q tile): lf_slot_of_block; under a causal mask the last q tile has the most kv tiles
   const int nqt = (p.Sq + LF_BM - 1) / LF_BM;
   const int nhv = p.Hq / LF_HEADS_PER_WG;     // head units per batch element (heads, or packs of heads)
-  const int nbh = p.B * nhv;
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  const int grp = slot / (LF_QGROUP * nqt);
-  const int in_grp = slot % (LF_QGROUP * nqt);
-  const int bh = (grp * LF_QGROUP + in_grp % LF_QGROUP) * 8 + xcd;
-  if (bh >= nbh) return;     // padding slot of the last group
-  const int slot_qt = nqt - 1 - in_grp / LF_QGROUP;
+  int bh, from_end;
+  if (!lf_slot_of_block(blockIdx.x, p.B * nhv, nqt, LF_QGROUP, bh, from_end)) return;
+  const int slot_qt = nqt - 1 - from_end;
   const int b = bh / nhv;
 #if LF_GQAPACK
   const int h = (bh % nhv) * LF_GQAPACK + wave % LF_GQAPACK;    // this wave's query head

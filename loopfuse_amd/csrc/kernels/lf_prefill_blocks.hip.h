@@ -100,6 +100,43 @@ __device__ __forceinline__ lf_u32x4 lf_make_buffer(const void* base, unsigned by
   return rs;
 }
 
+// Workgroup -> (unit, tile).  A unit is what shares K/V (or Q/dO) tiles in L2, a (batch, head) pair; its `tiles` work
+// items are numbered so that number 0 is the longest.  Workgroup ids with equal id % 8 run on one XCD, and all
+// tiles of a unit go to one XCD.  Inside an XCD the slots come in groups of `group` units -- so many that the
+// resident workgroups walk the K/V of few units at a time -- and inside a group by tile, the longest first
+// (dispatch is in id order: list scheduling); the last group holds the units that are left.
+//   Units that do not fill the XCDs evenly are cut: with 2^sh parts per unit, part p of a unit owns its tiles
+// p, p + 2^sh, ... and counts as a unit of its own, so few (or 9, or 12) units still load all eight XCDs alike.  sh
+// is the smallest value within 1/16 of the least number of slots per XCD.
+//   Measured on an MI355X (bf16 causal forward, S = 6001, 32 query / 8 kv heads packed by 4, i.e. one unit per
+// XCD): 694 us when the group was padded to 8 units -- the hardware deals an XCD's workgroups to its four shader
+// engines in turn, and padding left every eighth slot, always the same engine, real -- 312 us so; S = 8192,
+// window 512, 4 such units: 215 -> 55 us.
+// False: a padding slot, nothing to do.
+__device__ __forceinline__ bool lf_slot_of_block(unsigned block, int units, int tiles, int group, int& unit, int& tile) {
+  int sh = 0, slots = (units + 7) / 8 * tiles;
+#pragma unroll
+  for (int t = 1; t <= 3; ++t) {
+    const int n = ((units << t) + 7) / 8 * ((tiles + (1 << t) - 1) >> t);
+    if (17 * n <= 16 * slots) {
+      sh = t;
+      slots = n;
+    }
+  }
+  const int xcd = (int)(block & 7u), slot = (int)(block >> 3);
+  if (slot >= slots) return false;
+  const int part_tiles = (tiles + (1 << sh) - 1) >> sh;
+  const int per_xcd = ((units << sh) + 7) / 8;
+  const int g = slot / (group * part_tiles);
+  const int width = min(group, per_xcd - g * group);       // units of this group
+  const int in_g = slot - g * group * part_tiles;
+  const int t = in_g / width;
+  const int v = (g * group + in_g - t * width) * 8 + xcd;  // unit << sh | part
+  unit = v >> sh;
+  tile = (t << sh) + (v & ((1 << sh) - 1));
+  return unit < units && tile < tiles;
+}
+
 // Is score (query row q, key j) kept?  Top-left aligned masks of the reference
 // (loopfuse/torch_backend/ops.py:675-751) plus the bound of the key sequence.
 __device__ __forceinline__ bool lf_mask_keep(int q, int j, int Sk, int window) {

@@ -290,8 +290,17 @@ def _get_scratch(device: torch.device, nfloats: int) -> torch.Tensor:
     return t
 
 
-PREFILL_QGROUP = 8      # LF_QGROUP of lf_attn_prefill_swp.hip (its default)
-BWD_GROUP = 4           # LF_BW_GROUP of lf_attn_bwd.hip (its default)
+
+
+def xcd_slots(units: int, tiles: int) -> int:
+    """Grid of a kernel that maps its workgroups with ``lf_slot_of_block`` (csrc/kernels/lf_prefill_blocks.hip.h):
+    8 XCDs x the slots of one, with the units cut into as many parts as that function chooses."""
+    best = (units + 7) // 8 * tiles
+    for t in (1, 2, 3):
+        n = ((units << t) + 7) // 8 * ((tiles + (1 << t) - 1) >> t)
+        if 17 * n <= 16 * best:
+            best = n
+    return 8 * best
 
 
 def decode_split(units: int, Sk: int, cus: int = 256, per_cu: int = 2) -> int:
@@ -351,12 +360,18 @@ def _decode_rowload(paged: int, page_size: int, page_size_v: int, bias_bits: int
     return not paged or (page_size % 16 == 0 and (page_size_v or page_size) % 16 == 0)
 
 
-def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, workgroups: int = 1 << 30) -> int:
+def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, workgroups: int = 1 << 30,
+                    window: int = 0) -> int:
     """Keys per LDS tile of lf_attn_prefill_swp: 0 (the kernel's 64) or 32.  With 32-key tiles a
     workgroup needs 40 KB of LDS and at most 168 registers per lane, so three workgroups instead of
-    two share a CU; at head dimension 128 that outweighs the second barrier per 64 keys (config 2
-    -2.5 %, config 3 -10 %) once the launch has three workgroups for every CU -- a launch of 128
-    workgroups is a quarter slower with them -- and at head dimension 64 it does not.  The bias tile
+    two share a CU.  At head dimension 128 that pays (i) under a short sliding window (``window``,
+    0 = none) once the launch has three workgroups for every CU -- its q tiles are a few kv tiles long
+    and a third workgroup hides prologues and drains: window 256, S 1024 ... 4096, 768 ... 4096
+    workgroups: 0 ... 16 % faster; (ii) otherwise from 2048 workgroups on: causal B8 H32 S2048 301
+    against 313 us, B4 in front of its backward 750 against 768 us for both.  Between 768 and 2048
+    workgroups the tail of the launch counts more and two per CU win: causal S 4096, 768 workgroups
+    110 against 123 us; one 6001-token prompt, 1504 workgroups, 312 against 328 us.  At head
+    dimension 64 it does not pay.  The bias tile
     classes are per 64 keys, so biased calls keep 64.  ``choice["bn"]`` (the tuner) or
     ``LOOPFUSE_BN`` override the default."""
     if bias_bits:
@@ -364,7 +379,7 @@ def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, w
     want = (choice or {}).get("bn", os.environ.get("LOOPFUSE_BN"))
     if want is not None:
         return 32 if int(want) == 32 else 0
-    return 32 if D == 128 and workgroups >= 3 * 256 else 0
+    return 32 if D == 128 and workgroups >= (3 * 256 if 0 < window <= 512 else 8 * 256) else 0
 
 
 def prefill_variant(Sq: int, v_tr: bool = True) -> str:
@@ -793,7 +808,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                           page_size, table_i64, v_tr=v_tr if family == "prefill" else True, bias=bias_bits,
                           denom=plan.denom_add != 0.0, d2=d2, page_size_v=page_size_v, pack=pack, extra=extra,
                           safe=plan.zero_blind_rows and bool(bias_bits & 1),
-                          bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))))
+                          bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
+                                             P.window if mask == MASK_SLIDING else 0)
                           if family == "prefill_swp" else 0)
         bm, bn = TILE_SHAPES[family]
         nw = 4
@@ -812,18 +828,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         if record_visits:
             visits = torch.zeros((B * heads * nqt, nkt), dtype=torch.uint8, device=q.device)
             P.visits = visits.data_ptr()
-        # 8 XCD classes x (batch*head pairs per class, padded to the kernel's groups) x q tiles
-        per_xcd = (B * heads + 7) // 8
-        if family == "prefill_swp":
-            # one q tile per workgroup, groups of LF_QGROUP heads, longest q tiles first
-            qgroup = PREFILL_QGROUP
-            for e in spec.extra:
-                if e.startswith("-DLF_QGROUP="):
-                    qgroup = int(e.split("=")[1])
-            grid = 8 * ((per_xcd + qgroup - 1) // qgroup * qgroup) * nqt
-        else:
-            # lf_attn_prefill takes two q tiles (heavy + light) per workgroup, groups of 4 heads
-            grid = 8 * ((per_xcd + 3) // 4 * 4) * ((nqt + 1) // 2)
+        # lf_attn_prefill_swp: one q tile per workgroup; lf_attn_prefill: two (a long and a short one)
+        grid = xcd_slots(B * heads, nqt if family == "prefill_swp" else (nqt + 1) // 2)
         if lse is not None:
             if family != "prefill_swp" or paged:
                 raise UnsupportedPlan("the row log-sum-exp is written by lf_attn_prefill_swp for dense K/V only")
@@ -999,16 +1005,9 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     keep = (q, k, v, o, dout, lse, delta, dq, dk, dv)  # noqa: F841  (tensors stay alive until the launches are queued)
     rows = B * Hq * Sq
     get_kernel(spec, "lf_attn_bwd_delta").launch(((rows + 15) // 16, 1, 1), (256, 1, 1), P)
-    # 8 XCD classes x (batch, kv head) pairs per class, padded to the kernels' groups, x the
-    # workgroups of a pair (key blocks; query heads of the group x q tiles)
-    grp = BWD_GROUP
-    for e in spec.extra:
-        if e.startswith("-DLF_BW_GROUP="):
-            grp = int(e.split("=")[1])
-    pairs = ((B * Hkv + 7) // 8 + grp - 1) // grp * grp
-    get_kernel(spec, "lf_attn_bwd_dkdv").launch((8 * pairs * ((Sk + 127) // 128), 1, 1), (256, 1, 1), P)
+    get_kernel(spec, "lf_attn_bwd_dkdv").launch((xcd_slots(B * Hkv, (Sk + 127) // 128), 1, 1), (256, 1, 1), P)
     nt = bwd_dq_threads(mask, softcap is not None)
-    get_kernel(spec, "lf_attn_bwd_dq").launch((8 * pairs * (Hq // Hkv) * ((Sq + nt // 2 - 1) // (nt // 2)), 1, 1),
+    get_kernel(spec, "lf_attn_bwd_dq").launch((xcd_slots(B * Hkv, (Hq // Hkv) * ((Sq + nt // 2 - 1) // (nt // 2))), 1, 1),
                                               (nt, 1, 1), P)
     _last_launch.set({"kernels": ["lf_attn_bwd_delta", "lf_attn_bwd_dkdv", "lf_attn_bwd_dq"]})
     return dq, dk, dv
