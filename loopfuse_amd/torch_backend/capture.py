@@ -144,10 +144,11 @@ def _hint(sym) -> int:
         return 8
 
 
-def _stand_in_sizes(hints: dict) -> dict:
-    """Small concrete value per traced size, keeping small-ratio divisibility."""
+def _stand_in_sizes(hints: dict, taken: frozenset = frozenset()) -> dict:
+    """Small concrete value per traced size, keeping small-ratio divisibility; sizes without a ratio to
+    keep get a prime outside ``taken``."""
     distinct = sorted(set(hints.values()))
-    fresh = iter([5, 7, 3, 11, 13, 17, 19, 23, 29, 31, 37, 41])
+    fresh = iter([n for n in (5, 7, 3, 11, 13, 17, 19, 23, 29, 31, 37, 41, 43, 47, 53, 59, 61, 67, 71, 73) if n not in taken])
     small: dict[int, int] = {}
     for h in distinct:
         if h <= 4:
@@ -744,14 +745,24 @@ def _match_attention(gm: torch.fx.GraphModule) -> list:
     def _numel_as_is(val) -> int:
         return math.prod(int(d.node.expr.subs(sizes)) if isinstance(d, torch.SymInt) else int(d) for d in val.shape)
 
-    if any(isinstance(p.meta.get("val"), torch.Tensor) and _numel_as_is(p.meta["val"]) > CAP for p in placeholders):
-        statics = sorted({int(d) for p in placeholders if isinstance(p.meta.get("val"), torch.Tensor)
-                          for d in p.meta["val"].shape if not isinstance(d, torch.SymInt) and int(d) > 4})
-        joint = dict(hints)
-        joint.update({("static", v): v for v in statics})
-        both = _stand_in_sizes(joint)
-        sizes = {k: v for k, v in both.items() if not isinstance(k, tuple)}
-        fmap = {k[1]: v for k, v in both.items() if isinstance(k, tuple)}
+    tensors = [p.meta["val"] for p in placeholders if isinstance(p.meta.get("val"), torch.Tensor)]
+    if any(_numel_as_is(t) > CAP for t in tensors):
+        # Batch, head and group counts (dims up to 64) keep their values when the tensors then fit: the ratios
+        # between them (Hq = g * Hkv with a small batch of another size beside them) do not survive stand-ins
+        # chosen per value.  Only when they do not fit are all dims replaced.
+        statics = sorted({int(d) for t in tensors for d in t.shape if not isinstance(d, torch.SymInt) and int(d) > 4})
+        for keep in (64, 4):
+            kept = frozenset(v for v in statics if v <= keep)
+            joint = dict(hints)
+            joint.update({("static", v): v for v in statics if v > keep})
+            both = _stand_in_sizes(joint, kept)
+            sub = {k: v for k, v in both.items() if not isinstance(k, tuple)}
+            fmap = {k[1]: v for k, v in both.items() if isinstance(k, tuple)}
+            fmap.update({v: v for v in kept})
+            if max(math.prod(int(d.node.expr.subs(sub)) if isinstance(d, torch.SymInt) else fmap.get(int(d), int(d))
+                             for d in t.shape) for t in tensors) <= CAP:
+                break
+        sizes = sub
     shrink_static = bool(fmap)
 
     # Equalities the trace relies on without having solved them for one symbol (two page

@@ -886,3 +886,24 @@ def test_reference_import_path_is_a_drop_in():
     x = torch.randn(2, 3, 5, 5)
     fn = torch.compile(lambda a: torch.ops.loopfuse.causal_mask(a) + 1, backend=ref_path_backend, dynamic=True)
     assert torch.equal(fn(x), torch.ops.loopfuse.causal_mask(x) + 1)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(8, 16, 4, 1000, 64), (2, 12, 3, 4000, 64), (5, 6, 3, 3000, 128), (1, 64, 8, 2877, 128)])
+def test_static_grouped_heads_beside_an_unrelated_batch_size(B, Hq, Hkv, S, D):
+    """Traced with static shapes at real sizes (what a training graph is matched on): the ratio Hq = g * Hkv
+    survives the stand-ins although the batch size divides Hq in another ratio."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from loopfuse_amd.torch_backend import capture
+
+    def fn(q, k, v):
+        k, v = (t.repeat_interleave(Hq // Hkv, dim=1) for t in (k, v))
+        s = torch.ops.loopfuse.causal_mask(q @ k.transpose(-2, -1) * D ** -0.5)
+        return torch.softmax(s, dim=-1) @ v
+
+    q = torch.empty(B, Hq, S, D, dtype=torch.bfloat16)
+    k, v = (torch.empty(B, Hkv, S, D, dtype=torch.bfloat16) for _ in range(2))
+    with torch.no_grad():
+        gm = make_fx(fn, tracing_mode="fake")(q, k, v)
+    (m,) = capture.match_attention(gm)
+    assert m.mask == "causal" and [o.perm for o in (m.q, m.k, m.v)] == [(0, 1, 2, 3)] * 3
+    assert (m.q.group, m.k.group, m.v.group) == (1, Hq // Hkv, Hq // Hkv)
