@@ -29,7 +29,7 @@ struct LfAttnBwdParams {
   lf_elem* dk;
   lf_elem* dv;
   const float* lse;       // [B, Hq, Sq] row log-sum-exp of the scaled, masked scores, log2 units
-  float* delta;           // [B, Hq, Sq] scratch: rowsum(dO * O)
+  float* delta;           // [2, B, Hq, Sq] scratch: -rowsum(dO * O); what the accumulators of S start at, -L / cexp
   long long q_sb, q_sh, q_ss;      // element strides (d stride 1)
   long long k_sb, k_sh, k_ss;
   long long v_sb, v_sh, v_ss;
@@ -64,6 +64,16 @@ __device__ __forceinline__ bool lf_bw_keep(int t, int window) {
 #define LF_BW_DQ_NT 512     /* threads of lf_attn_bwd_dq: 8 waves x 32 query rows, two waves per SIMD */
 #endif
 
+// P = 2^(cexp * (S + start)): the row log-sum-exp enters through the start of the accumulators of S = Q K^T.  With a
+// softcap the exponent is not linear in S: there the second half of the scratch holds L itself.
+__device__ __forceinline__ float lf_bw_start_scale(const LfAttnBwdParams& p) {
+#if LF_SOFTCAP
+  return 1.0f;
+#else
+  return -1.0f / (p.scale * LF_LOG2E);
+#endif
+}
+
 // delta[row] = sum_d dO[row][d] * O[row][d]; 16 lanes per row, 8 elements per lane
 extern "C" __global__ void __launch_bounds__(LF_BW_NT) lf_attn_bwd_delta(const LfAttnBwdParams p) {
   const long long row = (long long)blockIdx.x * (LF_BW_NT / 16) + threadIdx.x / 16;
@@ -83,7 +93,10 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT) lf_attn_bwd_delta(const L
   s += __shfl_xor(s, 2, 64);
   s += __shfl_xor(s, 4, 64);
   s += __shfl_xor(s, 8, 64);
-  if (row < nrows && piece == 0) p.delta[row] = s;
+  if (row < nrows && piece == 0) {
+    p.delta[row] = -s;
+    p.delta[nrows + row] = p.lse[row] * lf_bw_start_scale(p);
+  }
 }
 
 // A 64-row tile of a [rows, D] matrix goes global -> LDS directly (buffer_load ... lds, the
@@ -211,11 +224,135 @@ __device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, lf_elem* 
   }
 }
 
+// ---- tiles that are kept in LDS once and read both ways.  A 64-row tile is row-major and unpadded; the 16-byte
+// chunks of a row are permuted by an XOR with lf_bw_swz(row), the low bits of the row (counted in 256-byte bank
+// spans) rotated so that both read patterns touch every bank once: 16 consecutive rows, one logical chunk
+// (ds_read_b128, rows = MFMA rows) get 16 different values, and the 4 rows x 64 bytes of a transposed read differ in
+// the bits above the two that its four chunks vary.  Against a copy per read pattern that is half the LDS and half
+// the L2 -> LDS traffic, and leaves room for a third stage.
+__device__ __forceinline__ int lf_bw_swz(int row) {
+  const int r = row / LF_RPS;
+#if LF_HEAD_DIM == 128
+  return ((r & 3) << 2) | ((r >> 2) & 3);
+#else
+  return ((r & 1) << 2) | ((r >> 1) & 3);
+#endif
+}
+#define LF_BW_ROWB (LF_D * 2)                       /* bytes per row of a tile */
+#define LF_BW_TILEB (64 * LF_BW_ROWB)               /* bytes per tile */
+typedef __attribute__((address_space(3))) const lf_u32x4* lf_bw_lds_u32x4;
+typedef __attribute__((address_space(3))) lf_s16x4* lf_bw_lds_s16x4;
+// This lane's offset for fragment (row block 0, 16-dim step 0) / (16-row step 0, 32-dim block 0); the other
+// fragments are an XOR of address bits below the row size and a constant away (tile addresses are multiples of it).
+__device__ __forceinline__ unsigned lf_bw_rm_off(int l32, int g) {
+  return (unsigned)(l32 * LF_BW_ROWB + 16 * (g ^ lf_bw_swz(l32)));
+}
+__device__ __forceinline__ unsigned lf_bw_tr_off(int lane) {
+  const int j = lane & 15, dh = (lane >> 4) & 1, row = 4 * (lane >> 5) + (j >> 2);
+  return (unsigned)(row * LF_BW_ROWB + 16 * ((2 * dh + ((j & 3) >> 1)) ^ lf_bw_swz(row)) + 8 * (j & 1));
+}
+// base ^ bits.  Volatile, so that equal addresses of different reads are formed again instead of being kept: a stage has
+// 24 of them and there are no registers to hold them in.
+__device__ __forceinline__ unsigned lf_bw_flip(unsigned base, int bits) {
+  if (bits == 0) return base;
+  unsigned a;
+  asm volatile("v_xor_b32 %0, %1, %2" : "=v"(a) : "i"(bits), "v"(base));
+  return a;
+}
+// rows 32*blk + lane % 32, d = 16*ks + 8*g .. +7 of the tile `disp` bytes into a stage; `base` = LDS address of the
+// stage + lf_bw_rm_off
+__device__ __forceinline__ lf_u32x4 lf_bw_read_rm(unsigned base, int disp, int blk, int ks) {
+  return *(lf_bw_lds_u32x4)(size_t)(lf_bw_flip(base, 32 * ks) + (unsigned)(disp + 32 * blk * LF_BW_ROWB));
+}
+// transposed: d = 32*db + lane % 32, rows 16*kk + 8*(s/4) + 4*g + s%4 for s = 0 .. 7; `base` = stage + lf_bw_tr_off
+__device__ __forceinline__ lf_u32x4 lf_bw_read_tr(unsigned base, int disp, int kk, int db) {
+  lf_u32x4 a;
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    const unsigned src = lf_bw_flip(base, 64 * db + 32 * half) + (unsigned)(disp + (16 * kk + 8 * half) * LF_BW_ROWB);
+    const lf_u32x2 t = __builtin_bit_cast(lf_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lf_bw_lds_s16x4)(size_t)src));
+    a[2 * half] = t[0];
+    a[2 * half + 1] = t[1];
+  }
+  return a;
+}
+// One direct load of a tile (256 threads: kRows whole rows per load of the workgroup): row row0 + srow + kRows * ps of
+// the matrix behind `rs`; rows past its end arrive as zeros.  `lane_off` = lf_bw_load_off.
+__device__ __forceinline__ unsigned lf_bw_load_off(unsigned rowb, int tid) {
+  const int srow = tid / LF_CPR, sch = tid % LF_CPR;       // a load is a multiple of 16 rows: the swizzle repeats
+  return (unsigned)srow * rowb + 16u * (unsigned)(sch ^ lf_bw_swz(srow));
+}
+__device__ __forceinline__ void lf_bw_load_rows(const lf_u32x4& rs, unsigned rowb, int row0, unsigned tile, unsigned lane_off,
+                                                int ps, int wave) {
+  constexpr int kRows = LF_BW_NT / LF_CPR, kRowsPerWave = 64 / LF_CPR;
+  static_assert(kRows % 16 == 0, "a load must keep the swizzle phase");
+  lf_dma_to_lds_at(rs, (unsigned)(row0 + kRows * ps) * rowb + lane_off,
+                   tile + (unsigned)((kRows * ps + kRowsPerWave * wave) * LF_BW_ROWB));
+}
+
+// One wave-level direct-to-LDS load of 64 floats: lane i's lands at lds_addr + 4 * i.
+__device__ __forceinline__ void lf_dma_dword_to_lds_at(const lf_u32x4& rs, unsigned voff, unsigned lds_addr) {
+  unsigned m0_written;
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dword %2, %3, 0 offen lds"
+               : "={m0}"(m0_written) : "s"(lds_addr), "v"(voff), "s"(rs) : "memory");
+}
+
+// MFMAs with every operand in VGPRs (the accumulator: VGPRs); first of a chain: started from `c0`, or from zero.  The
+// matrix core reads `c0` late: keep it alive (LF_BW_HOLD) until another MFMA has been issued behind its readers.
+#define LF_BW_HOLD(c0) asm volatile("" :: "v"(c0))
+__device__ __forceinline__ void lf_bw_mfma_vvv(lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b) {
+  asm volatile(LF_BW_MFMA " %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void lf_bw_mfma_from(lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b, const lf_f32x16& c0) {
+  asm volatile(LF_BW_MFMA " %0, %1, %2, %3" : "=&v"(c) : "v"(a), "v"(b), "v"(c0));
+}
+__device__ __forceinline__ void lf_bw_mfma_zero(lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b) {
+  asm volatile(LF_BW_MFMA " %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
+}
+
+// c (AGPRs) += a x b (VGPRs), with the accumulator handed over as an input: lf_attn_bwd_dkdv keeps up to all 256 AGPRs in
+// use from its first to its last instruction, and accumulators that the compiler sees change in the loop leave its
+// register allocator without a free tuple to resolve a control-flow merge with -- it spills a thousand registers.  So
+// it sees 16 values that are defined once, used throughout and defined anew by the drain behind the loop; they stay in
+// their registers for lack of any other (tests/test_kernel_codegen.py holds the generated code to that).
+__device__ __forceinline__ void lf_bw_mfma_hidden(const lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b) {
+  asm volatile(LF_BW_MFMA " %0, %1, %2, %0" ::"a"(c), "v"(a), "v"(b));
+}
+
+#ifndef LF_BW_W
+#define LF_BW_W 1        /* 32-key blocks per wave of lf_attn_bwd_dkdv: every fragment read from LDS feeds so many MFMAs */
+#endif
+#ifndef LF_BW_PF
+#define LF_BW_PF (LF_BW_W == 2 && LF_HEAD_DIM == 128 ? 3 : 4)   /* fragments read ahead of the MFMAs that take them (there, a fourth spills) */
+#endif
+
+#ifndef LF_BW_VL
+#define LF_BW_VL (LF_BW_W == 2 && LF_HEAD_DIM == 128 ? 5 : 0)    /* 16-dim steps of the V^T operand kept in LDS instead of registers */
+#endif
+
+// dK and dV of 128 * LF_BW_W keys of one (batch, kv head): 4 waves, one per SIMD, wave w the keys 32 * LF_BW_W * w ...
+// What bounds it: the four products' MFMAs and the power they draw.  At LF_BW_W = 2, D = 128 the 512 registers are spoken
+// for (dK^T, dV^T 256 AGPRs, K^T / V^T operands 96 VGPRs with half of V^T in LDS, S^T and dP^T 64, P and dS 32, fragments 12)
+// and an MFMA pair costs one LDS fragment read.  Causal bf16 B4 H32 S2048 D128: 390 us in the form before (a copy of each
+// tile per read pattern, one MFMA per fragment, a wait in front of every group of probabilities), 298 us now = 0.98
+// PFLOP/s executed at 0.39 of the MFMA cycles; without its LDS reads, direct loads, barrier and exponentials the same
+// stream still takes three quarters of that, and the read-ahead (2 ... 8 fragments) makes no difference.
+// Work of a wave: a stream of blocks of 32 queries, two per 64-query tile, and per block four phases of MFMAs whose
+// A fragments come through one read-ahead ring that runs on into the next block:
+//   S^T = Q K^T                      accumulators start at -L / c, so P = 2^(c S) needs no subtraction
+//   dP^T = dO V^T                    accumulators start at -delta; P between these MFMAs
+//   dV^T += dO^T P                   dS = P (dP - delta) between these
+//   dK^T += Q^T dS
+// Three LDS stages: a tile's loads are issued in the second half of the step two before its own, and the one barrier per
+// step, in its middle, says both that the next tile has landed and that the tile before this one is free.
 extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const LfAttnBwdParams p) {
-  // two stages of: Q tile in both layouts, dO tile in both layouts, L and delta of the 64 rows
-  __shared__ __attribute__((aligned(16))) lf_elem tiles[2][4][64 * LF_D];
-  __shared__ __attribute__((aligned(16))) float lse_st[2][64];
-  __shared__ __attribute__((aligned(16))) float delta_st[2][64];
+  constexpr int KB = LF_BW_W;
+  constexpr int kKeys = 128 * KB;
+  __shared__ __attribute__((aligned(256))) lf_elem tiles[3][2][64 * LF_D];        // Q, dO
+  __shared__ __attribute__((aligned(16))) float stats[3][2][64];                  // of the 64 rows: start of S, start of dP
+#if LF_BW_VL
+  __shared__ lf_u32x4 v_lds[LF_BW_VL][KB][LF_BW_NT];                               // V^T operands that the registers have no room for
+#endif
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -223,7 +360,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
-  const int nkt = (p.Sk + 127) / 128;
+  const int nkt = (p.Sk + kKeys - 1) / kKeys;
   // All key blocks of a (batch, kv head) share the Q / dO tiles they walk in one XCD's L2; the first key
   // block has the most steps under a causal mask.
   int bhkv, kt;
@@ -231,257 +368,363 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   const int hkv = bhkv % p.Hkv;
   const int b = bhkv / p.Hkv;
   const int group = p.Hq / p.Hkv;
-  const int key0 = 128 * kt + 32 * wave;           // first key of this wave
-  const int my_key = key0 + l32;
+  const int key0 = kKeys * kt + 32 * KB * wave;    // first key of this wave
+  const int klast = min(key0 + 32 * KB, p.Sk) - 1;
   const int nqt = (p.Sq + 63) / 64;
 
-  // K^T and V^T of this lane's key as B operands (d = 16*ks + 8*g .. +7), parked in AGPRs
-  lf_u32x4 kf[LF_NKS], vf[LF_NKS];
-  {
-    const int kr = min(my_key, p.Sk - 1);
+  // K^T and V^T of this lane's keys as B operands (d = 16*ks + 8*g .. +7)
+  constexpr int kVReg = LF_NKS - LF_BW_VL;
+  lf_u32x4 kf[KB][LF_NKS], vf[KB][kVReg];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int kr = min(key0 + 32 * kb + l32, p.Sk - 1);
     const lf_elem* krow = p.k + (long long)b * p.k_sb + (long long)hkv * p.k_sh + (long long)kr * p.k_ss;
     const lf_elem* vrow = p.v + (long long)b * p.v_sb + (long long)hkv * p.v_sh + (long long)kr * p.v_ss;
 #pragma unroll
     for (int ks = 0; ks < LF_NKS; ++ks) {
-      kf[ks] = *reinterpret_cast<const lf_u32x4*>(krow + 16 * ks + 8 * g);
-      vf[ks] = *reinterpret_cast<const lf_u32x4*>(vrow + 16 * ks + 8 * g);
+      kf[kb][ks] = *reinterpret_cast<const lf_u32x4*>(krow + 16 * ks + 8 * g);
+      const lf_u32x4 x = *reinterpret_cast<const lf_u32x4*>(vrow + 16 * ks + 8 * g);
+      if (ks < kVReg) vf[kb][ks] = x;
+#if LF_BW_VL
+      else v_lds[ks - kVReg][kb][tid] = x;
+#endif
     }
+  }
 #pragma unroll
-    for (int ks = 0; ks < LF_NKS; ++ks) asm volatile("" : "+a"(kf[ks]), "+a"(vf[ks]));
+  for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+    for (int ks = 0; ks < LF_NKS; ++ks) asm volatile("" : "+v"(kf[kb][ks]));
+#pragma unroll
+    for (int ks = 0; ks < kVReg; ++ks) asm volatile("" : "+v"(vf[kb][ks]));
   }
 #if LF_SOFTCAP
   const float sc_exp = p.scale / p.softcap * (2.0f * LF_LOG2E);   // 2^(s * sc_exp) = e^(2x)
   const float cexp = p.softcap * LF_LOG2E;                        // exponent of P: tanh x * cexp - L
 #else
-  const float cexp = p.scale * LF_LOG2E;
+  const float cexp = p.scale * LF_LOG2E;                          // exponent of P: (s - L / cexp) * cexp
 #endif
 
-  lf_f32x16 dk[LF_NDB], dv[LF_NDB];
+  lf_f32x16 dk[KB][LF_NDB], dv[KB][LF_NDB];
 #pragma unroll
-  for (int db = 0; db < LF_NDB; ++db) {
+  for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
-    asm volatile("" : "+a"(dk[db]), "+a"(dv[db]));
-  }
+    for (int db = 0; db < LF_NDB; ++db) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dk[kb][db][i] = dv[kb][db][i] = 0.0f;
+      asm volatile("" : "+a"(dk[kb][db]), "+a"(dv[kb][db]));
+    }
 
-  // q tiles (64 rows) that hold a query seeing one of the workgroup's 128 keys
+  // q tiles (64 rows) that hold a query seeing one of the workgroup's keys
   int qt_begin = 0, qt_end = nqt;
 #if LF_MASK >= 1
-  qt_begin = (128 * kt) / 64;                                   // q >= key
+  qt_begin = kKeys * kt / 64;                                   // q >= key
 #endif
 #if LF_MASK == 2
-  qt_end = min(nqt, (min(128 * kt + 127, p.Sk - 1) + p.window - 1) / 64 + 1);   // q - key < window
+  qt_end = min(nqt, (min(kKeys * kt + kKeys, p.Sk) - 1 + p.window - 1) / 64 + 1);   // q - key < window
 #endif
-
-  // the steps of this workgroup: query heads of the group x q tiles, one flat sequence; the
-  // direct loads of step it + 1 fill the other stage while step it is computed, one load after
-  // every pair of MFMAs of the first products (a wave owes LF_CPR loads per step, and that many
-  // pairs there are: the loads go through the CU's one texture path at 64 bytes per cycle, issued
-  // in one go they hold up the wave for as long as a quarter of its MFMAs take)
+  // the steps of this workgroup: query heads of the group x q tiles, one flat sequence
   const int ntq = max(qt_end - qt_begin, 0);
   const int nsteps = group * ntq;
+
   const unsigned q_bytes = (unsigned)(((long long)(p.Sq - 1) * p.q_ss + LF_D) * 2);
   const unsigned g_bytes = (unsigned)(((long long)(p.Sq - 1) * p.do_ss + LF_D) * 2);
-  const int wave_u = wave;
+  const unsigned q_rowb = (unsigned)p.q_ss * 2u, g_rowb = (unsigned)p.do_ss * 2u;
+  const unsigned q_loff = lf_bw_load_off(q_rowb, tid), g_loff = lf_bw_load_off(g_rowb, tid);
   constexpr int kPasses = 64 * LF_CPR / LF_BW_NT;      // loads of a wave per tile
-  static_assert(4 * kPasses == 2 * LF_NKS, "one direct load per pair of MFMAs of the first products");
-  float r_lse = 0.0f, r_delta = 0.0f;
-  lf_u32x4 q_rs, g_rs;        // rows of Q and dO of the step being loaded (zero bytes: nothing to load)
-  int q0_next = 0;
-  auto aim = [&](int it, bool real) {
-    const int h = hkv * group + it / ntq;
-    q0_next = 64 * (qt_begin + it % ntq);
-    q_rs = lf_make_buffer(p.q + (long long)b * p.q_sb + (long long)h * p.q_sh, real ? q_bytes : 0u);
-    g_rs = lf_make_buffer(p.dout + (long long)b * p.do_sb + (long long)h * p.do_sh, real ? g_bytes : 0u);
-    if (tid < 64) {            // into registers now, into the stage just before the barrier that opens it
-      const long long r = ((long long)b * p.Hq + h) * p.Sq + q0_next + tid;
-      const bool in = real && q0_next + tid < p.Sq;
-      r_lse = in ? p.lse[r] : __builtin_inff();                      // rows past Sq: P = 0
-      r_delta = in ? p.delta[r] : 0.0f;
+  constexpr int kLoads = 2 * kPasses;
+  const unsigned lds0 = lf_lds_addr(tiles);
+  auto q_tile = [&](int st) { return lds0 + (unsigned)(2 * st * LF_BW_TILEB); };
+  auto g_tile = [&](int st) { return lds0 + (unsigned)((2 * st + 1) * LF_BW_TILEB); };
+
+  // ---- what is loaded next: query head, q tile; past the last step the loads go out against an empty range.  Waves 0
+  // and 1 also bring the row statistics, the start of S and that of dP; those of rows past Sq are zeros: P is 1 there
+  // and meets dO = 0.
+  int ld_step = 0, ld_tile = qt_begin, ld_q0 = 0;
+  const lf_elem* ld_q = p.q + (long long)b * p.q_sb + (long long)(hkv * group) * p.q_sh;
+  const lf_elem* ld_g = p.dout + (long long)b * p.do_sb + (long long)(hkv * group) * p.do_sh;
+  const float* ld_stat = p.delta + ((wave == 0 ? (long long)p.B * p.Hq : 0ll) + (long long)b * p.Hq + hkv * group) * p.Sq;
+  lf_u32x4 q_rs, g_rs, stat_rs;
+  auto aim = [&]() {
+    const bool real = ld_step < nsteps;
+    ld_q0 = 64 * ld_tile;
+    q_rs = lf_make_buffer(ld_q, real ? q_bytes : 0u);
+    g_rs = lf_make_buffer(ld_g, real ? g_bytes : 0u);
+    stat_rs = lf_make_buffer(ld_stat, real && wave < 2 ? (unsigned)p.Sq * 4u : 0u);
+    ++ld_step;
+    if (++ld_tile == qt_end) {
+      ld_tile = qt_begin;
+      ld_q += p.q_sh;
+      ld_g += p.do_sh;
+      ld_stat += p.Sq;
     }
   };
-  const unsigned lane_off[4] = {lf_bw_dma_lane_off<LF_BW_NT>((unsigned)p.q_ss * 2u, false, tid),
-                                lf_bw_dma_lane_off<LF_BW_NT>((unsigned)p.q_ss * 2u, true, tid),
-                                lf_bw_dma_lane_off<LF_BW_NT>((unsigned)p.do_ss * 2u, false, tid),
-                                lf_bw_dma_lane_off<LF_BW_NT>((unsigned)p.do_ss * 2u, true, tid)};
-  auto issue_piece = [&](int st, int j) {      // load j of LF_CPR: tile j / kPasses (Q, Q, dO, dO), pass j % kPasses
-    const int t = j / kPasses;
-    lf_bw_dma_piece<LF_BW_NT>(t < 2 ? q_rs : g_rs, (unsigned)(t < 2 ? p.q_ss : p.do_ss) * 2u, q0_next, tiles[st][t],
-                              lane_off[t], j % kPasses, wave_u);
+  const unsigned stat0 = lf_lds_addr(stats);
+  auto issue = [&](int st, int j) {      // load j of kLoads
+    if (j < kPasses) lf_bw_load_rows(q_rs, q_rowb, ld_q0, q_tile(st), q_loff, j, wave);
+    else lf_bw_load_rows(g_rs, g_rowb, ld_q0, g_tile(st), g_loff, j - kPasses, wave);
+    if (j == kLoads - 1 && wave < 2)
+      lf_dma_dword_to_lds_at(stat_rs, (unsigned)(ld_q0 + lane) * 4u, stat0 + (unsigned)((2 * st + wave) * 256));
   };
-  auto publish = [&](int st) {
-    if (tid < 64) {
-      lse_st[st][tid] = r_lse;
-      delta_st[st][tid] = r_delta;
+  // values of the queries of block qb in accumulator order: element 4*i4 + e is query 32*qb + 8*i4 + 4*g + e
+  auto read_stats = [&](int st, int which, int qb) {
+    lf_f32x16 r;
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const lf_f32x4 x = *reinterpret_cast<const lf_f32x4*>(&stats[st][which][32 * qb + 8 * i4 + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[4 * i4 + e] = x[e];
     }
+    return r;
   };
-  // One step of a wave: S^T and dP^T of 32 keys x 64 queries in two blocks of 32 queries, P and dS,
-  // then dV^T += dO^T P and dK^T += Q^T dS.  With one wave per SIMD nothing else fills the matrix
-  // pipe while the wave computes P and dS, so the step is written as four phases of 16 MFMAs with
-  // that arithmetic placed between them: first products of block 0 | first products of block 1 with
-  // P, dS of block 0 | second products over block 0's queries with P, dS of block 1 | second
-  // products over block 1's queries.  dS is kept without the factor `scale`, which multiplies dK once
-  // at the end.
-  auto step = [&](bool masked, int st, int q0) {
-    // query minus key of element (qb, i4, e) is rel + 32*qb + 8*i4 + e; a key past Sk fails every test
-    const int rel = my_key < p.Sk ? q0 + 4 * g - my_key : -(1 << 30);
-    const lf_elem* q_rm = tiles[st][0];
-    const lf_elem* q_tr = tiles[st][1];
-    const lf_elem* g_rm = tiles[st][2];
-    const lf_elem* g_tr = tiles[st][3];
-    const float* lse_s = lse_st[st];
-    const float* delta_s = delta_st[st];
-    constexpr int kNF = LF_NKK * LF_NDB;
-    lf_u32x4 pf[LF_NKK], dsf[LF_NKK];
-    lf_f32x16 s[2], dp[2];
-    // P and dS of the four queries (qb, i4): elements 4*i4 .. +3 of the accumulators, query
-    // q0 + 32*qb + 8*i4 + 4*g + e, key my_key
-    auto soft4 = [&](int qb, int i4) {
-      const int ql = 32 * qb + 8 * i4 + 4 * g;
-      const lf_f32x4 l4 = *reinterpret_cast<const lf_f32x4*>(&lse_s[ql]);
-      const lf_f32x4 d4 = *reinterpret_cast<const lf_f32x4*>(&delta_s[ql]);
-      lf_elem4 pw, dw;
-      float pv[4];
-#if LF_SOFTCAP
-      float dcap[4];           // 1 - tanh^2
+
+  unsigned rm_off = lf_bw_rm_off(l32, g), tr_off = lf_bw_tr_off(lane);
+  asm volatile("" : "+v"(rm_off), "+v"(tr_off));
+  constexpr int NS = LF_NKS, NT = 2 * LF_NDB, NF = 2 * NS + 2 * NT;     // fragments of a block
+  static_assert(kLoads <= NS, "a block's loads go out during its first two phases");
+  static_assert(LF_BW_PF <= NS, "the read-ahead of a block's first phase");
+  // fragment i of block qb of the stage: Q rows, dO rows, dO^T, Q^T
+  auto frag = [&](int st, int qb, int i) {
+    const unsigned sb = q_tile(st);
+    if (i < NS) return lf_bw_read_rm(sb + rm_off, 0, qb, i);
+    if (i < 2 * NS) return lf_bw_read_rm(sb + rm_off, LF_BW_TILEB, qb, (i - NS + kVReg) % NS);      // steps of V^T in LDS first
+    const int j = i - 2 * NS;
+    if (j < NT) return lf_bw_read_tr(sb + tr_off, LF_BW_TILEB, 2 * qb + j / LF_NDB, j % LF_NDB);
+    return lf_bw_read_tr(sb + tr_off, 0, 2 * qb + (j - NT) / LF_NDB, j % LF_NDB);
+  };
+  lf_u32x4 pre[LF_BW_PF];            // the next block's first fragments
+  lf_f32x16 sinit;                   // and what its scores start at
+  auto read_ahead = [&](int st, int qb) {
+#pragma unroll
+    for (int f = 0; f < LF_BW_PF; ++f) pre[f] = frag(st, qb, f);
+    sinit = read_stats(st, 0, qb);
+  };
+
+  // One block of a wave: 32 queries (qb of stage st, first one q0) x its keys.  `loads`: those of stage `ld` are
+  // issued between the MFMAs; the block read ahead is (st_n, qb_n).
+  auto block = [&](const int qb, int st, int q0, const bool masked, const bool loads, int ld, int st_n, const int qb_n) {
+    lf_u32x4 fr[NF + LF_BW_PF];
+#pragma unroll
+    for (int f = 0; f < LF_BW_PF; ++f) fr[f] = pre[f];
+    lf_f32x16 s[KB], dp[KB], dinit;
+    lf_u32x4 pf[KB][2], dsf[KB][2];
+#if LF_BW_VL
+    lf_u32x4 vl[LF_BW_VL][KB];
 #endif
+    int rel[KB];                     // query minus key of element 0; a key past Sk fails every test
+    if (masked) {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const int my_key = key0 + 32 * kb + l32;
+        rel[kb] = my_key < p.Sk ? q0 + 4 * g - my_key : -(1 << 30);
+        asm volatile("" : "+v"(rel[kb]));      // formed per block: what derives from it is not kept over the loop
+      }
+    }
+    // P of elements 4*i4 .. +3 of key block kb; kept in fp32 in s for dS (with a cap: times its derivative)
+    auto soft4 = [&](int kb, int i4) {
+      lf_elem4 pw;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 4 * i4 + e;
 #if LF_SOFTCAP
-        const float r = __builtin_amdgcn_rcpf(1.0f + lf_exp2(s[qb][i] * sc_exp));     // 1 / (e^(2x) + 1), x = s * scale / cap
-        const float th = 1.0f - 2.0f * r;                                               // tanh x
-        pv[e] = lf_exp2(th * cexp - l4[e]);
-        dcap[e] = 4.0f * r * (1.0f - r);
+        const float r = __builtin_amdgcn_rcpf(1.0f + lf_exp2(s[kb][i] * sc_exp));     // 1 / (e^(2x) + 1), x = s * scale / cap
+        float pv = lf_exp2((1.0f - 2.0f * r) * cexp - sinit[i]);
+        const float dcap = 4.0f * r * (1.0f - r);                                      // 1 - tanh^2
 #else
-        pv[e] = lf_exp2(s[qb][i] * cexp - l4[e]);
+        float pv = lf_exp2(s[kb][i] * cexp);
 #endif
-      }
-      if (masked) {             // wave-uniform: most steps of a workgroup lie below the diagonal
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pv[e] = lf_bw_keep(rel + 32 * qb + 8 * i4 + e, p.window) ? pv[e] : 0.0f;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 4 * i4 + e;
-        pw[e] = lf_from_float(pv[e]);
+        if (masked) {
+          pv = lf_bw_keep(rel[kb] + 8 * i4 + e, p.window) ? pv : 0.0f;
+        }
+        pw[e] = lf_from_float(pv);
 #if LF_SOFTCAP
-        dw[e] = lf_from_float(pv[e] * (dp[qb][i] - d4[e]) * dcap[e]);
+        s[kb][i] = pv * dcap;
 #else
-        dw[e] = lf_from_float(pv[e] * (dp[qb][i] - d4[e]));
+        s[kb][i] = pv;
 #endif
       }
-      const lf_u32x2 pu = __builtin_bit_cast(lf_u32x2, pw), du = __builtin_bit_cast(lf_u32x2, dw);
-      pf[2 * qb + i4 / 2][2 * (i4 % 2)] = pu[0];
-      pf[2 * qb + i4 / 2][2 * (i4 % 2) + 1] = pu[1];
-      dsf[2 * qb + i4 / 2][2 * (i4 % 2)] = du[0];
-      dsf[2 * qb + i4 / 2][2 * (i4 % 2) + 1] = du[1];
+      const lf_u32x2 pu = __builtin_bit_cast(lf_u32x2, pw);
+      pf[kb][i4 / 2][2 * (i4 % 2)] = pu[0];
+      pf[kb][i4 / 2][2 * (i4 % 2) + 1] = pu[1];
     };
-    // phases 1 and 2
+    auto grad4 = [&](int kb, int i4) {      // dS, without the factor `scale`, which multiplies dK once at the end
+      lf_elem4 dw;
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
-      lf_u32x4 qa[LF_NKS], ga[LF_NKS];
-#pragma unroll
-      for (int ks = 0; ks < LF_BW_PF1; ++ks) {
-        qa[ks] = lf_read_k_frag(q_rm, l32, g, ks * LF_NKB + qb);
-        ga[ks] = lf_read_k_frag(g_rm, l32, g, ks * LF_NKB + qb);
-      }
+      for (int e = 0; e < 4; ++e) dw[e] = lf_from_float(s[kb][4 * i4 + e] * dp[kb][4 * i4 + e]);
+      const lf_u32x2 du = __builtin_bit_cast(lf_u32x2, dw);
+      dsf[kb][i4 / 2][2 * (i4 % 2)] = du[0];
+      dsf[kb][i4 / 2][2 * (i4 % 2) + 1] = du[1];
+    };
+    // per fragment: the read that is LF_BW_PF fragments ahead, and a direct load every other time
+    auto ahead = [&](int i) {
+      const int f = i + LF_BW_PF;
+      fr[f] = f < NF ? frag(st, qb, f) : frag(st_n, qb_n, f - NF);
+    };
+    auto load = [&](int i) {
+      if (loads && i % 2 == 0 && i / 2 < kLoads) issue(ld, i / 2);
       __builtin_amdgcn_sched_barrier(0);
+    };
+    // what is carried from block to block may have been moved between registers just now, by the vector ALU
 #pragma unroll
-      for (int ks = 0; ks < LF_NKS; ++ks) {
-        if (ks + LF_BW_PF1 < LF_NKS) {
-          qa[ks + LF_BW_PF1] = lf_read_k_frag(q_rm, l32, g, (ks + LF_BW_PF1) * LF_NKB + qb);
-          ga[ks + LF_BW_PF1] = lf_read_k_frag(g_rm, l32, g, (ks + LF_BW_PF1) * LF_NKB + qb);
-        }
-        if (ks == 0) {
-          lf_bw_mfma_first(s[qb], qa[ks], kf[ks]);
-          lf_bw_mfma_first(dp[qb], ga[ks], vf[ks]);
-        } else {
-          lf_bw_mfma_vva(s[qb], qa[ks], kf[ks]);
-          lf_bw_mfma_vva(dp[qb], ga[ks], vf[ks]);
-        }
-        issue_piece(st ^ 1, LF_NKS * qb + ks);
-        if (qb == 1 && ks * 4 % LF_NKS == 0) soft4(0, ks * 4 / LF_NKS);      // 4 groups over the LF_NKS pairs
-        __builtin_amdgcn_sched_barrier(0);
+    for (int f = 0; f < LF_BW_PF; ++f) asm volatile("" : "+v"(fr[f]));
+    asm volatile(LF_BW_VALU_SETTLE : "+v"(sinit));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      ahead(i);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+#if LF_SOFTCAP
+        if (i == 0) lf_bw_mfma_zero(s[kb], fr[i], kf[kb][i]);
+#else
+        if (i == 0) lf_bw_mfma_from(s[kb], fr[i], kf[kb][i], sinit);
+#endif
+        else lf_bw_mfma_vvv(s[kb], fr[i], kf[kb][i]);
       }
-      asm volatile(LF_BW_MFMA_DRAIN : "+v"(s[qb]), "+v"(dp[qb]));
+#if !LF_SOFTCAP
+      if (i == 1) LF_BW_HOLD(sinit);
+#endif
+      if (i == NS - 2) {
+        dinit = read_stats(st, 1, qb);
+#if LF_BW_VL
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) vl[0][kb] = v_lds[0][kb][tid];
+#endif
+      }
+      load(i);
     }
-    // phases 3 and 4
-    {
-      lf_u32x4 gt[kNF], qt2[kNF];
 #pragma unroll
-      for (int f = 0; f < LF_BW_PF2; ++f) {
-        gt[f] = __builtin_bit_cast(lf_u32x4, lf_read_v_frag_tr(g_tr, lane, g, f));
-        qt2[f] = __builtin_bit_cast(lf_u32x4, lf_read_v_frag_tr(q_tr, lane, g, f));
+    for (int ks = 0; ks < NS; ++ks) {
+      ahead(NS + ks);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+#if LF_BW_VL
+        const lf_u32x4 vop = ks < LF_BW_VL ? vl[ks][kb] : vf[kb][ks - LF_BW_VL];
+#else
+        const lf_u32x4 vop = vf[kb][ks];
+#endif
+        if (ks == 0) lf_bw_mfma_from(dp[kb], fr[NS + ks], vop, dinit);
+        else lf_bw_mfma_vvv(dp[kb], fr[NS + ks], vop);
+#if LF_BW_VL
+        if (ks + 1 < LF_BW_VL) vl[ks + 1][kb] = v_lds[ks + 1][kb][tid];
+#endif
       }
+      if (ks == 0) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) asm volatile(LF_BW_MFMA_DRAIN : "+v"(s[kb]));
+      } else if (ks == 1) {
+        LF_BW_HOLD(dinit);
+      }
+#pragma unroll
+      for (int t = ks * 4 * KB / NS; t < (ks + 1) * 4 * KB / NS; ++t) soft4(t % KB, t / KB);
+      load(NS + ks);
+    }
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) asm volatile(LF_BW_VALU_SETTLE : "+v"(pf[kb][0]), "+v"(pf[kb][1]), "+v"(s[kb]));     // (s: P takes its place)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      ahead(2 * NS + j);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) lf_bw_mfma_hidden(dv[kb][j % LF_NDB], fr[2 * NS + j], pf[kb][j / LF_NDB]);
+      if (j == 0) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) asm volatile(LF_BW_MFMA_DRAIN : "+v"(dp[kb]));
+      }
+#pragma unroll
+      for (int t = j * 4 * KB / NT; t < (j + 1) * 4 * KB / NT; ++t) grad4(t % KB, t / KB);
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int f = 0; f < kNF; ++f) {
-        if (f % (kNF / 2) == 0) {
-#pragma unroll
-          for (int kk = 0; kk < LF_NKK / 2; ++kk)
-            asm volatile(LF_BW_VALU_SETTLE : "+v"(pf[f / (kNF / 2) * (LF_NKK / 2) + kk]), "+v"(dsf[f / (kNF / 2) * (LF_NKK / 2) + kk]));
-        }
-        if (f + LF_BW_PF2 < kNF) {
-          gt[f + LF_BW_PF2] = __builtin_bit_cast(lf_u32x4, lf_read_v_frag_tr(g_tr, lane, g, f + LF_BW_PF2));
-          qt2[f + LF_BW_PF2] = __builtin_bit_cast(lf_u32x4, lf_read_v_frag_tr(q_tr, lane, g, f + LF_BW_PF2));
-        }
-        lf_bw_mfma_avv(dv[f % LF_NDB], gt[f], pf[f / LF_NDB]);
-        lf_bw_mfma_avv(dk[f % LF_NDB], qt2[f], dsf[f / LF_NDB]);
-        if (f < kNF / 2 && f * 8 % kNF == 0) soft4(1, f * 8 / kNF);              // 4 groups over the first kNF / 2 pairs
-        __builtin_amdgcn_sched_barrier(0);
-      }
     }
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) asm volatile(LF_BW_VALU_SETTLE : "+v"(dsf[kb][0]), "+v"(dsf[kb][1]));
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      ahead(2 * NS + NT + j);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) lf_bw_mfma_hidden(dk[kb][j % LF_NDB], fr[2 * NS + NT + j], dsf[kb][j / LF_NDB]);
+      if (j == 1) sinit = read_stats(st_n, 0, qb_n);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int f = 0; f < LF_BW_PF; ++f) pre[f] = fr[NF + f];
   };
+  // does the wave have a score to keep in queries q .. q + 31, and are all of them kept?
+  auto need = [&](int q) {
+    bool n = key0 < p.Sk && q < p.Sq;
+#if LF_MASK >= 1
+    n = n && q + 31 >= key0;
+#endif
+#if LF_MASK == 2
+    n = n && q - klast < p.window;
+#endif
+    return n;
+  };
+  auto full = [&](int q) {
+    bool n = key0 + 32 * KB <= p.Sk;
+#if LF_MASK >= 1
+    n = n && key0 + 32 * KB - 1 <= q;
+#endif
+#if LF_MASK == 2
+    n = n && q + 31 - key0 < p.window;
+#endif
+    return n;
+  };
+
   if (nsteps > 0) {
-    aim(0, true);
+    aim();
 #pragma unroll
-    for (int j = 0; j < LF_CPR; ++j) issue_piece(0, j);
-    publish(0);
-  }
-  LF_BW_BARRIER();
-  for (int it = 0; it < nsteps; ++it) {
-    const int st = it & 1;
-    const int q0 = 64 * (qt_begin + it % ntq);
-    // the other stage was last read in step it - 1, which every wave left at the barrier below;
-    // after the last step the loads still go out, against an empty range: they fetch nothing
-    aim(min(it + 1, nsteps - 1), it + 1 < nsteps);
-
-    bool need = key0 < p.Sk;
-#if LF_MASK >= 1
-    need = need && (q0 + 63 >= key0);
-#endif
-#if LF_MASK == 2
-    need = need && (q0 - min(key0 + 31, p.Sk - 1) < p.window);
-#endif
-    if (need) {                 // wave-uniform
-      // are all 32 x 64 scores of this wave kept?  Then the step runs without the mask arithmetic
-      bool full = key0 + 31 < p.Sk;
-#if LF_MASK >= 1
-      full = full && (key0 + 31 <= q0);
-#endif
-#if LF_MASK == 2
-      full = full && (q0 + 63 - key0 < p.window);
-#endif
-      step(!full, st, q0);
-    } else {
+    for (int j = 0; j < kLoads; ++j) issue(0, j);
+    aim();
 #pragma unroll
-      for (int j = 0; j < LF_CPR; ++j) issue_piece(st ^ 1, j);
+    for (int j = 0; j < kLoads; ++j) issue(1, j);
+    LF_BW_BARRIER();
+    read_ahead(0, 0);
+    int st = 0, q0 = 64 * qt_begin, left = ntq;
+    for (int it = 0; it < nsteps; ++it) {
+      const int st1 = st == 2 ? 0 : st + 1, st2 = st == 0 ? 2 : st - 1;
+      // (an instance each for the blocks that need the mask arithmetic and for those that do not: a branch per four
+      // scores costs registers that are not there)
+      if (!need(q0)) read_ahead(st, 1);
+      else if (full(q0)) block(0, st, q0, false, false, 0, st, 1);
+      else block(0, st, q0, true, false, 0, st, 1);
+      LF_BW_BARRIER();            // the next tile has landed; every wave is done with the one before this
+      aim();
+      if (!need(q0 + 32)) {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) issue(st2, j);
+        read_ahead(st1, 0);
+      } else if (full(q0 + 32)) {
+        block(1, st, q0 + 32, false, true, st2, st1, 0);
+      } else {
+        block(1, st, q0 + 32, true, true, st2, st1, 0);
+      }
+      st = st1;
+      q0 += 64;
+      if (--left == 0) {
+        left = ntq;
+        q0 = 64 * qt_begin;
+      }
     }
-    if (it + 1 < nsteps) publish(st ^ 1);
-    LF_BW_BARRIER();            // the next stage has landed; every wave is done with this one
+    __builtin_amdgcn_s_waitcnt(0x0070);      // the last loads, against an empty range, before the LDS is given back
   }
 #pragma unroll
-  for (int db = 0; db < LF_NDB; ++db) asm volatile(LF_BW_MFMA_DRAIN_LAST : "+a"(dk[db]), "+a"(dv[db]));
+  for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-  for (int db = 0; db < LF_NDB; ++db)
+    for (int db = 0; db < LF_NDB; ++db) asm volatile(LF_BW_MFMA_DRAIN_LAST : "+a"(dk[kb][db]), "+a"(dv[kb][db]));
+  // the parameters of the output are read only now: held over the loop they cost scalar registers it needs
+  auto ep = (const LfAttnBwdParams __attribute__((address_space(4)))*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ep));
+  const float scale = ep->scale;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dk[db][i] *= p.scale;
-
-  const bool valid = my_key < p.Sk;
-  const int kr = min(my_key, p.Sk - 1);
-  lf_bw_store_rows(dk, p.dk + (long long)b * p.dk_sb + (long long)hkv * p.dk_sh + (long long)kr * p.dk_ss, valid, g);
-  lf_bw_store_rows(dv, p.dv + (long long)b * p.dv_sb + (long long)hkv * p.dv_sh + (long long)kr * p.dv_ss, valid, g);
+  for (int kb = 0; kb < KB; ++kb) {
+    const int my_key = key0 + 32 * kb + l32;
+    const bool valid = my_key < p.Sk;
+    const int kr = min(my_key, p.Sk - 1);
+#pragma unroll
+    for (int db = 0; db < LF_NDB; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dk[kb][db][i] *= scale;
+    lf_bw_store_rows(dk[kb], ep->dk + (long long)b * ep->dk_sb + (long long)hkv * ep->dk_sh + (long long)kr * ep->dk_ss, valid, g);
+    lf_bw_store_rows(dv[kb], ep->dv + (long long)b * ep->dv_sb + (long long)hkv * ep->dv_sh + (long long)kr * ep->dv_ss, valid, g);
+  }
 }
 
 extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_attn_bwd_dq(const LfAttnBwdParams p) {
@@ -527,7 +770,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
   }
   const long long ridx = ((long long)b * p.Hq + h) * p.Sq + qr;
   const float lse_q = my_q < p.Sq ? p.lse[ridx] : __builtin_inff();
-  const float delta_q = my_q < p.Sq ? p.delta[ridx] : 0.0f;
+  const float delta_q = my_q < p.Sq ? -p.delta[ridx] : 0.0f;
 #if LF_SOFTCAP
   const float sc_exp = p.scale / p.softcap * (2.0f * LF_LOG2E);   // 2^(s * sc_exp) = e^(2x)
   const float cexp = p.softcap * LF_LOG2E;                        // exponent of P: tanh x * cexp - L

@@ -939,12 +939,29 @@ def bwd_dq_threads(mask: int, softcap: bool = False) -> int:
     return 256 if mask == MASK_SLIDING or softcap else 512
 
 
-def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False) -> KernelSpec:
-    return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap, extra=(f"-DLF_BW_DQ_NT={bwd_dq_threads(mask, softcap)}",))
+def bwd_key_blocks(D: int, mask: int, softcap: bool, units: int, Sk: int) -> int:
+    """32-key blocks a wave of lf_attn_bwd_dkdv holds: 2 (workgroups of 256 keys; every fragment read from
+    LDS feeds two MFMAs) or 1 (128 keys).  ``units`` = batch x kv heads.  Measured, all backward launches, 2 against 1:
+    causal B4 H32 S2048 541 / 570 us, B2 H32 S4096 946 / 1005 us, unmasked 6 % faster throughout, but the launch has to
+    stay balanced: causal with 256 such workgroups 1.13 ... 1.21 times slower (one long key block per CU), 512 of them at
+    S 1024 1.07 times, unmasked with a last round that is nearly empty (280 workgroups) 1.07 times.  A sliding window walks
+    more blocks than its waves need (0.95 ... 1.08 times), head dimension 64 runs two workgroups per CU with one block
+    (1.03 ... 1.3 times), and a softcap's values do not fit the registers beside two."""
+    n = units * -(-Sk // 256)
+    if D != 128 or softcap or mask == MASK_SLIDING:
+        return 1
+    if mask == MASK_CAUSAL:
+        return 2 if (n >= 512 and Sk >= 2048) or (n >= 1024 and Sk >= 1024) else 1
+    return 2 if n >= 256 and n >= 0.85 * 256 * -(-n // 256) else 1
+
+
+def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False, key_blocks: int = 1) -> KernelSpec:
+    return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap,
+                      extra=(f"-DLF_BW_DQ_NT={bwd_dq_threads(mask, softcap)}", f"-DLF_BW_W={key_blocks}"))
 
 
 def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
-                       dout: torch.Tensor, plan: AttnPlan):
+                       dout: torch.Tensor, plan: AttnPlan, *, key_blocks: Optional[int] = None):
     """Gradients of ``attention(q, k, v, plan)`` for dense K/V (mask none / causal / sliding, scale,
     softcap; no bias or paging): returns ``(dq, dk, dv)`` in the operands' dtype.  ``o`` and ``lse``
     are the forward's output and row log-sum-exp (``attention(..., lse=...)``).  Three launches
@@ -989,7 +1006,7 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     dq = torch.empty((B, Hq, Sq, D), dtype=dtype, device=q.device)
     dk = torch.empty((B, Hkv, Sk, D), dtype=dtype, device=q.device)
     dv = torch.empty((B, Hkv, Sk, D), dtype=dtype, device=q.device)
-    delta = torch.empty((B, Hq, Sq), dtype=torch.float32, device=q.device)
+    delta = torch.empty((2, B, Hq, Sq), dtype=torch.float32, device=q.device)     # row statistics of the kernels
     P = AttnBwdParams()
     for name, t in (("q", q), ("k", k), ("v", v), ("o", o), ("dout", dout), ("dq", dq), ("dk", dk), ("dv", dv),
                     ("lse", lse), ("delta", delta)):
@@ -1002,10 +1019,12 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     P.scale = float(plan.scale)
     P.softcap = softcap if softcap is not None else 0.0
     spec = bwd_spec(dtype, D, mask, softcap is not None)
+    keys = key_blocks or bwd_key_blocks(D, mask, softcap is not None, B * Hkv, Sk)
+    kv_spec = bwd_spec(dtype, D, mask, softcap is not None, keys)
     keep = (q, k, v, o, dout, lse, delta, dq, dk, dv)  # noqa: F841  (tensors stay alive until the launches are queued)
     rows = B * Hq * Sq
     get_kernel(spec, "lf_attn_bwd_delta").launch(((rows + 15) // 16, 1, 1), (256, 1, 1), P)
-    get_kernel(spec, "lf_attn_bwd_dkdv").launch((xcd_slots(B * Hkv, (Sk + 127) // 128), 1, 1), (256, 1, 1), P)
+    get_kernel(kv_spec, "lf_attn_bwd_dkdv").launch((xcd_slots(B * Hkv, -(-Sk // (128 * keys))), 1, 1), (256, 1, 1), P)
     nt = bwd_dq_threads(mask, softcap is not None)
     get_kernel(spec, "lf_attn_bwd_dq").launch((xcd_slots(B * Hkv, (Hq // Hkv) * ((Sq + nt // 2 - 1) // (nt // 2))), 1, 1),
                                               (nt, 1, 1), P)

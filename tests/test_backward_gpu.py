@@ -331,3 +331,27 @@ def test_module_with_projections_trains_with_the_fused_attention(spelling):
     for n, p in m.named_parameters():
         ref = p.grad.float()
         assert ((got[n] - ref).norm() / ref.norm()).item() <= 3e-2, n
+
+
+@pytest.mark.parametrize("key_blocks", [1, 2])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,mask,window,dtype", [
+    (1, 2, 2, 1, 1, "causal", 0, torch.bfloat16),              # a single score
+    (1, 2, 1, 31, 31, "causal", 0, torch.float16),             # less than one block of queries and keys
+    (1, 2, 2, 65, 65, "causal", 0, torch.bfloat16),            # one row into the second tile
+    (2, 2, 2, 257, 257, "causal", 0, torch.float16),           # one key into the second workgroup of 256
+    (1, 4, 2, 96, 290, None, 0, torch.bfloat16),               # Sq != Sk, an odd number of 32-query blocks
+    (1, 2, 2, 700, 513, None, 0, torch.bfloat16),
+])
+def test_key_blocks_per_wave_at_tile_edges(B, Hq, Hkv, Sq, Sk, mask, window, dtype, key_blocks):
+    g = torch.Generator().manual_seed(Sq + 3 * Sk)
+    q, k, v, dout = (torch.randn(s, generator=g).to(dtype).to(DEV)
+                     for s in ((B, Hq, Sq, 128), (B, Hkv, Sk, 128), (B, Hkv, Sk, 128), (B, Hq, Sq, 128)))
+    plan = lowering.AttnPlan(mask=mask, window=window, scale=128 ** -0.5)
+    lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=DEV)
+    o = lowering.attention(q, k, v, plan, lse=lse)
+    got = lowering.attention_backward(q, k, v, o, lse, dout, plan, key_blocks=key_blocks)
+    _, _, *want = _ref(q, k, v, dout, mask, window, 128 ** -0.5)
+    # as test_backward_matches_autograd: P, dS and the results are rounded once each (2^-9 bf16, 2^-12 fp16)
+    for name, a, w in zip(("dq", "dk", "dv"), got, want):
+        bound = (4e-2 if dtype == torch.bfloat16 else 1e-2) * max(1.0, w.abs().max().item())
+        assert (a.double() - w).abs().max().item() <= bound, name

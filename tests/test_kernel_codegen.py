@@ -127,3 +127,54 @@ def test_the_check_sees_an_early_read():
     with pytest.raises(AssertionError):
         _check("probe", chain + ["global_load_dwordx4 v[28:31], v[0:1], off", "s_nop 9", "s_nop 9"])
     _check("probe", chain + ["v_add_u32_e32 v1, v2, v3", "s_nop 9", "s_nop 9", "v_mov_b32_e32 v40, v17"])
+
+
+def _registers(operand):
+    m = re.match(r"v\[(\d+):(\d+)\]$", operand) or re.match(r"v(\d+)$", operand)
+    return set(range(int(m.group(1)), int(m.group(m.lastindex)) + 1)) if m else set()
+
+
+def _check_settled(name, lines):
+    """No MFMA reads a VGPR that the vector ALU wrote less than two wait states before: the compiler does not know that
+    an inline MFMA needs them, for instance behind a copy of its own."""
+    for i, ln in enumerate(lines):
+        if not ln.startswith("v_mfma"):
+            continue
+        read = set().union(*(_registers(x.strip()) for x in ln.split(None, 1)[1].split(",")[1:]))
+        states, j = 0, i - 1
+        while j >= 0 and states < 2:
+            x = lines[j]
+            if x.startswith("v_") and not x.startswith("v_mfma"):
+                dst = x.split(None, 1)[1].split(",")
+                wrote = _registers(dst[0].strip()) | (_registers(dst[1].strip()) if "swap" in x else set())
+                assert not wrote & read, f"{name}: '{ln}' reads what '{x}' wrote {states} wait states before"
+            nop = re.match(r"s_nop (\d+)", x)
+            states += int(nop.group(1)) + 1 if nop else 1
+            j -= 1
+
+
+@pytest.mark.parametrize("dtype,D,mask,softcap,blocks", [
+    (torch.bfloat16, 128, lowering.MASK_CAUSAL, False, 2), (torch.float16, 128, lowering.MASK_NONE, False, 2),
+    (torch.bfloat16, 128, lowering.MASK_CAUSAL, False, 1), (torch.float16, 128, lowering.MASK_SLIDING, True, 1),
+    (torch.float16, 64, lowering.MASK_CAUSAL, False, 1)])
+def test_hidden_accumulators_stay_in_their_registers(shim_built, dtype, D, mask, softcap, blocks):
+    """lf_attn_bwd_dkdv hands its accumulators to the MFMAs as inputs: between the first and the last MFMA no other
+    instruction may touch an AGPR, and nothing may be spilled."""
+    lines = _kernels(lowering.bwd_spec(dtype, D, mask, softcap, key_blocks=blocks))["lf_attn_bwd_dkdv"]
+    _check("lf_attn_bwd_dkdv", lines)
+    _check_settled("lf_attn_bwd_dkdv", lines)
+    mfma = [i for i, ln in enumerate(lines) if ln.startswith("v_mfma")]
+    for ln in lines[mfma[0]:mfma[-1]]:
+        assert ln.startswith("v_mfma") or not re.search(r"\ba(\d+|\[\d+:\d+\])", ln), ln
+    # every accumulator tuple is written by MFMAs that name it as source and destination alike
+    for ln in lines:
+        m = re.match(r"v_mfma_\S+ (a\[\d+:\d+\]),.*, (\S+)$", ln)
+        assert m is None or m.group(1) == m.group(2), ln
+
+
+def test_the_check_sees_an_unsettled_operand():
+    mfma = "v_mfma_f32_32x32x16_bf16 v[16:31], v[0:3], v[4:7], v[16:31]"
+    with pytest.raises(AssertionError):
+        _check_settled("probe", ["v_mov_b32_e32 v17, v9", "v_add_u32_e32 v40, v1, v2", mfma])
+    _check_settled("probe", ["v_mov_b32_e32 v17, v9", "s_nop 1", mfma])
+    _check_settled("probe", ["v_mov_b32_e32 v32, v9", mfma])
