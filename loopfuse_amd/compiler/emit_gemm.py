@@ -3,17 +3,19 @@
 cases ``tests/test_accuracy.py:56-82``: ``a @ b + c`` in two and three dims).
 
 A nest ``out[batch.., m, n] = f(sum_k A[batch.., m, k] * B[batch.., k, n], other reads)`` with bf16 /
-fp16 operands becomes one kernel.  A workgroup owns a tile of the output -- 128 x 128 on four waves (two
-workgroups per CU) or 256 x 256 on eight (one per CU, half the L2 -> LDS bytes per flop; ``TILES``), a
-compile-time choice -- and walks k in steps of 64.  Both operand tiles arrive by direct global -> LDS loads
+fp16 operands becomes one kernel.  A workgroup owns a tile of the output -- 128 x 128 on four waves or
+256 x 128 / 256 x 256 on eight (``TILES``), a compile-time choice -- and walks k, or a part of it, in
+steps of 64.  Both operand tiles arrive by direct global -> LDS loads
 (``buffer_load_dwordx4 ... lds``: 16-byte pieces, range-checked so that the edges arrive as zeros, the XOR
-permutation applied on the global side), double-buffered, one barrier per step, and come back as
+permutation applied on the global side), two to four stages, one barrier per step, and come back as
 ``v_mfma_f32_32x32x16`` operands -- by plain 16-byte reads where k is the contiguous dimension of the
 operand in memory, by transposed reads (``ds_read_b64_tr_b16``) where m / n is.  The product is formed
 transposed (C^T = B^T A^T); the fp32 accumulators then pass through LDS once so that a lane holds four
 consecutive n of one m and neighbouring lanes neighbouring n: the epilogue expression -- whatever the
 fused nest holds around the contraction -- is evaluated there per element, its reads coalesced, and the
-results leave in 8- or 16-byte stores along the rows of the output.  Tiles are walked in bands of a few
+results leave in 8- or 16-byte stores along the rows of the output.  Where the tiles alone would leave
+CUs idle, k is split into parts (``choose``): the workgroups then leave fp32 partial sums, which a second
+kernel adds up and runs the epilogue on.  Tiles are walked in bands of a few
 tile rows, an XCD taking a contiguous run of them, so that its resident workgroups share operand rows and
 columns in its L2.
 
@@ -26,25 +28,30 @@ one-thread-per-element kernel of the same nest.
 from __future__ import annotations
 
 import dataclasses
+import functools
+import math
 from typing import Optional
 
 from . import ir
 from .emit import _CT, MAX_N, MAX_PTR, Emitter, Kernel, NotLowerable
 
 BK = 64
-# workgroup tiles (waves along m, waves along n, 32 x 32 blocks per wave along m, along n): 128 x 128 on four waves at
-# two workgroups per CU; 256 x 256 on eight waves, one per CU, with half the L2 -> LDS bytes per flop
-TILES = {"s": (2, 2, 2, 2), "l": (4, 2, 2, 4)}
+# Workgroup tiles: waves along m, waves along n, 32 x 32 blocks per wave along m, along n, LDS stages.  128 x 128 on four
+# waves, at two workgroups per CU (s) or, where there are too few tiles for that, one with four stages in flight (d: a step
+# then no longer costs a memory latency); 256 x 128 on eight waves (m) and 256 x 256 (l), one per CU, with three quarters
+# and half the L2 -> LDS bytes per flop.
+TILES = {"s": (2, 2, 2, 2, 2), "d": (2, 2, 2, 2, 4), "m": (4, 2, 2, 2, 3), "l": (4, 2, 2, 4, 2)}
 
 
 def tile_extent(shape: str) -> tuple:
-    wm, wn, mb, nb = TILES[shape]
+    wm, wn, mb, nb, _ = TILES[shape]
     return 32 * wm * mb, 32 * wn * nb
 
 
-def tile_options(shape: str) -> list:
-    wm, wn, mb, nb = TILES[shape]
-    return [f"-DLFG_WGM={wm}", f"-DLFG_WGN={wn}", f"-DLFG_MB={mb}", f"-DLFG_NB={nb}"]
+def tile_options(shape: str, split: bool = False) -> list:
+    wm, wn, mb, nb, stages = TILES[shape]
+    return [f"-DLFG_WGM={wm}", f"-DLFG_WGN={wn}", f"-DLFG_MB={mb}", f"-DLFG_NB={nb}", f"-DLFG_STAGES={stages}"] + \
+        (["-DLFG_SPLIT=1"] if split else [])
 
 GEMM_PRELUDE = r"""
 typedef float lfg_f32x16 __attribute__((ext_vector_type(16)));
@@ -52,6 +59,9 @@ typedef unsigned int lfg_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int lfg_u32x2 __attribute__((ext_vector_type(2)));
 typedef float lfg_f32x4 __attribute__((ext_vector_type(4)));
 typedef short lfg_s16x4 __attribute__((ext_vector_type(4)));
+#ifndef LFG_SPLIT
+#define LFG_SPLIT 0      /* 1: a workgroup sums a part of k and leaves fp32 partials; a second kernel adds them up and runs the epilogue */
+#endif
 typedef __bf16 lfg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 lfg_f16x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ lfg_f32x16 lfg_mfma(__bf16, lfg_u32x4 a, lfg_u32x4 b, lfg_f32x16 c) {
@@ -142,9 +152,12 @@ class GemmInfo:
     a_batch_dims: list          # dims of A indexed by a batch atom
     b_batch_dims: list
     flags_at: int = 0           # n[flags_at]: the output's rows are contiguous and aligned for 8- / 16-byte stores;
-                                # n[flags_at + 1], n[flags_at + 2]: bytes of A / B reachable from a batch element's base
+                                # n[flags_at + 1], n[flags_at + 2]: bytes of A / B reachable from a batch element's base;
+                                # n[flags_at + 3], n[flags_at + 4]: parts that k is split into, steps of 64 k per part
     out_buf: object = None
     out_n_dim: int = -1         # dimension of the output indexed by n alone (-1: none)
+    ws_ptr: int = 0             # ptr[ws_ptr]: fp32 partials of a split product
+    sum_source: str = ""        # the kernel that adds them up
 
 
 def _single(atoms) -> Optional[ir.Atom]:
@@ -246,7 +259,8 @@ class GemmEmitter(Emitter):
                 g.out_n_dim = d
         na, ns = len(self.atoms), len(self.strides)
         g.flags_at = na + ns
-        if na + ns + 3 > MAX_N or len(self.bufs) > MAX_PTR:
+        g.ws_ptr = len(self.bufs)
+        if na + ns + 5 > MAX_N or len(self.bufs) + 1 > MAX_PTR:
             raise NotLowerable("nest touches too many buffers / dimensions")
         defs = [f"const long long N{k} = p.n[{k}];" for k in range(na)] + \
                [f"const long long S{k} = p.n[{na + k}];" for k in range(ns)]
@@ -264,10 +278,11 @@ class GemmEmitter(Emitter):
   constexpr int kBM = 32 * kWM * kMB, kBN = 32 * kWN * kNB, kWaves = kWM * kWN, kNT = 64 * kWaves;
   constexpr int kTileA = kBM * {BK}, kTileB = kBN * {BK};                    // elements of one operand tile
   constexpr int kPA = kBM * 8 / kNT, kPB = kBN * 8 / kNT;                   // 16-byte pieces per thread and tile
+  constexpr int kS = LFG_STAGES;
   static_assert(kNB % 2 == 0 && kBM * 8 % kNT == 0 && kBN * 8 % kNT == 0, "tile shape");
-  static_assert(kWaves * kMB * 8192 <= 4 * (kTileA + kTileB), "the accumulators pass through the tiles' LDS");
-  const bool row_stores = p.n[{g.flags_at}] != 0;
-  __shared__ __attribute__((aligned(16))) unsigned short lds[2 * (kTileA + kTileB)];     // A tiles [2], then B tiles [2]
+  static_assert(LFG_SPLIT || kWaves * kMB * 8192 <= 2 * kS * (kTileA + kTileB), "the accumulators pass through the tiles' LDS");
+  static_assert((kS - 2) * (kPA + kPB) < 64, "loads in flight behind a stage");
+  __shared__ __attribute__((aligned(16))) unsigned short lds[kS * (kTileA + kTileB)];     // A tiles [kS], then B tiles [kS]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % kWM, wn = wave / kWM;
   const long long M = N{km}, Nn = N{kn}, K = N{kk};
@@ -276,14 +291,17 @@ class GemmEmitter(Emitter):
   {' '.join(f'total *= N{self.atom(a)};' for a in g.batch)}
   // workgroups go to the 8 XCDs round-robin: each XCD takes a contiguous run of tiles (n fastest), so the
   // workgroups resident on it share rows of A and columns of B in its L2
-  const long long per_xcd = (total + 7) / 8;
+  const long long parts = LFG_SPLIT ? p.n[{g.flags_at + 3}] : 1, per_xcd = (total * parts + 7) / 8;
   long long blk = (long long)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((long long)(blockIdx.x >> 3) >= per_xcd || blk >= total) return;
+  if ((long long)(blockIdx.x >> 3) >= per_xcd || blk >= total * parts) return;
+  const long long part = LFG_SPLIT ? blk / total : 0;      // slowest: neighbouring tiles of one part share rows of A or columns of B
+  if (LFG_SPLIT) blk -= part * total;
   // inside a batch element the tiles run in bands of kBand tile rows, column by column: the workgroups resident
   // on an XCD at a time (32 or 64 consecutive tiles) then cover a block of the output that is a few tiles tall and
   // wide, and read correspondingly few rows of A and columns of B past its L2
   constexpr long long kBand = kNT <= 256 ? 8 : 4;
   const long long t = blk % (mt * nt); blk /= mt * nt;
+  const long long element = blk;      // of the batch
   const long long first = t / (kBand * nt) * kBand, tall = min(mt - first, kBand);
   const long long tm = first + (t % (kBand * nt)) % tall, tn = (t % (kBand * nt)) / tall;
   {' '.join(batch_decode)}
@@ -313,9 +331,21 @@ class GemmEmitter(Emitter):
   }}
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)lds;
   const unsigned stepa = (unsigned)(2 * {BK} * S{sak}), stepb = (unsigned)(2 * {BK} * S{sbk});
-  // tile of k step `st` into buffer `buf`
-  auto fetch = [&](int st, int buf) {{
-    const int k0 = st * {BK};
+  const int steps = (int)((K + {BK - 1}) / {BK});
+  const int st_begin = LFG_SPLIT ? (int)(part * p.n[{g.flags_at + 4}]) : 0;
+  const int st_end = LFG_SPLIT ? min(st_begin + (int)p.n[{g.flags_at + 4}], steps) : steps;
+  // With few rows of A the loads of B from memory are the time.  There a workgroup's walk over k starts at a step of its
+  // own, by tile column: with k contiguous and K a power of two every row of a step's window lies on the same few memory
+  // channels, and workgroups that walk k in step all ask those (M 64, N 4096, K 16384: 39 -> 33 us; from M 512 on, where
+  // matrix work is the time and tile columns share rows of A in an L2, it costs 4 ... 8 %).
+  const int nsteps = st_end - st_begin;
+  int ld_st = st_begin + (M <= 256 ? (int)(tn % nsteps) : 0), ld_left = nsteps;
+  // the next step's tiles into buffer `buf`; past the last step the loads go out against nothing, so that the number in
+  // flight behind a stage is always the same
+  auto fetch = [&](int buf) {{
+    const int st = ld_st, k0 = ld_left > 0 ? st * {BK} : 0x7fffffff;
+    --ld_left;
+    if (++ld_st == st_end) ld_st = st_begin;
 #pragma unroll
     for (int j = 0; j < kPA; ++j)
       lfg_dma(rs_a, k0 < rooma[j] ? offa[j] + (unsigned)st * stepa : 0xffffffffu,
@@ -323,7 +353,7 @@ class GemmEmitter(Emitter):
 #pragma unroll
     for (int j = 0; j < kPB; ++j)
       lfg_dma(rs_b, k0 < roomb[j] ? offb[j] + (unsigned)st * stepb : 0xffffffffu,
-              lds0 + 2u * (unsigned)(2 * kTileA + kTileB * buf) + 1024u * (unsigned)(wave + kWaves * j));
+              lds0 + 2u * (unsigned)(kS * kTileA + kTileB * buf) + 1024u * (unsigned)(wave + kWaves * j));
   }};
   lfg_f32x16 acc[kMB][kNB];
 #pragma unroll
@@ -332,14 +362,16 @@ class GemmEmitter(Emitter):
     for (int y = 0; y < kNB; ++y)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[x][y][i] = 0.0f;
-  fetch(0, 0);
-  asm volatile("s_waitcnt vmcnt(0)\\n\\ts_barrier" ::: "memory");
-  const int steps = (int)((K + {BK - 1}) / {BK});
-  for (int st = 0; st < steps; ++st) {{
-    const int cur = st & 1;
-    if (st + 1 < steps) fetch(st + 1, cur ^ 1);
+#define LFG_NEXT_STAGE() asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\\n\\ts_barrier" :: "n"((kS - 2) * (kPA + kPB)) : "memory")
+#pragma unroll
+  for (int s = 0; s < kS - 1; ++s) fetch(s);
+  LFG_NEXT_STAGE();
+  int cur = 0;
+  for (int i = 0; i < nsteps; ++i) {{
+    // into the stage that every wave left at the last barrier
+    fetch(cur == 0 ? kS - 1 : cur - 1);
     const unsigned short* ta = &lds[kTileA * cur];
-    const unsigned short* tb = &lds[2 * kTileA + kTileB * cur];
+    const unsigned short* tb = &lds[kS * kTileA + kTileB * cur];
 #pragma unroll
     for (int ks = 0; ks < {BK // 16}; ++ks) {{
       lfg_u32x4 fm[kMB], fn[kNB];
@@ -353,8 +385,29 @@ class GemmEmitter(Emitter):
         for (int y = 0; y < kNB; ++y) acc[x][y] = lfg_mfma(({elem})0.0f, fn[y], fm[x], acc[x][y]);
     }}
     // this wave's loads of the next tile have landed, every wave is done reading this one
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\\n\\ts_barrier" ::: "memory");
+    LFG_NEXT_STAGE();
+    cur = cur == kS - 1 ? 0 : cur + 1;
   }}
+#undef LFG_NEXT_STAGE
+  // the loads against nothing still write zeros: none may be left when the LDS changes its role or is given back
+  if (kS > 2) asm volatile("s_waitcnt vmcnt(0)\\n\\ts_barrier" ::: "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#if LFG_SPLIT
+  // partials in accumulator order: [part][tile][wave][32 x 32 block][4][64 lanes] x 4 floats, every store 1 KB in a row
+  float* ws = reinterpret_cast<float*>(p.ptr[{g.ws_ptr}]) +
+              (((part * (total / (mt * nt)) + element) * mt + tm) * nt + tn) * (kBM * kBN) + wave * (kMB * kNB * 1024) + 4 * lane;
+#pragma unroll
+  for (int x = 0; x < kMB; ++x)
+#pragma unroll
+    for (int y = 0; y < kNB; ++y)
+      if (m0 + 32 * (kMB * wm + x) < M && n0 + 32 * (kNB * wn + y) < Nn) {{
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<lfg_f32x4*>(&ws[((x * kNB + y) * 4 + q) * 256]) =
+              lfg_f32x4{{acc[x][y][4 * q], acc[x][y][4 * q + 1], acc[x][y][4 * q + 2], acc[x][y][4 * q + 3]}};
+      }}
+#else
+  const bool row_stores = p.n[{g.flags_at}] != 0;
   // acc[x][y][i] = C[m][n], m = 32 * (kMB * wm + x) + lane % 32, n = 32 * (kNB * wn + y) + 8 * (i / 4) + 4 * (lane / 32) + i % 4.
   // Two n blocks at a time through the wave's own part of LDS ([32 * kMB m][64 n] fp32, 16-byte pieces permuted by the
   // row): afterwards a lane holds four consecutive n of one m and 16 neighbouring lanes cover 64 consecutive n.
@@ -398,6 +451,89 @@ class GemmEmitter(Emitter):
       }}
     }}
   }}
+#endif
+}}
+"""
+        g.sum_source = f"""
+// The parts of a 32 x 32 block of the output, one block per workgroup, added in fp32 in the order of k, and the epilogue on
+// the sum.  Bound by its reads (written just before, mostly still in the last-level cache): a wave takes 8 rows x 32
+// columns, so that it reads whole 128-byte lines and writes 64-byte pieces of rows.
+extern "C" __global__ void __launch_bounds__(256) {self.name}_sum(const LfGenParams p) {{
+  {' '.join(defs)}
+  constexpr int kWM = LFG_WGM, kWN = LFG_WGN, kMB = LFG_MB, kNB = LFG_NB;
+  constexpr int kBM = 32 * kWM * kMB, kBN = 32 * kWN * kNB;
+  const long long M = N{km}, Nn = N{kn};
+  const long long mt = (M + kBM - 1) / kBM, nt = (Nn + kBN - 1) / kBN, mb = (M + 31) / 32, nb = (Nn + 31) / 32;
+  long long total = mt * nt;
+  {' '.join(f'total *= N{self.atom(a)};' for a in g.batch)}
+  long long blk = blockIdx.x;
+  const int bn = (int)(blk % nb); blk /= nb;
+  const int bm = (int)(blk % mb); blk /= mb;
+  const int tm = bm / (kWM * kMB), wm = bm / kMB % kWM, x = bm % kMB, tn = bn / (kWN * kNB), wn = bn / kNB % kWN, y = bn % kNB;
+  const int lane = threadIdx.x & 63, row = 8 * (threadIdx.x >> 6) + (lane & 7), q = lane >> 4, gg = (lane >> 3) & 1;
+  const float* ws = reinterpret_cast<const float*>(p.ptr[{g.ws_ptr}]) + ((blk * mt + tm) * nt + tn) * (kBM * kBN) +
+                    (wm + kWM * wn) * (kMB * kNB * 1024) + ((x * kNB + y) * 4 + q) * 256 + 4 * (32 * gg + row);
+  const long long m = 32 * bm + row, n = 32 * bn + 8 * q + 4 * gg, stride = total * (kBM * kBN);
+  {' '.join(batch_decode)}
+  if (m >= M || n >= Nn) return;
+  lfg_f32x4 c = {{0.0f, 0.0f, 0.0f, 0.0f}};
+  const int parts = (int)p.n[{g.flags_at + 3}];
+  for (int z = 0; z < parts; z += 4) {{
+    lfg_f32x4 t[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) t[u] = *reinterpret_cast<const lfg_f32x4*>(&ws[min(z + u, parts - 1) * stride]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (z + u < parts) c += t[u];
+  }}
+  auto epilogue = [&](float accv, long long i{km}, long long i{kn}) -> float {{ return {val}; }};
+  auto out_at = [&](long long i{km}, long long i{kn}) -> long long {{ return {ooff}; }};
+  float r[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = epilogue(c[e], m, n + e < Nn ? n + e : n);
+  if (p.n[{g.flags_at}] != 0 && n + 3 < Nn) {{
+    lfg_st4<{out_t}>(p.ptr[{o}], out_at(m, n), r);
+  }} else {{
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < Nn) lfg_st<{out_t}>(p.ptr[{o}], out_at(m, n + e), r[e]);
+  }}
 }}
 """
         return Kernel(self.name, src, self.bufs, self.atoms, self.strides, self.scalars, par)
+
+
+
+# us per step of 64 k with every CU busy (s: see choose), us per workgroup besides (first loads, results), workgroups resident at a time
+_COST = {"s": (0.0, 4.0, 512), "d": (0.80, 5.0, 256), "m": (1.02, 5.0, 256), "l": (1.95, 8.0, 256)}
+_MAX_PARTIALS = 1 << 26         # floats that the parts of a split product may take
+
+
+@functools.lru_cache(maxsize=4096)
+def choose(M: int, N: int, K: int, batch: int) -> tuple:
+    """(tile shape, parts that k is split into) of a product: the candidate with the least time in a model of rounds of
+    resident workgroups, plus, for a split product, the sum's launch and the traffic of its partials.  The constants are
+    fitted to a sweep of both over 16 shapes (M 16 ... 8192, N and K 1024 ... 16384, weights from HBM), where the choice is
+    within 4 % of the best candidate.  What it is for: a product whose tiles leave most CUs idle, or alone with the latency
+    of their loads.  M 256, us: N 4096 K 16384 241 (64 tiles s) -> 52 (m, 8 parts); N 16384 K 4096 72 -> 54 (m, 2 parts);
+    M 64, N 4096 K 16384 235 -> 33 (d, 8 parts); M 1024, N 4096 K 16384 246 -> 145 (m, 2 parts)."""
+    steps = -(-K // BK)
+    best, best_t = ("s", 1), math.inf
+    for shape, (step, fixed, slots) in _COST.items():
+        bm, bn = tile_extent(shape)
+        if shape in "ml" and M <= bm // 2 or shape == "l" and N <= bn // 2:
+            continue                         # half of the tile would be padding
+        tiles = -(-M // bm) * -(-N // bn) * batch
+        for parts in range(1, max(1, min(32, steps // 4)) + 1):
+            if parts > 1 and (tiles * parts > slots or parts * tiles * bm * bn > _MAX_PARTIALS):
+                break
+            if shape == "s":
+                step = 1.5 if M <= 128 else 1.3 if M <= 256 else (0.85 if tiles * parts <= 256 else 1.05)     # two stages: the latency of memory shows
+            elif shape == "d" and M <= 128:
+                step = 0.72
+            t = -(-tiles * parts // slots) * (-(-steps // parts) * step + fixed)
+            if parts > 1:
+                t += 4.0 + parts * M * N * batch * 8 / 6e6
+            if t < best_t:
+                best, best_t = (shape, parts), t
+    return best

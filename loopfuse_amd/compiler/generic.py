@@ -116,27 +116,30 @@ class GenericProgram:
             self._loaded[dev] = ([mod.kernel(k.name) for k in self.kernels], {i: mod.kernel(k.name) for i, k in self.wave.items()})
         return self._loaded[dev]
 
-    def _gemm_kernel(self, ni: int, layouts, shape: str):
+    def _gemm_kernel(self, ni: int, layouts, shape: str, split: bool = False):
+        """The product kernel of nest ``ni`` and, for a split product, the kernel that adds up the parts."""
         from .. import lowering, runtime
-        key = (torch.cuda.current_device(), tuple(layouts), shape)
+        key = (torch.cuda.current_device(), tuple(layouts), shape, split)
         if key not in self._gemm_loaded:
             opts = list(lowering.COMMON_OPTS) + [f"-DLFG_A_ROWS={layouts[0]}", f"-DLFG_B_ROWS={layouts[1]}"] + \
-                emit_gemm.tile_options(shape)
-            code, _, _ = runtime.compile_source(self.gemm_source, "lf_generic_mfma", opts)
+                emit_gemm.tile_options(shape, split)
+            src = self.gemm_source + ("".join(info.sum_source for _, info in self.gemm.values()) if split else "")
+            code, _, _ = runtime.compile_source(src, "lf_generic_mfma", opts)
             mod = runtime.Module(code)
-            self._gemm_loaded[key] = {i: mod.kernel(k.name) for i, (k, _) in self.gemm.items()}
+            self._gemm_loaded[key] = {i: (mod.kernel(k.name), mod.kernel(k.name + "_sum") if split else None)
+                                      for i, (k, _) in self.gemm.items()}
         return self._gemm_loaded[key][ni]
 
     @staticmethod
-    def _gemm_shape(info, ext: dict) -> str:
-        """256 x 256 tiles when they fill most of the CUs, else 128 x 128."""
+    def _gemm_shape(info, ext: dict) -> tuple:
+        """(tile shape, parts that k is split into); LOOPFUSE_GEMM_TILE / LOOPFUSE_GEMM_PARTS override the rule."""
         import os
+        M, N, K = ext[info.m.id], ext[info.n.id], ext[info.k.id]
+        batch = math.prod(ext[a.id] for a in info.batch)
         forced = os.environ.get("LOOPFUSE_GEMM_TILE")
         if forced in emit_gemm.TILES:
-            return forced
-        bm, bn = emit_gemm.tile_extent("l")
-        tiles = -(-ext[info.m.id] // bm) * -(-ext[info.n.id] // bn) * math.prod(ext[a.id] for a in info.batch)
-        return "l" if tiles >= 192 and ext[info.m.id] >= bm and ext[info.n.id] >= bn else "s"
+            return forced, max(1, min(int(os.environ.get("LOOPFUSE_GEMM_PARTS", "1")), -(-K // emit_gemm.BK)))
+        return emit_gemm.choose(M, N, K, batch)
 
     @staticmethod
     def _gemm_layouts(info, bufs: dict, ext: dict):
@@ -247,9 +250,9 @@ class GenericProgram:
                 except KeyError:
                     layouts = None
                 if layouts is not None and all(ext.get(a.id, 0) > 0 for a in self.gemm[ni][0].atoms):
-                    shape = self._gemm_shape(self.gemm[ni][1], ext)
-                    steps.append(self._launch_gemm(self._gemm_kernel(ni, layouts, shape), shape, *self.gemm[ni], bufs, ext, args)
-                                 + ([b.name for b in self.gemm[ni][0].bufs],))
+                    shape, parts = self._gemm_shape(self.gemm[ni][1], ext)
+                    steps += self._launch_gemm(self._gemm_kernel(ni, layouts, shape, parts > 1), shape, parts, *self.gemm[ni],
+                                               bufs, ext, args, lambda name, n: allocs.append((len(steps), name, (n,), torch.float32)))
                     counters["mfma"] += 1
                     n_mfma += 1
                     info = self.gemm[ni][1]
@@ -303,6 +306,7 @@ class GenericProgram:
             while at < len(allocs) and allocs[at][0] <= i:
                 bufs[allocs[at][1]] = torch.empty(allocs[at][2], dtype=allocs[at][3], device=dev)
                 at += 1
+            prm = emit.GenParams.from_buffer_copy(prm)      # (another thread may be replaying the same plan)
             for slot, name in enumerate(names):
                 prm.ptr[slot] = bufs[name].data_ptr()
             fn.launch((blocks, 1, 1), (threads, 1, 1), prm)
@@ -315,10 +319,28 @@ class GenericProgram:
         return bufs[out_name].view(view)
 
     @staticmethod
-    def _launch_gemm(fn, shape: str, k, info, bufs: dict, ext: dict, args) -> tuple:
+    def _launch_gemm(fns, shape: str, parts: int, k, info, bufs: dict, ext: dict, args, allocated) -> list:
+        """Launch the product (and, with ``parts`` > 1, the sum over its parts); returns the launches."""
+        fn, fn_sum = fns
+        M, N, K = ext[info.m.id], ext[info.n.id], ext[info.k.id]
+        batch = math.prod(ext[a.id] for a in info.batch)
         prm = emit.GenParams()
-        for i, b in enumerate(k.bufs):
-            prm.ptr[i] = bufs[b.name].data_ptr()
+        names = [b.name for b in k.bufs]
+        bm, bn = emit_gemm.tile_extent(shape)
+        tiles = -(-M // bm) * -(-N // bn) * batch
+        steps = -(-K // emit_gemm.BK)
+        per_part = -(-steps // parts)
+        parts = -(-steps // per_part)
+        blocks = 8 * -(-(tiles * parts) // 8)
+        if blocks >= 1 << 31:
+            raise NotLowerable("more tiles than one grid dimension holds")
+        if fn_sum is not None:
+            ws = f"{k.name} partial sums"
+            bufs[ws] = torch.empty((parts * tiles * bm * bn,), dtype=torch.float32, device=bufs[info.out_buf.name].device)
+            allocated(ws, bufs[ws].numel())
+            names.append(ws)
+        for i, name in enumerate(names):
+            prm.ptr[i] = bufs[name].data_ptr()
         for i, a in enumerate(k.atoms):
             prm.n[i] = ext[a.id]
         for i, (b, d) in enumerate(k.strides):
@@ -326,20 +348,21 @@ class GenericProgram:
         # rows of the output contiguous along n, every row start and the extent a multiple of four elements:
         # results leave four at a time
         o = bufs[info.out_buf.name]
-        prm.n[info.flags_at] = int(info.out_n_dim >= 0 and o.stride(info.out_n_dim) == 1 and ext[info.n.id] % 4 == 0
+        prm.n[info.flags_at] = int(info.out_n_dim >= 0 and o.stride(info.out_n_dim) == 1 and N % 4 == 0
                                    and o.data_ptr() % 16 == 0
                                    and all(st % 4 == 0 for d, st in enumerate(o.stride()) if d != info.out_n_dim and o.shape[d] > 1))
-        for j, (buf, (d_outer, d_k), outer) in enumerate(((info.a_buf, info.a_dims, ext[info.m.id]),
-                                                          (info.b_buf, info.b_dims, ext[info.n.id]))):
+        for j, (buf, (d_outer, d_k), outer) in enumerate(((info.a_buf, info.a_dims, M), (info.b_buf, info.b_dims, N))):
             t = bufs[buf.name]
-            prm.n[info.flags_at + 1 + j] = 2 * ((outer - 1) * t.stride(d_outer) + (ext[info.k.id] - 1) * t.stride(d_k) + 1)
+            prm.n[info.flags_at + 1 + j] = 2 * ((outer - 1) * t.stride(d_outer) + (K - 1) * t.stride(d_k) + 1)
+        prm.n[info.flags_at + 3], prm.n[info.flags_at + 4] = parts, per_part
         for i, s in enumerate(k.scalars):
             prm.f[i] = float(s.fn(args))
-        bm, bn = emit_gemm.tile_extent(shape)
-        tiles = -(-ext[info.m.id] // bm) * -(-ext[info.n.id] // bn) * math.prod(ext[a.id] for a in info.batch)
-        blocks = 8 * -(-tiles // 8)
-        if blocks >= 1 << 31:
-            raise NotLowerable("more tiles than one grid dimension holds")
-        wm, wn, _, _ = emit_gemm.TILES[shape]
-        fn.launch((blocks, 1, 1), (64 * wm * wn, 1, 1), prm)
-        return fn, blocks, 64 * wm * wn, prm
+        wm, wn = emit_gemm.TILES[shape][:2]
+        launches = [(fn, blocks, 64 * wm * wn, prm, names)]
+        if fn_sum is not None:
+            launches.append((fn_sum, -(-M // 32) * -(-N // 32) * batch, 256, prm, names))
+            if launches[1][1] >= 1 << 31:
+                raise NotLowerable("more blocks of results than one grid dimension holds")
+        for f, grid, threads, _, _ in launches:
+            f.launch((grid, 1, 1), (threads, 1, 1), prm)
+        return launches

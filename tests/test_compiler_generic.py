@@ -332,3 +332,23 @@ def test_mfma_kernel_compiles_for_every_operand_layout(shim_built, layouts, shap
     assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", notes).group(1)) == 0
     assert int(re.search(r"\.vgpr_count:\s+(\d+)", notes).group(1)) <= 256
     assert int(re.search(r"\.group_segment_fixed_size:\s+(\d+)", notes).group(1)) == {"s": 65536, "l": 131072}[shape]
+
+
+def test_tile_and_parts_of_a_product_stay_within_their_limits():
+    """``emit_gemm.choose`` over sizes from 1 on: every part holds at least four steps, a split launch is one round of
+    resident workgroups, its partials stay under their bound, and tiles that are half padding are not taken."""
+    from loopfuse_amd.compiler import emit_gemm
+
+    sizes = [1, 17, 64, 129, 257, 700, 2048, 8191, 65536]
+    for M in sizes:
+        for N in sizes:
+            for K in (1, 64, 65, 1000, 16384, 300000):
+                for batch in (1, 33):
+                    shape, parts = emit_gemm.choose(M, N, K, batch)
+                    bm, bn = emit_gemm.tile_extent(shape)
+                    tiles = -(-M // bm) * -(-N // bn) * batch
+                    steps = -(-K // emit_gemm.BK)
+                    assert 1 <= parts <= 32 and (parts == 1 or steps // parts >= 4)
+                    if parts > 1:
+                        assert tiles * parts <= 512 and parts * tiles * bm * bn <= 1 << 26
+                    assert shape in "sd" or M > bm // 2

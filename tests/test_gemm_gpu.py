@@ -221,6 +221,28 @@ def test_random_products_on_mfma(chunk, monkeypatch):
         _close(got, want, dtype)
 
 
+@pytest.mark.parametrize("dtype", [BF, HF])
+@pytest.mark.parametrize("tile,parts,M,N,K", [("d", 1, 130, 136, 200), ("d", 3, 17, 264, 8 * 125), ("d", 5, 256, 128, 64 * 5),
+                                              ("m", 1, 257, 128, 192), ("m", 4, 300, 392, 64 * 9 + 8), ("m", 2, 255, 40, 128),
+                                              ("s", 7, 31, 520, 64 * 13), ("l", 3, 300, 264, 64 * 8 + 8), ("l", 32, 40, 24, 2048)])
+def test_split_products_and_tile_shapes(tile, parts, M, N, K, dtype, monkeypatch):
+    """The tile shapes with three and four stages, and products whose k is split: more parts than an even division has,
+    a last part shorter than the others, k that ends inside a step, rows and columns past the last tile, fewer steps than
+    stages, a batch, an odd N (results one at a time).  Same bound as the unsplit products; a call of a known signature
+    (which replays its launches with a new workspace) gives the same bits."""
+    monkeypatch.setenv("LOOPFUSE_GEMM_TILE", tile)
+    monkeypatch.setenv("LOOPFUSE_GEMM_PARTS", str(parts))
+    for n, batch in ((N, ()), (N + 1, (2,))):
+        a, b, c = rand(batch + (M, K), dtype, 1, 0.5).to(DEV), rand(batch + (n, K), dtype, 2, 0.5).to(DEV), rand((n,), dtype, 3).to(DEV)
+        run = _compiled(lambda a, b, c: torch.tanh((a @ b.transpose(-1, -2)) * 0.125 + c))
+        before = dict(generic.counters)
+        got = run(a, b, c)
+        assert generic.counters["mfma"] == before["mfma"] + 1 and generic.counters["plain"] == before["plain"]
+        want = torch.tanh(torch.matmul(a.double().cpu(), b.double().cpu().transpose(-1, -2)) * 0.125 + c.double().cpu())
+        _close(got, want, dtype)
+        assert torch.equal(run(a, b, c), got)
+
+
 def test_softmax_times_matrix_at_the_reference_size():
     """``softmax(x) @ y`` with x [4, 8, 1024, 64], y [4, 8, 64, 1024] in bf16 (reference tests/test_accuracy.py:197-211,
     its own size): 2^31 multiply-adds, which the plain kernels are not allowed.  The row maxima and sums are plain
