@@ -430,7 +430,7 @@ def tuned_attention(q, k, v, plan: AttnPlan, k_table=None, v_table=None, **kw):
     of a shape class each candidate is timed on the call's own tensors (HIP events, a few
     launches), the winner is remembered in the process and in ``autotune.json`` beside
     the code-object cache.  Used by the backend under ``mode="max-autotune"``."""
-    if kw.get("score_bias") is not None or kw.get("out_bias") is not None or kw.get("record_visits") \
+    if kw.get("score_bias") is not None or kw.get("score_mask") is not None or kw.get("out_bias") is not None or kw.get("record_visits") \
             or kw.get("force_family") or kw.get("num_splits") or kw.get("choice") or plan.denom_add != 0.0 or kw.get("q2") is not None:
         return attention(q, k, v, plan, k_table, v_table, **kw)
     _load_tuned()
@@ -534,7 +534,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
               score_bias: Optional[torch.Tensor] = None, out_bias: Optional[torch.Tensor] = None,
               choice: Optional[dict] = None, merge_splits: bool = True,
               q2: Optional[torch.Tensor] = None, k2: Optional[torch.Tensor] = None,
-              static_scratch: bool = False, lse: Optional[torch.Tensor] = None):
+              static_scratch: bool = False, lse: Optional[torch.Tensor] = None,
+              score_mask: Optional[torch.Tensor] = None, mask_keep: bool = True):
     """Run fused attention on the GPU.
 
     q : [B, Hq, Sq, D];  k, v : [B, Hkv, Sk, D], or page pools [N, P, Hkv, D]
@@ -543,6 +544,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     scaled / capped scores before the mask, ``out_bias`` (broadcastable to
     [B, Hq, Sq, D]) to the result -- the reference's "modified attention" graph
     (tests/test_accuracy.py:172-196).  Both are served by ``lf_attn_prefill`` only.
+    ``score_mask`` (torch.bool, broadcastable to [B, Hq, Sq, Sk]; not together with ``score_bias``) stands for the score
+    bias that is 0 where a key is visible -- True, or False with ``mask_keep=False`` -- and -inf elsewhere.
     ``q2`` [B, Hq, Sq, D2] and ``k2`` [B, H2, Sk, D2] (H2 divides Hq; D2 in 16, 32, 64) add a
     second product to the scores, ``Q K^T + Q2 K2^T`` before the scale -- the two-part scores
     of multi-head latent attention (reference tests/test_attention.py:126-151); served by
@@ -580,7 +583,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             raise UnsupportedPlan(f"head dim {D} not supported (64 and 128; up to 128 by padding for dense operands)")
         grow = lambda t: None if t is None else torch.nn.functional.pad(t, (0, Dp - D))
         res = attention(grow(q), grow(k), grow(v), plan, None, None, record_visits=record_visits, score_bias=score_bias,
-                        out_bias=grow(out_bias), force_family=force_family, num_splits=num_splits, v_tr=v_tr,
+                        score_mask=score_mask, mask_keep=mask_keep, out_bias=grow(out_bias), force_family=force_family, num_splits=num_splits, v_tr=v_tr,
                         choice=choice, merge_splits=merge_splits)
         o_p, vis = res if record_visits else (res, None)
         if out is None:
@@ -601,7 +604,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     _check_tensor("K", k, dtype)
     _check_tensor("V", v, dtype)
     for name, t in (("K", k), ("V", v), ("K page table", k_table), ("V page table", v_table), ("score bias", score_bias),
-                    ("output bias", out_bias), ("Q2", q2), ("K2", k2), ("O", out)):
+                    ("score mask", score_mask), ("output bias", out_bias), ("Q2", q2), ("K2", k2), ("O", out)):
         if t is not None and t.device != q.device:
             raise RuntimeError(f"loopfuse_amd: {name} is on {t.device}, Q on {q.device}")
 
@@ -720,6 +723,31 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         P.bias = score_bias.data_ptr()
         P.bias_sb, P.bias_sh, P.bias_sq = score_bias.stride(0), score_bias.stride(1), score_bias.stride(2)
         bias_bits |= 1
+    mask_own = None        # the mask without the dims it is shared over, while its bias buffer is not written yet
+    if score_mask is not None:
+        if score_bias is not None:
+            raise UnsupportedPlan("a score mask and a score bias")
+        if score_mask.dtype != torch.bool:
+            raise UnsupportedPlan("the score mask must be a boolean tensor")
+        try:
+            score_mask = score_mask.expand(B, Hq, Sq, Sk)
+        except RuntimeError:
+            raise UnsupportedPlan(f"score mask does not broadcast to [{B}, {Hq}, {Sq}, {Sk}]")
+        mask_own = score_mask[tuple(slice(0, 1) if st == 0 else slice(None) for st in score_mask.stride()[:3])]
+        mask_buf = torch.empty((*mask_own.shape[:3], (Sk + 7) // 8 * 8), dtype=dtype, device=q.device)[..., :Sk]
+        score_bias = mask_buf.expand(B, Hq, Sq, Sk)
+        P.bias = mask_buf.data_ptr()
+        P.bias_sb, P.bias_sh, P.bias_sq = score_bias.stride(0), score_bias.stride(1), score_bias.stride(2)
+        bias_bits |= 1
+
+    def write_mask_bias():
+        """The whole bias of a boolean mask, for the kernels that read every element of it."""
+        nonlocal mask_own
+        if mask_own is not None:
+            shown, hidden = 0.0, float("-inf")
+            mask_buf.fill_(hidden if mask_keep else shown).masked_fill_(mask_own, shown if mask_keep else hidden)
+            mask_own = None
+
     if out_bias is not None:
         out_bias = bias_layout(out_bias, "output bias", D)
         P.obias = out_bias.data_ptr()
@@ -752,7 +780,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         # a caller that wants the row log-sum-exp (a forward that a backward will follow) gets the
         # prefill kernel, which writes it; the decode kernels do not
         family = "decode" if (mask == MASK_NONE and few and Sk >= 16 and lse is None) else "prefill"
-    keep = (q, k, v, out, kt, vt, score_bias, out_bias, q2, k2)  # noqa: F841  (tensors stay alive until the launch is queued)
+    keep = (q, k, v, out, kt, vt, score_bias, score_mask, out_bias, q2, k2)  # noqa: F841  (tensors stay alive until the launch is queued)
 
     if family == "prefill" and not bias_bits and plan.denom_add == 0.0 and not d2:
         family = {"swp": "prefill_swp", "w32": "prefill"}.get(choice.get("prefill"), None) or prefill_variant(Sq, v_tr)
@@ -804,6 +832,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             pack = 4 if group % 4 == 0 else 2
         if family == "prefill_swp" and bias_bits and not bias_tiles:
             family = "prefill"                          # swp was refused above (spans): the register-staged kernel
+        if family != "prefill_swp" or (mask_own is not None and mask_own.stride(3) != 1):
+            write_mask_bias()
         spec = KernelSpec(family, _DTYPE_CODE[dtype], D, mask, plan.softcap is not None, paged,
                           page_size, table_i64, v_tr=v_tr if family == "prefill" else True, bias=bias_bits,
                           denom=plan.denom_add != 0.0, d2=d2, page_size_v=page_size_v, pack=pack, extra=extra,
@@ -843,8 +873,14 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             table = torch.empty((nb_ * nh_ * nqt * nkt,), dtype=torch.int32, device=q.device)
             keep += (table,)
             P.part_acc = table.data_ptr()
-            get_kernel(spec, "lf_bias_classify").launch((nqt, nb_ * nh_, (nkt + 3) // 4), (256, 1, 1), P)
-            names.insert(0, "lf_bias_classify")
+            classify = "lf_bias_classify"
+            if mask_own is not None:
+                # classes straight from the mask's bytes, the bias only where the attention kernel reads it
+                classify = "lf_mask_tiles"
+                P.obias, P.rows = mask_own.data_ptr(), int(mask_keep)
+                P.ob_sb, P.ob_sh, P.ob_sq = (st if n > 1 else 0 for n, st in zip(mask_own.shape, mask_own.stride()[:3]))
+            get_kernel(spec, classify).launch((nqt, nb_ * nh_, (nkt + 3) // 4), (256, 1, 1), P)
+            names.insert(0, classify)
         get_kernel(spec, spec.entry()).launch((grid, 1, 1), (64 * nw, 1, 1), P)
         _last_launch.set({"kernels": names, "grid": grid, "block": 64 * nw, "q_tile_rows": bm, "kv_tile_rows": bn,
                                  "heads_per_workgroup": spec.pack or 1})
@@ -856,6 +892,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         raise UnsupportedPlan("the decode kernels do not write the row log-sum-exp")
     if mask != MASK_NONE:
         raise UnsupportedPlan("the decode kernel takes no mask")
+    write_mask_bias()
     # query rows of one unit: the group's heads (Sq == 1) or the Sq rows (group == 1)
     if Sq == 1:
         rows = group

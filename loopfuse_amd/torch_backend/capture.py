@@ -293,18 +293,18 @@ class AttentionMatch:
             t = t.clone(memory_format=torch.contiguous_format)
         return t, None
 
-    def _bias_view(self, bo: Optional[BiasOperand], vals, shape, dtype=None):
+    def _bias_view(self, bo: Optional[BiasOperand], vals, shape, as_mask=False):
+        """The [B, Hq, Sq, X] view of a bias; a boolean mask as the float32 term 0 / -inf it stands for, or as it is
+        (``as_mask``: the kernels take its bytes for that term, tiles that are all -inf are never walked)."""
         if bo is None:
             return None
         t = vals[bo.index]
         if bo.keep:
-            # a boolean mask written with masked_fill / where: the kernels take it as the additive
-            # term 0 / -inf (of the mask's own, possibly broadcast, shape; tiles that are all -inf
-            # are never walked)
+            # written with masked_fill / where, or given to torch's fused attention op
             if t.dtype != torch.bool:
                 raise lowering.UnsupportedPlan("the mask is not the boolean tensor seen at trace time")
-            t = torch.zeros(t.shape, dtype=dtype or torch.float32, device=t.device).masked_fill_(
-                t if bo.keep < 0 else ~t, float("-inf"))
+            if not as_mask:
+                t = torch.zeros(t.shape, dtype=torch.float32, device=t.device).masked_fill_(t if bo.keep < 0 else ~t, float("-inf"))
         # ("merged", k) / ("inner", k): batch and heads share source dim k ([B*H, ..], what baddbmm takes)
         def stride_of(d):
             if d is None:
@@ -364,8 +364,12 @@ class AttentionMatch:
         B, Hq, Sq, Sk, D = self._shapes(vals)
         run = lowering.tuned_attention if self.tune else lowering.attention
         given = {"out": self.empty_out(vals, q.dtype, q.device)} if self.out_order else {}
+        added = self._bias_view(self.bias, vals, (B, Hq, Sq, Sk), as_mask=True)
+        if added is not None and self.bias.keep:
+            given.update(score_mask=added, mask_keep=self.bias.keep > 0)
+        else:
+            given["score_bias"] = added
         out = run(q, k, v, self.plan_for(vals), kt, vt, **given,
-                                 score_bias=self._bias_view(self.bias, vals, (B, Hq, Sq, Sk), q.dtype),
                                  out_bias=self._bias_view(self.out_bias, vals, (B, Hq, Sq, D)),
                                  **self._second_product(vals))
         if self.out_rank == 3:
@@ -874,6 +878,36 @@ def _match_attention(gm: torch.fx.GraphModule) -> list:
                     return dataclasses.replace(st, mask="sliding", window=int(lo_hi[1]) + 1)
         return dataclasses.replace(st, bias=(ids, st.shape), bias_keep=keep)
 
+    def boolean_of(node, ids):
+        """(ids, +1 / -1) of the boolean tensor behind a 0 / -inf term that torch made of it for one of its fused
+        attention ops -- ``where(mask, 0, -inf)``, or a slice that cuts off the columns added to pad its rows --
+        or None.  A stand-in element of the term is the mask's element of the same place."""
+        same = lambda x, y: [str(d) for d in x] == [str(d) for d in y]
+        size = lambda n: n.meta["val"].shape if isinstance(n, torch.fx.Node) and isinstance(n.meta.get("val"), torch.Tensor) else None
+        while isinstance(node, torch.fx.Node) and node.target is aten.expand.default:
+            node = node.args[0]
+        src = node
+        if ids.src.kind != "node" or ids.src.node is not src:
+            return None
+        if node.target is aten.slice.Tensor and len(node.args) in (3, 4) and not node.kwargs \
+                and node.args[1] in (-1, len(size(node)) - 1) and node.args[2] in (0, None):
+            pad = node.args[0]
+            if not (isinstance(pad, torch.fx.Node) and pad.target is aten.constant_pad_nd.default and len(pad.args[1]) == 2
+                    and pad.args[1][0] == 0 and size(pad.args[0]) is not None and same(size(pad.args[0]), size(node))):
+                return None
+            node = pad.args[0]
+        if not (isinstance(node, torch.fx.Node) and node.target is aten.where.self and len(node.args) == 3):
+            return None
+        cond, x, y = node.args
+        is_zero = lambda n: (is_number(n) and n == 0) or (isinstance(n, Scalar) and n.expr == ("lit", 0.0))
+        x, y = arg(x), arg(y)
+        keep = 1 if is_zero(x) and is_neg_inf(y) else (-1 if is_neg_inf(x) and is_zero(y) else 0)
+        given = env.get(cond)
+        if not keep or not isinstance(given, Ids) or not is_bool(given) or size(cond) is None or not same(size(cond), size(node)) \
+                or tuple(given.t.shape) != tuple(ids.src.shape):
+            return None
+        return Ids(given.src, given.t.reshape(-1)[ids.t]), keep
+
     def meta_view(target, shape, args, kwargs):
         m = torch.empty(shape, device="meta")
         return tuple(target(m, *args, **kwargs).shape)
@@ -939,10 +973,17 @@ def _match_attention(gm: torch.fx.GraphModule) -> list:
             raise _Skip("fused attention op: scale not understood")
         sq, sk = qi.t.shape[-2], ki.t.shape[-2]
         # a mask tensor reaches the op as an additive term in the query's dtype (torch turns
-        # boolean masks into 0 / -inf before it dispatches): the kernels' score bias
+        # boolean masks into 0 / -inf before it dispatches): the kernels' score bias, or the boolean itself
+        keep = 0
+        if bias is not None:
+            raw = dict(zip(names, node.args))
+            raw.update(node.kwargs)
+            found = boolean_of(raw.get("attn_mask") if raw.get("attn_mask") is not None else raw.get("attn_bias"), bias)
+            if found is not None:
+                bias, keep = found
         return Stage("out", tuple(qi.t.shape[:-1]) + (vi.t.shape[-1],), qi, Ids(ki.src, ki.t.transpose(-1, -2)), vi,
                      factors=[scale], mask="causal" if given.get("is_causal", False) else None, mat=(sq, sk),
-                     bias=None if bias is None else (bias, tuple(qi.t.shape[:-1]) + (sk,)), zero_blind_rows=True)
+                     bias=None if bias is None else (bias, tuple(qi.t.shape[:-1]) + (sk,)), bias_keep=keep, zero_blind_rows=True)
 
     def pattern_step(node, tgt, a, kw, first):
         """The abstract value of ``node`` if it continues a pattern; raises _Skip otherwise."""

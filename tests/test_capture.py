@@ -426,6 +426,28 @@ def test_rewritten_graphs_compute_the_same(which, monkeypatch):
         torch.testing.assert_close(g, w, rtol=2e-4, atol=2e-4)
 
 
+@pytest.mark.parametrize("S,dynamic,keep", [(40, False, 1), (41, False, 1), (41, True, 1), (40, True, -1)])
+def test_the_boolean_behind_a_fused_ops_mask_is_found(S, dynamic, keep, monkeypatch):
+    """F.scaled_dot_product_attention's boolean mask reaches the graph as where(mask, 0, -inf), with padded rows where
+    the length is odd or dynamic: the fused call takes the boolean; a term with another fill stays what it is."""
+    import torch.nn.functional as F
+    monkeypatch.setattr(capture.AttentionMatch, "run", _oracle_run)
+    q, k, v = (torch.randn(2, 3, S, 64, generator=torch.Generator().manual_seed(s)) for s in range(3))
+    m = torch.rand(2, 1, S, S, generator=torch.Generator().manual_seed(5)) > 0.3
+    m[..., 0] = keep > 0
+    for fill in (float("-inf"), -3.0):
+        def fn(q, k, v, m):
+            if fill == -3.0 or keep < 0:
+                m = torch.where(m, 0.0, fill) if keep > 0 else torch.where(m, fill, 0.0)
+            return F.scaled_dot_product_attention(q, k, v, attn_mask=m)
+
+        torch._dynamo.reset()
+        got = torch.compile(fn, backend=loopfuse_amd.loopfuse_backend, dynamic=dynamic)(q, k, v, m)
+        (match,) = interface.last_matches
+        assert match.bias.keep == (keep if fill == float("-inf") else 0)
+        torch.testing.assert_close(got, fn(q, k, v, m), rtol=2e-4, atol=2e-4)
+
+
 @pytest.mark.parametrize("which", ["buffer_eq_zero", "tril_in_graph", "arange_where", "where_full_like",
                                    "where_masked_first", "key_padding", "band_not_causal"])
 def test_boolean_masks_written_by_hand_are_fused(which, monkeypatch):

@@ -1096,6 +1096,61 @@ def test_bias_tile_classes(i, monkeypatch):
     assert (other[~blind] - gotc[~blind]).abs().max().item() <= TOL[dt] if (~blind).any() else True
 
 
+@pytest.mark.parametrize("Sq,Sk,mshape,group,keep,strided", [
+    (128, 64, "b1qk", 1, True, False),       # one block
+    (300, 333, "b1qk", 1, True, False),      # odd rows: byte loads, last key block of 13 keys
+    (300, 336, "b1qk", 1, False, False),     # 16-byte loads, last key block of 16 keys, True = masked
+    (515, 1104, "bhqk", 1, True, False),     # a mask per head
+    (515, 1104, "11qk", 4, True, False),     # 32-row q tiles (packed heads)
+    (300, 401, "b1qk", 2, False, False),     # 64-row q tiles, byte loads
+    (200, 640, "b11k", 1, True, False),      # one row for all queries
+    (200, 639, "111k", 4, True, False),      # ... shared by the whole batch, byte loads
+    (300, 320, "b1qk", 1, True, True),       # rows of a wider buffer that start off 16-byte borders
+    (17, 4, "b1qk", 1, True, False),         # the smallest
+])
+def test_boolean_masks_equal_the_bias_they_stand_for(Sq, Sk, mshape, group, keep, strided):
+    """lf_mask_tiles: classes and mixed blocks from the bytes of a boolean mask.  Walked tiles and results are bit for
+    bit those of the 0 / -inf bias through lf_bias_classify."""
+    g = torch.Generator().manual_seed(Sq + Sk)
+    B, H, D = 2, 4, 64
+    q, k, v = (rand((B, h, n, D), torch.bfloat16, s).to(dev()) for h, n, s in ((H, Sq, 1), (H // group, Sk, 2), (H // group, Sk, 3)))
+    shape = tuple({"b": B, "h": H, "q": Sq, "k": Sk, "1": 1}[x] for x in mshape)
+    i, j = torch.arange(shape[2])[:, None], torch.arange(Sk)[None, :]
+    shown = ((j <= i + Sk // 3) & (j >= i - 150)).expand(shape).clone()
+    shown[..., Sk // 2: Sk // 2 + 70] &= torch.rand((*shape[:3], 1), generator=g) < 0.5
+    if shape[0] > 1:
+        shown[1, ..., Sk - Sk // 5:] = False                       # padding at the end of the second sequence
+    shown[..., 0] = True
+    bias = torch.zeros(shape).masked_fill(~shown, float("-inf")).to(torch.bfloat16).to(dev())
+    mask = (shown if keep else ~shown).to(dev())
+    if strided:
+        wide = torch.zeros((*shape[:3], Sk + 9), dtype=torch.bool, device=dev())
+        wide[..., 3:3 + Sk] = mask
+        mask = wide[..., 3:3 + Sk]
+    plan = lowering.AttnPlan(scale=D ** -0.5, zero_blind_rows=True)
+    got, walked = lowering.attention(q, k, v, plan, score_mask=mask, mask_keep=keep, record_visits=True)
+    assert lowering.attention.last_launch["kernels"] == ["lf_mask_tiles", "lf_attn_prefill_swp"]
+    want, want_walked = lowering.attention(q, k, v, plan, score_bias=bias, record_visits=True)
+    assert lowering.attention.last_launch["kernels"] == ["lf_bias_classify", "lf_attn_prefill_swp"]
+    assert torch.equal(walked, want_walked) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("case", ["decode", "key_stride", "register_staged"])
+def test_boolean_masks_where_the_whole_bias_is_read(case, monkeypatch):
+    B, H, Sq, Sk, D = 2, 3, 1 if case == "decode" else 130, 700, 64
+    q, k, v = (rand((B, H, n, D), torch.bfloat16, s).to(dev()) for n, s in ((Sq, 1), (Sk, 2), (Sk, 3)))
+    shown = (torch.rand((B, 1, Sq, Sk), generator=torch.Generator().manual_seed(9)) < 0.7).to(dev())
+    bias = torch.zeros(shown.shape, device=dev()).masked_fill(~shown, float("-inf")).to(torch.bfloat16)
+    if case == "key_stride":
+        shown = shown.transpose(2, 3).contiguous().transpose(2, 3)
+    if case == "register_staged":
+        monkeypatch.setenv("LOOPFUSE_BIAS_TILES", "0")
+    plan = lowering.AttnPlan(scale=D ** -0.5)
+    got = lowering.attention(q, k, v, plan, score_mask=shown)
+    assert "lf_mask_tiles" not in lowering.attention.last_launch["kernels"]
+    assert torch.equal(got, lowering.attention(q, k, v, plan, score_bias=bias))
+
+
 @pytest.mark.parametrize("per_head", [False, True])
 @pytest.mark.parametrize("group", [2, 4])
 def test_bias_tiles_with_grouped_query_heads(group, per_head):
