@@ -78,8 +78,8 @@ struct LfDecIds {            // page ids of one step
 };
 
 #ifndef LF_COOP
-#define LF_COOP 0            /* 1 (with LF_HEADWAVE, K and V paged, pages of a multiple of 16 tokens, token-major
-                                pools): the workgroup loads each 16-token step of its LF_DW heads as ONE
+#define LF_COOP 0            /* 1 (with LF_HEADWAVE, K and V in pages of one size, token-major pools, a token row of at
+                                least 1 KB over the LF_DW heads): the workgroup loads each 16-token step of its LF_DW heads as ONE
                                 contiguous block (16 token rows x LF_DW heads x D), every load instruction 1 KB
                                 of consecutive bytes, and hands the rows to the waves through LDS.  Reading
                                 the same bytes head by head -- 256-byte pieces 2 KB apart per wave -- costs
@@ -87,8 +87,8 @@ struct LfDecIds {            // page ids of one step
 #endif
 
 #if LF_COOP
-#if !LF_HEADWAVE || LF_PAGED != 3 || LF_BIAS || (LF_PAGE_SIZE % 16) || (LF_PAGE_SIZE_V % 16)
-#error "LF_COOP needs LF_HEADWAVE, paged K and V with pages of a multiple of 16 tokens, and no score bias"
+#if !LF_HEADWAVE || LF_PAGED != 3 || LF_BIAS || LF_PAGE_SIZE != LF_PAGE_SIZE_V || LF_DW * LF_D < 512
+#error "LF_COOP needs LF_HEADWAVE, K and V in pages of one size, no score bias, and whole waves per token row"
 #endif
 
 struct LfCoopStage {
@@ -96,6 +96,9 @@ struct LfCoopStage {
   lf_u32x4 v[LF_NJ];
 };
 
+// Bound: HBM.  B64 Hq32 S2048 D128 bf16, 1 ... 4-token pages: 8 kv heads 106 -> 88 us (6.1 TB/s with the combine
+// launch), 4 kv heads 60 -> 48 us; before, four waves shared a head and fetched 64-byte quarters of 256-byte rows.
+//
 // Split decode step, cooperative loads.  Layout of the work as in the kernel below with
 // LF_HEADWAVE: grid = (B * Hkv/LF_DW, nsplit), wave w owns kv head LF_DW*hc + w and writes its
 // own result or partial.  What differs is the way K and V reach the waves:
@@ -107,7 +110,7 @@ struct LfCoopStage {
 //   LDS -> MFMA         : S^T = K Q^T with ds_read_b128 (row = token, 32 d per k-step) on the
 //                         16x16x32 MFMA; O^T += V^T P^T with transposed 8-byte reads on the
 //                         16x16x16 MFMA, whose k extent is the 16 tokens of a step
-extern "C" __global__ void __launch_bounds__(LF_DT, 1) lf_attn_decode(const LfAttnParams p) {
+extern "C" __global__ void __launch_bounds__(LF_DT, 8 / LF_DW) lf_attn_decode(const LfAttnParams p) {
   constexpr int kRowB = LF_DW * LF_D * 2;            // bytes of one token row over the workgroup's heads
   constexpr int kPieces = kRowB / 16;                // 16-byte pieces per row
   constexpr int kKStride = kRowB + 16;               // LDS row strides
@@ -164,19 +167,26 @@ extern "C" __global__ void __launch_bounds__(LF_DT, 1) lf_attn_decode(const LfAt
   float l_part = 0.0f;         // this lane's share of the sum
 
   // ---- loads: piece u of this thread is piece tid + LF_DT*u of the step's block
-  // Page ids: one register holds the ids of 32 steps (lane l: step l % 32 of the chunk, K for
-  // l < 32, V for l >= 32), issue() picks its pair with v_readlane.  The next chunk's register
-  // is loaded 32 steps ahead.  So the loop's only vector memory operations are the K/V loads:
+  // Page ids: one register holds the ids of kChunk steps (K in lanes 0 .. 31, V in lanes 32 .. 63), issue()
+  // picks its ids with v_readlane.  A step of 16 tokens lies inside one page, or (short pages) has a page of its
+  // own for each of the kIds token rows this wave loads pieces of: rows row_w + kRowStep * u.  The next chunk's
+  // register is loaded one chunk ahead.  So the loop's only vector memory operations are the K/V loads:
   // these complete in order, and a table load consumed between them would make the wave wait
   // for every load in flight.
+  constexpr int kIds = LF_PAGE_SIZE % 16 == 0 ? 1 : LF_NJ;
+  constexpr int kChunk = 32 / kIds;
+  constexpr int kRowStep = LF_DT / kPieces;
+  const int row_w = __builtin_amdgcn_readfirstlane(tid / kPieces);
   auto load_ids = [&](int st0) -> lf_table_t {
-    const int tok = min(tok_begin + 16 * (st0 + (lane & 31)), p.Sk - 1);   // steps past the end: the last page (never issued)
+    const int l = lane & 31;
+    const int row = kIds == 1 ? 0 : row_w + kRowStep * (l % kIds);
+    const int tok = min(tok_begin + 16 * (st0 + l / kIds) + row, p.Sk - 1);   // steps past the end: the last page (never issued)
     return lane < 32 ? reinterpret_cast<const lf_table_t*>(p.k_table)[(long long)b * p.kt_stride + tok / LF_PAGE_SIZE]
                      : reinterpret_cast<const lf_table_t*>(p.v_table)[(long long)b * p.vt_stride + tok / LF_PAGE_SIZE_V];
   };
-  lf_table_t ids_cur = load_ids(0), ids_nxt = load_ids(32);
-  auto id_of = [&](int st, int which) -> long long {
-    const int l = (st & 31) + 32 * which;
+  lf_table_t ids_cur = load_ids(0), ids_nxt = load_ids(kChunk);
+  auto id_of = [&](int st, int u, int which) -> long long {
+    const int l = (st % kChunk) * kIds + u + 32 * which;
 #if LF_TABLE_I64
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(ids_cur & 0xffffffffll), l);
     const int hi = __builtin_amdgcn_readlane((int)(ids_cur >> 32), l);
@@ -185,17 +195,20 @@ extern "C" __global__ void __launch_bounds__(LF_DT, 1) lf_attn_decode(const LfAt
     return (long long)__builtin_amdgcn_readlane(ids_cur, l);
 #endif
   };
-  auto issue = [&](LfCoopStage& sg, int st) {
-    if ((st & 31) == 0 && st > 0) {       // next chunk of ids (workgroup-uniform)
+  // Chunks start at multiples of 4 steps, which stage s0 holds: only its refill (`first`) looks for a new one, so that the
+  // compiler sees four steps of K/V loads between the load of a chunk and its use and does not wait for those in flight.
+  auto issue = [&](LfCoopStage& sg, int st, bool first) {
+    if (first && st % kChunk == 0 && st > 0) {       // next chunk of ids (workgroup-uniform)
       ids_cur = ids_nxt;
-      ids_nxt = load_ids(st + 32);
+      ids_nxt = load_ids(st + kChunk);
     }
-    const long long idk = id_of(st, 0), idv = id_of(st, 1);
     const int tok0 = tok_begin + 16 * st;
 #pragma unroll
     for (int u = 0; u < LF_NJ; ++u) {
+      const long long idk = id_of(st, kIds == 1 ? 0 : u, 0), idv = id_of(st, kIds == 1 ? 0 : u, 1);
       const int piece = tid + LF_DT * u;
-      const int tk = min(tok0 + piece / kPieces, p.Sk - 1);  // rows past Sk: clamped, masked later
+      const int row = row_w + kRowStep * u;                  // the same for the whole wave: scalar addresses
+      const int tk = min(tok0 + row, p.Sk - 1);              // rows past Sk: clamped, masked later
       const int within = 8 * (piece % kPieces);              // elements
       // every byte is read once, whole lines at a time: streaming (non-temporal) loads
       sg.k[u] = __builtin_nontemporal_load(reinterpret_cast<const lf_u32x4*>(
@@ -278,7 +291,7 @@ extern "C" __global__ void __launch_bounds__(LF_DT, 1) lf_attn_decode(const LfAt
 #define LF_COOP_STEP(sg, st, refill)                                         \
     {                                                                        \
       to_lds(sg, (st) & 1);                                                  \
-      if (refill) issue(sg, (st) + 4);                                       \
+      if (refill) issue(sg, (st) + 4, &(sg) == &s0);                         \
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");        \
       consume((st) & 1, (st));                                               \
     }
@@ -287,10 +300,10 @@ extern "C" __global__ void __launch_bounds__(LF_DT, 1) lf_attn_decode(const LfAt
     // path, as if the stage being written were the last one loaded (i.e. for everything).
     int st = 0;
     if (nsteps >= 8) {
-      issue(s0, 0);
-      issue(s1, 1);
-      issue(s2, 2);
-      issue(s3, 3);
+      issue(s0, 0, false);
+      issue(s1, 1, false);
+      issue(s2, 2, false);
+      issue(s3, 3, false);
       do {
         LF_COOP_STEP(s0, st, true)
         LF_COOP_STEP(s1, st + 1, true)
@@ -299,10 +312,10 @@ extern "C" __global__ void __launch_bounds__(LF_DT, 1) lf_attn_decode(const LfAt
         st += 4;
       } while (st + 8 <= nsteps);
     } else {
-      if (0 < nsteps) issue(s0, 0);
-      if (1 < nsteps) issue(s1, 1);
-      if (2 < nsteps) issue(s2, 2);
-      if (3 < nsteps) issue(s3, 3);
+      if (0 < nsteps) issue(s0, 0, false);
+      if (1 < nsteps) issue(s1, 1, false);
+      if (2 < nsteps) issue(s2, 2, false);
+      if (3 < nsteps) issue(s3, 3, false);
     }
     for (; st < nsteps; st += 4) {
       if (st < nsteps) LF_COOP_STEP(s0, st, st + 4 < nsteps)

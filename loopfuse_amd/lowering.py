@@ -320,6 +320,26 @@ def decode_split(units: int, Sk: int, cus: int = 256, per_cu: int = 2) -> int:
     return max(1, min(want, most))
 
 
+def decode_coop_split(units: int, Sk: int, rows: int, cus: int = 256) -> int:
+    """KV splits of a decode step with cooperative loads (``units`` workgroups per split).  One workgroup per CU streams at
+    the card's rate and fewer at their own (48 / 96 / 144 / 192 / 240 workgroups: 2.2 / 4.1 / 5.7 / 6.6 / 6.3 TB/s), more
+    than one per CU add a round (320 instead of 200 of 4 waves: 57 against 45 us), a split costs its pipeline's fill and the
+    partial results of its rows: the count with the smallest sum, with at least 160 tokens per split (40 sequences of
+    1000 tokens in one-token pages, 8 heads: 6 splits 35 us, 3 splits 44 us)."""
+    env = os.environ.get("LOOPFUSE_DECODE_SPLITS")
+    if env:
+        return max(1, int(env))
+
+    def cost(n):
+        size = (-(-Sk // n) + 31) // 32 * 32
+        full, rest = divmod(units * -(-Sk // size), cus)
+        return (size + 64 + (4 * rows if n > 1 else 0)) * (full + (max(0.6, 0.1 + 0.9 * rest / cus) if rest else 0.0))
+
+    # one round of all CUs, of three quarters of them, two rounds, or no split
+    most = max(1, min(64, Sk // 160))
+    return min({max(1, min(most, n)) for n in (1, cus // units, 3 * cus // (4 * units), 2 * cus // units)}, key=cost)
+
+
 def _decode_headwave(paged: int, page_size: int, Hkv: int, D: int, P: "AttnParams", units_hw: int = 1 << 30,
                      Sk: int = 1 << 30, cus: int = 256) -> bool:
     """One kv head per wave pays when K and V are paged, token-major (head stride D,
@@ -334,20 +354,20 @@ def _decode_headwave(paged: int, page_size: int, Hkv: int, D: int, P: "AttnParam
             and units_hw * max(1, min(8, Sk // 512)) >= cus)
 
 
-def _decode_coop(headwave: bool, page_size: int, page_size_v: int, bias_bits: int, Hkv: int, waves: int,
-                 P: "AttnParams", D: int) -> bool:
-    """With one kv head per wave the workgroup reads every 16-token block of its 8 heads as one
-    contiguous piece and hands the rows to the waves through LDS (``-DLF_COOP=1``) when a block
-    lies inside a page (pages of a multiple of 16 tokens) and there is no score bias to carry
-    along: a wave that fetches its own head reads 256-byte pieces 2 KB apart, which costs about a
-    tenth of the HBM rate.  LOOPFUSE_DECODE_COOP=0 keeps the per-wave loads."""
-    if os.environ.get("LOOPFUSE_DECODE_COOP", "1") != "1":
-        return False
-    # the block loads take a token's 8 heads as one run of 8 * D elements: the pool must hold the heads of a
-    # token side by side (a permuted [pages, Hkv, page, D] pool view goes to the per-wave loads, which follow
-    # the head stride)
-    token_major = P.k_sh == D and P.v_sh == D and P.k_ss >= Hkv * D and P.v_ss >= Hkv * D
-    return headwave and page_size % 16 == 0 and not page_size_v and not bias_bits and Hkv % waves == 0 and token_major
+def _decode_coop_waves(paged: int, page_size: int, page_size_v: int, bias_bits: int, Hkv: int, P: "AttnParams", D: int) -> int:
+    """Waves of a workgroup that reads every 16-token block of its heads as one contiguous piece per token, one kv head
+    per wave, and hands the rows to the waves through LDS (``-DLF_COOP=1``): 8, 4 (Hkv a multiple of 4 only), or 0 where
+    that form does not serve the call -- pools of different page sizes, a score bias to carry along, heads of a token
+    not side by side (a permuted [pages, Hkv, page, D] pool view goes to the per-wave loads, which follow the head
+    stride), or less than 1 KB per token row, where a wave would need the page ids of several tokens per load (and
+    where it gains nothing with longer pages: 4 heads of 64, 34 against 28 us).  A wave that fetches its own head reads 256-byte pieces 2 KB apart, which costs
+    about a tenth of the HBM rate.  LOOPFUSE_DECODE_COOP=0 keeps the per-wave loads."""
+    if os.environ.get("LOOPFUSE_DECODE_COOP", "1") != "1" or paged != 3 or page_size_v or bias_bits:
+        return 0
+    if P.k_sh != D or P.v_sh != D or (page_size > 1 and (P.k_ss < Hkv * D or P.v_ss < Hkv * D)):
+        return 0
+    waves = 8 if Hkv % 8 == 0 else (4 if Hkv % 4 == 0 else 0)
+    return 0 if waves * D < 512 else waves
 
 
 def _decode_rowload(paged: int, page_size: int, page_size_v: int, bias_bits: int) -> bool:
@@ -911,20 +931,32 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     waves = int(os.environ.get("LOOPFUSE_DECODE_WAVES", "4"))
     # Token-major page pools ([pages, page, Hkv, D]: the heads of a token side by side)
     # are read whole-page-wise when the 8 waves of a workgroup take 8 consecutive heads.
+    coop = _decode_coop_waves(paged, page_size, page_size_v, bias_bits, Hkv, P, D)
     headwave = _decode_headwave(paged, page_size, Hkv, D, P, B * ((Hkv + 7) // 8) * chunks, Sk) and not page_size_v
     if "head_per_wave" in choice:
-        headwave = bool(choice["head_per_wave"]) and paged == 3 and Hkv % 8 == 0
+        headwave = bool(choice["head_per_wave"]) and paged == 3 and (Hkv % 8 == 0 or coop > 0)
+    elif coop and os.environ.get("LOOPFUSE_DECODE_HEADWAVE") is None:
+        # whole token rows pay once there are about as many workgroups as CUs, below that the four waves of a workgroup
+        # share one head.  Pages of 16 tokens and more, where those read whole pages too: at up to 8 splits of 512 tokens
+        # (28 sequences of 4096 tokens, 8 heads, D 128: 79 against 84 us; 16 of 2048 32 against 29).  Shorter pages: at
+        # up to 32 splits of 160 tokens (16 of 8192: 90 against 111 us; 8 of 8192 54 against 58; 8 of 4096 37 against 33)
+        most = min(8, Sk // 512) if page_size % 16 == 0 else min(32, Sk // 160)
+        headwave = B * (Hkv // coop) * chunks * max(1, most) >= 224
+    coop = coop if headwave else 0
     if headwave:
-        waves = 8
+        waves = coop or 8
         units = B * ((Hkv + waves - 1) // waves) * chunks
     num_splits = num_splits or choice.get("splits")
-    nsplit = num_splits if num_splits else decode_split(units, Sk, per_cu=1 if headwave else 2)
+    if not num_splits:
+        num_splits = decode_coop_split(units, Sk, min(rows, DECODE_QROWS)) if coop else \
+            decode_split(units, Sk, per_cu=1 if headwave else 2)
+    nsplit = num_splits
     split_len = ((Sk + nsplit - 1) // nsplit + 31) // 32 * 32     # whole pairs of 16-token steps
     nsplit = (Sk + split_len - 1) // split_len
     P.rows, P.nsplit, P.split_len = rows, nsplit, split_len
     spec = KernelSpec("decode", _DTYPE_CODE[dtype], D, MASK_NONE, plan.softcap is not None, paged,
                       page_size, table_i64, rows=DECODE_QROWS, waves=waves, headwave=headwave, page_size_v=page_size_v,
-                      coop=(coop := _decode_coop(headwave, page_size, page_size_v, bias_bits, Hkv, waves, P, D)),
+                      coop=coop > 0,
                       rowload=not coop and _decode_rowload(paged, page_size, page_size_v, bias_bits),
                       bias=bias_bits, safe=plan.zero_blind_rows and bool(bias_bits),
                       extra=tuple(os.environ.get("LOOPFUSE_KOPTS", "").split()))

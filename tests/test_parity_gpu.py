@@ -515,6 +515,36 @@ def test_mixed_page_sizes(pk, pv):
     check(rand((B, Hq, S, D), torch.bfloat16, 4), kp, vp, mask="causal", k_table=kt, v_table=vt)
 
 
+@pytest.mark.parametrize("B,Hkv,group,Sk,D,page,i64,dt,cap", [
+    (64, 4, 8, 700, 128, 1, False, torch.bfloat16, None),      # 4 waves, last step of 12 tokens
+    (40, 4, 2, 1024, 128, 4, True, torch.float16, None),       # several tokens per page, 64-bit ids
+    (56, 4, 1, 2064, 128, 16, False, torch.bfloat16, None),    # 4 waves, whole blocks per page
+    (40, 8, 4, 1001, 128, 1, True, torch.bfloat16, 30.0),      # 8 waves, odd length
+    (48, 16, 1, 808, 64, 8, False, torch.float16, None),       # one wave per token row
+    (16, 8, 20, 2300, 128, 2, False, torch.bfloat16, None),    # two row chunks, splits that cross the id chunks
+])
+def test_decode_with_cooperative_loads_of_short_pages(B, Hkv, group, Sk, D, page, i64, dt, cap):
+    """-DLF_COOP=1 where a 16-token step spans several pages, and with 4 waves: equal to the oracle and, by error, no
+    further from it than the kernel whose waves share a head; splits of every length down to less than a trip."""
+    n = Sk // page
+    g = torch.Generator().manual_seed(Sk)
+    q = rand((B, Hkv * group, 1, D), dt, 1)
+    pool = (B * n, Hkv, D) if page == 1 else (B * n, page, Hkv, D)
+    k, v = rand(pool, dt, 2), rand(pool, dt, 3)
+    table = torch.randperm(B * n, generator=g).view(B, n).to(torch.int64 if i64 else torch.int32)
+    plan = lowering.AttnPlan(scale=D ** -0.5, softcap=cap, k_paged=True, v_paged=True)
+    rows = [x[table.long()].reshape(B, n * page, Hkv, D).transpose(1, 2) for x in (k, v)]
+    want = O.attention_reference(q, *rows, softcap=cap)
+    on = [t.to(dev()) for t in (q, k, v, table)]
+    got = lowering.attention(*on[:3], plan, on[3], on[3])
+    assert lowering.attention.last_launch["cooperative_loads"]
+    assert lowering.attention.last_launch["block"] == (512 if Hkv % 8 == 0 else 256)
+    for splits in (None, 1, 3, 7, 16):
+        got = lowering.attention(*on[:3], plan, on[3], on[3], choice={"head_per_wave": True, **({"splits": splits} if splits else {})})
+        assert lowering.attention.last_launch["cooperative_loads"]
+        assert (got.float().cpu() - want).abs().max().item() <= TOL[dt], splits
+
+
 def test_decode_head_major_pool_keeps_per_wave_loads():
     """A page pool whose storage is [pages, Hkv, page, D] (viewed as [pages, page, Hkv, D]): the cooperative
     block loads assume the heads of a token side by side, so even when one head per wave is asked for the
