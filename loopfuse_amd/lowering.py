@@ -39,6 +39,18 @@ _DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1}
 COMMON_OPTS = ("-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops")
 
 
+_ENVIRON = os.environ._data if os.name == "posix" and isinstance(getattr(os.environ, "_data", None), dict) else None
+
+
+def _env(name: str, default=None):
+    """``os.environ.get``, without the exception that raises and catches for each variable that is not set: 0.6 us, half a
+    dozen times per call of ``attention``."""
+    if _ENVIRON is not None and name.encode() not in _ENVIRON:
+        return default
+    return os.environ.get(name, default)
+
+
+
 class AttnParams(ctypes.Structure):
     """Mirror of ``struct LfAttnParams`` in csrc/kernels/lf_common.hip.h."""
 
@@ -185,7 +197,7 @@ def compile_spec(spec: KernelSpec, arch: str = runtime.DEFAULT_ARCH) -> Compiled
     # two threads asking for the same one both compile, the results are identical)
     code, hit, log = runtime.compile_source(spec.source(), spec.name(), spec.options(), arch)
     ck = CompiledKernel(spec, code, hit, log)
-    record = os.environ.get("LOOPFUSE_RECORD_SPECS")
+    record = _env("LOOPFUSE_RECORD_SPECS")
     with _lock:
         if record and spec not in _compiled:
             # one JSON line per specialisation a workload asked for: specs_from_file() reads
@@ -290,8 +302,6 @@ def _get_scratch(device: torch.device, nfloats: int) -> torch.Tensor:
     return t
 
 
-
-
 def xcd_slots(units: int, tiles: int) -> int:
     """Grid of a kernel that maps its workgroups with ``lf_slot_of_block`` (csrc/kernels/lf_prefill_blocks.hip.h):
     8 XCDs x the slots of one, with the units cut into as many parts as that function chooses."""
@@ -309,7 +319,7 @@ def decode_split(units: int, Sk: int, cus: int = 256, per_cu: int = 2) -> int:
     in flight: two workgroups of 4 waves, or one of 8); below that the KV range is
     split, down to 512 tokens per split and up to 64 splits, and a second kernel merges
     the partial results."""
-    env = os.environ.get("LOOPFUSE_DECODE_SPLITS")
+    env = _env("LOOPFUSE_DECODE_SPLITS")
     if env:
         return max(1, int(env))
     want = max(1, (per_cu * cus + units - 1) // units)
@@ -326,7 +336,7 @@ def decode_coop_split(units: int, Sk: int, rows: int, cus: int = 256) -> int:
     than one per CU add a round (320 instead of 200 of 4 waves: 57 against 45 us), a split costs its pipeline's fill and the
     partial results of its rows: the count with the smallest sum, with at least 160 tokens per split (40 sequences of
     1000 tokens in one-token pages, 8 heads: 6 splits 35 us, 3 splits 44 us)."""
-    env = os.environ.get("LOOPFUSE_DECODE_SPLITS")
+    env = _env("LOOPFUSE_DECODE_SPLITS")
     if env:
         return max(1, int(env))
 
@@ -346,7 +356,7 @@ def _decode_headwave(paged: int, page_size: int, Hkv: int, D: int, P: "AttnParam
     token stride Hkv*D), there are at least 8 heads to fill the 8 waves, and the
     (batch, head-chunk) units times at most 8 KV splits of >= 256 tokens still give one
     workgroup per CU (measured: below that, 4 waves per head with more splits win)."""
-    env = os.environ.get("LOOPFUSE_DECODE_HEADWAVE")
+    env = _env("LOOPFUSE_DECODE_HEADWAVE")
     if env is not None:
         return env == "1"
     return (paged == 3 and Hkv % 8 == 0 and P.k_sh == D and P.v_sh == D
@@ -362,7 +372,7 @@ def _decode_coop_waves(paged: int, page_size: int, page_size_v: int, bias_bits: 
     stride), or less than 1 KB per token row, where a wave would need the page ids of several tokens per load (and
     where it gains nothing with longer pages: 4 heads of 64, 34 against 28 us).  A wave that fetches its own head reads 256-byte pieces 2 KB apart, which costs
     about a tenth of the HBM rate.  LOOPFUSE_DECODE_COOP=0 keeps the per-wave loads."""
-    if os.environ.get("LOOPFUSE_DECODE_COOP", "1") != "1" or paged != 3 or page_size_v or bias_bits:
+    if paged != 3 or page_size_v or bias_bits or _env("LOOPFUSE_DECODE_COOP", "1") != "1":
         return 0
     if P.k_sh != D or P.v_sh != D or (page_size > 1 and (P.k_ss < Hkv * D or P.v_ss < Hkv * D)):
         return 0
@@ -375,7 +385,7 @@ def _decode_rowload(paged: int, page_size: int, page_size_v: int, bias_bits: int
     non-temporal loads and passes K through a wave-private LDS tile (``-DLF_ROWLOAD=1``) when a
     16-token step lies inside one page (or K/V are dense) and there is no score bias.
     LOOPFUSE_DECODE_ROWLOAD=0 keeps the loads in MFMA operand layout."""
-    if os.environ.get("LOOPFUSE_DECODE_ROWLOAD", "1") != "1" or bias_bits:
+    if _env("LOOPFUSE_DECODE_ROWLOAD", "1") != "1" or bias_bits:
         return False
     return not paged or (page_size % 16 == 0 and (page_size_v or page_size) % 16 == 0)
 
@@ -396,7 +406,7 @@ def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, w
     ``LOOPFUSE_BN`` override the default."""
     if bias_bits:
         return 0
-    want = (choice or {}).get("bn", os.environ.get("LOOPFUSE_BN"))
+    want = (choice or {}).get("bn", _env("LOOPFUSE_BN"))
     if want is not None:
         return 32 if int(want) == 32 else 0
     return 32 if D == 128 and workgroups >= (3 * 256 if 0 < window <= 512 else 8 * 256) else 0
@@ -407,7 +417,7 @@ def prefill_variant(Sq: int, v_tr: bool = True) -> str:
     with direct-to-LDS staging (``prefill_swp``; dense K/V only, ``attention`` falls
     back to ``prefill`` for paged operands).  LOOPFUSE_PREFILL=w32 selects the
     register-staged kernel for comparison."""
-    env = os.environ.get("LOOPFUSE_PREFILL", "swp")
+    env = _env("LOOPFUSE_PREFILL", "swp")
     if not v_tr or env == "w32":
         return "prefill"
     return "prefill_swp"
@@ -648,7 +658,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             raise RuntimeError(f"loopfuse_amd: {which} page table is not on the GPU")
         if table.stride(1) != 1:
             table = table.contiguous()
-        if os.environ.get("LOOPFUSE_CHECK_TABLES", "0") == "1" and table.numel():
+        if _env("LOOPFUSE_CHECK_TABLES", "0") == "1" and table.numel():
             # debugging aid (waits for the stream): the kernels trust page ids, an id outside
             # the pool is a read outside the allocation
             lo, hi = int(table.min()), int(table.max())
@@ -721,7 +731,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             raise UnsupportedPlan(f"{what} must be a {dtype} GPU tensor")
         if t.dim() > 4:
             raise UnsupportedPlan(f"{what} has more than 4 dims")
-        if os.environ.get("LOOPFUSE_BIAS_COPY", "1") == "1" and \
+        if _env("LOOPFUSE_BIAS_COPY", "1") == "1" and \
                 t.dim() >= 2 and t.shape[-1] == last and t.stride(-1) == 1 and t.numel() <= (1 << 25) and \
                 (t.data_ptr() % 8 or any(st % 4 for n, st in zip(t.shape[:-1], t.stride()[:-1]) if n > 1)):
             # rows that do not start on 8-byte borders (a mask over an odd number of keys) would
@@ -808,7 +818,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     # classified tile by tile first (lf_bias_classify) -- what a mask given as a tensor needs
     bias_tiles = (family == "prefill" and bias_bits == 1 and plan.denom_add == 0.0 and not d2
                   and lse is None and Sk >= 4 and (Sk + 63) // 64 <= 65535 * 4 and B * Hq <= 65535
-                  and os.environ.get("LOOPFUSE_BIAS_TILES", "1") == "1" and choice.get("prefill") != "w32"
+                  and _env("LOOPFUSE_BIAS_TILES", "1") == "1" and choice.get("prefill") != "w32"
                   and prefill_variant(Sq, v_tr) == "prefill_swp")
     if bias_tiles:
         family = "prefill_swp"
@@ -826,7 +836,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             return ss >= 0 and reach < (1 << 32) and (Sk - 1) * abs(ss) * 2 + 2 * D < (1 << 31)
         if not (swp_ok(k, plan.k_paged, page_size, P.k_ss)
                 and swp_ok(v, plan.v_paged, page_size_v or page_size, P.v_ss)) \
-                or (paged and os.environ.get("LOOPFUSE_PAGED_SWP", "1") != "1"):
+                or (paged and _env("LOOPFUSE_PAGED_SWP", "1") != "1"):
             family = "prefill"
         if plan.k_paged:
             P.k_span = sum((n - 1) * st for n, st in zip(k.shape, k.stride())) + 1
@@ -835,7 +845,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     if family in ("prefill", "prefill_swp"):
         P.q_sb, P.q_sh, P.q_ss = q.stride(0), q.stride(1), q.stride(2)
         P.o_sb, P.o_sh, P.o_ss = out.stride(0), out.stride(1), out.stride(2)
-        extra = tuple(os.environ.get("LOOPFUSE_KOPTS", "").split())
+        extra = tuple(_env("LOOPFUSE_KOPTS", "").split())
         # buffer loads address a (batch, kv head) span with 32-bit byte offsets
         span = max((Sk - 1) * abs(P.k_ss), (Sk - 1) * abs(P.v_ss)) * 2 + 2 * D
         if family == "prefill" and span >= (1 << 31):
@@ -846,7 +856,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         # group over the same query rows and share every K/V tile in LDS
         pack = 0
         if family == "prefill_swp" and group % 2 == 0 and not any(e.startswith("-DLF_NW=") for e in extra) and \
-                choice.get("pack", os.environ.get("LOOPFUSE_GQAPACK", "1") == "1") and (not bias_bits or P.bias_sh == 0):
+                choice.get("pack", _env("LOOPFUSE_GQAPACK", "1") == "1") and (not bias_bits or P.bias_sh == 0):
             # (with a score bias only when all heads share it: the tile classes are then the same for the
             # packed heads of a workgroup)
             pack = 4 if group % 4 == 0 else 2
@@ -928,14 +938,15 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         raise UnsupportedPlan("decode needs Sq == 1 or group == 1")
     chunks = (rows + DECODE_QROWS - 1) // DECODE_QROWS
     units = B * Hkv * chunks
-    waves = int(os.environ.get("LOOPFUSE_DECODE_WAVES", "4"))
+    waves = int(_env("LOOPFUSE_DECODE_WAVES", "4"))
     # Token-major page pools ([pages, page, Hkv, D]: the heads of a token side by side)
     # are read whole-page-wise when the 8 waves of a workgroup take 8 consecutive heads.
     coop = _decode_coop_waves(paged, page_size, page_size_v, bias_bits, Hkv, P, D)
-    headwave = _decode_headwave(paged, page_size, Hkv, D, P, B * ((Hkv + 7) // 8) * chunks, Sk) and not page_size_v
     if "head_per_wave" in choice:
         headwave = bool(choice["head_per_wave"]) and paged == 3 and (Hkv % 8 == 0 or coop > 0)
-    elif coop and os.environ.get("LOOPFUSE_DECODE_HEADWAVE") is None:
+    elif not coop or _env("LOOPFUSE_DECODE_HEADWAVE") is not None:
+        headwave = _decode_headwave(paged, page_size, Hkv, D, P, B * ((Hkv + 7) // 8) * chunks, Sk) and not page_size_v
+    else:
         # whole token rows pay once there are about as many workgroups as CUs, below that the four waves of a workgroup
         # share one head.  Pages of 16 tokens and more, where those read whole pages too: at up to 8 splits of 512 tokens
         # (28 sequences of 4096 tokens, 8 heads, D 128: 79 against 84 us; 16 of 2048 32 against 29).  Shorter pages: at
@@ -959,7 +970,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                       coop=coop > 0,
                       rowload=not coop and _decode_rowload(paged, page_size, page_size_v, bias_bits),
                       bias=bias_bits, safe=plan.zero_blind_rows and bool(bias_bits),
-                      extra=tuple(os.environ.get("LOOPFUSE_KOPTS", "").split()))
+                      extra=tuple(_env("LOOPFUSE_KOPTS", "").split()))
     rows_per_block = 1024 // D       # combine kernel: 256 threads, 4 consecutive d each
     combine_grid = (B * Hkv * rows + rows_per_block - 1) // rows_per_block
     if static_scratch:
