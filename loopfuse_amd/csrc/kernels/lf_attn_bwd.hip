@@ -8,14 +8,13 @@
 // dS picks up the derivative of the cap: dS = scale * (1 - tanh^2) * P * (dP - delta).
 // Three kernels, no atomics, every result written once (deterministic):
 //   lf_attn_bwd_delta : delta[b, h, q]
-//   lf_attn_bwd_dkdv  : a workgroup owns 128 keys of one (batch, kv head) -- 4 waves x 32 keys,
-//                       K^T and V^T of its keys in registers as MFMA B operands -- and walks the
+//   lf_attn_bwd_dkdv  : a workgroup owns 128 or 256 keys of one (batch, kv head) -- 4 waves x 32 or 64
+//                       keys, K^T and V^T of its keys in registers as MFMA B operands -- and walks the
 //                       q tiles (64 rows) of the query heads of the group that can see them
-//   lf_attn_bwd_dq    : a workgroup owns 128 query rows of one (batch, head), Q^T and dO^T in
-//                       registers, and walks the kv tiles (64 keys) as the forward does
-// The tiles that are walked go through LDS in the two layouts of lf_prefill_blocks.hip.h: the
-// K layout (ds_read_b128, rows of the tile = MFMA rows) and the V layout (transposed reads,
-// rows of the tile = MFMA k).  As in the forward, the accumulator of the first product is, as
+//   lf_attn_bwd_dq    : a workgroup owns 128 or 256 query rows of one (batch, head) -- 4 or 8 waves x
+//                       32 rows, Q^T and dO^T in registers -- and walks the kv tiles (64 keys)
+// The tiles that are walked are kept in LDS once and read both ways: along their rows (ds_read_b128,
+// rows of the tile = MFMA rows) and transposed (rows of the tile = MFMA k).  As in the forward, the accumulator of the first product is, as
 // held, the B operand of the second, so P and dS never leave registers.
 // L and the exponent are in log2 units (the forward writes L2 = offset + log2(sum)).
 
@@ -60,9 +59,6 @@ __device__ __forceinline__ bool lf_bw_keep(int t, int window) {
   return (unsigned)t < (unsigned)window;
 #endif
 }
-#ifndef LF_BW_DQ_NT
-#define LF_BW_DQ_NT 512     /* threads of lf_attn_bwd_dq: 8 waves x 32 query rows, two waves per SIMD */
-#endif
 
 // P = 2^(cexp * (S + start)): the row log-sum-exp enters through the start of the accumulators of S = Q K^T.  With a
 // softcap the exponent is not linear in S: there the second half of the scratch holds L itself.
@@ -99,28 +95,6 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT) lf_attn_bwd_delta(const L
   }
 }
 
-// A 64-row tile of a [rows, D] matrix goes global -> LDS directly (buffer_load ... lds, the
-// forward's staging): per pass the workgroup's NT threads move NT / LF_CPR whole rows, a wave
-// 64 lanes x 16 B that land contiguously; the XOR swizzle of the K layout (`tr` false:
-// ds_read_b128, tile rows = MFMA rows) or of the V layout (`tr` true: transposed reads, tile
-// rows = MFMA k) is applied on the global side.  `rs` covers rows 0 .. nrows-1 of the matrix
-// (row stride `rowb` bytes): rows past the end get an offset beyond it and arrive as zeros.
-// Not tracked by the compiler's wait counters: callers wait with s_waitcnt vmcnt(0).
-template <int NT>
-__device__ __forceinline__ unsigned lf_bw_dma_lane_off(unsigned rowb, bool tr, int tid) {
-  // byte offset of this lane's 16 bytes in the first pass of a tile that starts at row 0; the
-  // swizzles repeat every 16 rows and a pass is a multiple of 16 rows, so every pass adds rows only
-  const int srow = tid / LF_CPR, sch = tid % LF_CPR;
-  return (unsigned)srow * rowb + 16u * (unsigned)(tr ? lf_v_phys(srow, sch) : lf_k_phys(srow, sch));
-}
-template <int NT>
-__device__ __forceinline__ void lf_bw_dma_piece(const lf_u32x4& rs, unsigned rowb, int row0, lf_elem* tile,
-                                                unsigned lane_off, int ps, int wave) {
-  constexpr int kRowsPerPass = NT / LF_CPR, kRowsPerWave = 64 / LF_CPR;
-  static_assert(kRowsPerPass % 16 == 0, "a pass must keep the swizzle phase");
-  const unsigned off = (unsigned)(row0 + kRowsPerPass * ps) * rowb + lane_off;
-  lf_dma_to_lds(rs, off, &tile[(kRowsPerPass * ps + kRowsPerWave * wave) * LF_D]);
-}
 // wait for this wave's direct loads and LDS writes, then meet the other waves.  The wait is the
 // builtin, not inline asm, so that the compiler's wait-counter pass sees that nothing is
 // outstanding afterwards: otherwise it waits again inside the step -- for the operands loaded
@@ -134,15 +108,8 @@ __device__ __forceinline__ void lf_bw_dma_piece(const lf_u32x4& rs, unsigned row
     asm volatile("" ::: "memory");           \
   } while (0)
 
-// Fragment read-ahead of the two product loops (LDS reads in flight ahead of the MFMA that
-// consumes them; the order of reads and MFMAs is pinned with scheduling barriers, left to
-// itself the compiler issues read, wait, MFMA one after the other)
-#define LF_BW_PF1 3      /* first products: pairs of K-layout fragments */
-#define LF_BW_PF2 4      /* second products: V-layout fragments */
-#define LF_BW_DQ_PF1 2   /* lf_attn_bwd_dq, first products: 3 do not fit its 256 registers */
-
-// MFMAs of lf_attn_bwd_dkdv with the register file of every operand spelled out.  At one wave per
-// SIMD the kernel has 512 registers per lane, and the compiler then gives every MFMA an AGPR
+// MFMAs of both product kernels with the register file of every operand spelled out.  At one wave per
+// SIMD a kernel has 512 registers per lane, and the compiler then gives every MFMA an AGPR
 // destination while keeping what it computes with in VGPRs: left to it, the loop carries hundreds
 // of v_accvgpr moves per step.  Here dK^T / dV^T (written in the loop, read after it) and the
 // loop-invariant K^T / V^T operands live in AGPRs, S^T / dP^T (read by the VALU right away) in VGPRs.
@@ -168,37 +135,6 @@ __device__ __forceinline__ void lf_bw_mfma_first(lf_f32x16& c, const lf_u32x4& a
 __device__ __forceinline__ void lf_bw_mfma_vva(lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b) {
   asm volatile(LF_BW_MFMA " %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(b));
 }
-// c (AGPRs) += a (VGPRs) x b (VGPRs)
-__device__ __forceinline__ void lf_bw_mfma_avv(lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b) {
-  asm volatile(LF_BW_MFMA " %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-
-// lf_attn_bwd_dq in its 8-wave form runs two waves per SIMD on 256 registers: the compiler then uses
-// no AGPRs and its own MFMAs are as good; the 4-wave form has 512 and gets the explicit ones
-#if LF_BW_DQ_NT == 256
-#define LF_BW_DQ_ASM 1
-#else
-#define LF_BW_DQ_ASM 0
-#endif
-__device__ __forceinline__ void lf_bw_dq_mfma_s(lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b, bool first) {
-#if LF_BW_DQ_ASM
-  if (first) lf_bw_mfma_first(c, a, b); else lf_bw_mfma_vva(c, a, b);
-#else
-  if (first) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) c[i] = 0.0f;
-  }
-  c = lf_mfma32(__builtin_bit_cast(lf_elem8, a), __builtin_bit_cast(lf_elem8, b), c);
-#endif
-}
-__device__ __forceinline__ void lf_bw_dq_mfma_acc(lf_f32x16& c, const lf_u32x4& a, const lf_u32x4& b) {
-#if LF_BW_DQ_ASM
-  lf_bw_mfma_avv(c, a, b);
-#else
-  c = lf_mfma32(__builtin_bit_cast(lf_elem8, a), __builtin_bit_cast(lf_elem8, b), c);
-#endif
-}
-
 // accumulators X^T[d][n] (lane n = lane % 32; element i of block db is d = 32*db + 8*(i/4) + 4*g + i%4)
 // -> rows n of a [rows, D] matrix, 16 bytes per store (the exchange of the forward's epilogue)
 __device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, lf_elem* row_ptr, bool valid, int g) {
@@ -276,15 +212,16 @@ __device__ __forceinline__ lf_u32x4 lf_bw_read_tr(unsigned base, int disp, int k
   }
   return a;
 }
-// One direct load of a tile (256 threads: kRows whole rows per load of the workgroup): row row0 + srow + kRows * ps of
+// One direct load of a tile (NT threads: kRows whole rows per load of the workgroup): row row0 + srow + kRows * ps of
 // the matrix behind `rs`; rows past its end arrive as zeros.  `lane_off` = lf_bw_load_off.
 __device__ __forceinline__ unsigned lf_bw_load_off(unsigned rowb, int tid) {
   const int srow = tid / LF_CPR, sch = tid % LF_CPR;       // a load is a multiple of 16 rows: the swizzle repeats
   return (unsigned)srow * rowb + 16u * (unsigned)(sch ^ lf_bw_swz(srow));
 }
+template <int NT>
 __device__ __forceinline__ void lf_bw_load_rows(const lf_u32x4& rs, unsigned rowb, int row0, unsigned tile, unsigned lane_off,
                                                 int ps, int wave) {
-  constexpr int kRows = LF_BW_NT / LF_CPR, kRowsPerWave = 64 / LF_CPR;
+  constexpr int kRows = NT / LF_CPR, kRowsPerWave = 64 / LF_CPR;
   static_assert(kRows % 16 == 0, "a load must keep the swizzle phase");
   lf_dma_to_lds_at(rs, (unsigned)(row0 + kRows * ps) * rowb + lane_off,
                    tile + (unsigned)((kRows * ps + kRowsPerWave * wave) * LF_BW_ROWB));
@@ -310,7 +247,7 @@ __device__ __forceinline__ void lf_bw_mfma_zero(lf_f32x16& c, const lf_u32x4& a,
   asm volatile(LF_BW_MFMA " %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
 }
 
-// c (AGPRs) += a x b (VGPRs), with the accumulator handed over as an input: lf_attn_bwd_dkdv keeps up to all 256 AGPRs in
+// c (AGPRs) += a x b (VGPRs), with the accumulator handed over as an input: the kernels keep up to all of their AGPRs in
 // use from its first to its last instruction, and accumulators that the compiler sees change in the loop leave its
 // register allocator without a free tuple to resolve a control-flow merge with -- it spills a thousand registers.  So
 // it sees 16 values that are defined once, used throughout and defined anew by the drain behind the loop; they stay in
@@ -460,8 +397,8 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   };
   const unsigned stat0 = lf_lds_addr(stats);
   auto issue = [&](int st, int j) {      // load j of kLoads
-    if (j < kPasses) lf_bw_load_rows(q_rs, q_rowb, ld_q0, q_tile(st), q_loff, j, wave);
-    else lf_bw_load_rows(g_rs, g_rowb, ld_q0, g_tile(st), g_loff, j - kPasses, wave);
+    if (j < kPasses) lf_bw_load_rows<LF_BW_NT>(q_rs, q_rowb, ld_q0, q_tile(st), q_loff, j, wave);
+    else lf_bw_load_rows<LF_BW_NT>(g_rs, g_rowb, ld_q0, g_tile(st), g_loff, j - kPasses, wave);
     if (j == kLoads - 1 && wave < 2)
       lf_dma_dword_to_lds_at(stat_rs, (unsigned)(ld_q0 + lane) * 4u, stat0 + (unsigned)((2 * st + wave) * 256));
   };
@@ -727,9 +664,29 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   }
 }
 
+#ifndef LF_BW_DQ_NT
+#define LF_BW_DQ_NT 512  /* threads of lf_attn_bwd_dq, 32 query rows per wave */
+#endif
+#define LF_BW_DQ_PF 4    /* fragments read ahead of the MFMAs that take them */
+
+// dQ of LF_BW_DQ_NT / 2 query rows of one (batch, head), 32 per wave.
+// A wave walks blocks of 32 keys, two per 64-key tile, as lf_attn_bwd_dkdv walks blocks of queries: fragments through one
+// read-ahead ring, three LDS stages, one barrier in the middle of a step.  Per block:
+//   S^T = K Q^T
+//   dP^T = V dO^T                    P between these MFMAs
+//   dQ^T += K^T dS^T of the block before (it has no other product to hide dS behind); dS of this block between these
+// What bounds it: an LDS fragment read (16 ... 24 cycles of the CU's LDS) per MFMA of a wave and the matrix work, with two
+// waves per SIMD: 512 threads, or 256 with two workgroups per CU where their LDS fits (head dimension 64).  A wave's 256
+// registers are dQ^T, Q^T and dO^T in 128 AGPRs and S^T, dP^T, two dS^T, fragments and addresses in 118 VGPRs.  Two row
+// blocks per wave, half the LDS reads with one wave per SIMD, are slower (causal bf16 B4 H32 S2048 D128: 246 us): then
+// nothing fills the gaps of a wave's own stream.  Against the form before (a copy of the K tile per read pattern, two
+// stages, dS in front of its product; 4 waves per CU under a window or a softcap), us:
+//   causal B4 H32 S2048 D128 223 -> 222, B2 32/8 S4096 378 -> 373, B2 16/8 S777 35 -> 25, B1 32/8 S2048 85 -> 71
+//   the same with a softcap 383 -> 275; window 256 B4 32/8 S2048 151 -> 107, window 1024 259 -> 179
+//   causal B8 16/4 S1000 D64 fp16 47 -> 42, B16 32/8 S300 48 -> 32
 extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_attn_bwd_dq(const LfAttnBwdParams p) {
-  // two stages of: K tile in both layouts, V tile in the K layout
-  __shared__ __attribute__((aligned(16))) lf_elem tiles[2][3][64 * LF_D];
+  constexpr int kBM = LF_BW_DQ_NT / 2;                           // query rows of a workgroup
+  __shared__ __attribute__((aligned(256))) lf_elem tiles[3][2][64 * LF_D];        // K, V
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -737,7 +694,6 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
-  constexpr int kBM = LF_BW_DQ_NT / 2;                    // query rows of a workgroup
   const int nqt = (p.Sq + kBM - 1) / kBM;
   // As in lf_attn_bwd_dkdv: the q tiles of all query heads of a (batch, kv head) share its K / V tiles in one
   // XCD's L2, the long q tiles first.
@@ -749,12 +705,12 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
   const int b = bhkv / p.Hkv;
   const int h = hkv * (p.Hq / p.Hkv) + row % (p.Hq / p.Hkv);
   const int q0 = kBM * qt;
-  const int wq0 = q0 + 32 * wave;
-  const int my_q = wq0 + l32;
-  const int qr = min(my_q, p.Sq - 1);
+  const int wq0 = q0 + 32 * wave;                    // first row of this wave
   const int nkt = (p.Sk + 63) / 64;
 
+  // Q^T and dO^T of this lane's rows as B operands (d = 16*ks + 8*g .. +7)
   lf_u32x4 qf[LF_NKS], gf[LF_NKS];
+  const int my_q = wq0 + l32, qr = min(my_q, p.Sq - 1);
   {
     const lf_elem* qrow = p.q + (long long)b * p.q_sb + (long long)h * p.q_sh + (long long)qr * p.q_ss;
     const lf_elem* grow = p.dout + (long long)b * p.do_sb + (long long)h * p.do_sh + (long long)qr * p.do_ss;
@@ -763,10 +719,8 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
       qf[ks] = *reinterpret_cast<const lf_u32x4*>(qrow + 16 * ks + 8 * g);
       gf[ks] = *reinterpret_cast<const lf_u32x4*>(grow + 16 * ks + 8 * g);
     }
-#if LF_BW_DQ_ASM
 #pragma unroll
     for (int ks = 0; ks < LF_NKS; ++ks) asm volatile("" : "+a"(qf[ks]), "+a"(gf[ks]));
-#endif
   }
   const long long ridx = ((long long)b * p.Hq + h) * p.Sq + qr;
   const float lse_q = my_q < p.Sq ? p.lse[ridx] : __builtin_inff();
@@ -783,9 +737,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
   for (int db = 0; db < LF_NDB; ++db) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[db][i] = 0.0f;
-#if LF_BW_DQ_ASM
     asm volatile("" : "+a"(dq[db]));
-#endif
   }
 
   int kt_begin = 0, kt_end = nkt;
@@ -800,158 +752,215 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
 #endif
     (void)qlast;
   }
-  const lf_elem* kbase = p.k + (long long)b * p.k_sb + (long long)hkv * p.k_sh;
-  const lf_elem* vbase = p.v + (long long)b * p.v_sb + (long long)hkv * p.v_sh;
-  const lf_u32x4 k_rs = lf_make_buffer(kbase, (unsigned)(((long long)(p.Sk - 1) * p.k_ss + LF_D) * 2));
-  const lf_u32x4 v_rs = lf_make_buffer(vbase, (unsigned)(((long long)(p.Sk - 1) * p.v_ss + LF_D) * 2));
-  // the direct loads of tile kt + 1 go out one by one behind MFMA pairs of the first products of
-  // tile kt (a wave owes 3 * kPasses per tile); past the last tile they go out against an empty
-  // range and fetch nothing
-  constexpr int kPasses = 64 * LF_CPR / LF_BW_DQ_NT;
-  constexpr int kLoads = 3 * kPasses;
-  static_assert(kLoads <= 2 * LF_NKS, "one direct load per pair of MFMAs of the first products");
-  lf_u32x4 k_cur = k_rs, v_cur = v_rs;
-  const unsigned lane_off[3] = {lf_bw_dma_lane_off<LF_BW_DQ_NT>((unsigned)p.k_ss * 2u, false, tid),
-                                lf_bw_dma_lane_off<LF_BW_DQ_NT>((unsigned)p.k_ss * 2u, true, tid),
-                                lf_bw_dma_lane_off<LF_BW_DQ_NT>((unsigned)p.v_ss * 2u, false, tid)};
-  auto issue_piece = [&](int kt, int st, int j) {      // tile j / kPasses (K, K transposed, V), pass j % kPasses
-    const int t = j / kPasses;
-    lf_bw_dma_piece<LF_BW_DQ_NT>(t < 2 ? k_cur : v_cur, (unsigned)(t < 2 ? p.k_ss : p.v_ss) * 2u, 64 * kt, tiles[st][t],
-                                 lane_off[t], j % kPasses, wave);
+  const unsigned k_bytes = (unsigned)(((long long)(p.Sk - 1) * p.k_ss + LF_D) * 2);
+  const unsigned v_bytes = (unsigned)(((long long)(p.Sk - 1) * p.v_ss + LF_D) * 2);
+  lf_u32x4 k_rs = lf_make_buffer(p.k + (long long)b * p.k_sb + (long long)hkv * p.k_sh, k_bytes);
+  lf_u32x4 v_rs = lf_make_buffer(p.v + (long long)b * p.v_sb + (long long)hkv * p.v_sh, v_bytes);
+  const unsigned k_rowb = (unsigned)p.k_ss * 2u, v_rowb = (unsigned)p.v_ss * 2u;
+  const unsigned k_loff = lf_bw_load_off(k_rowb, tid), v_loff = lf_bw_load_off(v_rowb, tid);
+  constexpr int kPasses = 64 * LF_CPR / LF_BW_DQ_NT;      // loads of a wave per tile
+  constexpr int kLoads = 2 * kPasses;
+  const unsigned lds0 = lf_lds_addr(tiles);
+  auto k_tile = [&](int st) { return lds0 + (unsigned)(2 * st * LF_BW_TILEB); };
+  auto v_tile = [&](int st) { return lds0 + (unsigned)((2 * st + 1) * LF_BW_TILEB); };
+  // the tile that is loaded next; past the last one the loads go out against an empty range
+  int ld_kt = kt_begin - 1;
+  auto aim = [&]() {
+    if (++ld_kt >= kt_end) k_rs[2] = v_rs[2] = 0u;
   };
+  auto issue = [&](int st, int j) {      // load j of kLoads
+    if (j < kPasses) lf_bw_load_rows<LF_BW_DQ_NT>(k_rs, k_rowb, 64 * ld_kt, k_tile(st), k_loff, j, wave);
+    else lf_bw_load_rows<LF_BW_DQ_NT>(v_rs, v_rowb, 64 * ld_kt, v_tile(st), v_loff, j - kPasses, wave);
+  };
+
+  unsigned rm_off = lf_bw_rm_off(l32, g), tr_off = lf_bw_tr_off(lane);
+  asm volatile("" : "+v"(rm_off), "+v"(tr_off));
+  constexpr int NS = LF_NKS, NT = 2 * LF_NDB, NF = 2 * NS + NT, PF = LF_BW_DQ_PF;      // fragments of a block
+  static_assert(kLoads <= NS, "a block's loads go out during its first two phases");
+  static_assert(PF <= NS, "the read-ahead of a block's first phase");
+  // dS^T of the first / second block of a tile: B operands of the block after it
+  lf_u32x4 ds[2][2];
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb) ds[kb][0] = ds[kb][1] = lf_u32x4{0u, 0u, 0u, 0u};
+  constexpr unsigned kNone = ~0u;
+  unsigned last = kNone;           // K rows in LDS of the block whose dS waits for its product
+  auto frag_kt = [&](unsigned rows, int j) { return lf_bw_read_tr(rows + tr_off, 0, j / LF_NDB, j % LF_NDB); };
+  // fragment i of block kb of the stage: K rows, V rows
+  auto frag = [&](int st, int kb, int i) {
+    if (i < NS) return lf_bw_read_rm(k_tile(st) + rm_off, 0, kb, i);
+    return lf_bw_read_rm(k_tile(st) + rm_off, LF_BW_TILEB, kb, i - NS);
+  };
+  lf_u32x4 pre[PF];                // the next block's first fragments
+  auto read_ahead = [&](int st, int kb) {
+#pragma unroll
+    for (int f = 0; f < PF; ++f) pre[f] = frag(st, kb, f);
+  };
+  // dQ of the last block before one that has nothing for this wave
+  auto flush = [&](const int kb) {
+    lf_u32x4 fr[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) fr[j] = frag_kt(last, j);
+    asm volatile(LF_BW_VALU_SETTLE : "+v"(ds[kb][0]), "+v"(ds[kb][1]));
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      lf_bw_mfma_hidden(dq[j % LF_NDB], fr[j], ds[kb][j / LF_NDB]);
+    last = kNone;
+  };
+
+  // One block of a wave: 32 keys (kb of stage st, first one k0) x its rows.  `loads`: those of stage `ld` are issued
+  // between the MFMAs; the block read ahead is (st_n, kb_n).
+  auto block = [&](const int kb, int st, int k0, const bool masked, const bool loads, int ld, int st_n, const int kb_n) {
+    lf_u32x4 fr[NF + PF];
+#pragma unroll
+    for (int f = 0; f < PF; ++f) fr[f] = pre[f];
+    lf_f32x16 s, dp;
+    const unsigned own = k_tile(st) + (unsigned)(32 * kb * LF_BW_ROWB);
+    // the first block of a wave adds zeros times its own keys (any other tile may hold no numbers yet)
+    const unsigned before = last != kNone ? last : own;
+    int rel = 0, room = 0;
+    if (masked) {
+      room = p.Sk - k0 - 4 * g;
+      rel = my_q - k0 - 4 * g;            // query minus key of element 0
+      asm volatile("" : "+v"(rel), "+v"(room));      // formed per block: what derives from them is not kept over the loop
+    }
+    // P of elements 4*i4 .. +3 in s (with a cap: times its derivative)
+    auto soft4 = [&](int i4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * i4 + e;
+#if LF_SOFTCAP
+        const float r = __builtin_amdgcn_rcpf(1.0f + lf_exp2(s[i] * sc_exp));     // 1 / (e^(2x) + 1), x = s * scale / cap
+        float pv = lf_exp2((1.0f - 2.0f * r) * cexp - lse_q);
+#else
+        float pv = lf_exp2(s[i] * cexp - lse_q);
+#endif
+        if (masked) {
+          pv = (8 * i4 + e < room && lf_bw_keep(rel - 8 * i4 - e, p.window)) ? pv : 0.0f;
+        }
+#if LF_SOFTCAP
+        s[i] = pv * (4.0f * r * (1.0f - r));             // 1 - tanh^2
+#else
+        s[i] = pv;
+#endif
+      }
+    };
+    auto grad4 = [&](int i4) {      // dS, without the factor `scale`, which multiplies dQ once at the end
+      lf_elem4 dw;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dw[e] = lf_from_float(s[4 * i4 + e] * (dp[4 * i4 + e] - delta_q));
+      const lf_u32x2 du = __builtin_bit_cast(lf_u32x2, dw);
+      ds[kb][i4 / 2][2 * (i4 % 2)] = du[0];
+      ds[kb][i4 / 2][2 * (i4 % 2) + 1] = du[1];
+    };
+    // per fragment: the read that is PF fragments ahead, and a direct load every other time
+    auto ahead = [&](int i) {
+      const int f = i + PF;
+      fr[f] = f < 2 * NS ? frag(st, kb, f) : f < NF ? frag_kt(before, f - 2 * NS) : frag(st_n, kb_n, f - NF);
+    };
+    auto load = [&](int i) {
+      if (loads && i % 2 == 0 && i / 2 < kLoads) issue(ld, i / 2);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // what is carried from block to block may have been moved between registers just now, by the vector ALU
+#pragma unroll
+    for (int f = 0; f < PF; ++f) asm volatile("" : "+v"(fr[f]));
+    asm volatile(LF_BW_VALU_SETTLE : "+v"(fr[0]));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      ahead(i);
+      if (i == 0) lf_bw_mfma_first(s, fr[i], qf[i]);         // S^T[key][q]
+      else lf_bw_mfma_vva(s, fr[i], qf[i]);
+      load(i);
+    }
+#pragma unroll
+    for (int ks = 0; ks < NS; ++ks) {
+      ahead(NS + ks);
+      if (ks == 0) lf_bw_mfma_first(dp, fr[NS + ks], gf[ks]);   // dP^T[key][q]
+      else lf_bw_mfma_vva(dp, fr[NS + ks], gf[ks]);
+      if (ks == 0) asm volatile(LF_BW_MFMA_DRAIN : "+v"(s));
+#pragma unroll
+      for (int t = ks * 4 / NS; t < (ks + 1) * 4 / NS; ++t) soft4(t);
+      load(NS + ks);
+    }
+    asm volatile(LF_BW_VALU_SETTLE : "+v"(ds[kb ^ 1][0]), "+v"(ds[kb ^ 1][1]), "+v"(s));
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      ahead(2 * NS + j);
+      lf_bw_mfma_hidden(dq[j % LF_NDB], fr[2 * NS + j], ds[kb ^ 1][j / LF_NDB]);
+      if (j == 0) {
+        asm volatile(LF_BW_MFMA_DRAIN : "+v"(dp));
+      }
+#pragma unroll
+      for (int t = j * 4 / NT; t < (j + 1) * 4 / NT; ++t) grad4(t);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    last = own;
+#pragma unroll
+    for (int f = 0; f < PF; ++f) pre[f] = fr[NF + f];
+  };
+  // does the wave have a score to keep in keys k .. k + 31, and are all of them kept?
+  auto need = [&](int k) {
+    bool n = wq0 < p.Sq && k < p.Sk;
+#if LF_MASK >= 1
+    n = n && k <= min(wq0 + 32, p.Sq) - 1;
+#endif
+#if LF_MASK == 2
+    n = n && min(k + 32, p.Sk) - 1 >= wq0 - p.window + 1;
+#endif
+    return n;
+  };
+  auto full = [&](int k) {
+    bool n = k + 31 < p.Sk;
+#if LF_MASK >= 1
+    n = n && k + 31 <= wq0;
+#endif
+#if LF_MASK == 2
+    n = n && wq0 + 32 - 1 - k < p.window;
+#endif
+    return n;
+  };
+
   if (kt_begin < kt_end) {
+    aim();
 #pragma unroll
-    for (int j = 0; j < kLoads; ++j) issue_piece(kt_begin, 0, j);
-  }
-  LF_BW_BARRIER();
-  for (int kt = kt_begin; kt < kt_end; ++kt) {
-    const int k0 = 64 * kt;
-    const int st = (kt - kt_begin) & 1;
-    const lf_elem* k_rm = tiles[st][0];
-    const lf_elem* k_tr = tiles[st][1];
-    const lf_elem* v_rm = tiles[st][2];
-    if (kt + 1 >= kt_end) k_cur[2] = v_cur[2] = 0u;   // the other stage is free: every wave left it at the last barrier
-#if !LF_BW_DQ_ASM      // 8 waves: a wave owes few loads and has no registers to spare for their offsets
+    for (int j = 0; j < kLoads; ++j) issue(0, j);
+    aim();
 #pragma unroll
-    for (int j = 0; j < kLoads; ++j) issue_piece(kt + 1, st ^ 1, j);
-#endif
-
-    bool need = wq0 < p.Sq;
-#if LF_MASK >= 1
-    need = need && (k0 <= min(wq0 + 31, p.Sq - 1));
-#endif
-#if LF_MASK == 2
-    need = need && (min(k0 + 64, p.Sk) - 1 >= wq0 - p.window + 1);
-#endif
-    if (need) {
-    // are all 64 x 32 scores of this wave kept?  Then the tile runs without the mask arithmetic
-    bool full = k0 + 63 < p.Sk;
-#if LF_MASK >= 1
-    full = full && (k0 + 63 <= wq0);
-#endif
-#if LF_MASK == 2
-    full = full && (wq0 + 31 - k0 < p.window);
-#endif
-    const bool masked = !full;
-
-    lf_u32x4 dsf[LF_NKK];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      lf_f32x16 s, dp;
-      lf_u32x4 ka[LF_NKS], va[LF_NKS];
-#pragma unroll
-      for (int ks = 0; ks < LF_BW_DQ_PF1; ++ks) {
-        ka[ks] = lf_read_k_frag(k_rm, l32, g, ks * LF_NKB + kb);
-        va[ks] = lf_read_k_frag(v_rm, l32, g, ks * LF_NKB + kb);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < LF_NKS; ++ks) {
-        if (ks + LF_BW_DQ_PF1 < LF_NKS) {
-          ka[ks + LF_BW_DQ_PF1] = lf_read_k_frag(k_rm, l32, g, (ks + LF_BW_DQ_PF1) * LF_NKB + kb);
-          va[ks + LF_BW_DQ_PF1] = lf_read_k_frag(v_rm, l32, g, (ks + LF_BW_DQ_PF1) * LF_NKB + kb);
-        }
-        lf_bw_dq_mfma_s(s, ka[ks], qf[ks], ks == 0);         // S^T[key][q]
-        lf_bw_dq_mfma_s(dp, va[ks], gf[ks], ks == 0);        // dP^T[key][q]
-#if LF_BW_DQ_ASM
-        if (LF_NKS * kb + ks < kLoads) issue_piece(kt + 1, st ^ 1, LF_NKS * kb + ks);
-#endif
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#if LF_BW_DQ_ASM
-      asm volatile(LF_BW_MFMA_DRAIN : "+v"(s), "+v"(dp));
-#endif
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        lf_elem4 dw;
-        float pv[4];
-#if LF_SOFTCAP
-        float dcap[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float r = __builtin_amdgcn_rcpf(1.0f + lf_exp2(s[4 * i4 + e] * sc_exp));
-          pv[e] = lf_exp2((1.0f - 2.0f * r) * cexp - lse_q);
-          dcap[e] = 4.0f * r * (1.0f - r);
-        }
-#else
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pv[e] = lf_exp2(s[4 * i4 + e] * cexp - lse_q);
-#endif
-        if (masked) {           // wave-uniform: most tiles of a q tile lie below the diagonal
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int j = k0 + 32 * kb + 8 * i4 + 4 * g + e;
-            pv[e] = (j < p.Sk && lf_bw_keep(my_q - j, p.window)) ? pv[e] : 0.0f;
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-#if LF_SOFTCAP
-          dw[e] = lf_from_float(pv[e] * (dp[4 * i4 + e] - delta_q) * dcap[e]);
-#else
-          dw[e] = lf_from_float(pv[e] * (dp[4 * i4 + e] - delta_q));   // dS without `scale`
-#endif
-        }
-        const lf_u32x2 du = __builtin_bit_cast(lf_u32x2, dw);
-        dsf[2 * kb + i4 / 2][2 * (i4 % 2)] = du[0];
-        dsf[2 * kb + i4 / 2][2 * (i4 % 2) + 1] = du[1];
-      }
-    }
-    // dQ^T += K^T dS^T (k = the 64 keys of the tile)
-    {
-      constexpr int kNF = LF_NKK * LF_NDB;
-      lf_u32x4 kt2[kNF];
-      // the addresses of the transposed reads are formed again in every step: held across the
-      // first products they do not fit the 256 registers of a wave and end up in scratch memory
-      int lane_r = lane;
-      asm volatile("" : "+v"(lane_r));
-      const int g_r = lane_r >> 5;
-#pragma unroll
-      for (int f = 0; f < LF_BW_PF2; ++f) kt2[f] = __builtin_bit_cast(lf_u32x4, lf_read_v_frag_tr(k_tr, lane_r, g_r, f));
-      __builtin_amdgcn_sched_barrier(0);
-#if LF_BW_DQ_ASM
-#pragma unroll
-      for (int kk = 0; kk < LF_NKK; ++kk) asm volatile(LF_BW_VALU_SETTLE : "+v"(dsf[kk]));
-#endif
-#pragma unroll
-      for (int f = 0; f < kNF; ++f) {
-        if (f + LF_BW_PF2 < kNF) kt2[f + LF_BW_PF2] = __builtin_bit_cast(lf_u32x4, lf_read_v_frag_tr(k_tr, lane_r, g_r, f + LF_BW_PF2));
-        lf_bw_dq_mfma_acc(dq[f % LF_NDB], kt2[f], dsf[f / LF_NDB]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    } else {
-#if LF_BW_DQ_ASM
-#pragma unroll
-      for (int j = 0; j < kLoads; ++j) issue_piece(kt + 1, st ^ 1, j);
-#endif
-    }
+    for (int j = 0; j < kLoads; ++j) issue(1, j);
     LF_BW_BARRIER();
+    read_ahead(0, 0);
+    int st = 0;
+    for (int kt = kt_begin; kt < kt_end; ++kt) {
+      const int k0 = 64 * kt;
+      const int st1 = st == 2 ? 0 : st + 1, st2 = st == 0 ? 2 : st - 1;
+      if (!need(k0)) {
+        if (last != kNone) flush(1);
+        read_ahead(st, 1);
+      } else if (full(k0)) {
+        block(0, st, k0, false, false, 0, st, 1);
+      } else {
+        block(0, st, k0, true, false, 0, st, 1);
+      }
+      LF_BW_BARRIER();            // the next tile has landed; every wave is done with the one before this
+      aim();
+      if (!need(k0 + 32)) {
+        if (last != kNone) flush(0);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) issue(st2, j);
+        read_ahead(st1, 0);
+      } else if (full(k0 + 32)) {
+        block(1, st, k0 + 32, false, true, st2, st1, 0);
+      } else {
+        block(1, st, k0 + 32, true, true, st2, st1, 0);
+      }
+      st = st1;
+    }
+    if (last != kNone) flush(1);
+    __builtin_amdgcn_s_waitcnt(0x0070);      // the last loads, against an empty range, before the LDS is given back
   }
-#if LF_BW_DQ_ASM
 #pragma unroll
   for (int db = 0; db < LF_NDB; ++db) asm volatile(LF_BW_MFMA_DRAIN_LAST : "+a"(dq[db]));
-#endif
 #pragma unroll
   for (int db = 0; db < LF_NDB; ++db)
 #pragma unroll

@@ -1011,12 +1011,18 @@ class AttnBwdParams(ctypes.Structure):
     )
 
 
-def bwd_dq_threads(mask: int, softcap: bool = False) -> int:
-    """Workgroup size of lf_attn_bwd_dq: 8 waves (256 query rows, two waves per SIMD on one K/V
-    tile stream) except under a sliding window, where a 256-row tile walks too many kv tiles
-    that only part of its rows can see, and with a softcap, whose extra values do not fit the
-    256 registers a wave has at two per SIMD."""
-    return 256 if mask == MASK_SLIDING or softcap else 512
+def bwd_dq_threads(D: int, mask: int, softcap: bool, units: int, Sq: int, Sk: int) -> int:
+    """Workgroup size of lf_attn_bwd_dq: 512 (256 query rows, two waves per SIMD on one K/V tile stream) or 256 (128 rows,
+    twice the workgroups).  ``units`` = batch x query heads.  Head dimension 128: a CU's LDS holds one workgroup of either,
+    so the larger one wins once all CUs have work -- more than 128 of them, and more than 256 under a causal mask, where
+    the longest q tile is the launch: 512 against 256 threads, us, causal 64 workgroups 74 / 57, 256 80 / 71, 384 61 / 73,
+    1024 233 / 294; unmasked 64 77 / 59, 192 157 / 218; window 256: 64 25 / 18, 192 28 / 38, 1024 112 / 144.  Head
+    dimension 64: two workgroups of 256 threads fit and balance better (B16 32/8 S300 41 / 32, window 256 B4 H32 S2048
+    71 / 62) except over long sequences, where halving the K/V traffic counts (causal B2 H16 S4096 121 / 133)."""
+    n = units * -(-Sq // 256)
+    if n <= (256 if mask == MASK_CAUSAL else 128) or (D == 64 and (Sk < 4096 or softcap or mask == MASK_SLIDING)):
+        return 256
+    return 512
 
 
 def bwd_key_blocks(D: int, mask: int, softcap: bool, units: int, Sk: int) -> int:
@@ -1035,18 +1041,20 @@ def bwd_key_blocks(D: int, mask: int, softcap: bool, units: int, Sk: int) -> int
     return 2 if n >= 256 and n >= 0.85 * 256 * -(-n // 256) else 1
 
 
-def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False, key_blocks: int = 1) -> KernelSpec:
+def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False, key_blocks: int = 1,
+             dq_threads: int = 512) -> KernelSpec:
     return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap,
-                      extra=(f"-DLF_BW_DQ_NT={bwd_dq_threads(mask, softcap)}", f"-DLF_BW_W={key_blocks}"))
+                      extra=(f"-DLF_BW_DQ_NT={dq_threads}", f"-DLF_BW_W={key_blocks}"))
 
 
 def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
-                       dout: torch.Tensor, plan: AttnPlan, *, key_blocks: Optional[int] = None):
+                       dout: torch.Tensor, plan: AttnPlan, *, key_blocks: Optional[int] = None,
+                       dq_threads: Optional[int] = None):
     """Gradients of ``attention(q, k, v, plan)`` for dense K/V (mask none / causal / sliding, scale,
     softcap; no bias or paging): returns ``(dq, dk, dv)`` in the operands' dtype.  ``o`` and ``lse``
     are the forward's output and row log-sum-exp (``attention(..., lse=...)``).  Three launches
-    (csrc/kernels/lf_attn_bwd.hip): delta = rowsum(dO * O); dK and dV, one workgroup per 128 keys of
-    a (batch, kv head); dQ, one workgroup per 128 query rows.  No atomics: results are
+    (csrc/kernels/lf_attn_bwd.hip): delta = rowsum(dO * O); dK and dV, one workgroup per 128 or 256
+    keys of a (batch, kv head); dQ, one workgroup per 128 or 256 query rows.  No atomics: results are
     reproducible bit for bit."""
     dtype = q.dtype
     if dtype not in _DTYPE_CODE:
@@ -1098,15 +1106,15 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     P.B, P.Hq, P.Hkv, P.Sq, P.Sk, P.window = B, Hq, Hkv, Sq, Sk, window
     P.scale = float(plan.scale)
     P.softcap = softcap if softcap is not None else 0.0
-    spec = bwd_spec(dtype, D, mask, softcap is not None)
-    keys = key_blocks or bwd_key_blocks(D, mask, softcap is not None, B * Hkv, Sk)
-    kv_spec = bwd_spec(dtype, D, mask, softcap is not None, keys)
+    cap = softcap is not None
+    keys = key_blocks or bwd_key_blocks(D, mask, cap, B * Hkv, Sk)
+    nt = dq_threads or bwd_dq_threads(D, mask, cap, B * Hq, Sq, Sk)
+    spec = bwd_spec(dtype, D, mask, cap, keys, nt)
     keep = (q, k, v, o, dout, lse, delta, dq, dk, dv)  # noqa: F841  (tensors stay alive until the launches are queued)
     rows = B * Hq * Sq
     get_kernel(spec, "lf_attn_bwd_delta").launch(((rows + 15) // 16, 1, 1), (256, 1, 1), P)
-    get_kernel(kv_spec, "lf_attn_bwd_dkdv").launch((xcd_slots(B * Hkv, -(-Sk // (128 * keys))), 1, 1), (256, 1, 1), P)
-    nt = bwd_dq_threads(mask, softcap is not None)
-    get_kernel(spec, "lf_attn_bwd_dq").launch((xcd_slots(B * Hkv, (Hq // Hkv) * ((Sq + nt // 2 - 1) // (nt // 2))), 1, 1),
+    get_kernel(spec, "lf_attn_bwd_dkdv").launch((xcd_slots(B * Hkv, -(-Sk // (128 * keys))), 1, 1), (256, 1, 1), P)
+    get_kernel(spec, "lf_attn_bwd_dq").launch((xcd_slots(B * Hkv, (Hq // Hkv) * -(-Sq // (nt // 2))), 1, 1),
                                               (nt, 1, 1), P)
     _last_launch.set({"kernels": ["lf_attn_bwd_delta", "lf_attn_bwd_dkdv", "lf_attn_bwd_dq"]})
     return dq, dk, dv

@@ -355,3 +355,34 @@ def test_key_blocks_per_wave_at_tile_edges(B, Hq, Hkv, Sq, Sk, mask, window, dty
     for name, a, w in zip(("dq", "dk", "dv"), got, want):
         bound = (4e-2 if dtype == torch.bfloat16 else 1e-2) * max(1.0, w.abs().max().item())
         assert (a.double() - w).abs().max().item() <= bound, name
+
+
+@pytest.mark.parametrize("threads", [256, 512])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,mask,window,softcap,dtype", [
+    (1, 2, 2, 1, 1, 128, "causal", 0, None, torch.bfloat16),             # one row, one key
+    (1, 2, 1, 129, 129, 64, "causal", 0, None, torch.float16),           # one row into the second workgroup, one key into the third tile
+    (2, 2, 2, 257, 257, 128, "causal", 0, 30.0, torch.float16),
+    (1, 4, 2, 290, 95, 128, None, 0, None, torch.bfloat16),              # an odd number of 32-key blocks: the last one waits for its product
+    (1, 2, 2, 300, 33, 64, "causal", 0, None, torch.bfloat16),           # more rows than keys
+    (1, 2, 2, 40, 200, 128, "causal", 0, None, torch.float16),           # waves without a row
+    (1, 2, 1, 520, 520, 128, "sliding", 33, None, torch.bfloat16),       # waves that start and end inside the walk
+    (1, 2, 2, 333, 333, 64, "sliding", 1, None, torch.float16),          # a block or two per wave
+])
+def test_dq_workgroup_sizes_at_tile_edges(B, Hq, Hkv, Sq, Sk, D, mask, window, softcap, dtype, threads):
+    g = torch.Generator().manual_seed(Sq + 3 * Sk)
+    q, k, v, dout = (torch.randn(s, generator=g).to(dtype).to(DEV)
+                     for s in ((B, Hq, Sq, D), (B, Hkv, Sk, D), (B, Hkv, Sk, D), (B, Hq, Sq, D)))
+    plan = lowering.AttnPlan(mask=mask, window=window, scale=D ** -0.5, softcap=softcap)
+    lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=DEV)
+    o = lowering.attention(q, k, v, plan, lse=lse)
+    dq, _, _ = lowering.attention_backward(q, k, v, o, lse, dout, plan, dq_threads=threads)
+    want = _ref(q, k, v, dout, mask, window, D ** -0.5, softcap)[2]
+    # as test_backward_matches_autograd: P, dS and the results are rounded once each (2^-9 bf16, 2^-12 fp16)
+    bound = (4e-2 if dtype == torch.bfloat16 else 1e-2) * max(1.0, want.abs().max().item())
+    assert (dq.double() - want).abs().max().item() <= bound
+
+
+@pytest.mark.parametrize("units,Sq,want", [(12, 4096, 256), (24, 4096, 512)])
+def test_dq_workgroup_size_rule(units, Sq, want):
+    assert lowering.bwd_dq_threads(128, lowering.MASK_CAUSAL, False, units, Sq, Sq) == want
+    assert lowering.bwd_dq_threads(64, lowering.MASK_SLIDING, False, units, Sq, Sq) == 256

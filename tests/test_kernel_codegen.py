@@ -172,6 +172,22 @@ def test_hidden_accumulators_stay_in_their_registers(shim_built, dtype, D, mask,
         assert m is None or m.group(1) == m.group(2), ln
 
 
+@pytest.mark.parametrize("threads", [256, 512])
+@pytest.mark.parametrize("dtype,D,mask,softcap", [
+    (torch.bfloat16, 128, lowering.MASK_CAUSAL, False), (torch.float16, 128, lowering.MASK_SLIDING, True),
+    (torch.bfloat16, 128, lowering.MASK_NONE, True), (torch.float16, 64, lowering.MASK_SLIDING, False)])
+def test_hidden_accumulators_of_dq_stay_in_their_registers(shim_built, dtype, D, mask, softcap, threads):
+    lines = _kernels(lowering.bwd_spec(dtype, D, mask, softcap, dq_threads=threads))["lf_attn_bwd_dq"]
+    _check("lf_attn_bwd_dq", lines)
+    _check_settled("lf_attn_bwd_dq", lines)
+    mfma = [i for i, ln in enumerate(lines) if ln.startswith("v_mfma")]
+    for ln in lines[mfma[0]:mfma[-1]]:
+        assert ln.startswith("v_mfma") or not re.search(r"\ba(\d+|\[\d+:\d+\])", ln), ln
+    for ln in lines:
+        m = re.match(r"v_mfma_\S+ (a\[\d+:\d+\]),.*, (\S+)$", ln)
+        assert m is None or m.group(1) == m.group(2), ln
+
+
 def test_the_check_sees_an_unsettled_operand():
     mfma = "v_mfma_f32_32x32x16_bf16 v[16:31], v[0:3], v[4:7], v[16:31]"
     with pytest.raises(AssertionError):
