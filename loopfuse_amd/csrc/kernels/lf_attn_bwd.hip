@@ -28,7 +28,7 @@ struct LfAttnBwdParams {
   lf_elem* dk;
   lf_elem* dv;
   const float* lse;       // [B, Hq, Sq] row log-sum-exp of the scaled, masked scores, log2 units
-  float* delta;           // [2, B, Hq, Sq] scratch: -rowsum(dO * O); what the accumulators of S start at, -L / cexp
+  float* delta;           // [B, Hq, Sq] scratch: -rowsum(dO * O)
   long long q_sb, q_sh, q_ss;      // element strides (d stride 1)
   long long k_sb, k_sh, k_ss;
   long long v_sb, v_sh, v_ss;
@@ -60,16 +60,6 @@ __device__ __forceinline__ bool lf_bw_keep(int t, int window) {
 #endif
 }
 
-// P = 2^(cexp * (S + start)): the row log-sum-exp enters through the start of the accumulators of S = Q K^T.  With a
-// softcap the exponent is not linear in S: there the second half of the scratch holds L itself.
-__device__ __forceinline__ float lf_bw_start_scale(const LfAttnBwdParams& p) {
-#if LF_SOFTCAP
-  return 1.0f;
-#else
-  return -1.0f / (p.scale * LF_LOG2E);
-#endif
-}
-
 // delta[row] = sum_d dO[row][d] * O[row][d]; 16 lanes per row, 8 elements per lane
 extern "C" __global__ void __launch_bounds__(LF_BW_NT) lf_attn_bwd_delta(const LfAttnBwdParams p) {
   const long long row = (long long)blockIdx.x * (LF_BW_NT / 16) + threadIdx.x / 16;
@@ -89,10 +79,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT) lf_attn_bwd_delta(const L
   s += __shfl_xor(s, 2, 64);
   s += __shfl_xor(s, 4, 64);
   s += __shfl_xor(s, 8, 64);
-  if (row < nrows && piece == 0) {
-    p.delta[row] = -s;
-    p.delta[nrows + row] = p.lse[row] * lf_bw_start_scale(p);
-  }
+  if (row < nrows && piece == 0) p.delta[row] = -s;
 }
 
 // wait for this wave's direct loads and LDS writes, then meet the other waves.  The wait is the
@@ -286,7 +273,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   constexpr int KB = LF_BW_W;
   constexpr int kKeys = 128 * KB;
   __shared__ __attribute__((aligned(256))) lf_elem tiles[3][2][64 * LF_D];        // Q, dO
-  __shared__ __attribute__((aligned(16))) float stats[3][2][64];                  // of the 64 rows: start of S, start of dP
+  __shared__ __attribute__((aligned(16))) float stats[3][2][64];                  // of the 64 rows: L, start of dP
 #if LF_BW_VL
   __shared__ lf_u32x4 v_lds[LF_BW_VL][KB][LF_BW_NT];                               // V^T operands that the registers have no room for
 #endif
@@ -374,12 +361,12 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   auto g_tile = [&](int st) { return lds0 + (unsigned)((2 * st + 1) * LF_BW_TILEB); };
 
   // ---- what is loaded next: query head, q tile; past the last step the loads go out against an empty range.  Waves 0
-  // and 1 also bring the row statistics, the start of S and that of dP; those of rows past Sq are zeros: P is 1 there
+  // and 1 also bring the row statistics, L and the start of dP; those of rows past Sq are zeros: P is 1 there
   // and meets dO = 0.
   int ld_step = 0, ld_tile = qt_begin, ld_q0 = 0;
   const lf_elem* ld_q = p.q + (long long)b * p.q_sb + (long long)(hkv * group) * p.q_sh;
   const lf_elem* ld_g = p.dout + (long long)b * p.do_sb + (long long)(hkv * group) * p.do_sh;
-  const float* ld_stat = p.delta + ((wave == 0 ? (long long)p.B * p.Hq : 0ll) + (long long)b * p.Hq + hkv * group) * p.Sq;
+  const float* ld_stat = (wave == 0 ? p.lse : p.delta) + ((long long)b * p.Hq + hkv * group) * p.Sq;
   lf_u32x4 q_rs, g_rs, stat_rs;
   auto aim = [&]() {
     const bool real = ld_step < nsteps;
@@ -413,6 +400,18 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     }
     return r;
   };
+  // P = 2^(cexp * (S + start)), start = -L / cexp: the row log-sum-exp enters through the start of the accumulators of S.
+  // With a softcap the exponent is not linear in S: there L itself is kept.
+#if !LF_SOFTCAP
+  const float start_scale = -1.0f / (p.scale * LF_LOG2E);
+#endif
+  auto to_start = [&](lf_f32x16 r) {
+#if !LF_SOFTCAP
+#pragma unroll
+    for (int i = 0; i < 16; ++i) r[i] *= start_scale;
+#endif
+    return r;
+  };
 
   unsigned rm_off = lf_bw_rm_off(l32, g), tr_off = lf_bw_tr_off(lane);
   asm volatile("" : "+v"(rm_off), "+v"(tr_off));
@@ -433,7 +432,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   auto read_ahead = [&](int st, int qb) {
 #pragma unroll
     for (int f = 0; f < LF_BW_PF; ++f) pre[f] = frag(st, qb, f);
-    sinit = read_stats(st, 0, qb);
+    sinit = to_start(read_stats(st, 0, qb));
   };
 
   // One block of a wave: 32 queries (qb of stage st, first one q0) x its keys.  `loads`: those of stage `ld` are
@@ -578,6 +577,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) lf_bw_mfma_hidden(dk[kb][j % LF_NDB], fr[2 * NS + NT + j], dsf[kb][j / LF_NDB]);
       if (j == 1) sinit = read_stats(st_n, 0, qb_n);
+      if (j == NT - 1) sinit = to_start(sinit);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll

@@ -1094,7 +1094,7 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     dq = torch.empty((B, Hq, Sq, D), dtype=dtype, device=q.device)
     dk = torch.empty((B, Hkv, Sk, D), dtype=dtype, device=q.device)
     dv = torch.empty((B, Hkv, Sk, D), dtype=dtype, device=q.device)
-    delta = torch.empty((2, B, Hq, Sq), dtype=torch.float32, device=q.device)     # row statistics of the kernels
+    delta = torch.empty((B, Hq, Sq), dtype=torch.float32, device=q.device)
     P = AttnBwdParams()
     for name, t in (("q", q), ("k", k), ("v", v), ("o", o), ("dout", dout), ("dq", dq), ("dk", dk), ("dv", dv),
                     ("lse", lse), ("delta", delta)):
