@@ -62,8 +62,9 @@ typedef struct LfAttnParamsHost {
 /*
  * Parameter block of the backward kernels lf_attn_bwd_delta, lf_attn_bwd_dkdv and
  * lf_attn_bwd_dq (loopfuse_amd/csrc/kernels/lf_attn_bwd.hip, `struct LfAttnBwdParams`;
- * loopfuse_amd/lowering.py::AttnBwdParams is the ctypes mirror).  The three kernels take
- * the same block and run in that order on one stream.  The reference has no backward:
+ * loopfuse_amd/lowering.py::AttnBwdParams is the ctypes mirror).  The kernels take the same
+ * block and run on one stream: delta, then dkdv and dq; built with -DLF_BW_DQ_NT=256, dq forms delta itself, and dq, dkdv
+ * will do.  The reference has no backward:
  * its backend traces inference graphs only (reference loopfuse/torch_backend/interface.py:600-621).
  */
 typedef struct LfAttnBwdParamsHost {
@@ -76,7 +77,7 @@ typedef struct LfAttnBwdParamsHost {
   void* dk;             /* [B, Hkv, Sk, D]: summed over the query heads of a group */
   void* dv;
   const float* lse;     /* [B, Hq, Sq] row log-sum-exp of the scaled, masked scores in log2 units (part_ml of the forward) */
-  float* delta;         /* [B, Hq, Sq] scratch, written by lf_attn_bwd_delta */
+  float* delta;         /* [B, Hq, Sq] scratch, written by lf_attn_bwd_delta and by lf_attn_bwd_dq with 256 threads, read by the others */
   int64_t q_sb, q_sh, q_ss;
   int64_t k_sb, k_sh, k_ss;
   int64_t v_sb, v_sh, v_ss;

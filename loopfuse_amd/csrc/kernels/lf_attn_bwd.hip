@@ -7,12 +7,12 @@
 // With a softcap (LF_SOFTCAP) the scores are T = cap * tanh(scale * Q K^T / cap), P = exp(T - L), and
 // dS picks up the derivative of the cap: dS = scale * (1 - tanh^2) * P * (dP - delta).
 // Three kernels, no atomics, every result written once (deterministic):
-//   lf_attn_bwd_delta : delta[b, h, q]
+//   lf_attn_bwd_delta : delta[b, h, q], in front of the other two unless lf_attn_bwd_dq has 256 threads and forms it itself
+//   lf_attn_bwd_dq    : a workgroup owns 128 or 256 query rows of one (batch, head) -- 4 or 8 waves x
+//                       32 rows, Q^T and dO^T in registers -- and walks the kv tiles (64 keys)
 //   lf_attn_bwd_dkdv  : a workgroup owns 128 or 256 keys of one (batch, kv head) -- 4 waves x 32 or 64
 //                       keys, K^T and V^T of its keys in registers as MFMA B operands -- and walks the
 //                       q tiles (64 rows) of the query heads of the group that can see them
-//   lf_attn_bwd_dq    : a workgroup owns 128 or 256 query rows of one (batch, head) -- 4 or 8 waves x
-//                       32 rows, Q^T and dO^T in registers -- and walks the kv tiles (64 keys)
 // The tiles that are walked are kept in LDS once and read both ways: along their rows (ds_read_b128,
 // rows of the tile = MFMA rows) and transposed (rows of the tile = MFMA k).  As in the forward, the accumulator of the first product is, as
 // held, the B operand of the second, so P and dS never leave registers.
@@ -710,6 +710,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
 
   // Q^T and dO^T of this lane's rows as B operands (d = 16*ks + 8*g .. +7)
   lf_u32x4 qf[LF_NKS], gf[LF_NKS];
+  float delta_q;
   const int my_q = wq0 + l32, qr = min(my_q, p.Sq - 1);
   {
     const lf_elem* qrow = p.q + (long long)b * p.q_sb + (long long)h * p.q_sh + (long long)qr * p.q_ss;
@@ -719,12 +720,38 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
       qf[ks] = *reinterpret_cast<const lf_u32x4*>(qrow + 16 * ks + 8 * g);
       gf[ks] = *reinterpret_cast<const lf_u32x4*>(grow + 16 * ks + 8 * g);
     }
+#if LF_BW_DQ_NT == 256
+    // delta of the row, half of its elements in each of two lanes: eight sums of LF_NKS products, then a tree, i.e. chains
+    // as short as those of lf_attn_bwd_delta.  dO is in registers here anyway, so this costs a read of O, where a launch of
+    // its own reads both.  Both launches against this one, us: causal B8 16/4 S1000 D64 52 / 43, B2 16/8 S777 D128 31 / 26,
+    // B16 H8 S256 D128 20 / 16, unmasked B8 H16 S1024 D64 75 / 64.  The single workgroup that a CU holds of the larger
+    // form has nothing to run beside these reads (causal B4 H32 S2048 D128 238 / 243): there delta has its launch.
+    const lf_elem* orow = p.o + (long long)b * p.o_sb + (long long)h * p.o_sh + (long long)qr * p.o_ss;
+    lf_u32x4 of[LF_NKS];
+#pragma unroll
+    for (int ks = 0; ks < LF_NKS; ++ks) of[ks] = *reinterpret_cast<const lf_u32x4*>(orow + 16 * ks + 8 * g);
+    float t[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t[e] = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < LF_NKS; ++ks) {
+      const lf_elem8 ov = __builtin_bit_cast(lf_elem8, of[ks]), gv = __builtin_bit_cast(lf_elem8, gf[ks]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) t[e] += (float)ov[e] * (float)gv[e];
+    }
+    const float half = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+    delta_q = half + __shfl_xor(half, 32, 64);
+#endif
 #pragma unroll
     for (int ks = 0; ks < LF_NKS; ++ks) asm volatile("" : "+a"(qf[ks]), "+a"(gf[ks]));
   }
   const long long ridx = ((long long)b * p.Hq + h) * p.Sq + qr;
   const float lse_q = my_q < p.Sq ? p.lse[ridx] : __builtin_inff();
-  const float delta_q = my_q < p.Sq ? -p.delta[ridx] : 0.0f;
+#if LF_BW_DQ_NT == 256
+  if (my_q < p.Sq && g == 0) p.delta[ridx] = -delta_q;     // for lf_attn_bwd_dkdv
+#else
+  delta_q = my_q < p.Sq ? -p.delta[ridx] : 0.0f;
+#endif
 #if LF_SOFTCAP
   const float sc_exp = p.scale / p.softcap * (2.0f * LF_LOG2E);   // 2^(s * sc_exp) = e^(2x)
   const float cexp = p.softcap * LF_LOG2E;                        // exponent of P: tanh x * cexp - L

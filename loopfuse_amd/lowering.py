@@ -1052,10 +1052,10 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
                        dq_threads: Optional[int] = None):
     """Gradients of ``attention(q, k, v, plan)`` for dense K/V (mask none / causal / sliding, scale,
     softcap; no bias or paging): returns ``(dq, dk, dv)`` in the operands' dtype.  ``o`` and ``lse``
-    are the forward's output and row log-sum-exp (``attention(..., lse=...)``).  Three launches
-    (csrc/kernels/lf_attn_bwd.hip): delta = rowsum(dO * O); dK and dV, one workgroup per 128 or 256
-    keys of a (batch, kv head); dQ, one workgroup per 128 or 256 query rows.  No atomics: results are
-    reproducible bit for bit."""
+    are the forward's output and row log-sum-exp (``attention(..., lse=...)``).  Two or
+    three launches (csrc/kernels/lf_attn_bwd.hip): delta = rowsum(dO * O), together with dQ where that has small
+    workgroups; dK and dV, one workgroup per 128 or 256 keys of a (batch, kv head); dQ, one workgroup per 128
+    or 256 query rows.  No atomics: results are reproducible bit for bit."""
     dtype = q.dtype
     if dtype not in _DTYPE_CODE:
         raise UnsupportedPlan(f"dtype {dtype} not supported by the MFMA kernels (bf16/fp16 only)")
@@ -1111,10 +1111,13 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     nt = dq_threads or bwd_dq_threads(D, mask, cap, B * Hq, Sq, Sk)
     spec = bwd_spec(dtype, D, mask, cap, keys, nt)
     keep = (q, k, v, o, dout, lse, delta, dq, dk, dv)  # noqa: F841  (tensors stay alive until the launches are queued)
-    rows = B * Hq * Sq
-    get_kernel(spec, "lf_attn_bwd_delta").launch(((rows + 15) // 16, 1, 1), (256, 1, 1), P)
-    get_kernel(spec, "lf_attn_bwd_dkdv").launch((xcd_slots(B * Hkv, -(-Sk // (128 * keys))), 1, 1), (256, 1, 1), P)
-    get_kernel(spec, "lf_attn_bwd_dq").launch((xcd_slots(B * Hkv, (Hq // Hkv) * -(-Sq // (nt // 2))), 1, 1),
-                                              (nt, 1, 1), P)
-    _last_launch.set({"kernels": ["lf_attn_bwd_delta", "lf_attn_bwd_dkdv", "lf_attn_bwd_dq"]})
+    steps = {"lf_attn_bwd_delta": (-(-B * Hq * Sq // 16), 256),
+             "lf_attn_bwd_dkdv": (xcd_slots(B * Hkv, -(-Sk // (128 * keys))), 256),
+             "lf_attn_bwd_dq": (xcd_slots(B * Hkv, (Hq // Hkv) * -(-Sq // (nt // 2))), nt)}
+    # with 256 threads lf_attn_bwd_dq forms delta itself, and lf_attn_bwd_dkdv reads it
+    names = ["lf_attn_bwd_dq", "lf_attn_bwd_dkdv"] if nt == 256 else list(steps)
+    for name in names:
+        grid, block = steps[name]
+        get_kernel(spec, name).launch((grid, 1, 1), (block, 1, 1), P)
+    _last_launch.set({"kernels": names})
     return dq, dk, dv
