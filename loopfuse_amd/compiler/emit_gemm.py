@@ -219,10 +219,21 @@ class GemmEmitter(Emitter):
     def __init__(self, nest: ir.Nest, dtypes: dict, name: str, info: GemmInfo):
         super().__init__(nest, dtypes, name)
         self.info = info
+        self.reads: list = []       # what the epilogue reads besides the product, loaded ahead of it (rd[k])
+        self.conditional = 0
 
     def expr(self, e: ir.Expr) -> str:
         if isinstance(e, ir.Dot):
             return "accv"
+        if isinstance(e, ir.Select):
+            self.conditional += 1
+            try:
+                return super().expr(e)
+            finally:
+                self.conditional -= 1
+        if isinstance(e, ir.Read) and e.gather is None and not self.conditional:
+            self.reads.append(super().expr(e))
+            return f"rd[{len(self.reads) - 1}]"
         return super().expr(e)
 
     def emit(self) -> Kernel:
@@ -249,6 +260,14 @@ class GemmEmitter(Emitter):
         val = self.expr(n.stmt.value)              # epilogue on `accv`; registers its buffers, strides, scalars
         if self.lines:
             raise NotLowerable("a second contraction inside the epilogue")
+        # The reads of all elements go out before the first of them is needed: an activation with branches (erf) keeps the
+        # compiler from moving the loads of the next element above it, which then waits for memory once per element.  With
+        # the sum's block numbers divided in 32 bits, linear -> gelu -> linear with 256 rows, 4096 / 16384 wide: 106.4 -> 104.9
+        # us, 1024 rows 287.9 -> 282.4, 64 rows 65.0 -> 64.0.  (Two blocks of columns per workgroup of the sum: no more at 256
+        # and 1024 rows, 64 rows 64.9 -> 66.1: half the workgroups.)
+        lambdas = f"""constexpr int kRd = {max(1, len(self.reads))};
+  auto read = [&](float* rd, long long i{km}, long long i{kn}) {{ {' '.join(f'rd[{j}] = {r};' for j, r in enumerate(self.reads))} }};
+  auto epilogue = [&](float accv, const float* rd, long long i{km}, long long i{kn}) -> float {{ return {val}; }};"""
         out = n.writes()
         o = self.buf(out)
         ooff = self.offset(out, out.dims, None)
@@ -412,7 +431,7 @@ class GemmEmitter(Emitter):
   // Two n blocks at a time through the wave's own part of LDS ([32 * kMB m][64 n] fp32, 16-byte pieces permuted by the
   // row): afterwards a lane holds four consecutive n of one m and 16 neighbouring lanes cover 64 consecutive n.
   float* mine = reinterpret_cast<float*>(lds) + wave * (kMB * 2048);
-  auto epilogue = [&](float accv, long long i{km}, long long i{kn}) -> float {{ return {val}; }};
+  {lambdas}
   auto out_at = [&](long long i{km}, long long i{kn}) -> long long {{ return {ooff}; }};
 #pragma unroll
   for (int pass = 0; pass < kNB / 2; ++pass) {{
@@ -438,9 +457,11 @@ class GemmEmitter(Emitter):
       const lfg_f32x4 c = __builtin_bit_cast(lfg_f32x4, *reinterpret_cast<const lfg_u32x4*>(&mine[row * 64 + 4 * (piece ^ (row & 15))]));
       const long long m = m0 + 32 * kMB * wm + row, n = n0 + 32 * kNB * wn + 64 * pass + 4 * piece;
       if (m < M && n < Nn) {{
-        float r[4];
+        float r[4], rd[4][kRd];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = epilogue(c[e], m, n + e < Nn ? n + e : n);
+        for (int e = 0; e < 4; ++e) read(rd[e], m, n + e < Nn ? n + e : n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = epilogue(c[e], rd[e], m, n + e < Nn ? n + e : n);
         if (row_stores && n + 3 < Nn) {{
           lfg_st4<{out_t}>(p.ptr[{o}], out_at(m, n), r);
         }} else {{
@@ -463,12 +484,12 @@ extern "C" __global__ void __launch_bounds__(256) {self.name}_sum(const LfGenPar
   constexpr int kWM = LFG_WGM, kWN = LFG_WGN, kMB = LFG_MB, kNB = LFG_NB;
   constexpr int kBM = 32 * kWM * kMB, kBN = 32 * kWN * kNB;
   const long long M = N{km}, Nn = N{kn};
-  const long long mt = (M + kBM - 1) / kBM, nt = (Nn + kBN - 1) / kBN, mb = (M + 31) / 32, nb = (Nn + 31) / 32;
+  const long long mt = (M + kBM - 1) / kBM, nt = (Nn + kBN - 1) / kBN;
+  const unsigned mb = (unsigned)((M + 31) / 32), nb = (unsigned)((Nn + 31) / 32);   // at most the grid, which has 31 bits
   long long total = mt * nt;
   {' '.join(f'total *= N{self.atom(a)};' for a in g.batch)}
-  long long blk = blockIdx.x;
-  const int bn = (int)(blk % nb); blk /= nb;
-  const int bm = (int)(blk % mb); blk /= mb;
+  const int bn = (int)(blockIdx.x % nb), bm = (int)(blockIdx.x / nb % mb);
+  long long blk = blockIdx.x / nb / mb;
   const int tm = bm / (kWM * kMB), wm = bm / kMB % kWM, x = bm % kMB, tn = bn / (kWN * kNB), wn = bn / kNB % kWN, y = bn % kNB;
   const int lane = threadIdx.x & 63, row = 8 * (threadIdx.x >> 6) + (lane & 7), q = lane >> 4, gg = (lane >> 3) & 1;
   const float* ws = reinterpret_cast<const float*>(p.ptr[{g.ws_ptr}]) + ((blk * mt + tm) * nt + tn) * (kBM * kBN) +
@@ -476,6 +497,10 @@ extern "C" __global__ void __launch_bounds__(256) {self.name}_sum(const LfGenPar
   const long long m = 32 * bm + row, n = 32 * bn + 8 * q + 4 * gg, stride = total * (kBM * kBN);
   {' '.join(batch_decode)}
   if (m >= M || n >= Nn) return;
+  {lambdas}
+  float r[4], rd[4][kRd];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) read(rd[e], m, n + e < Nn ? n + e : n);
   lfg_f32x4 c = {{0.0f, 0.0f, 0.0f, 0.0f}};
   const int parts = (int)p.n[{g.flags_at + 3}];
   for (int z = 0; z < parts; z += 4) {{
@@ -486,11 +511,9 @@ extern "C" __global__ void __launch_bounds__(256) {self.name}_sum(const LfGenPar
     for (int u = 0; u < 4; ++u)
       if (z + u < parts) c += t[u];
   }}
-  auto epilogue = [&](float accv, long long i{km}, long long i{kn}) -> float {{ return {val}; }};
   auto out_at = [&](long long i{km}, long long i{kn}) -> long long {{ return {ooff}; }};
-  float r[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = epilogue(c[e], m, n + e < Nn ? n + e : n);
+  for (int e = 0; e < 4; ++e) r[e] = epilogue(c[e], rd[e], m, n + e < Nn ? n + e : n);
   if (p.n[{g.flags_at}] != 0 && n + 3 < Nn) {{
     lfg_st4<{out_t}>(p.ptr[{o}], out_at(m, n), r);
   }} else {{
