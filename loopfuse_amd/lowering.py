@@ -1025,6 +1025,13 @@ def bwd_dq_threads(D: int, mask: int, softcap: bool, units: int, Sq: int, Sk: in
     return 512
 
 
+def bwd_two_key_blocks(D: int, mask: int, softcap: bool) -> bool:
+    """Is lf_attn_bwd_dkdv built with two key blocks per wave?  Its accumulators are right only while the compiler leaves
+    them where they are, and beside the values of a window or a softcap it has no registers left to do so: with both it
+    spills accumulators and drops what the loop adds to them."""
+    return D == 128 and not softcap and mask != MASK_SLIDING
+
+
 def bwd_key_blocks(D: int, mask: int, softcap: bool, units: int, Sk: int) -> int:
     """32-key blocks a wave of lf_attn_bwd_dkdv holds: 2 (workgroups of 256 keys; every fragment read from
     LDS feeds two MFMAs) or 1 (128 keys).  ``units`` = batch x kv heads.  Measured, all backward launches, 2 against 1:
@@ -1034,7 +1041,7 @@ def bwd_key_blocks(D: int, mask: int, softcap: bool, units: int, Sk: int) -> int
     more blocks than its waves need (0.95 ... 1.08 times), head dimension 64 runs two workgroups per CU with one block
     (1.03 ... 1.3 times), and a softcap's values do not fit the registers beside two."""
     n = units * -(-Sk // 256)
-    if D != 128 or softcap or mask == MASK_SLIDING:
+    if not bwd_two_key_blocks(D, mask, softcap):
         return 1
     if mask == MASK_CAUSAL:
         return 2 if (n >= 512 and Sk >= 2048) or (n >= 1024 and Sk >= 1024) else 1
@@ -1084,6 +1091,11 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     window = int(plan.window or 0)
     if mask == MASK_SLIDING and window < 1:
         raise UnsupportedPlan("sliding window must be >= 1")
+    cap = softcap is not None
+    if key_blocks and key_blocks != 1 and (key_blocks != 2 or not bwd_two_key_blocks(D, mask, cap)):
+        raise UnsupportedPlan(f"key_blocks {key_blocks!r}: 1, or 2 at head dim 128 without a window and a softcap")
+    if dq_threads and dq_threads not in (256, 512):
+        raise UnsupportedPlan(f"dq_threads {dq_threads!r}: 256 or 512")
     for name, t in (("Q", q), ("K", k), ("V", v), ("O", o), ("dO", dout)):
         _check_tensor(name, t, dtype)
     # the tiles travel global -> LDS with 32-bit byte offsets inside one (batch, head) span, rows
@@ -1106,7 +1118,6 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     P.B, P.Hq, P.Hkv, P.Sq, P.Sk, P.window = B, Hq, Hkv, Sq, Sk, window
     P.scale = float(plan.scale)
     P.softcap = softcap if softcap is not None else 0.0
-    cap = softcap is not None
     keys = key_blocks or bwd_key_blocks(D, mask, cap, B * Hkv, Sk)
     nt = dq_threads or bwd_dq_threads(D, mask, cap, B * Hq, Sq, Sk)
     spec = bwd_spec(dtype, D, mask, cap, keys, nt)

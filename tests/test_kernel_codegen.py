@@ -194,3 +194,17 @@ def test_the_check_sees_an_unsettled_operand():
         _check_settled("probe", ["v_mov_b32_e32 v17, v9", "v_add_u32_e32 v40, v1, v2", mfma])
     _check_settled("probe", ["v_mov_b32_e32 v17, v9", "s_nop 1", mfma])
     _check_settled("probe", ["v_mov_b32_e32 v32, v9", mfma])
+
+
+@pytest.mark.parametrize("D,mask,softcap,window,kw", [
+    (128, "sliding", 30.0, 64, {"key_blocks": 2}), (128, "sliding", None, 64, {"key_blocks": 2}),
+    (128, "causal", 30.0, 0, {"key_blocks": 2}), (64, "causal", None, 0, {"key_blocks": 2}),
+    (128, "causal", None, 0, {"key_blocks": 3}),
+    (128, "causal", None, 0, {"dq_threads": 128})])
+def test_backward_refuses_work_splits_that_no_kernel_is_built_for(D, mask, softcap, window, kw):
+    """A build with two key blocks per wave has no registers for a window's or a softcap's values: it would move its
+    accumulators.  Refused before anything else is looked at (the tensors here are not even on a GPU)."""
+    q, k, v, o, dout = (torch.zeros((1, 2, 64, D), dtype=torch.bfloat16) for _ in range(5))
+    plan = lowering.AttnPlan(mask=mask, window=window, scale=D ** -0.5, softcap=softcap)
+    with pytest.raises(lowering.UnsupportedPlan, match=next(iter(kw))):
+        lowering.attention_backward(q, k, v, o, torch.zeros((1, 2, 64)), dout, plan, **kw)
