@@ -196,6 +196,13 @@ def compile_spec(spec: KernelSpec, arch: str = runtime.DEFAULT_ARCH) -> Compiled
     # outside the lock: different specialisations compile concurrently (the shim is re-entrant;
     # two threads asking for the same one both compile, the results are identical)
     code, hit, log = runtime.compile_source(spec.source(), spec.name(), spec.options(), arch)
+    if spec.family == "bwd" and _env("USE_HARDCODE_KERNEL", "0") != "1":
+        # the product kernels hand their accumulators to inline MFMAs as inputs: one that is spilled loses what the loop
+        # added to it, and nothing at run time says so
+        spilled = {name: n for name, n in runtime.private_segment_bytes(code).items() if n}
+        if spilled:
+            raise RuntimeError(f"loopfuse_amd: this compiler spills registers of the backward kernels ({spec.name()}: {spilled} "
+                               "bytes per lane); their results would be wrong")
     ck = CompiledKernel(spec, code, hit, log)
     record = _env("LOOPFUSE_RECORD_SPECS")
     with _lock:

@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 from typing import Sequence
 
@@ -135,6 +136,32 @@ def compile_source(src: str, name: str, opts: Sequence[str], arch: str | None = 
     finally:
         L.lf_free_code(code)
     return data, bool(hit.value), log.value.decode("utf-8", "replace")
+
+
+def private_segment_bytes(code: bytes) -> dict:
+    """Scratch memory per lane of every kernel of a code object, by name: what its registers did not hold.  Read from the
+    kernel descriptors (ELF symbols ``<kernel>.kd``; the second 32-bit word of a descriptor is its private segment's size)."""
+    if code[:6] != b"\x7fELF\x02\x01":
+        raise ValueError("not a 64-bit little-endian ELF code object")
+    shoff, = struct.unpack_from("<Q", code, 0x28)
+    shentsize, shnum = struct.unpack_from("<HH", code, 0x3a)
+    # type, address, file offset, size, link, entry size of each section
+    sections = []
+    for i in range(shnum):
+        _, kind, _, addr, off, size, link, _, _, entsize = struct.unpack_from("<IIQQQQIIQQ", code, shoff + i * shentsize)
+        sections.append((kind, addr, off, size, link, entsize))
+    out = {}
+    for kind, _, off, size, link, entsize in sections:
+        if kind not in (2, 11):                      # SHT_SYMTAB, SHT_DYNSYM
+            continue
+        strings = sections[link][2]
+        for at in range(off, off + size, entsize):
+            name_at, _, _, shndx, value, _ = struct.unpack_from("<IBBHQQ", code, at)
+            name = code[strings + name_at:code.index(b"\0", strings + name_at)].decode()
+            if name.endswith(".kd") and 0 < shndx < shnum:
+                _, addr, start = sections[shndx][:3]
+                out[name[:-3]], = struct.unpack_from("<I", code, start + value - addr + 4)
+    return out
 
 
 def current_stream_handle() -> int:

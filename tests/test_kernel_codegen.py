@@ -20,7 +20,7 @@ import subprocess
 import pytest
 import torch
 
-from loopfuse_amd import lowering
+from loopfuse_amd import lowering, runtime
 
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 MIN_GAP = 24     # instructions; 12 wait states for the result plus one MFMA that may run ahead of it
@@ -208,3 +208,15 @@ def test_backward_refuses_work_splits_that_no_kernel_is_built_for(D, mask, softc
     plan = lowering.AttnPlan(mask=mask, window=window, scale=D ** -0.5, softcap=softcap)
     with pytest.raises(lowering.UnsupportedPlan, match=next(iter(kw))):
         lowering.attention_backward(q, k, v, o, torch.zeros((1, 2, 64)), dout, plan, **kw)
+
+
+def test_backward_code_that_spills_is_refused(shim_built):
+    """An accumulator that the compiler spills loses what the loop adds to it: ``compile_spec`` raises instead of handing
+    out such code, here the build with two key blocks per wave beside a softcap, and passes the one without."""
+    spec = lowering.bwd_spec(torch.bfloat16, 128, lowering.MASK_SLIDING, True, key_blocks=2)
+    with pytest.raises(RuntimeError, match="lf_attn_bwd_dkdv"):
+        lowering.compile_spec(spec)
+    code = lowering.compile_spec(lowering.bwd_spec(torch.bfloat16, 128, lowering.MASK_CAUSAL, key_blocks=2)).code_object
+    assert runtime.private_segment_bytes(code) == {"lf_attn_bwd_delta": 0, "lf_attn_bwd_dkdv": 0, "lf_attn_bwd_dq": 0}
+    with pytest.raises(ValueError):
+        runtime.private_segment_bytes(b"no code object")
