@@ -263,10 +263,14 @@ __device__ __forceinline__ void lf_bw_mfma_hidden(const lf_f32x16& c, const lf_u
 // stream still takes three quarters of that, and the read-ahead (2 ... 8 fragments) makes no difference.
 // Work of a wave: a stream of blocks of 32 queries, two per 64-query tile, and per block four phases of MFMAs whose
 // A fragments come through one read-ahead ring that runs on into the next block:
-//   S^T = Q K^T                      accumulators start at -L / c, so P = 2^(c S) needs no subtraction
+//   S^T = Q K^T
 //   dP^T = dO V^T                    accumulators start at -delta; P between these MFMAs
 //   dV^T += dO^T P                   dS = P (dP - delta) between these
 //   dK^T += Q^T dS
+// L is subtracted in the exponent (one fused multiply-add, P = 2^(c S - L)), not by starting S at -L / c: there every step of
+// the product rounds at the size of L / c (dV in fp16 at exponents of 1e5: 1.2e-3 off instead of 2.9e-4), a scale of 0 gives
+// NaN, and it is no faster (all launches, us, started / subtracted: causal B4 H32 S2048 D128 538 / 537, B8 16/4 S1000 D64
+// 129 / 127, unmasked B2 32/8 S4096 1627 / 1618, softcap B4 32/8 S2048 631 / 628).
 // Three LDS stages: a tile's loads are issued in the second half of the step two before its own, and the one barrier per
 // step, in its middle, says both that the next tile has landed and that the tile before this one is free.
 extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const LfAttnBwdParams p) {
@@ -325,7 +329,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   const float sc_exp = p.scale / p.softcap * (2.0f * LF_LOG2E);   // 2^(s * sc_exp) = e^(2x)
   const float cexp = p.softcap * LF_LOG2E;                        // exponent of P: tanh x * cexp - L
 #else
-  const float cexp = p.scale * LF_LOG2E;                          // exponent of P: (s - L / cexp) * cexp
+  const float cexp = p.scale * LF_LOG2E;                          // exponent of P: s * cexp - L
 #endif
 
   lf_f32x16 dk[KB][LF_NDB], dv[KB][LF_NDB];
@@ -361,7 +365,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   auto g_tile = [&](int st) { return lds0 + (unsigned)((2 * st + 1) * LF_BW_TILEB); };
 
   // ---- what is loaded next: query head, q tile; past the last step the loads go out against an empty range.  Waves 0
-  // and 1 also bring the row statistics, L and the start of dP; those of rows past Sq are zeros: P is 1 there
+  // and 1 also bring the row statistics, L and -delta; those of rows past Sq are zeros: P is 1 there
   // and meets dO = 0.
   int ld_step = 0, ld_tile = qt_begin, ld_q0 = 0;
   const lf_elem* ld_q = p.q + (long long)b * p.q_sb + (long long)(hkv * group) * p.q_sh;
@@ -389,27 +393,18 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     if (j == kLoads - 1 && wave < 2)
       lf_dma_dword_to_lds_at(stat_rs, (unsigned)(ld_q0 + lane) * 4u, stat0 + (unsigned)((2 * st + wave) * 256));
   };
-  // values of the queries of block qb in accumulator order: element 4*i4 + e is query 32*qb + 8*i4 + 4*g + e
+  // statistic `which` of the queries of block qb in accumulator order: element 4*i4 + e is query 32*qb + 8*i4 + 4*g + e
+  auto read_stat4 = [&](int st, int which, int qb, int i4) {
+    return *reinterpret_cast<const lf_f32x4*>(&stats[st][which][32 * qb + 8 * i4 + 4 * g]);
+  };
   auto read_stats = [&](int st, int which, int qb) {
     lf_f32x16 r;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
-      const lf_f32x4 x = *reinterpret_cast<const lf_f32x4*>(&stats[st][which][32 * qb + 8 * i4 + 4 * g]);
+      const lf_f32x4 x = read_stat4(st, which, qb, i4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) r[4 * i4 + e] = x[e];
     }
-    return r;
-  };
-  // P = 2^(cexp * (S + start)), start = -L / cexp: the row log-sum-exp enters through the start of the accumulators of S.
-  // With a softcap the exponent is not linear in S: there L itself is kept.
-#if !LF_SOFTCAP
-  const float start_scale = -1.0f / (p.scale * LF_LOG2E);
-#endif
-  auto to_start = [&](lf_f32x16 r) {
-#if !LF_SOFTCAP
-#pragma unroll
-    for (int i = 0; i < 16; ++i) r[i] *= start_scale;
-#endif
     return r;
   };
 
@@ -428,11 +423,9 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     return lf_bw_read_tr(sb + tr_off, 0, 2 * qb + (j - NT) / LF_NDB, j % LF_NDB);
   };
   lf_u32x4 pre[LF_BW_PF];            // the next block's first fragments
-  lf_f32x16 sinit;                   // and what its scores start at
   auto read_ahead = [&](int st, int qb) {
 #pragma unroll
     for (int f = 0; f < LF_BW_PF; ++f) pre[f] = frag(st, qb, f);
-    sinit = to_start(read_stats(st, 0, qb));
   };
 
   // One block of a wave: 32 queries (qb of stage st, first one q0) x its keys.  `loads`: those of stage `ld` are
@@ -442,6 +435,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
 #pragma unroll
     for (int f = 0; f < LF_BW_PF; ++f) fr[f] = pre[f];
     lf_f32x16 s[KB], dp[KB], dinit;
+    lf_f32x4 lse4[4];                // L of elements 4*i4 .. +3, read one group ahead of its first use
     lf_u32x4 pf[KB][2], dsf[KB][2];
 #if LF_BW_VL
     lf_u32x4 vl[LF_BW_VL][KB];
@@ -463,10 +457,10 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
         const int i = 4 * i4 + e;
 #if LF_SOFTCAP
         const float r = __builtin_amdgcn_rcpf(1.0f + lf_exp2(s[kb][i] * sc_exp));     // 1 / (e^(2x) + 1), x = s * scale / cap
-        float pv = lf_exp2((1.0f - 2.0f * r) * cexp - sinit[i]);
+        float pv = lf_exp2((1.0f - 2.0f * r) * cexp - lse4[i4][e]);
         const float dcap = 4.0f * r * (1.0f - r);                                      // 1 - tanh^2
 #else
-        float pv = lf_exp2(s[kb][i] * cexp);
+        float pv = lf_exp2(s[kb][i] * cexp - lse4[i4][e]);
 #endif
         if (masked) {
           pv = lf_bw_keep(rel[kb] + 8 * i4 + e, p.window) ? pv : 0.0f;
@@ -502,25 +496,19 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     // what is carried from block to block may have been moved between registers just now, by the vector ALU
 #pragma unroll
     for (int f = 0; f < LF_BW_PF; ++f) asm volatile("" : "+v"(fr[f]));
-    asm volatile(LF_BW_VALU_SETTLE : "+v"(sinit));
+    asm volatile(LF_BW_VALU_SETTLE : "+v"(fr[0]));
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
       ahead(i);
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
-#if LF_SOFTCAP
         if (i == 0) lf_bw_mfma_zero(s[kb], fr[i], kf[kb][i]);
-#else
-        if (i == 0) lf_bw_mfma_from(s[kb], fr[i], kf[kb][i], sinit);
-#endif
         else lf_bw_mfma_vvv(s[kb], fr[i], kf[kb][i]);
       }
-#if !LF_SOFTCAP
-      if (i == 1) LF_BW_HOLD(sinit);
-#endif
       if (i == NS - 2) {
         dinit = read_stats(st, 1, qb);
+        lse4[0] = read_stat4(st, 0, qb, 0);
 #if LF_BW_VL
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) vl[0][kb] = v_lds[0][kb][tid];
@@ -551,7 +539,10 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
         LF_BW_HOLD(dinit);
       }
 #pragma unroll
-      for (int t = ks * 4 * KB / NS; t < (ks + 1) * 4 * KB / NS; ++t) soft4(t % KB, t / KB);
+      for (int t = ks * 4 * KB / NS; t < (ks + 1) * 4 * KB / NS; ++t) {
+        if (t % KB == 0 && t / KB < 3) lse4[t / KB + 1] = read_stat4(st, 0, qb, t / KB + 1);
+        soft4(t % KB, t / KB);
+      }
       load(NS + ks);
     }
 #pragma unroll
@@ -576,8 +567,6 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
       ahead(2 * NS + NT + j);
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) lf_bw_mfma_hidden(dk[kb][j % LF_NDB], fr[2 * NS + NT + j], dsf[kb][j / LF_NDB]);
-      if (j == 1) sinit = read_stats(st_n, 0, qb_n);
-      if (j == NT - 1) sinit = to_start(sinit);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll

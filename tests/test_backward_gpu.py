@@ -386,3 +386,28 @@ def test_dq_workgroup_sizes_at_tile_edges(B, Hq, Hkv, Sq, Sk, D, mask, window, s
 def test_dq_workgroup_size_rule(units, Sq, want):
     assert lowering.bwd_dq_threads(128, lowering.MASK_CAUSAL, False, units, Sq, Sq) == want
     assert lowering.bwd_dq_threads(64, lowering.MASK_SLIDING, False, units, Sq, Sq) == 256
+
+
+@pytest.mark.parametrize("scale", [64.0, 0.0])
+@pytest.mark.parametrize("Hkv,D,mask,key_blocks", [(2, 128, "causal", 1), (2, 128, "causal", 2), (1, 64, None, 1)])
+def test_dv_rounds_a_large_exponent_once(Hkv, D, mask, key_blocks, scale):
+    """Scores that fp32 sums hold exactly (products of small integers), exponents up to 2^17 (or all zero, scale 0): the
+    error of P = 2^(c S - L) is then the rounding of one fused multiply-add, at most 2^-8 where L has a unit of 2^-7, and
+    exp2's.  Most rows see one key, where c S - L is a small multiple of L's unit and exact, so what is left is P and dV
+    rounded to fp16 (2^-11 each); a form that rounds at the size of L in every step of the product shows 1e-3."""
+    S, Hq = 320, 2
+    g = torch.Generator().manual_seed(S + D)
+    q, k = (torch.randint(-8, 9, (1, h, S, D), generator=g).half().to(DEV) for h in (Hq, Hkv))
+    v, dout = (torch.randn((1, h, S, D), generator=g).half().to(DEV) for h in (Hkv, Hq))
+    o, lse2, *_ = _ref(q, k, v, dout, mask, 0, scale)
+    lse = lse2.float()
+    dq, dk, dv = lowering.attention_backward(q, k, v, o.half(), lse, dout, lowering.AttnPlan(mask=mask, scale=scale),
+                                             key_blocks=key_blocks)
+    s = torch.matmul(q.double(), k.double().repeat_interleave(Hq // Hkv, 1).transpose(-1, -2).contiguous())
+    c = scale * torch.tensor(1.4426950408889634, dtype=torch.float32).item()
+    p = torch.exp2(c * s - lse.double()[..., None])
+    if mask:
+        p = p.tril()
+    want = torch.matmul(p.transpose(-1, -2).contiguous(), dout.double()).view(1, Hkv, Hq // Hkv, S, D).sum(2)
+    assert torch.isfinite(dq).all() and torch.isfinite(dk).all()
+    assert ((dv.double() - want).norm() / want.norm()).item() <= 2 ** -11
