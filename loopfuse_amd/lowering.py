@@ -1034,8 +1034,8 @@ def bwd_dq_threads(D: int, mask: int, softcap: bool, units: int, Sq: int, Sk: in
 
 def bwd_two_key_blocks(D: int, mask: int, softcap: bool) -> bool:
     """Is lf_attn_bwd_dkdv built with two key blocks per wave?  Its accumulators are right only while the compiler leaves
-    them where they are, and beside the values of a window or a softcap it has no registers left to do so: with both it
-    spills accumulators and drops what the loop adds to them."""
+    them where they are, so the forms that are built are those whose code is checked; beside the values of a window or a
+    softcap two blocks leave it next to no registers, and gain nothing."""
     return D == 128 and not softcap and mask != MASK_SLIDING
 
 

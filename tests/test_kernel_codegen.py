@@ -12,6 +12,7 @@ compiled as the library compiles them (hipRTC, no GPU needed), disassembled, and
   * no instruction other than the chain's own MFMAs touching the VGPR destination of an MFMA
     between that MFMA and the drain behind its chain.
 """
+import dataclasses
 import os
 import re
 import shutil
@@ -202,8 +203,8 @@ def test_the_check_sees_an_unsettled_operand():
     (128, "causal", None, 0, {"key_blocks": 3}),
     (128, "causal", None, 0, {"dq_threads": 128})])
 def test_backward_refuses_work_splits_that_no_kernel_is_built_for(D, mask, softcap, window, kw):
-    """A build with two key blocks per wave has no registers for a window's or a softcap's values: it would move its
-    accumulators.  Refused before anything else is looked at (the tensors here are not even on a GPU)."""
+    """Two key blocks per wave are built and measured at head dim 128 without a window and a softcap only.  Anything else
+    is refused before a kernel is built (the tensors here are not even on a GPU)."""
     q, k, v, o, dout = (torch.zeros((1, 2, 64, D), dtype=torch.bfloat16) for _ in range(5))
     plan = lowering.AttnPlan(mask=mask, window=window, scale=D ** -0.5, softcap=softcap)
     with pytest.raises(lowering.UnsupportedPlan, match=next(iter(kw))):
@@ -212,8 +213,9 @@ def test_backward_refuses_work_splits_that_no_kernel_is_built_for(D, mask, softc
 
 def test_backward_code_that_spills_is_refused(shim_built):
     """An accumulator that the compiler spills loses what the loop adds to it: ``compile_spec`` raises instead of handing
-    out such code, here the build with two key blocks per wave beside a softcap, and passes the one without."""
+    out such code, here a build that reads twice as many fragments ahead as there are registers for."""
     spec = lowering.bwd_spec(torch.bfloat16, 128, lowering.MASK_SLIDING, True, key_blocks=2)
+    spec = dataclasses.replace(spec, extra=spec.extra + ("-DLF_BW_PF=8",))
     with pytest.raises(RuntimeError, match="lf_attn_bwd_dkdv"):
         lowering.compile_spec(spec)
     code = lowering.compile_spec(lowering.bwd_spec(torch.bfloat16, 128, lowering.MASK_CAUSAL, key_blocks=2)).code_object
