@@ -357,6 +357,25 @@ def decode_coop_split(units: int, Sk: int, rows: int, cus: int = 256) -> int:
     return min({max(1, min(most, n)) for n in (1, cus // units, 3 * cus // (4 * units), 2 * cus // units)}, key=cost)
 
 
+def _split_lengths(n: int, Sk: int) -> tuple:
+    """(splits, keys per split) of a decode step asked to make ``n``: whole pairs of 16-token steps."""
+    size = (-(-Sk // n) + 31) // 32 * 32
+    return -(-Sk // size), size
+
+
+def decode_static_split(n: int, plain: int, Sk: int, rows: int, D: int, room: int) -> int:
+    """KV splits of a step whose partials live in the library's static array of ``room`` bytes (``rows`` output rows, whose
+    partials per split are D + 2 floats): ``n``, what ``decode_coop_split`` chose, where the step is then split and fits;
+    otherwise, for a step that ``decode_split`` splits (into ``plain``) within the array, its count for an unsplit one and
+    the largest count with room for one that does not fit.  So every step that the per-wave loads' rule can run there runs."""
+    upto = lambda region: (region + 255) // 256 * 256
+    fits = lambda n: upto(4 * rows * n * D) + upto(8 * rows * n) <= room
+    splits, plain_splits = _split_lengths(n, Sk)[0], _split_lengths(plain, Sk)[0]
+    if (splits > 1 and fits(splits)) or plain_splits < 2 or not fits(plain_splits):
+        return n
+    return plain if splits < 2 else max(m for m in range(plain_splits, n) if fits(m))
+
+
 def _decode_headwave(paged: int, page_size: int, Hkv: int, D: int, P: "AttnParams", units_hw: int = 1 << 30,
                      Sk: int = 1 << 30, cus: int = 256) -> bool:
     """One kv head per wave pays when K and V are paged, token-major (head stride D,
@@ -965,12 +984,16 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         waves = coop or 8
         units = B * ((Hkv + waves - 1) // waves) * chunks
     num_splits = num_splits or choice.get("splits")
-    if not num_splits:
-        num_splits = decode_coop_split(units, Sk, min(rows, DECODE_QROWS)) if coop else \
-            decode_split(units, Sk, per_cu=1 if headwave else 2)
-    nsplit = num_splits
-    split_len = ((Sk + nsplit - 1) // nsplit + 31) // 32 * 32     # whole pairs of 16-token steps
-    nsplit = (Sk + split_len - 1) // split_len
+    if not num_splits and coop:
+        num_splits = decode_coop_split(units, Sk, min(rows, DECODE_QROWS))
+        if static_scratch:
+            eight = bool(choice["head_per_wave"]) and Hkv % 8 == 0 if "head_per_wave" in choice else \
+                _decode_headwave(paged, page_size, Hkv, D, P, B * ((Hkv + 7) // 8) * chunks, Sk)
+            plain = decode_split(B * ((Hkv + 7) // 8 if eight else Hkv) * chunks, Sk, per_cu=1 if eight else 2)
+            num_splits = decode_static_split(num_splits, plain, Sk, B * Hkv * rows, D, runtime.static_scratch_bytes())
+    elif not num_splits:
+        num_splits = decode_split(units, Sk, per_cu=1 if headwave else 2)
+    nsplit, split_len = _split_lengths(num_splits, Sk)
     P.rows, P.nsplit, P.split_len = rows, nsplit, split_len
     spec = KernelSpec("decode", _DTYPE_CODE[dtype], D, MASK_NONE, plan.softcap is not None, paged,
                       page_size, table_i64, rows=DECODE_QROWS, waves=waves, headwave=headwave, page_size_v=page_size_v,

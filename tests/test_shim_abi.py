@@ -5,8 +5,9 @@ import os
 import re
 
 import pytest
+import torch
 
-from loopfuse_amd import runtime
+from loopfuse_amd import lowering, runtime
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -113,3 +114,54 @@ def test_c_header_matches_the_ctypes_mirror_and_the_device_struct(tmp_path, host
         if decl:
             fields += [re.sub(r"[^A-Za-z0-9_]", "", x.split()[-1]) for x in decl.split(",")]
     assert fields == names
+
+
+def _stubbed_static_step(monkeypatch, B, Hq, Hkv, S, page, D=128):
+    """``attention(..., static_scratch=True)`` on the CPU with the launch replaced by the library's own size check;
+    returns the number of splits."""
+    room, seen = runtime.static_scratch_bytes(), []
+
+    def launch(decode, combine, P, acc, ml, grid, *rest):
+        if (acc + 255) // 256 * 256 + (ml + 255) // 256 * 256 > room:
+            raise runtime.ShimError("static", -4, "too large")
+        seen.append((P.nsplit, P.split_len, grid[1]))
+
+    monkeypatch.setattr(lowering, "_check_tensor", lambda *a: None)
+    monkeypatch.setattr(lowering, "get_kernel", lambda *a: None)
+    monkeypatch.setattr(runtime, "launch_decode_static", launch)
+    q = torch.empty((B, Hq, 1, D), dtype=torch.bfloat16)
+    pool = torch.empty((1, page, Hkv, D) if page > 1 else (1, Hkv, D), dtype=torch.bfloat16)
+    pool = pool.expand(B * S // page, *pool.shape[1:])
+
+    class Table(torch.Tensor):
+        is_cuda = True
+
+    table = torch.zeros((B, S // page), dtype=torch.int32).as_subclass(Table)
+    plan = lowering.AttnPlan(scale=D ** -0.5, k_paged=True, v_paged=True)
+    lowering.attention(q, pool, pool, plan, table, table, out=torch.empty_like(q), static_scratch=True)
+    (nsplit, split_len, gy), = seen
+    assert nsplit == gy == -(-S // split_len)
+    return nsplit
+
+
+# what decode_split made of these with the per-wave loads: two splits, or as many as have room
+@pytest.mark.parametrize("B,Hq,Hkv,S,page", [(96, 16, 16, 1024, 16), (112, 16, 16, 8192, 64), (180, 8, 8, 1024, 16), (224, 8, 8, 8192, 16),
+                                             (16, 64, 8, 8192, 1), (16, 32, 4, 8192, 1), (4, 64, 8, 8192, 2)])
+def test_static_scratch_serves_what_the_general_split_rule_fits(shim_built, monkeypatch, B, Hq, Hkv, S, page):
+    splits = _stubbed_static_step(monkeypatch, B, Hq, Hkv, S, page)
+    assert splits >= 2 and 4 * B * Hq * splits * 130 <= runtime.static_scratch_bytes()
+
+
+def test_static_scratch_split_rule():
+    """Over sizes: a step that the general rule splits within the array is split within it, any other is left as it is."""
+    room, D = 8 << 20, 128
+    upto = lambda n: -(-n // 256) * 256
+    for rows in (1, 8, 100, 1000, 2000, 4096, 10000):
+        for Sk in (64, 1000, 1024, 2048, 8192, 32768):
+            runs = lambda n: (k := lowering._split_lengths(n, Sk)[0]) > 1 and upto(4 * rows * k * D) + upto(8 * rows * k) <= room
+            for n in (1, 2, 5, 16, 33, 64):
+                for plain in (1, 2, 4, 16, 64):
+                    got = lowering.decode_static_split(n, plain, Sk, rows, D, room)
+                    assert runs(got) if runs(plain) or runs(n) else got == n
+                    assert got == n or not runs(n)
+    assert lowering.decode_static_split(16, 4, 8192, 1024, D, room) == 15

@@ -47,3 +47,18 @@ def test_static_scratch_refuses_oversized_steps():
     # and an unsplit step is not what this entry point is for
     with pytest.raises(lowering.UnsupportedPlan):
         _step(w, 1, out=out, static_scratch=True)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,page", [(96, 16, 16, 1024, 16), (16, 64, 8, 8192, 1)])
+def test_static_scratch_chooses_splits_that_fit(B, Hq, Hkv, S, page):
+    """No count given: a step that would run unsplit, and one whose partials would not fit."""
+    g = torch.Generator(device="cuda").manual_seed(B)
+    q = torch.randn((B, Hq, 1, 128), generator=g, device="cuda").bfloat16()
+    shape = (B * S // page, page, Hkv, 128) if page > 1 else (B * S, Hkv, 128)
+    k, v = (torch.randn(shape, generator=g, device="cuda").bfloat16() for _ in range(2))
+    table = torch.randperm(B * S // page, generator=g, device="cuda").view(B, S // page).int()
+    plan = lowering.AttnPlan(scale=128 ** -0.5, k_paged=True, v_paged=True)
+    out = torch.empty_like(q)
+    lowering.attention(q, k, v, plan, table, table, out=out, static_scratch=True)
+    splits = lowering.attention.last_launch["grid"][1]
+    assert splits > 1 and torch.equal(out, lowering.attention(q, k, v, plan, table, table, num_splits=splits))
