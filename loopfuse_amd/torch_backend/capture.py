@@ -680,14 +680,23 @@ def match_attention(gm: torch.fx.GraphModule) -> list:
     from torch.utils._python_dispatch import _disable_current_modes
 
     with _disable_current_modes():
-        return _match_attention(gm)
+        try:
+            return _match_attention(gm)
+        except _StandInTooLarge:
+            # a tensor the graph computes (a bias over all batches, heads, queries and keys) is large although the inputs
+            # are not: once more without the counts that were kept as traced
+            return _match_attention(gm, keep_counts=False)
+
+
+class _StandInTooLarge(NoMatch):
+    """An ordinary tensor of the graph has too many elements on the stand-in sizes."""
 
 
 class _Skip(Exception):
     """This node does not continue an attention pattern: treat it as an ordinary op."""
 
 
-def _match_attention(gm: torch.fx.GraphModule) -> list:
+def _match_attention(gm: torch.fx.GraphModule, keep_counts: bool = True) -> list:
     graph = gm.graph
     placeholders = [n for n in graph.nodes if n.op == "placeholder"]
     outputs = [n for n in graph.nodes if n.op == "output"]
@@ -755,7 +764,7 @@ def _match_attention(gm: torch.fx.GraphModule) -> list:
         # between them (Hq = g * Hkv with a small batch of another size beside them) do not survive stand-ins
         # chosen per value.  Only when they do not fit are all dims replaced.
         statics = sorted({int(d) for t in tensors for d in t.shape if not isinstance(d, torch.SymInt) and int(d) > 4})
-        for keep in (64, 4):
+        for keep in (64, 4) if keep_counts else (4,):
             kept = frozenset(v for v in statics if v <= keep)
             joint = dict(hints)
             joint.update({("static", v): v for v in statics if v > keep})
@@ -831,7 +840,7 @@ def _match_attention(gm: torch.fx.GraphModule) -> list:
         shape = tuple(concrete(d) for d in val.shape)
         n = math.prod(shape)
         if n > CAP:
-            raise NoMatch("stand-in tensor too large")
+            raise _StandInTooLarge("stand-in tensor too large")
         return Ids(Source("node", node, shape=shape), torch.arange(n, dtype=torch.int64).reshape(shape))
 
     env: dict[torch.fx.Node, Any] = {}

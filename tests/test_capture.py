@@ -929,3 +929,21 @@ def test_static_grouped_heads_beside_an_unrelated_batch_size(B, Hq, Hkv, S, D):
     (m,) = capture.match_attention(gm)
     assert m.mask == "causal" and [o.perm for o in (m.q, m.k, m.v)] == [(0, 1, 2, 3)] * 3
     assert (m.q.group, m.k.group, m.v.group) == (1, Hq // Hkv, Hq // Hkv)
+
+
+@pytest.mark.parametrize("B,H,S", [(64, 64, 64), (48, 64, 64), (8, 8, 2048)])
+def test_static_graph_with_a_bias_it_computes_for_every_score(B, H, S):
+    """A bias per head formed in the graph, [B, H, S, S]: with batch, heads and length all as traced it has more elements
+    than a stand-in may have, while the inputs have few enough; the graph is matched on smaller sizes then."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    def fn(q, k, v, slopes):
+        i = torch.arange(S, device="meta")
+        bias = -(i[:, None] - i[None, :]).abs() * slopes[:, :, None, None]
+        return torch.softmax(q @ k.transpose(-2, -1) * 0.125 + bias.to(q.dtype), dim=-1) @ v
+
+    q, k, v = (torch.empty(B, H, S, 128, dtype=torch.bfloat16, device="meta") for _ in range(3))
+    with torch.no_grad():
+        gm = make_fx(fn, tracing_mode="fake")(q, k, v, torch.empty(B, H, device="meta"))
+    (m,) = capture.match_attention(gm)
+    assert m.mask is None and m.bias.dims == (0, 1, 2, 3)
