@@ -134,6 +134,7 @@ _SHAPE_ONLY_VIEW_OPS = {aten.view.default, aten._unsafe_view.default, aten.resha
 _SDPA_OPS = {getattr(aten, name).default for name in (
     "_scaled_dot_product_flash_attention", "_scaled_dot_product_efficient_attention",
     "_scaled_dot_product_flash_attention_for_cpu") if hasattr(aten, name)}
+_SOFTMAX_OPS = {aten._softmax.default, aten.exp.default, aten.exp2.default}
 _CAST_OPS = {prims.convert_element_type.default, aten._to_copy.default}
 
 
@@ -680,23 +681,33 @@ def match_attention(gm: torch.fx.GraphModule) -> list:
     from torch.utils._python_dispatch import _disable_current_modes
 
     with _disable_current_modes():
+        kept: list = []
+        found, reason = [], None
         try:
-            return _match_attention(gm)
-        except _StandInTooLarge:
-            # a tensor the graph computes (a bias over all batches, heads, queries and keys) is large although the inputs
-            # are not: once more without the counts that were kept as traced
-            return _match_attention(gm, keep_counts=False)
-
-
-class _StandInTooLarge(NoMatch):
-    """An ordinary tensor of the graph has too many elements on the stand-in sizes."""
+            found = _match_attention(gm, kept=kept)
+        except NoMatch as e:
+            reason = e
+        # Counts kept as traced lose a graph that smaller sizes serve where a tensor it computes is large although the
+        # inputs are not (a bias over all batches, heads, queries and keys) or a ratio leaves their range (84 = 7 * 12
+        # heads): where an attention may be left over, once more without them.
+        softmaxes = sum(n.op == "call_function" and (n.target in _SDPA_OPS or n.target in _SOFTMAX_OPS) for n in gm.graph.nodes)
+        if kept and len(found) < max(1, softmaxes):
+            try:
+                again = _match_attention(gm)
+                found = again if len(again) > len(found) else found
+            except NoMatch:
+                pass
+        if not found:
+            raise reason
+        return found
 
 
 class _Skip(Exception):
     """This node does not continue an attention pattern: treat it as an ordinary op."""
 
 
-def _match_attention(gm: torch.fx.GraphModule, keep_counts: bool = True) -> list:
+def _match_attention(gm: torch.fx.GraphModule, kept: Optional[list] = None) -> list:
+    """With ``kept``, static batch, head and group counts may stay as traced; the list then receives them."""
     graph = gm.graph
     placeholders = [n for n in graph.nodes if n.op == "placeholder"]
     outputs = [n for n in graph.nodes if n.op == "output"]
@@ -764,16 +775,18 @@ def _match_attention(gm: torch.fx.GraphModule, keep_counts: bool = True) -> list
         # between them (Hq = g * Hkv with a small batch of another size beside them) do not survive stand-ins
         # chosen per value.  Only when they do not fit are all dims replaced.
         statics = sorted({int(d) for t in tensors for d in t.shape if not isinstance(d, torch.SymInt) and int(d) > 4})
-        for keep in (64, 4) if keep_counts else (4,):
-            kept = frozenset(v for v in statics if v <= keep)
+        for keep in (64, 4) if kept is not None else (4,):
+            as_traced = frozenset(v for v in statics if v <= keep)
             joint = dict(hints)
             joint.update({("static", v): v for v in statics if v > keep})
-            both = _stand_in_sizes(joint, kept)
+            both = _stand_in_sizes(joint, as_traced)
             sub = {k: v for k, v in both.items() if not isinstance(k, tuple)}
             fmap = {k[1]: v for k, v in both.items() if isinstance(k, tuple)}
-            fmap.update({v: v for v in kept})
+            fmap.update({v: v for v in as_traced})
             if max(math.prod(int(d.node.expr.subs(sub)) if isinstance(d, torch.SymInt) else fmap.get(int(d), int(d))
                              for d in t.shape) for t in tensors) <= CAP:
+                if as_traced:
+                    kept += as_traced
                 break
         sizes = sub
     shrink_static = bool(fmap)
@@ -840,7 +853,7 @@ def _match_attention(gm: torch.fx.GraphModule, keep_counts: bool = True) -> list
         shape = tuple(concrete(d) for d in val.shape)
         n = math.prod(shape)
         if n > CAP:
-            raise _StandInTooLarge("stand-in tensor too large")
+            raise NoMatch("stand-in tensor too large")
         return Ids(Source("node", node, shape=shape), torch.arange(n, dtype=torch.int64).reshape(shape))
 
     env: dict[torch.fx.Node, Any] = {}

@@ -910,7 +910,8 @@ def test_reference_import_path_is_a_drop_in():
     assert torch.equal(fn(x), torch.ops.loopfuse.causal_mask(x) + 1)
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(8, 16, 4, 1000, 64), (2, 12, 3, 4000, 64), (5, 6, 3, 3000, 128), (1, 64, 8, 2877, 128)])
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(8, 16, 4, 1000, 64), (2, 12, 3, 4000, 64), (5, 6, 3, 3000, 128), (1, 64, 8, 2877, 128),
+                                              (48, 96, 12, 128, 64), (3, 84, 12, 2048, 128), (100, 84, 12, 60, 128)])
 def test_static_grouped_heads_beside_an_unrelated_batch_size(B, Hq, Hkv, S, D):
     """Traced with static shapes at real sizes (what a training graph is matched on): the ratio Hq = g * Hkv
     survives the stand-ins although the batch size divides Hq in another ratio."""
