@@ -165,3 +165,14 @@ def test_static_scratch_split_rule():
                     assert runs(got) if runs(plain) or runs(n) else got == n
                     assert got == n or not runs(n)
     assert lowering.decode_static_split(16, 4, 8192, 1024, D, room) == 15
+
+
+def test_switches_are_read_from_the_environment_of_the_moment(monkeypatch):
+    """Set, unset, and with ``os.environ`` itself replaced by another mapping."""
+    assert lowering.decode_split(1, 1 << 16) == 64
+    monkeypatch.setenv("LOOPFUSE_DECODE_SPLITS", "5")
+    assert lowering.decode_split(1, 1 << 16) == 5
+    monkeypatch.delenv("LOOPFUSE_DECODE_SPLITS")
+    assert lowering.decode_split(1, 1 << 16) == 64
+    monkeypatch.setattr(os, "environ", {"LOOPFUSE_DECODE_SPLITS": "3"})
+    assert lowering.decode_split(1, 1 << 16) == 3
