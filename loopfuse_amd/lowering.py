@@ -301,7 +301,11 @@ _scratch: dict[tuple[int, int], torch.Tensor] = {}
 
 def _get_scratch(device: torch.device, nfloats: int) -> torch.Tensor:
     """Split-K scratch, one buffer per (device, stream): launches on one stream are
-    ordered, so they can share it; launches on different streams must not."""
+    ordered, so they can share it; launches on different streams must not.  A graph keeps the address
+    for all its replays, while the shared buffer is let go of when a later call needs a larger one, so a
+    captured call takes its own from torch's allocator: what is allocated under capture stays the graph's."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(nfloats, dtype=torch.float32, device=device)
     key = (device.index or 0, runtime.current_stream_handle())
     t = _scratch.get(key)
     if t is None or t.numel() < nfloats:

@@ -176,3 +176,20 @@ def test_switches_are_read_from_the_environment_of_the_moment(monkeypatch):
     assert lowering.decode_split(1, 1 << 16) == 64
     monkeypatch.setattr(os, "environ", {"LOOPFUSE_DECODE_SPLITS": "3"})
     assert lowering.decode_split(1, 1 << 16) == 3
+
+
+def test_a_captured_call_keeps_no_scratch_that_a_later_call_lets_go_of(monkeypatch):
+    """Under graph capture the split-K scratch is neither taken from nor put into the buffer that calls on a stream share:
+    that one is replaced, and its memory given back, as soon as a larger one is needed, and the graph goes on writing to it."""
+    monkeypatch.setattr(lowering, "_scratch", {})
+    monkeypatch.setattr(runtime, "current_stream_handle", lambda: 7)
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    dev = torch.device("cpu")
+    shared = lowering._get_scratch(dev, 10)
+    assert lowering._get_scratch(dev, 1 << 20) is shared
+    capturing[0] = True
+    own = lowering._get_scratch(dev, 1 << 22)
+    assert own.numel() == 1 << 22 and own.data_ptr() != shared.data_ptr()
+    assert list(lowering._scratch.values()) == [shared]
+    assert lowering._get_scratch(dev, 10).data_ptr() != shared.data_ptr()

@@ -62,3 +62,31 @@ def test_static_scratch_chooses_splits_that_fit(B, Hq, Hkv, S, page):
     lowering.attention(q, k, v, plan, table, table, out=out, static_scratch=True)
     splits = lowering.attention.last_launch["grid"][1]
     assert splits > 1 and torch.equal(out, lowering.attention(q, k, v, plan, table, table, num_splits=splits))
+
+
+def test_captured_split_steps_keep_their_scratch():
+    """A split decode step captured into a graph, then a larger one on the same stream (which replaces the buffer that calls
+    on a stream share) and other tensors in the memory that is free afterwards: every replay gives the eager result and
+    leaves those tensors alone."""
+    w, big = (workloads.make("c5", seed=7, B=B, S=2048).to(torch.device("cuda")) for B in (2, 24))
+    want, want_big = _step(w, 4).clone(), _step(big, 16).clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        _step(w, 4)                      # the shared buffer of this stream
+    torch.cuda.synchronize()
+    g, g_big = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        got = _step(w, 4)
+    with torch.cuda.stream(s):
+        _step(big, 16)
+    with torch.cuda.graph(g_big, stream=s):
+        got_big = _step(big, 16)
+    others = [torch.full((1 << 20,), 3.0, device="cuda") for _ in range(8)]
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        g_big.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got_big, want_big) and all(bool((t == 3.0).all()) for t in others)
