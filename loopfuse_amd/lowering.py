@@ -422,16 +422,16 @@ def _decode_rowload(paged: int, page_size: int, page_size_v: int, bias_bits: int
 
 
 def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, workgroups: int = 1 << 30,
-                    window: int = 0) -> int:
+                    keys: int = 1 << 30) -> int:
     """Keys per LDS tile of lf_attn_prefill_swp: 0 (the kernel's 64) or 32.  With 32-key tiles a
     workgroup needs 40 KB of LDS and at most 168 registers per lane, so three workgroups instead of
-    two share a CU.  At head dimension 128 that pays (i) under a short sliding window (``window``,
-    0 = none) once the launch has three workgroups for every CU -- its q tiles are a few kv tiles long
-    and a third workgroup hides prologues and drains: window 256, S 1024 ... 4096, 768 ... 4096
-    workgroups: 0 ... 16 % faster; (ii) otherwise from 2048 workgroups on: causal B8 H32 S2048 301
-    against 313 us, B4 in front of its backward 750 against 768 us for both.  Between 768 and 2048
-    workgroups the tail of the launch counts more and two per CU win: causal S 4096, 768 workgroups
-    110 against 123 us; one 6001-token prompt, 1504 workgroups, 312 against 328 us.  At head
+    two share a CU.  ``keys`` = most keys a query can see (the sequence or the window).  At head dimension 128 that pays
+    once the launch has three workgroups for every CU (768): a third workgroup hides prologues and drains.  Long walks
+    have few of these, and there two per CU and a shorter tail win until the launch has 2048 workgroups.  Times with 32
+    over times with 64, geometric mean (extremes) over 194 launches with and without masks, caps and packed heads:
+    768 ... 2047 workgroups, up to 700 keys 0.91 (0.80 ... 1.02), 700 ... 2047 0.97 (0.82 ... 1.10), 2048 and more 1.02 (0.92 ... 1.13: 784
+    workgroups of 6211 keys; one 6001-token prompt, 1504 workgroups, 328 against 312 us); from 2048 workgroups on 0.94
+    (0.79 ... 1.05).  Below 768 both ways.  At head
     dimension 64 it does not pay.  The bias tile
     classes are per 64 keys, so biased calls keep 64.  ``choice["bn"]`` (the tuner) or
     ``LOOPFUSE_BN`` override the default."""
@@ -440,7 +440,7 @@ def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, w
     want = (choice or {}).get("bn", _env("LOOPFUSE_BN"))
     if want is not None:
         return 32 if int(want) == 32 else 0
-    return 32 if D == 128 and workgroups >= (3 * 256 if 0 < window <= 512 else 8 * 256) else 0
+    return 32 if D == 128 and workgroups >= (3 * 256 if keys < 2048 else 8 * 256) else 0
 
 
 def prefill_variant(Sq: int, v_tr: bool = True) -> str:
@@ -900,7 +900,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                           denom=plan.denom_add != 0.0, d2=d2, page_size_v=page_size_v, pack=pack, extra=extra,
                           safe=plan.zero_blind_rows and bool(bias_bits & 1),
                           bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
-                                             P.window if mask == MASK_SLIDING else 0)
+                                             min(Sk, P.window) if mask == MASK_SLIDING else Sk)
                           if family == "prefill_swp" else 0)
         bm, bn = TILE_SHAPES[family]
         nw = 4

@@ -429,7 +429,7 @@ class AttentionMatch:
         bn = 0
         if family == "prefill_swp":       # the tile shape the launch would take for a grid of this size
             bn = lowering.prefill_kv_tile(D, bias, None, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
-                                          plan.window if plan.mask == "sliding" else 0)
+                                          min(Sk, plan.window) if plan.mask == "sliding" else Sk)
         return [lowering.KernelSpec(family, dt, D, mask, plan.softcap is not None, paged, ps, i64, bias=bias, d2=d2,
                                     page_size_v=psv, pack=pack, extra=extra, bn=bn,
                                     safe=plan.zero_blind_rows and bool(bias & 1) and family == "prefill")]

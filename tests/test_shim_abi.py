@@ -193,3 +193,9 @@ def test_a_captured_call_keeps_no_scratch_that_a_later_call_lets_go_of(monkeypat
     assert own.numel() == 1 << 22 and own.data_ptr() != shared.data_ptr()
     assert list(lowering._scratch.values()) == [shared]
     assert lowering._get_scratch(dev, 10).data_ptr() != shared.data_ptr()
+
+
+@pytest.mark.parametrize("workgroups,keys,tile", [(767, 100, 0), (768, 2047, 32), (768, 2048, 0), (2047, 8192, 0), (2048, 8192, 32)])
+def test_kv_tile_rule(workgroups, keys, tile):
+    assert lowering.prefill_kv_tile(128, workgroups=workgroups, keys=keys) == tile
+    assert lowering.prefill_kv_tile(64, workgroups=workgroups, keys=keys) == 0
