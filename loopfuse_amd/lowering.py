@@ -342,24 +342,53 @@ def decode_split(units: int, Sk: int, cus: int = 256, per_cu: int = 2) -> int:
     return max(1, min(want, most))
 
 
+def _coop_cost(n: int, units: int, Sk: int, rows: int, cus: int = 256) -> float:
+    """Time of a decode step with cooperative loads in ``n`` KV splits (``units`` workgroups each), in tokens streamed by
+    one workgroup per CU: rounds of one workgroup per CU, a last one that is not full costing nine tenths of one (fewer
+    workgroups stream at their own rate, not at the card's), of a split's keys, the fill of its pipeline (160 tokens) and
+    the partial results of its rows (8 each).  Constants fitted on 269 steps of 1 ... 128 sequences, 200 ... 16384 keys, 4 ... 32
+    kv heads, pages of 1 ... 64 tokens: the count with the least cost is within 0.3 % of the best measured one in the mean (1.5 % at
+    the 95th percentile) with token rows of 2 KB, within 1.6 % (10 %) with 1 KB."""
+    splits, size = _split_lengths(n, Sk)
+    full, rest = divmod(units * splits, cus)
+    return (size + 160 + (8 * rows if n > 1 else 0)) * (full + (0.9 if rest else 0.0))
+
+
+@functools.lru_cache(maxsize=1024)          # (every layer of a model asks for the same step)
+def _coop_best(units: int, Sk: int, rows: int, cus: int = 256) -> tuple:
+    """(splits, cost) of the cheapest count."""
+    # one round of all CUs, of three quarters of them, two rounds, or no split; at least 160 tokens per split
+    most = max(1, min(64, Sk // 160))
+    cost, n = min((_coop_cost(n, units, Sk, rows, cus), n)
+                  for n in {max(1, min(most, n)) for n in (1, cus // units, 3 * cus // (4 * units), 2 * cus // units)})
+    return n, cost
+
+
 def decode_coop_split(units: int, Sk: int, rows: int, cus: int = 256) -> int:
-    """KV splits of a decode step with cooperative loads (``units`` workgroups per split).  One workgroup per CU streams at
-    the card's rate and fewer at their own (48 / 96 / 144 / 192 / 240 workgroups: 2.2 / 4.1 / 5.7 / 6.6 / 6.3 TB/s), more
-    than one per CU add a round (320 instead of 200 of 4 waves: 57 against 45 us), a split costs its pipeline's fill and the
-    partial results of its rows: the count with the smallest sum, with at least 160 tokens per split (40 sequences of
-    1000 tokens in one-token pages, 8 heads: 6 splits 35 us, 3 splits 44 us)."""
+    """KV splits of a decode step with cooperative loads (``units`` workgroups per split)."""
     env = _env("LOOPFUSE_DECODE_SPLITS")
     if env:
         return max(1, int(env))
+    return _coop_best(units, Sk, rows, cus)[0]
 
-    def cost(n):
-        size = (-(-Sk // n) + 31) // 32 * 32
-        full, rest = divmod(units * -(-Sk // size), cus)
-        return (size + 64 + (4 * rows if n > 1 else 0)) * (full + (max(0.6, 0.1 + 0.9 * rest / cus) if rest else 0.0))
 
-    # one round of all CUs, of three quarters of them, two rounds, or no split
-    most = max(1, min(64, Sk // 160))
-    return min({max(1, min(most, n)) for n in (1, cus // units, 3 * cus // (4 * units), 2 * cus // units)}, key=cost)
+def decode_coop_fills(units: int, Sk: int, page_size: int) -> bool:
+    most = min(8, Sk // 512) if page_size % 16 == 0 else min(32, Sk // 160)
+    return units * max(1, most) >= 224
+
+
+def decode_coop_pays(units: int, Sk: int, rows: int, page_size: int, cus: int = 256) -> bool:
+    """Does a step with ``units`` workgroups per split pay with cooperative loads, against four waves per head?
+    First, there must be about as many workgroups as CUs.  Pages of 16 tokens and more, where the other form reads whole
+    pages too: at up to 8 splits of 512 tokens (28 sequences of 4096 tokens, 8 heads, D 128: 79 against 84 us; 16 of 2048 32
+    against 29).  Shorter pages: at up to 32 splits of 160 tokens (16 of 8192: 90 against 111 us).
+    Second, the rounds must not be too empty nor the splits too short, against an even stream: less than 1.8 times with pages
+    of 16 tokens and more, 2.4 times with shorter ones, which the other form reads in quarter rows.  Just over 256
+    workgroups that cannot be split make a second round of a few (66 sequences of 228 tokens, 32 heads: 64 against 46 us; 92
+    of 2192, 12 heads, pages of 16: 262 against 210), many short splits are mostly fill.  Of 454 steps, most of them next to
+    the lines, 24 are more than 4 % slower than the other form without this, by up to 41 %, and 15 with it, by up to 12 %."""
+    even = (1.8 if page_size % 16 == 0 else 2.4) * units * Sk
+    return decode_coop_fills(units, Sk, page_size) and _coop_best(units, Sk, rows, cus)[1] * cus < even
 
 
 def _split_lengths(n: int, Sk: int) -> tuple:
@@ -368,17 +397,25 @@ def _split_lengths(n: int, Sk: int) -> tuple:
     return -(-Sk // size), size
 
 
-def decode_static_split(n: int, plain: int, Sk: int, rows: int, D: int, room: int) -> int:
-    """KV splits of a step whose partials live in the library's static array of ``room`` bytes (``rows`` output rows, whose
-    partials per split are D + 2 floats): ``n``, what ``decode_coop_split`` chose, where the step is then split and fits;
-    otherwise, for a step that ``decode_split`` splits (into ``plain``) within the array, its count for an unsplit one and
-    the largest count with room for one that does not fit.  So every step that the per-wave loads' rule can run there runs."""
+def static_split_runs(n: int, Sk: int, rows: int, D: int, room: int) -> bool:
+    """Does a step asked to make ``n`` splits run with its partials in the library's static array of ``room`` bytes: it is
+    split, and the partials (``rows`` output rows, D + 2 floats each per split) fit?"""
     upto = lambda region: (region + 255) // 256 * 256
-    fits = lambda n: upto(4 * rows * n * D) + upto(8 * rows * n) <= room
-    splits, plain_splits = _split_lengths(n, Sk)[0], _split_lengths(plain, Sk)[0]
-    if (splits > 1 and fits(splits)) or plain_splits < 2 or not fits(plain_splits):
+    n = _split_lengths(n, Sk)[0]
+    return n > 1 and upto(4 * rows * n * D) + upto(8 * rows * n) <= room
+
+
+def decode_static_split(n: int, plain: int, Sk: int, rows: int, D: int, room: int) -> int:
+    """KV splits of a step with cooperative loads whose partials live in the static array: ``n``, what
+    ``decode_coop_split`` chose, where that runs; for an unsplit step ``plain``, what ``decode_split`` makes of it with
+    the other loads; for one that does not fit the largest count that does.  So every step runs that one of the two rules
+    can run there (``n`` is returned, to be refused, for one that no such count serves)."""
+    runs = lambda m: static_split_runs(m, Sk, rows, D, room)
+    if runs(n):
         return n
-    return plain if splits < 2 else max(m for m in range(plain_splits, n) if fits(m))
+    if _split_lengths(n, Sk)[0] < 2:
+        return plain if runs(plain) else n
+    return next((m for m in range(n - 1, 1, -1) if runs(m)), n)
 
 
 def _decode_headwave(paged: int, page_size: int, Hkv: int, D: int, P: "AttnParams", units_hw: int = 1 << 30,
@@ -428,10 +465,10 @@ def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, w
     two share a CU.  ``keys`` = most keys a query can see (the sequence or the window).  At head dimension 128 that pays
     once the launch has three workgroups for every CU (768): a third workgroup hides prologues and drains.  Long walks
     have few of these, and there two per CU and a shorter tail win until the launch has 2048 workgroups.  Times with 32
-    over times with 64, geometric mean (extremes) over 194 launches with and without masks, caps and packed heads:
-    768 ... 2047 workgroups, up to 700 keys 0.91 (0.80 ... 1.02), 700 ... 2047 0.97 (0.82 ... 1.10), 2048 and more 1.02 (0.92 ... 1.13: 784
-    workgroups of 6211 keys; one 6001-token prompt, 1504 workgroups, 328 against 312 us); from 2048 workgroups on 0.94
-    (0.79 ... 1.05).  Below 768 both ways.  At head
+    over times with 64, geometric mean (extremes) over 320 launches with and without masks, caps and packed heads:
+    768 ... 2047 workgroups, up to 700 keys 0.90 (0.80 ... 1.10), 700 ... 2047 0.97 (0.90 ... 1.04), 2048 and more 1.02 (0.94 ... 1.13: 784
+    workgroups of 6211 keys; one 6001-token prompt, 1504 workgroups, 328 against 312 us); from 2048 workgroups on 0.95
+    (0.79 ... 1.05); 500 ... 767 either way (0.72 ... 1.15).  At head
     dimension 64 it does not pay.  The bias tile
     classes are per 64 keys, so biased calls keep 64.  ``choice["bn"]`` (the tuner) or
     ``LOOPFUSE_BN`` override the default."""
@@ -978,12 +1015,11 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     elif not coop or _env("LOOPFUSE_DECODE_HEADWAVE") is not None:
         headwave = _decode_headwave(paged, page_size, Hkv, D, P, B * ((Hkv + 7) // 8) * chunks, Sk) and not page_size_v
     else:
-        # whole token rows pay once there are about as many workgroups as CUs, below that the four waves of a workgroup
-        # share one head.  Pages of 16 tokens and more, where those read whole pages too: at up to 8 splits of 512 tokens
-        # (28 sequences of 4096 tokens, 8 heads, D 128: 79 against 84 us; 16 of 2048 32 against 29).  Shorter pages: at
-        # up to 32 splits of 160 tokens (16 of 8192: 90 against 111 us; 8 of 8192 54 against 58; 8 of 4096 37 against 33)
-        most = min(8, Sk // 512) if page_size % 16 == 0 else min(32, Sk // 160)
-        headwave = B * (Hkv // coop) * chunks * max(1, most) >= 224
+        units_coop = B * (Hkv // coop) * chunks
+        headwave = decode_coop_pays(units_coop, Sk, min(rows, DECODE_QROWS), page_size)
+        if static_scratch and not (headwave or num_splits or choice.get("splits")) and decode_coop_fills(units_coop, Sk, page_size):
+            # more splits of fewer workgroups: a step that does not run in the static array with the other loads may with these
+            headwave = not static_split_runs(decode_split(units, Sk), Sk, B * Hkv * rows, D, runtime.static_scratch_bytes())
     coop = coop if headwave else 0
     if headwave:
         waves = coop or 8

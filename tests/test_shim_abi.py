@@ -153,7 +153,7 @@ def test_static_scratch_serves_what_the_general_split_rule_fits(shim_built, monk
 
 
 def test_static_scratch_split_rule():
-    """Over sizes: a step that the general rule splits within the array is split within it, any other is left as it is."""
+    """Over sizes: a step runs wherever one of the two rules' counts does, with the cooperative rule's if that one runs."""
     room, D = 8 << 20, 128
     upto = lambda n: -(-n // 256) * 256
     for rows in (1, 8, 100, 1000, 2000, 4096, 10000):
@@ -162,7 +162,7 @@ def test_static_scratch_split_rule():
             for n in (1, 2, 5, 16, 33, 64):
                 for plain in (1, 2, 4, 16, 64):
                     got = lowering.decode_static_split(n, plain, Sk, rows, D, room)
-                    assert runs(got) if runs(plain) or runs(n) else got == n
+                    assert runs(got) if runs(plain) or runs(n) else got == n or (1 < got < n and runs(got))
                     assert got == n or not runs(n)
     assert lowering.decode_static_split(16, 4, 8192, 1024, D, room) == 15
 
@@ -193,6 +193,25 @@ def test_a_captured_call_keeps_no_scratch_that_a_later_call_lets_go_of(monkeypat
     assert own.numel() == 1 << 22 and own.data_ptr() != shared.data_ptr()
     assert list(lowering._scratch.values()) == [shared]
     assert lowering._get_scratch(dev, 10).data_ptr() != shared.data_ptr()
+
+
+@pytest.mark.parametrize("units,Sk,page,pays", [
+    (64, 2048, 1, True), (64, 2048, 16, True), (28, 4096, 16, True),      # whole rounds of even splits
+    (264, 228, 1, False), (276, 2192, 16, False), (285, 1728, 16, False),  # a second round of a few workgroups
+    (8, 1200, 4, False), (16, 2048, 16, False), (250, 2048, 16, True)])    # too few workgroups; almost a round
+def test_cooperative_decode_is_chosen_where_its_rounds_are_full(units, Sk, page, pays):
+    assert lowering.decode_coop_pays(units, Sk, 1, page) == pays
+
+
+@pytest.mark.parametrize("units,Sk,rows", [(64, 2048, 8), (66, 871, 8), (50, 1142, 8), (8, 8192, 4), (300, 100, 1), (1, 32768, 16)])
+def test_cooperative_split_count(units, Sk, rows):
+    """Within its bounds, and of the counts it looks at the one with the least cost."""
+    n = lowering.decode_coop_split(units, Sk, rows)
+    most = max(1, min(64, Sk // 160))
+    assert 1 <= n <= most
+    for m in (1, 256 // units, 512 // units):
+        m = max(1, min(most, m))
+        assert lowering._coop_cost(n, units, Sk, rows) <= lowering._coop_cost(m, units, Sk, rows)
 
 
 @pytest.mark.parametrize("workgroups,keys,tile", [(767, 100, 0), (768, 2047, 32), (768, 2048, 0), (2047, 8192, 0), (2048, 8192, 32)])
