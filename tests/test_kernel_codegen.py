@@ -1,5 +1,5 @@
 """Static checks on the code objects of the kernels whose MFMAs are inline asm with explicit
-register files (lf_attn_bwd_dkdv, the 4-wave lf_attn_bwd_dq).
+register files (lf_attn_bwd_dkdv and lf_attn_bwd_dq, in every form that is built).
 
 The compiler does not know the latency of those MFMAs: a register copy or a spill it decides
 to place right behind one reads the accumulator before the result is there, and nothing at run
@@ -10,7 +10,11 @@ compiled as the library compiles them (hipRTC, no GPU needed), disassembled, and
   * every read of an MFMA's AGPR result by a non-MFMA instruction at least MIN_GAP
     instructions behind the MFMA that wrote it, or behind an explicit drain (s_nop >= 9),
   * no instruction other than the chain's own MFMAs touching the VGPR destination of an MFMA
-    between that MFMA and the drain behind its chain.
+    between that MFMA and the drain behind its chain,
+  * no instruction but MFMAs touching an AGPR between the first and the last of them, and every MFMA with an AGPR
+    destination naming the same tuple as its source: the accumulators are handed over as inputs there, so the compiler
+    takes them for constants, and
+  * two wait states between a vector instruction and an MFMA that reads what it wrote.
 """
 import dataclasses
 import os
@@ -187,6 +191,42 @@ def test_hidden_accumulators_of_dq_stay_in_their_registers(shim_built, dtype, D,
     for ln in lines:
         m = re.match(r"v_mfma_\S+ (a\[\d+:\d+\]),.*, (\S+)$", ln)
         assert m is None or m.group(1) == m.group(2), ln
+
+
+def _backward_builds():
+    import __graft_entry__
+
+    return sorted({s for s in __graft_entry__.standard_specs() if s.family == "bwd"}, key=lambda s: s.name())
+
+
+@pytest.mark.parametrize("spec", _backward_builds(), ids=lambda s: s.name())
+def test_every_backward_build_keeps_its_accumulators(shim_built, spec):
+    """All checks of this file over every backward specialisation that the build compiles and a call can ask for."""
+    kernels = _kernels(spec)
+    for name in ("lf_attn_bwd_dkdv", "lf_attn_bwd_dq"):
+        lines = kernels[name]
+        _check(name, lines)
+        _check_settled(name, lines)
+        mfma = [i for i, ln in enumerate(lines) if ln.startswith("v_mfma")]
+        for ln in lines[mfma[0]:mfma[-1]]:
+            assert ln.startswith("v_mfma") or not re.search(r"\ba(\d+|\[\d+:\d+\])", ln), f"{name}: {ln}"
+        for ln in lines:
+            m = re.match(r"v_mfma_\S+ (a\[\d+:\d+\]),.*, (\S+)$", ln)
+            assert m is None or m.group(1) == m.group(2), f"{name}: {ln}"
+
+
+def test_every_split_the_rules_choose_is_built():
+    """The rules for the work split never leave the set of builds that the test above covers."""
+    built = set(_backward_builds())
+    for dtype in (torch.bfloat16, torch.float16):
+        for D in (64, 128):
+            for mask in (lowering.MASK_NONE, lowering.MASK_CAUSAL, lowering.MASK_SLIDING):
+                for cap in (False, True):
+                    for units in (1, 31, 100, 256, 4096):
+                        for S in (1, 300, 1024, 2048, 8192):
+                            spec = lowering.bwd_spec(dtype, D, mask, cap, lowering.bwd_key_blocks(D, mask, cap, units, S),
+                                                     lowering.bwd_dq_threads(D, mask, cap, units, S, S))
+                            assert spec in built, spec
 
 
 def test_the_check_sees_an_unsettled_operand():
