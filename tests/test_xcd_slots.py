@@ -33,7 +33,7 @@ def slot_of_block(tmp_path_factory):
 def test_every_tile_once(slot_of_block, units, tiles, group):
     grid = lowering.xcd_slots(units, tiles)
     # a host that still launches the padded grid of whole groups starts at least as many workgroups
-    assert grid <= 8 * ((units + 7) // 8 + group - 1) // group * group * tiles
+    assert grid <= 8 * (((units + 7) // 8 + group - 1) // group * group) * tiles
     seen, per_xcd = {}, [0] * 8
     unit, tile = ctypes.c_int(), ctypes.c_int()
     for b in range(grid + 16):
@@ -43,6 +43,7 @@ def test_every_tile_once(slot_of_block, units, tiles, group):
             seen[key] = b
             per_xcd[b % 8] += 1
     assert len(seen) == units * tiles
+    assert grid == 8 * (max(seen.values()) // 8 + 1)                   # no slot row of the grid is padding alone
     if units * tiles >= 64 and tiles >= 8:
         assert max(per_xcd) <= 1.125 * units * tiles / 8 + 1           # no XCD carries much more than its share
     for u in range(units):                                             # dispatch order: a unit's tiles in order per part
