@@ -529,7 +529,6 @@ extern "C" __global__ void __launch_bounds__(256) {self.name}_sum(const LfGenPar
 
 # us per step of 64 k with every CU busy (s: see choose), us per workgroup besides (first loads, results), workgroups resident at a time
 _COST = {"s": (0.0, 4.0, 512), "d": (0.80, 5.0, 256), "m": (1.02, 5.0, 256), "l": (1.95, 8.0, 256)}
-_MAX_PARTIALS = 1 << 26         # floats that the parts of a split product may take
 
 
 @functools.lru_cache(maxsize=4096)
@@ -548,7 +547,7 @@ def choose(M: int, N: int, K: int, batch: int) -> tuple:
             continue                         # half of the tile would be padding
         tiles = -(-M // bm) * -(-N // bn) * batch
         for parts in range(1, max(1, min(32, steps // 4)) + 1):
-            if parts > 1 and (tiles * parts > slots or parts * tiles * bm * bn > _MAX_PARTIALS):
+            if parts > 1 and tiles * parts > slots:      # one round, whose partials are 2^24 floats at most
                 break
             if shape == "s":
                 step = 1.5 if M <= 128 else 1.3 if M <= 256 else (0.85 if tiles * parts <= 256 else 1.05)     # two stages: the latency of memory shows

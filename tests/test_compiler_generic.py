@@ -334,9 +334,43 @@ def test_mfma_kernel_compiles_for_every_operand_layout(shim_built, layouts, shap
     assert int(re.search(r"\.group_segment_fixed_size:\s+(\d+)", notes).group(1)) == {"s": 65536, "l": 131072}[shape]
 
 
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("shape", ["s", "d", "m", "l"])
+def test_every_tile_of_a_product_fits_its_registers_and_lds(shim_built, shape, split):
+    """All four tiles, whole and split with the kernel that adds up the parts: no scratch memory, two waves per SIMD, LDS as
+    the stages of the tile say."""
+    import re
+    import subprocess
+
+    from loopfuse_amd.compiler import emit_gemm
+
+    prog = generic.GenericProgram(_bf16_graph(lambda a, b, c: torch.nn.functional.gelu(a @ b + c), [(256, 512), (512, 192), (192,)]))
+    src = prog.gemm_source + ("".join(info.sum_source for _, info in prog.gemm.values()) if split else "")
+    for layouts in ((1, 1), (1, 0), (0, 1), (0, 0)):
+        opts = list(lowering.COMMON_OPTS) + [f"-DLFG_A_ROWS={layouts[0]}", f"-DLFG_B_ROWS={layouts[1]}"] + emit_gemm.tile_options(shape, split)
+        code, _, _ = runtime.compile_source(src, "lf_generic_mfma", opts)
+        kernels = runtime.private_segment_bytes(code)
+        assert len(kernels) == 1 + split and not any(kernels.values())
+        readelf = "/opt/rocm/llvm/bin/llvm-readelf"
+        if not os.path.exists(readelf):
+            continue
+        path = os.path.join(os.environ.get("TMPDIR", "/tmp"), f"lf_gemm_{os.getpid()}.hsaco")
+        with open(path, "wb") as fh:
+            fh.write(code)
+        try:
+            notes = subprocess.run([readelf, "--notes", path], capture_output=True, text=True, check=True).stdout
+        finally:
+            os.unlink(path)
+        assert all(int(n) <= 256 for n in re.findall(r"\.vgpr_count:\s+(\d+)", notes))
+        bm, bn = emit_gemm.tile_extent(shape)
+        lds = sorted(int(n) for n in re.findall(r"\.group_segment_fixed_size:\s+(\d+)", notes))
+        assert lds == [0] * split + [emit_gemm.TILES[shape][4] * 2 * emit_gemm.BK * (bm + bn)]
+
+
 def test_tile_and_parts_of_a_product_stay_within_their_limits():
     """``emit_gemm.choose`` over sizes from 1 on: every part holds at least four steps, a split launch is one round of
-    resident workgroups, its partials stay under their bound, and tiles that are half padding are not taken."""
+    resident workgroups of its tile (which bounds its partials, 2^24 floats at most), and tiles that are half padding are
+    not taken."""
     from loopfuse_amd.compiler import emit_gemm
 
     sizes = [1, 17, 64, 129, 257, 700, 2048, 8191, 65536]
@@ -350,5 +384,5 @@ def test_tile_and_parts_of_a_product_stay_within_their_limits():
                     steps = -(-K // emit_gemm.BK)
                     assert 1 <= parts <= 32 and (parts == 1 or steps // parts >= 4)
                     if parts > 1:
-                        assert tiles * parts <= 512 and parts * tiles * bm * bn <= 1 << 26
+                        assert tiles * parts <= emit_gemm._COST[shape][2] and parts * tiles * bm * bn <= 1 << 24
                     assert shape in "sd" or M > bm // 2
