@@ -241,15 +241,23 @@ def load_spec(spec: KernelSpec) -> runtime.Module:
     return mod
 
 
-_kernels: dict[tuple[KernelSpec, int, str], runtime.Kernel] = {}
+_kernels: dict[tuple[KernelSpec, int], dict[str, runtime.Kernel]] = {}
 
 
-def get_kernel(spec: KernelSpec, symbol: str) -> runtime.Kernel:
-    key = (spec, torch.cuda.current_device(), symbol)
-    k = _kernels.get(key)
+def _kernels_of(spec: KernelSpec) -> dict:
+    key = (spec, torch.cuda.current_device())
+    named = _kernels.get(key)
+    return _kernels.setdefault(key, {}) if named is None else named
+
+
+def get_kernel(spec: KernelSpec, symbol: str, named: Optional[dict] = None) -> runtime.Kernel:
+    """A kernel of a specialisation on the current device.  ``named``: ``_kernels_of(spec)``, for a caller that takes
+    several (the key's hash costs 0.6 us)."""
+    if named is None:
+        named = _kernels_of(spec)
+    k = named.get(symbol)
     if k is None:
-        k = load_spec(spec).kernel(symbol)
-        _kernels[key] = k
+        k = named[symbol] = load_spec(spec).kernel(symbol)
     return k
 
 
@@ -297,11 +305,13 @@ def _check_tensor(name: str, t: torch.Tensor, dtype: torch.dtype) -> None:
 
 
 _scratch: dict[tuple[int, int], torch.Tensor] = {}
+_scratch_lock = threading.Lock()
 
 
 def _get_scratch(device: torch.device, nfloats: int) -> torch.Tensor:
     """Split-K scratch, one buffer per (device, stream): launches on one stream are
-    ordered, so they can share it; launches on different streams must not.  A graph keeps the address
+    ordered, so they can share it (a step and its merge are launched under ``_scratch_lock``, or another
+    thread's step on the stream could come between them); launches on different streams must not.  A graph keeps the address
     for all its replays, while the shared buffer is let go of when a later call needs a larger one, so a
     captured call takes its own from torch's allocator: what is allocated under capture stays the graph's."""
     if torch.cuda.is_current_stream_capturing():
@@ -1054,14 +1064,19 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                                  "block": 64 * spec.waves, "head_per_wave": headwave, "cooperative_loads": spec.coop,
                                  "static_scratch": True})
         return out
+    named = _kernels_of(spec)
+    step, combine = get_kernel(spec, "lf_attn_decode", named), get_kernel(spec, "lf_attn_decode_combine", named)
     if nsplit > 1:
         nrow = B * Hkv * rows * nsplit
-        scratch = _get_scratch(q.device, nrow * (D + 2))
-        P.part_acc = scratch.data_ptr()
-        P.part_ml = scratch.data_ptr() + 4 * nrow * D
-    get_kernel(spec, "lf_attn_decode").launch((units, nsplit, 1), (64 * spec.waves, 1, 1), P)
-    if nsplit > 1 and merge_splits:
-        get_kernel(spec, "lf_attn_decode_combine").launch((combine_grid, 1, 1), (256, 1, 1), P)
+        with _scratch_lock:        # no other thread's step on this stream between the two launches
+            scratch = _get_scratch(q.device, nrow * (D + 2))
+            P.part_acc = scratch.data_ptr()
+            P.part_ml = scratch.data_ptr() + 4 * nrow * D
+            step.launch((units, nsplit, 1), (64 * spec.waves, 1, 1), P)
+            if merge_splits:
+                combine.launch((combine_grid, 1, 1), (256, 1, 1), P)
+    else:
+        step.launch((units, nsplit, 1), (64 * spec.waves, 1, 1), P)
     _last_launch.set({"kernels": ["lf_attn_decode"] + (["lf_attn_decode_combine"] if nsplit > 1 and merge_splits else []),
                              "grid": (units, nsplit), "block": 64 * spec.waves, "head_per_wave": headwave,
                              "cooperative_loads": spec.coop})

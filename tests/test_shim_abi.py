@@ -218,3 +218,39 @@ def test_cooperative_split_count(units, Sk, rows):
 def test_kv_tile_rule(workgroups, keys, tile):
     assert lowering.prefill_kv_tile(128, workgroups=workgroups, keys=keys) == tile
     assert lowering.prefill_kv_tile(64, workgroups=workgroups, keys=keys) == 0
+
+
+def test_a_split_step_and_its_merge_are_launched_together(shim_built, monkeypatch):
+    """Threads that decode on one stream share its scratch: no step of another thread comes between a step and its merge."""
+    import threading
+    import time
+
+    order = []
+
+    class Fake:
+        def __init__(self, name):
+            self.name = name
+
+        def launch(self, *args):
+            order.append((threading.get_ident(), self.name))
+            time.sleep(0.002)
+
+    monkeypatch.setattr(lowering, "_check_tensor", lambda *a: None)
+    monkeypatch.setattr(lowering, "_kernels_of", lambda spec: {n: Fake(n) for n in ("lf_attn_decode", "lf_attn_decode_combine")})
+    monkeypatch.setattr(lowering, "_scratch", {})
+    monkeypatch.setattr(runtime, "current_stream_handle", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    q, k = torch.zeros((1, 2, 1, 64), dtype=torch.bfloat16), torch.zeros((1, 2, 256, 64), dtype=torch.bfloat16)
+
+    def work():
+        for _ in range(5):
+            lowering.attention(q, k, k, lowering.AttnPlan(scale=0.125), num_splits=2)
+
+    threads = [threading.Thread(target=work) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(order) == 30
+    for (a, first), (b, second) in zip(order[::2], order[1::2]):
+        assert (a, first, second) == (b, "lf_attn_decode", "lf_attn_decode_combine")
