@@ -39,17 +39,17 @@ _DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1}
 COMMON_OPTS = ("-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops")
 
 
+_ENVIRON = os.environ
+_VARIABLES = _ENVIRON._data if os.name == "posix" and isinstance(getattr(_ENVIRON, "_data", None), dict) else None
+
+
 def _env(name: str, default=None):
     """``os.environ.get``, without the exception that raises and catches for each variable that is not set: 0.6 us, half a
-    dozen times per call of ``attention``.  (CPython's environment keeps its variables as bytes in ``_data``; any other mapping
-    in its place is asked in the ordinary way.)"""
-    env = os.environ
-    if type(env) is _ENVIRON_TYPE and name.encode() not in env._data:
+    dozen times per call of ``attention``.  (CPython's environment keeps its variables as bytes in ``_data``; another mapping
+    put in its place is asked in the ordinary way.)"""
+    if os.environ is _ENVIRON and _VARIABLES is not None and name.encode() not in _VARIABLES:
         return default
-    return env.get(name, default)
-
-
-_ENVIRON_TYPE = type(os.environ) if os.name == "posix" and isinstance(getattr(os.environ, "_data", None), dict) else None
+    return os.environ.get(name, default)
 
 
 class AttnParams(ctypes.Structure):
