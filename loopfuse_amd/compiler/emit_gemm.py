@@ -3,8 +3,8 @@
 cases ``tests/test_accuracy.py:56-82``: ``a @ b + c`` in two and three dims).
 
 A nest ``out[batch.., m, n] = f(sum_k A[batch.., m, k] * B[batch.., k, n], other reads)`` with bf16 /
-fp16 operands becomes one kernel.  A workgroup owns a tile of the output -- 128 x 128 on four waves or
-256 x 128 / 256 x 256 on eight (``TILES``), a compile-time choice -- and walks k, or a part of it, in
+fp16 operands becomes one kernel.  A workgroup owns a tile of the output -- 64 x 128 to 256 x 256,
+four or eight waves (``TILES``), a compile-time choice -- and walks k, or a part of it, in
 steps of 64.  Both operand tiles arrive by direct global -> LDS loads
 (``buffer_load_dwordx4 ... lds``: 16-byte pieces, range-checked so that the edges arrive as zeros, the XOR
 permutation applied on the global side), two to four stages, one barrier per step, and come back as
@@ -37,10 +37,11 @@ from .emit import _CT, MAX_N, MAX_PTR, Emitter, Kernel, NotLowerable
 
 BK = 64
 # Workgroup tiles: waves along m, waves along n, 32 x 32 blocks per wave along m, along n, LDS stages.  128 x 128 on four
-# waves, at two workgroups per CU (s) or, where there are too few tiles for that, one with four stages in flight (d: a step
-# then no longer costs a memory latency); 256 x 128 on eight waves (m) and 256 x 256 (l), one per CU, with three quarters
-# and half the L2 -> LDS bytes per flop.
-TILES = {"s": (2, 2, 2, 2, 2), "d": (2, 2, 2, 2, 4), "m": (4, 2, 2, 2, 3), "l": (4, 2, 2, 4, 2)}
+# waves at two workgroups per CU (s), or on eight with four stages, one per CU (d: a step does not cost a memory latency where
+# there are too few tiles for two); 256 x 128 on eight waves (m) and 256 x 256 (l), one per CU, with three quarters and half
+# the L2 -> LDS bytes per flop; 64 x 128 on four (n), up to two per CU, for few rows of A, where the tiles' number, not their
+# bytes, is the time.
+TILES = {"s": (2, 2, 2, 2, 2), "d": (4, 2, 1, 2, 4), "m": (4, 2, 2, 2, 3), "l": (4, 2, 2, 4, 2), "n": (2, 2, 1, 2, 3)}
 
 
 def tile_extent(shape: str) -> tuple:
@@ -48,10 +49,10 @@ def tile_extent(shape: str) -> tuple:
     return 32 * wm * mb, 32 * wn * nb
 
 
-def tile_options(shape: str, split: bool = False) -> list:
+def tile_options(shape: str, split: bool = False, b_streams: bool = False) -> list:
     wm, wn, mb, nb, stages = TILES[shape]
     return [f"-DLFG_WGM={wm}", f"-DLFG_WGN={wn}", f"-DLFG_MB={mb}", f"-DLFG_NB={nb}", f"-DLFG_STAGES={stages}"] + \
-        (["-DLFG_SPLIT=1"] if split else [])
+        (["-DLFG_SPLIT=1"] if split else []) + (["-DLFG_B_NT=1"] if b_streams else [])
 
 GEMM_PRELUDE = r"""
 typedef float lfg_f32x16 __attribute__((ext_vector_type(16)));
@@ -61,6 +62,9 @@ typedef float lfg_f32x4 __attribute__((ext_vector_type(4)));
 typedef short lfg_s16x4 __attribute__((ext_vector_type(4)));
 #ifndef LFG_SPLIT
 #define LFG_SPLIT 0      /* 1: a workgroup sums a part of k and leaves fp32 partials; a second kernel adds them up and runs the epilogue */
+#endif
+#ifndef LFG_B_NT
+#define LFG_B_NT 0       /* 1: B by non-temporal loads */
 #endif
 typedef __bf16 lfg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 lfg_f16x8 __attribute__((ext_vector_type(8)));
@@ -74,16 +78,18 @@ __device__ __forceinline__ lfg_f32x16 lfg_mfma(_Float16, lfg_u32x4 a, lfg_u32x4 
 //   k-contiguous operand ("rows"): [kExtent rows][64 k]; the eight 16-byte pieces of a row are permuted by the
 //   row pair, so that the 16-byte reads of 16 consecutive rows touch every bank once.
 //   m/n-contiguous operand ("cols"): [64 k][kExtent]; the 64-byte groups of a row are permuted by the row, for the
-//   transposed reads (4 consecutive rows x 64 contiguous bytes per 32 lanes).
+//   transposed reads (4 consecutive rows x 64 contiguous bytes per 32 lanes); of 64 columns two rows share the banks' span.
 __device__ __forceinline__ int lfg_rows_at(int row, int piece) { return row * 64 + 8 * (piece ^ ((row >> 1) & 7)); }
 template <int kExtent>
-__device__ __forceinline__ int lfg_cols_at(int row, int piece) { return row * kExtent + 8 * (piece ^ (4 * (row & 3))); }
+__device__ __forceinline__ int lfg_cols_swz(int row) { return kExtent >= 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); }
+template <int kExtent>
+__device__ __forceinline__ int lfg_cols_at(int row, int piece) { return row * kExtent + 8 * (piece ^ lfg_cols_swz<kExtent>(row)); }
 // Tiles arrive by direct global -> LDS loads: a wave-level load writes 64 lanes x 16 bytes at M0 + 16 * lane, i.e. 64
 // consecutive 16-byte positions `idx` of the tile, and the permutation is applied on the global side: the lane that
 // fills position idx fetches the piece (outer = m or n, k) that lives there.
 template <bool kRows, int kExtent> struct LfgPiece {
   static __device__ __forceinline__ int outer(int idx) {
-    return kRows ? (idx >> 3) : 8 * ((idx % (kExtent / 8)) ^ (4 * ((idx / (kExtent / 8)) & 3)));
+    return kRows ? (idx >> 3) : 8 * ((idx % (kExtent / 8)) ^ lfg_cols_swz<kExtent>(idx / (kExtent / 8)));
   }
   static __device__ __forceinline__ int k(int idx) {
     return kRows ? 8 * ((idx & 7) ^ ((idx >> 4) & 7)) : idx / (kExtent / 8);
@@ -100,12 +106,27 @@ __device__ __forceinline__ lfg_u32x4 lfg_make_buffer(const void* base, unsigned 
   rs[3] = 0x00020000u;
   return rs;
 }
-// One wave-level direct-to-LDS load (not tracked by the compiler's wait counters: callers wait with s_waitcnt vmcnt)
+// One wave-level direct-to-LDS load (not tracked by the compiler's wait counters: callers wait with s_waitcnt vmcnt);
+// kNt: non-temporal, for an operand that one workgroup alone reads
+template <bool kNt>
 __device__ __forceinline__ void lfg_dma(const lfg_u32x4& rs, unsigned voff, unsigned lds_addr) {
   unsigned m0_written;
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
-               : "={m0}"(m0_written) : "s"(lds_addr), "v"(voff), "s"(rs) : "memory");
+  if (kNt)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen nt lds"
+                 : "={m0}"(m0_written) : "s"(lds_addr), "v"(voff), "s"(rs) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
+                 : "={m0}"(m0_written) : "s"(lds_addr), "v"(voff), "s"(rs) : "memory");
 }
+// This wave's loads but the newest `n` have landed and its LDS reads are done; then the workgroup's barrier.  The wait is
+// the builtin, so that the compiler knows its own reads to be done and does not wait for them again.
+#define LFG_STAGE_BARRIER(n)                                                         \
+  do {                                                                               \
+    asm volatile("" ::: "memory");                                                   \
+    __builtin_amdgcn_s_waitcnt(((n) & 15) | 0x70 | (((n) >> 4) << 14));              \
+    __builtin_amdgcn_s_barrier();                                                    \
+    asm volatile("" ::: "memory");                                                   \
+  } while (0)
 // MFMA operand (either side: 32 rows or columns `blk`, lane % 32 picks one, lane / 32 the half of the 16-step `ks`):
 // k = 16 * ks + 8 * (lane / 32) .. + 7 in both layouts
 template <bool kRows, int kExtent>
@@ -300,31 +321,33 @@ class GemmEmitter(Emitter):
   constexpr int kS = LFG_STAGES;
   static_assert(kNB % 2 == 0 && kBM * 8 % kNT == 0 && kBN * 8 % kNT == 0, "tile shape");
   static_assert(LFG_SPLIT || kWaves * kMB * 8192 <= 2 * kS * (kTileA + kTileB), "the accumulators pass through the tiles' LDS");
-  static_assert((kS - 2) * (kPA + kPB) < 64, "loads in flight behind a stage");
+  static_assert((kS - 1) * (kPA + kPB) < 64, "loads in flight behind a stage");
   __shared__ __attribute__((aligned(16))) unsigned short lds[kS * (kTileA + kTileB)];     // A tiles [kS], then B tiles [kS]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % kWM, wn = wave / kWM;
   const long long M = N{km}, Nn = N{kn}, K = N{kk};
-  const long long mt = (M + kBM - 1) / kBM, nt = (Nn + kBN - 1) / kBN;
-  long long total = mt * nt;
-  {' '.join(f'total *= N{self.atom(a)};' for a in g.batch)}
+  // tiles, and workgroups, number less than 2^31 (the launcher's grid): 32-bit arithmetic, whose divisions are short
+  const unsigned mt = (unsigned)((M + kBM - 1) / kBM), nt = (unsigned)((Nn + kBN - 1) / kBN);
+  unsigned total = mt * nt;
+  {' '.join(f'total *= (unsigned)N{self.atom(a)};' for a in g.batch)}
   // workgroups go to the 8 XCDs round-robin: each XCD takes a contiguous run of tiles (n fastest), so the
   // workgroups resident on it share rows of A and columns of B in its L2
-  const long long parts = LFG_SPLIT ? p.n[{g.flags_at + 3}] : 1, per_xcd = (total * parts + 7) / 8;
-  long long blk = (long long)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((long long)(blockIdx.x >> 3) >= per_xcd || blk >= total * parts) return;
-  const long long part = LFG_SPLIT ? blk / total : 0;      // slowest: neighbouring tiles of one part share rows of A or columns of B
-  if (LFG_SPLIT) blk -= part * total;
+  const unsigned parts = LFG_SPLIT ? (unsigned)p.n[{g.flags_at + 3}] : 1, per_xcd = (total * parts + 7) / 8;
+  unsigned t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (blockIdx.x >> 3 >= per_xcd || t >= total * parts) return;
+  const unsigned part = LFG_SPLIT ? t / total : 0;      // slowest: neighbouring tiles of one part share rows of A or columns of B
+  if (LFG_SPLIT) t -= part * total;
   // inside a batch element the tiles run in bands of kBand tile rows, column by column: the workgroups resident
   // on an XCD at a time (32 or 64 consecutive tiles) then cover a block of the output that is a few tiles tall and
   // wide, and read correspondingly few rows of A and columns of B past its L2
-  constexpr long long kBand = kNT <= 256 ? 8 : 4;
-  const long long t = blk % (mt * nt); blk /= mt * nt;
-  const long long element = blk;      // of the batch
-  const long long first = t / (kBand * nt) * kBand, tall = min(mt - first, kBand);
-  const long long tm = first + (t % (kBand * nt)) % tall, tn = (t % (kBand * nt)) / tall;
+  constexpr unsigned kBand = kNT <= 256 ? 8 : 4;
+  const unsigned element = {'t / (mt * nt)' if g.batch else '0'};      // of the batch
+  t -= element * (mt * nt);
+  const unsigned band = (unsigned)min(kBand * (unsigned long long)nt, 0xffffffffull), first = t / band * kBand, at = t % band;
+  const unsigned tall = min(mt - first, kBand), tm = first + at % tall, tn = at / tall;
+  {'long long blk = element;' if g.batch else ''}
   {' '.join(batch_decode)}
-  const long long m0 = tm * kBM, n0 = tn * kBN;
+  const long long m0 = (long long)tm * kBM, n0 = (long long)tn * kBN;
   const {elem}* A = {a_base};
   const {elem}* B = {b_base};
   // this thread's pieces of a tile: byte offset at k = 0 and how many k are left from the piece's own k (0: the
@@ -351,28 +374,28 @@ class GemmEmitter(Emitter):
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)lds;
   const unsigned stepa = (unsigned)(2 * {BK} * S{sak}), stepb = (unsigned)(2 * {BK} * S{sbk});
   const int steps = (int)((K + {BK - 1}) / {BK});
-  const int st_begin = LFG_SPLIT ? (int)(part * p.n[{g.flags_at + 4}]) : 0;
+  const int st_begin = LFG_SPLIT ? (int)part * (int)p.n[{g.flags_at + 4}] : 0;
   const int st_end = LFG_SPLIT ? min(st_begin + (int)p.n[{g.flags_at + 4}], steps) : steps;
   // With few rows of A the loads of B from memory are the time.  There a workgroup's walk over k starts at a step of its
   // own, by tile column: with k contiguous and K a power of two every row of a step's window lies on the same few memory
   // channels, and workgroups that walk k in step all ask those (M 64, N 4096, K 16384: 39 -> 33 us; from M 512 on, where
   // matrix work is the time and tile columns share rows of A in an L2, it costs 4 ... 8 %).
   const int nsteps = st_end - st_begin;
-  int ld_st = st_begin + (M <= 256 ? (int)(tn % nsteps) : 0), ld_left = nsteps;
-  // the next step's tiles into buffer `buf`; past the last step the loads go out against nothing, so that the number in
-  // flight behind a stage is always the same
-  auto fetch = [&](int buf) {{
-    const int st = ld_st, k0 = ld_left > 0 ? st * {BK} : 0x7fffffff;
-    --ld_left;
+  int ld_st = st_begin + (M <= 256 ? (int)(tn % (unsigned)nsteps) : 0), ld_left = nsteps;
+  // A step's tiles, one wave-level load at a time (load j of kPA + kPB into buffer `buf`); past the last step the loads go
+  // out against nothing, so that the number in flight behind a stage is always the same
+  int k0 = ld_st * {BK};
+  auto issue = [&](int buf, int j) {{
+    if (j < kPA)
+      lfg_dma<false>(rs_a, k0 < rooma[j] ? offa[j] + (unsigned)ld_st * stepa : 0xffffffffu,
+                     lds0 + 2u * (unsigned)(kTileA * buf) + 1024u * (unsigned)(wave + kWaves * j));
+    else
+      lfg_dma<LFG_B_NT != 0>(rs_b, k0 < roomb[j - kPA] ? offb[j - kPA] + (unsigned)ld_st * stepb : 0xffffffffu,
+                             lds0 + 2u * (unsigned)(kS * kTileA + kTileB * buf) + 1024u * (unsigned)(wave + kWaves * (j - kPA)));
+  }};
+  auto advance = [&]() {{
     if (++ld_st == st_end) ld_st = st_begin;
-#pragma unroll
-    for (int j = 0; j < kPA; ++j)
-      lfg_dma(rs_a, k0 < rooma[j] ? offa[j] + (unsigned)st * stepa : 0xffffffffu,
-              lds0 + 2u * (unsigned)(kTileA * buf) + 1024u * (unsigned)(wave + kWaves * j));
-#pragma unroll
-    for (int j = 0; j < kPB; ++j)
-      lfg_dma(rs_b, k0 < roomb[j] ? offb[j] + (unsigned)st * stepb : 0xffffffffu,
-              lds0 + 2u * (unsigned)(kS * kTileA + kTileB * buf) + 1024u * (unsigned)(wave + kWaves * j));
+    k0 = --ld_left > 0 ? ld_st * {BK} : 0x7fffffff;
   }};
   lfg_f32x16 acc[kMB][kNB];
 #pragma unroll
@@ -381,40 +404,60 @@ class GemmEmitter(Emitter):
     for (int y = 0; y < kNB; ++y)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[x][y][i] = 0.0f;
-#define LFG_NEXT_STAGE() asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\\n\\ts_barrier" :: "n"((kS - 2) * (kPA + kPB)) : "memory")
+  // operand f of step-of-16 ks of the stage in buffer `buf`: the kMB blocks of A (lane = m), then the kNB of B (lane = n:
+  // the A operand of C^T = B^T A^T)
+  constexpr int kF = kMB + kNB, kMF = kMB * kNB, kP = kPA + kPB, kKS = {BK // 16};
+  auto operand = [&](int buf, int ks, int f) -> lfg_u32x4 {{
+    if (f < kMB) return lfg_operand<a_rows, kBM>(&lds[kTileA * buf], kMB * wm + f, ks, lane);
+    return lfg_operand<b_rows, kBN>(&lds[kS * kTileA + kTileB * buf], kNB * wn + f - kMB, ks, lane);
+  }};
+  // The operands of a step of 16 are read during the MFMAs of the one before, across stages too, so that no MFMA waits for a
+  // read just issued.  The barrier of a stage stands in front of its last 16: by then every wave has read them, the next stage
+  // has landed, and the loads of the stage kS on go out into this one's buffer between those MFMAs.  Against a barrier at the
+  // end of a stage with its reads behind it, same tile, in a loop of its own: 8192^3 l 866 -> 829 us (1.33 PFLOP/s), m 1009 ->
+  // 950; M 1024, N 4096, K 16384 m in 2 parts 133 -> 127.  What bounds it: matrix work at the clock it gets (large M); with few
+  // rows of A the loads, which return in order per CU, so that A's, from L2, take their time beside B's from memory: 256 x
+  // 16384 x 4096 d 39 us of loads alone (24 B's, 11 A's), 19 of products alone, 43 together.
 #pragma unroll
-  for (int s = 0; s < kS - 1; ++s) fetch(s);
-  LFG_NEXT_STAGE();
+  for (int s = 0; s < kS; ++s) {{
+#pragma unroll
+    for (int j = 0; j < kP; ++j) issue(s, j);
+    advance();
+  }}
+  LFG_STAGE_BARRIER((kS - 1) * kP);
+  lfg_u32x4 fr[2][kF];
+#pragma unroll
+  for (int f = 0; f < kF; ++f) fr[0][f] = operand(0, 0, f);
   int cur = 0;
   for (int i = 0; i < nsteps; ++i) {{
-    // into the stage that every wave left at the last barrier
-    fetch(cur == 0 ? kS - 1 : cur - 1);
-    const unsigned short* ta = &lds[kTileA * cur];
-    const unsigned short* tb = &lds[kS * kTileA + kTileB * cur];
+    const int next = cur == kS - 1 ? 0 : cur + 1;
 #pragma unroll
-    for (int ks = 0; ks < {BK // 16}; ++ks) {{
-      lfg_u32x4 fm[kMB], fn[kNB];
+    for (int ks = 0; ks < kKS; ++ks) {{
+      if (ks == kKS - 1) LFG_STAGE_BARRIER((kS - 2) * kP);
 #pragma unroll
-      for (int x = 0; x < kMB; ++x) fm[x] = lfg_operand<a_rows, kBM>(ta, kMB * wm + x, ks, lane);       // lane = m
+      for (int j = 0; j < kMF; ++j) {{
 #pragma unroll
-      for (int y = 0; y < kNB; ++y) fn[y] = lfg_operand<b_rows, kBN>(tb, kNB * wn + y, ks, lane);       // lane = n: the A operand of C^T = B^T A^T
+        for (int f = j * kF / kMF; f < (j + 1) * kF / kMF; ++f)
+          fr[(ks + 1) & 1][f] = ks < kKS - 1 ? operand(cur, ks + 1, f) : operand(next, 0, f);
+        const int x = j / kNB, y = j % kNB;
+        acc[x][y] = lfg_mfma(({elem})0.0f, fr[ks & 1][kMB + y], fr[ks & 1][x], acc[x][y]);
+        if (ks == kKS - 1) {{
 #pragma unroll
-      for (int x = 0; x < kMB; ++x)
-#pragma unroll
-        for (int y = 0; y < kNB; ++y) acc[x][y] = lfg_mfma(({elem})0.0f, fn[y], fm[x], acc[x][y]);
+          for (int l = j * kP / kMF; l < (j + 1) * kP / kMF; ++l) issue(cur, l);
+        }}
+        __builtin_amdgcn_sched_barrier(0);
+      }}
     }}
-    // this wave's loads of the next tile have landed, every wave is done reading this one
-    LFG_NEXT_STAGE();
-    cur = cur == kS - 1 ? 0 : cur + 1;
+    advance();
+    cur = next;
   }}
-#undef LFG_NEXT_STAGE
-  // the loads against nothing still write zeros: none may be left when the LDS changes its role or is given back
-  if (kS > 2) asm volatile("s_waitcnt vmcnt(0)\\n\\ts_barrier" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // the loads against nothing still write zeros, and the last operands read are of such a stage: nothing may be left of
+  // either when the LDS changes its role or is given back
+  LFG_STAGE_BARRIER(0);
 #if LFG_SPLIT
   // partials in accumulator order: [part][tile][wave][32 x 32 block][4][64 lanes] x 4 floats, every store 1 KB in a row
   float* ws = reinterpret_cast<float*>(p.ptr[{g.ws_ptr}]) +
-              (((part * (total / (mt * nt)) + element) * mt + tm) * nt + tn) * (kBM * kBN) + wave * (kMB * kNB * 1024) + 4 * lane;
+              ((part * (long long)total + (long long)element * (mt * nt)) + (long long)tm * nt + tn) * (kBM * kBN) + wave * (kMB * kNB * 1024) + 4 * lane;
 #pragma unroll
   for (int x = 0; x < kMB; ++x)
 #pragma unroll
@@ -527,35 +570,46 @@ extern "C" __global__ void __launch_bounds__(256) {self.name}_sum(const LfGenPar
 
 
 
-# us per step of 64 k with every CU busy (s: see choose), us per workgroup besides (first loads, results), workgroups resident at a time
-_COST = {"s": (0.0, 4.0, 512), "d": (0.80, 5.0, 256), "m": (1.02, 5.0, 256), "l": (1.95, 8.0, 256)}
+# us per step of 64 k with every CU busy (s, n: up to 256 workgroups, one per CU, and beyond), us per workgroup besides (first
+# loads, results), workgroups resident at a time
+_COST = {"s": ((0.65, 1.01), 7.0, 512), "d": ((0.53, 0.53), 7.4, 256), "m": ((0.84, 0.84), 8.2, 256),
+         "l": ((1.38, 1.38), 9.5, 256), "n": ((0.46, 0.94), 5.2, 512)}
 
 
 @functools.lru_cache(maxsize=4096)
 def choose(M: int, N: int, K: int, batch: int) -> tuple:
     """(tile shape, parts that k is split into) of a product: the candidate with the least time in a model of rounds of
-    resident workgroups, plus, for a split product, the sum's launch and the traffic of its partials.  Against every
-    candidate on 22 shapes (M 16 ... 8192, N and K 1024 ... 16384, weights from HBM) the choice is the best on 13, within 4 % of
-    it on 17 and 13 % off at worst (1024 x 1024 x 1024: s in 4 parts 18.3, d in 2 16.1, s whole 17.6 us).  What it is for: a product whose tiles leave most CUs idle, or alone with the latency
-    of their loads.  M 256, us: N 4096 K 16384 241 (64 tiles s) -> 52 (m, 8 parts); N 16384 K 4096 72 -> 54 (m, 2 parts);
-    M 64, N 4096 K 16384 235 -> 33 (d, 8 parts); M 1024, N 4096 K 16384 246 -> 145 (m, 2 parts)."""
+    resident workgroups, plus, for a split product, the sum's launch and the traffic of its partials.  The model's constants
+    are fitted to every candidate on 42 shapes (M 16 ... 8192, N 640 ... 16384, K 512 ... 16384, weights from HBM); there the
+    choice is within 3 % of the best on 39, the others are 5 % (777 x 3000, K 5000), 10 % (6388 x 2880, K 1472, with gelu: m 98.9,
+    s 90.3 us) and 11 % off (100 x 1024, K 4096: n in 16 parts 12.8, in 8 11.5).  What it is for: a product whose tiles leave
+    most CUs idle, or alone with the latency of their loads.  M 256, us: N 4096 K 16384 218 (64 tiles s) -> 49 (d, 4 parts);
+    N 16384 K 4096 66 -> 46 (d); M 64, N 4096 K 16384 214 -> 29 (n, 8 parts); M 1024, N 4096 K 16384 218 -> 130 (l, 4 parts);
+    M 2000, N 1024 K 512 17 -> 11 (n)."""
     steps = -(-K // BK)
     best, best_t = ("s", 1), math.inf
-    for shape, (step, fixed, slots) in _COST.items():
+    for shape, ((step_1, step_2), fixed, slots) in _COST.items():
         bm, bn = tile_extent(shape)
-        if shape in "ml" and M <= bm // 2 or shape == "l" and N <= bn // 2:
+        if shape in "mln" and M <= bm // 2 or shape == "l" and N <= bn // 2:
             continue                         # half of the tile would be padding
         tiles = -(-M // bm) * -(-N // bn) * batch
         for parts in range(1, max(1, min(32, steps // 4)) + 1):
             if parts > 1 and tiles * parts > slots:      # one round, whose partials are 2^24 floats at most
                 break
-            if shape == "s":
-                step = 1.5 if M <= 128 else 1.3 if M <= 256 else (0.85 if tiles * parts <= 256 else 1.05)     # two stages: the latency of memory shows
-            elif shape == "d" and M <= 128:
-                step = 0.72
-            t = -(-tiles * parts // slots) * (-(-steps // parts) * step + fixed)
+            per_part = -(-steps // parts)
+            rounds, rest = divmod(tiles * parts, slots)
+            t = rounds * (per_part * step_2 + fixed)
+            if rest:
+                t += per_part * (step_1 if rest <= 256 else step_2) + fixed
             if parts > 1:
-                t += 4.0 + parts * M * N * batch * 8 / 6e6
+                t += 1.1 + 0.087 * parts + parts * M * N * batch * 8 / 5.8e6
             if t < best_t:
                 best, best_t = (shape, parts), t
     return best
+
+
+def stream_b(M: int) -> bool:
+    """B by non-temporal loads: where at most four tile rows, resident at the same time, read it, so that it need not stay in an
+    L2 it would push A out of.  us, plain / non-temporal, M x N x K: 16 x 4096 x 4096 14.1 / 13.3, 64 x 16384 x 4096 33.7 /
+    30.4, 256 x 16384 x 4096 48.3 / 46.2; 512 x 4096 x 4096 32.6 / 33.1, 400 x 2048 x 8192 30.0 / 31.3."""
+    return M <= 256

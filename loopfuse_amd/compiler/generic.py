@@ -116,13 +116,13 @@ class GenericProgram:
             self._loaded[dev] = ([mod.kernel(k.name) for k in self.kernels], {i: mod.kernel(k.name) for i, k in self.wave.items()})
         return self._loaded[dev]
 
-    def _gemm_kernel(self, ni: int, layouts, shape: str, split: bool = False):
+    def _gemm_kernel(self, ni: int, layouts, shape: str, split: bool = False, b_streams: bool = False):
         """The product kernel of nest ``ni`` and, for a split product, the kernel that adds up the parts."""
         from .. import lowering, runtime
-        key = (torch.cuda.current_device(), tuple(layouts), shape, split)
+        key = (torch.cuda.current_device(), tuple(layouts), shape, split, b_streams)
         if key not in self._gemm_loaded:
             opts = list(lowering.COMMON_OPTS) + [f"-DLFG_A_ROWS={layouts[0]}", f"-DLFG_B_ROWS={layouts[1]}"] + \
-                emit_gemm.tile_options(shape, split)
+                emit_gemm.tile_options(shape, split, b_streams)
             src = self.gemm_source + ("".join(info.sum_source for _, info in self.gemm.values()) if split else "")
             code, _, _ = runtime.compile_source(src, "lf_generic_mfma", opts)
             mod = runtime.Module(code)
@@ -251,7 +251,8 @@ class GenericProgram:
                     layouts = None
                 if layouts is not None and all(ext.get(a.id, 0) > 0 for a in self.gemm[ni][0].atoms):
                     shape, parts = self._gemm_shape(self.gemm[ni][1], ext)
-                    steps += self._launch_gemm(self._gemm_kernel(ni, layouts, shape, parts > 1), shape, parts, *self.gemm[ni],
+                    fns = self._gemm_kernel(ni, layouts, shape, parts > 1, emit_gemm.stream_b(ext[self.gemm[ni][1].m.id]))
+                    steps += self._launch_gemm(fns, shape, parts, *self.gemm[ni],
                                                bufs, ext, args, lambda name, n: allocs.append((len(steps), name, (n,), torch.float32)))
                     counters["mfma"] += 1
                     n_mfma += 1

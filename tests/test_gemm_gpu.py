@@ -243,6 +243,25 @@ def test_split_products_and_tile_shapes(tile, parts, M, N, K, dtype, monkeypatch
         assert torch.equal(run(a, b, c), got)
 
 
+@pytest.mark.parametrize("tile,M,N", [("n", 33, 136), ("n", 130, 72), ("s", 200, 136), ("d", 129, 264), ("m", 272, 136), ("l", 264, 392)])
+@pytest.mark.parametrize("a_rows,b_rows", [(True, True), (True, False), (False, True), (False, False)])
+def test_operands_read_across_stages(tile, M, N, a_rows, b_rows, monkeypatch):
+    """The loop that reads a step's first operands before the barrier of the step's stage: every tile and operand layout, fewer
+    steps of 64 than LDS stages, as many and more, k ending inside a step, one part and two, B by plain (M > 256) and by
+    non-temporal loads.  Same bound as the other products."""
+    monkeypatch.setenv("LOOPFUSE_GEMM_TILE", tile)
+    for K, parts in ((40, 1), (64, 1), (64 * 3, 1), (64 * 6 + 8, 1), (64 * 9 + 24, 2)):
+        monkeypatch.setenv("LOOPFUSE_GEMM_PARTS", str(parts))
+        m = M if a_rows else -(-M // 8) * 8       # the contiguous extent is a multiple of 8
+        a = (rand((m, K), BF, 1, 0.5) if a_rows else rand((K, m), BF, 1, 0.5).t()).to(DEV)
+        b = (rand((N, K), BF, 2, 0.5).t() if b_rows else rand((K, N), BF, 2, 0.5)).to(DEV)
+        c = rand((N,), BF, 3).to(DEV)
+        before = dict(generic.counters)
+        got = _compiled(lambda a, b, c: torch.tanh((a @ b) * 0.125 + c))(a, b, c)
+        assert generic.counters["mfma"] == before["mfma"] + 1 and generic.counters["plain"] == before["plain"]
+        _close(got, torch.tanh((a.double().cpu() @ b.double().cpu()) * 0.125 + c.double().cpu()), BF)
+
+
 def test_softmax_times_matrix_at_the_reference_size():
     """``softmax(x) @ y`` with x [4, 8, 1024, 64], y [4, 8, 64, 1024] in bf16 (reference tests/test_accuracy.py:197-211,
     its own size): 2^31 multiply-adds, which the plain kernels are not allowed.  The row maxima and sums are plain
