@@ -49,6 +49,41 @@ def _host_build(prog: generic.GenericProgram, tmp_path):
     return out
 
 
+def test_gelu_without_branches(tmp_path):
+    """``lfg_gelu`` (host build of the device text) against float64: over the whole line no further off than the same formula with
+    an erff correctly rounded (absolute, 2-norm), digits kept where the result is small (1e-5 relative down to x = -4, which
+    1 + erff loses to 5e-4), the two pieces' border at |x| = sqrt 2, signed zeros, infinities and NaN as x (1 + erf) / 2 gives them."""
+    import math
+
+    import numpy as np
+
+    src = tmp_path / "gelu.cpp"
+    src.write_text(HOST_PRELUDE + emit.PRELUDE +
+                   'extern "C" void run(const float* x, float* y, long n) { for (long i = 0; i < n; ++i) y[i] = lfg_gelu(x[i]); }')
+    so = tmp_path / "gelu.so"
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", str(src), "-o", str(so)], check=True)
+    edge = np.float32(math.sqrt(2.0))
+    special = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 7.0710, 7.0712, -7.0710, -7.0712, 1e-30, -1e-30, 3e38, -3e38], np.float32)
+    near = np.nextafter(edge, np.float32(0)) + np.arange(-50, 50, dtype=np.float32) * np.spacing(edge)
+    x = np.concatenate([np.random.default_rng(1).standard_normal(200000).astype(np.float32), np.linspace(-9, 9, 200001, dtype=np.float32), near, -near, special])
+    y = np.empty_like(x)
+    ctypes.CDLL(str(so)).run(ctypes.c_void_p(x.ctypes.data), ctypes.c_void_p(y.ctypes.data), ctypes.c_long(x.size))
+    xd = torch.from_numpy(x).double()
+    want = (xd * 0.5 * torch.special.erfc(-xd / math.sqrt(2.0))).numpy()
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isnan(want), np.isnan(y)) and np.array_equal(want[~fin & ~np.isnan(want)], y[~fin & ~np.isnan(want)])
+    assert np.array_equal(np.signbit(y[-13:-11]), [False, True])
+    z32 = (x * np.float32(0.70710678)).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        plain = np.float32(0.5) * x * (np.float32(1) + torch.erf(torch.from_numpy(z32)).numpy().astype(np.float32))
+        err, err_plain = np.abs(y - want), np.abs(plain - want)
+    n = 200000
+    assert np.linalg.norm(err[:n]) <= np.linalg.norm(err_plain[:n])
+    assert err[n:2 * n + 200].max() <= err_plain[n:2 * n + 200].max()
+    small = fin & (np.abs(x) < 4) & (x != 0)
+    assert (err[small] / np.abs(want[small])).max() < 1e-5
+
+
 def _softmax64(x):
     e = torch.exp(x - x.amax(dim=-1, keepdim=True))
     return e / e.sum(dim=-1, keepdim=True)
