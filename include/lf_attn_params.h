@@ -92,12 +92,14 @@ typedef struct LfAttnBwdParamsHost {
   int32_t window;       /* sliding-window width (LF_MASK == 2) */
   float scale;
   float softcap;        /* LF_SOFTCAP: cap of cap * tanh(s / cap) */
+  void* ds;             /* LF_BW_DS: scratch for dS, 32 x 32 blocks, written by lf_attn_bwd_dkdv and read by lf_attn_bwd_dq behind it */
+  int64_t ds_sh;        /* elements of it per (batch, query head): 1024 * the blocks that hold a visible score */
 } LfAttnBwdParamsHost;
 
 #ifdef __cplusplus
-static_assert(sizeof(LfAttnBwdParamsHost) == 304, "LfAttnBwdParamsHost must match the device struct");
+static_assert(sizeof(LfAttnBwdParamsHost) == 320, "LfAttnBwdParamsHost must match the device struct");
 #else
-_Static_assert(sizeof(LfAttnBwdParamsHost) == 304, "LfAttnBwdParamsHost must match the device struct");
+_Static_assert(sizeof(LfAttnBwdParamsHost) == 320, "LfAttnBwdParamsHost must match the device struct");
 #endif
 
 #ifdef __cplusplus

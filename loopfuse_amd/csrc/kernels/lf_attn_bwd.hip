@@ -8,8 +8,10 @@
 // dS picks up the derivative of the cap: dS = scale * (1 - tanh^2) * P * (dP - delta).
 // Three kernels, no atomics, every result written once (deterministic):
 //   lf_attn_bwd_delta : delta[b, h, q], in front of the other two unless lf_attn_bwd_dq has 256 threads and forms it itself
+//                       (never with LF_BW_DS)
 //   lf_attn_bwd_dq    : a workgroup owns 128 or 256 query rows of one (batch, head) -- 4 or 8 waves x
-//                       32 rows, Q^T and dO^T in registers -- and walks the kv tiles (64 keys)
+//                       32 rows, Q^T and dO^T in registers -- and walks the kv tiles (64 keys); with LF_BW_DS it
+//                       reads the dS that lf_attn_bwd_dkdv has left instead of forming it, and runs behind it
 //   lf_attn_bwd_dkdv  : a workgroup owns 128 or 256 keys of one (batch, kv head) -- 4 waves x 32 or 64
 //                       keys, K^T and V^T of its keys in registers as MFMA B operands -- and walks the
 //                       q tiles (64 rows) of the query heads of the group that can see them
@@ -41,6 +43,8 @@ struct LfAttnBwdParams {
   int window;
   float scale;
   float softcap;          // LF_SOFTCAP: cap of cap * tanh(s / cap)
+  lf_elem* ds;            // LF_BW_DS: dS as lf_attn_bwd_dkdv leaves it for lf_attn_bwd_dq, lf_bw_ds_row below
+  long long ds_sh;        // elements of it per (batch, query head)
 };
 
 #define LF_BW_NT 256
@@ -58,6 +62,30 @@ __device__ __forceinline__ bool lf_bw_keep(int t, int window) {
 #else
   return (unsigned)t < (unsigned)window;
 #endif
+}
+
+#ifndef LF_BW_DS
+#define LF_BW_DS 0         /* 1: lf_attn_bwd_dkdv leaves dS in memory, lf_attn_bwd_dq is the one product dQ = dS K */
+#endif
+// dS in memory: per (batch, query head) the 32 x 32 blocks (2 KB) that hold a visible score, those of 32 queries in a row in the
+// order of their keys.  Blocks in front of block (qb, 0) of a head, nkb = key blocks; under a window a row starts at key
+// block qb - (window + 30) / 32, which may lie before the first.
+__device__ __forceinline__ int lf_bw_ds_row(int qb, int nkb, int window) {
+#if LF_MASK == 0
+  return qb * nkb;
+#elif LF_MASK == 1
+  const int m = min(qb, nkb);
+  return m * (m + 1) / 2 + (qb - m) * nkb;
+#else
+  const int before = (window + 30) / 32;
+  return qb * (before + 1) - (qb - before);
+#endif
+}
+// A block holds what the lanes of lf_attn_bwd_dkdv hold as the B operand of dK^T += Q^T dS, 16-byte chunks (half h of the 32
+// queries, lane half g, key) of 8 queries, permuted so that the transposed reads of lf_attn_bwd_dq (4 keys, all 16 queries
+// of both halves at a time) touch every LDS bank once: byte offset of lane (g, key)'s chunk of half 0; half 1 is (it ^ 128) + 1024.
+__device__ __forceinline__ unsigned lf_bw_ds_chunk(int key, int g) {
+  return 16u * (unsigned)(32 * g + 16 * (key >> 4) + 4 * (((key >> 2) & 3) ^ g) + (key & 3));
 }
 
 // delta[row] = sum_d dO[row][d] * O[row][d]; 16 lanes per row, 8 elements per lane
@@ -221,6 +249,13 @@ __device__ __forceinline__ void lf_dma_dword_to_lds_at(const lf_u32x4& rs, unsig
                : "={m0}"(m0_written) : "s"(lds_addr), "v"(voff), "s"(rs) : "memory");
 }
 
+// lf_dma_to_lds_at for bytes that are read once: they do not push what is shared out of the L2
+__device__ __forceinline__ void lf_dma_nt_to_lds_at(const lf_u32x4& rs, unsigned voff, unsigned lds_addr) {
+  unsigned m0_written;
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen nt lds"
+               : "={m0}"(m0_written) : "s"(lds_addr), "v"(voff), "s"(rs) : "memory");
+}
+
 // MFMAs with every operand in VGPRs (the accumulator: VGPRs); first of a chain: started from `c0`, or from zero.  The
 // matrix core reads `c0` late: keep it alive (LF_BW_HOLD) until another MFMA has been issued behind its readers.
 #define LF_BW_HOLD(c0) asm volatile("" :: "v"(c0))
@@ -273,6 +308,8 @@ __device__ __forceinline__ void lf_bw_mfma_hidden(const lf_f32x16& c, const lf_u
 // 129 / 127, unmasked B2 32/8 S4096 1627 / 1618, softcap B4 32/8 S2048 631 / 628).
 // Three LDS stages: a tile's loads are issued in the second half of the step two before its own, and the one barrier per
 // step, in its middle, says both that the next tile has landed and that the tile before this one is free.
+// With LF_BW_DS the B operands dS also leave for memory, two stores per 32 x 32 block between the MFMAs that take them, and the
+// barrier does not wait for them: 297 -> 340 us of the above for 545 MB (352 with plain stores, which take L2 from Q and dO).
 extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const LfAttnBwdParams p) {
   constexpr int KB = LF_BW_W;
   constexpr int kKeys = 128 * KB;
@@ -428,6 +465,14 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     for (int f = 0; f < LF_BW_PF; ++f) pre[f] = frag(st, qb, f);
   };
 
+#if LF_BW_DS
+  const int nkb = (p.Sk + 31) / 32;
+  lf_elem* ds_head = p.ds + ((long long)b * p.Hq + hkv * group) * p.ds_sh;      // of the query head that is walked
+  int ds_young = 0;                // stores of this wave behind its last direct loads
+  unsigned ds_off = lf_bw_ds_chunk(l32, g);
+  asm volatile("" : "+v"(ds_off));
+#endif
+
   // One block of a wave: 32 queries (qb of stage st, first one q0) x its keys.  `loads`: those of stage `ld` are
   // issued between the MFMAs; the block read ahead is (st_n, qb_n).
   auto block = [&](const int qb, int st, int q0, const bool masked, const bool loads, int ld, int st_n, const int qb_n) {
@@ -567,6 +612,26 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
       ahead(2 * NS + NT + j);
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) lf_bw_mfma_hidden(dk[kb][j % LF_NDB], fr[2 * NS + NT + j], dsf[kb][j / LF_NDB]);
+#if LF_BW_DS
+      if (j % (NT / (2 * KB)) == 0) {
+        const int t = j / (NT / (2 * KB)), kb = t / 2, half = t % 2, key = key0 + 32 * kb;
+        bool store = true;
+        if (masked) {
+          store = key < p.Sk;
+#if LF_MASK >= 1
+          store = store && key <= q0;
+#endif
+#if LF_MASK == 2
+          store = store && q0 - (min(key + 32, p.Sk) - 1) < p.window;
+#endif
+        }
+        if (store) {
+          ++ds_young;
+          char* at = reinterpret_cast<char*>(ds_head) + 2048ll * (lf_bw_ds_row(q0 / 32, nkb, p.window) + key / 32);
+          __builtin_nontemporal_store(dsf[kb][half], reinterpret_cast<lf_u32x4*>(at + 1024 * half + (half ? ds_off ^ 128u : ds_off)));
+        }
+      }
+#endif
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -611,7 +676,18 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
       if (!need(q0)) read_ahead(st, 1);
       else if (full(q0)) block(0, st, q0, false, false, 0, st, 1);
       else block(0, st, q0, true, false, 0, st, 1);
-      LF_BW_BARRIER();            // the next tile has landed; every wave is done with the one before this
+      // the next tile has landed; every wave is done with the one before this
+#if LF_BW_DS
+      // (stores of dS behind the loads stay in flight: the counter retires in order)
+      asm volatile("" ::: "memory");
+      if (ds_young == 4 * KB) __builtin_amdgcn_s_waitcnt(0x0070 | 4 * KB);
+      else __builtin_amdgcn_s_waitcnt(0x0070);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      ds_young = 0;
+#else
+      LF_BW_BARRIER();
+#endif
       aim();
       if (!need(q0 + 32)) {
 #pragma unroll
@@ -627,6 +703,9 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
       if (--left == 0) {
         left = ntq;
         q0 = 64 * qt_begin;
+#if LF_BW_DS
+        ds_head += p.ds_sh;
+#endif
       }
     }
     __builtin_amdgcn_s_waitcnt(0x0070);      // the last loads, against an empty range, before the LDS is given back
@@ -658,6 +737,147 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
 #endif
 #define LF_BW_DQ_PF 4    /* fragments read ahead of the MFMAs that take them */
 
+#if LF_BW_DS
+// dQ of LF_BW_DQ_NT / 2 query rows of one (batch, head), 32 per wave, from the dS that lf_attn_bwd_dkdv left: dQ^T += K^T dS^T.
+// Bound by its loads: dS once, 2 bytes per visible score, and a K tile from L2 per 64 keys and workgroup, which return to a CU
+// in order.  Causal bf16 B4 H32 S2048 D128, 545 MB of dS: 131 us (126 with the products left out; 152 where the loads of dS
+// are plain ones and push K out of the L2), against 222 us of the kernel below, which forms dS again.  A step is 64 keys: the
+// K tile, and every wave's own two blocks of dS, 4 KB in a row of memory; three LDS stages, one barrier.  Steps of 32 keys in
+// 3 ... 6 stages: 143 ... 148 us.
+extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_attn_bwd_dq(const LfAttnBwdParams p) {
+  constexpr int kBM = LF_BW_DQ_NT / 2, kWaves = LF_BW_DQ_NT / 64, kS = 3;
+  __shared__ __attribute__((aligned(256))) lf_elem k_tiles[kS][64 * LF_D];
+  __shared__ __attribute__((aligned(256))) lf_elem ds_tiles[kS][kWaves][2 * 1024];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31;
+  const int g = lane >> 5;
+
+  const int nqt = (p.Sq + kBM - 1) / kBM;
+  const int group = p.Hq / p.Hkv;
+  int bhkv, row;
+  if (!lf_slot_of_block(blockIdx.x, p.B * p.Hkv, group * nqt, LF_BW_GROUP, bhkv, row)) return;
+  const int qt = nqt - 1 - row / group;
+  const int hkv = bhkv % p.Hkv;
+  const int b = bhkv / p.Hkv;
+  const int h = hkv * group + row % group;
+  const int q0 = kBM * qt;
+  const int wq0 = q0 + 32 * wave;                    // first row of this wave
+  const int my_q = wq0 + l32, qr = min(my_q, p.Sq - 1);
+
+  int kt_begin = 0, kt_end = (p.Sk + 63) / 64;
+  {
+    const int qlast = min(q0 + kBM, p.Sq) - 1;
+#if LF_MASK >= 1
+    kt_end = min(kt_end, qlast / 64 + 1);
+#endif
+#if LF_MASK == 2
+    const int lo = q0 - p.window + 1;
+    if (lo > 0) kt_begin = lo / 64;
+#endif
+    (void)qlast;
+  }
+  const unsigned k_rowb = (unsigned)p.k_ss * 2u;
+  const unsigned k_bytes = (unsigned)(((long long)(p.Sk - 1) * p.k_ss + LF_D) * 2);
+  lf_u32x4 k_rs = lf_make_buffer(p.k + (long long)b * p.k_sb + (long long)hkv * p.k_sh, k_bytes);
+  const unsigned k_loff = lf_bw_load_off(k_rowb, tid);
+  // the wave's row of blocks; what it does not hold (keys behind the diagonal, past the last, in front of the window) lies
+  // outside the range and arrives as zeros
+  const int nkb = (p.Sk + 31) / 32, qb = wq0 / 32;
+  const int row0 = lf_bw_ds_row(qb, nkb, p.window), row1 = lf_bw_ds_row(qb + 1, nkb, p.window);
+  const int first = LF_MASK == 2 ? max(0, qb - (p.window + 30) / 32) : 0;      // its first key block
+  const bool rows = wq0 < p.Sq;
+  const lf_elem* ds_row = p.ds + ((long long)b * p.Hq + h) * p.ds_sh + 1024ll * (row0 + first);
+#if LF_MASK == 2
+  const int count = min(qb + 1, nkb) - first;
+  (void)row1;
+#else
+  const int count = row1 - row0;
+#endif
+  lf_u32x4 ds_rs = lf_make_buffer(ds_row, rows && count > 0 ? 2048u * (unsigned)count : 0u);
+
+  constexpr int kPasses = 64 * LF_CPR / LF_BW_DQ_NT;      // K loads of a wave per tile
+  constexpr int kLoads = kPasses + 4;
+  static_assert(kLoads * (kS - 2) < 16, "loads left in flight");
+  const unsigned k0_lds = lf_lds_addr(k_tiles), ds0_lds = lf_lds_addr(ds_tiles);
+  auto k_tile = [&](int st) { return k0_lds + (unsigned)(st * LF_BW_TILEB); };
+  auto ds_tile = [&](int st) { return ds0_lds + (unsigned)((st * kWaves + wave) * 4096); };
+  int ld_kt = kt_begin;
+  auto issue = [&](int st) {
+    if (ld_kt >= kt_end) k_rs[2] = ds_rs[2] = 0u;       // past the last tile: against an empty range
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      lf_dma_nt_to_lds_at(ds_rs, (unsigned)(2 * ld_kt - first) * 2048u + 1024u * (unsigned)j + 16u * (unsigned)lane,
+                          ds_tile(st) + 1024u * (unsigned)j);
+#pragma unroll
+    for (int j = 0; j < kPasses; ++j) lf_bw_load_rows<LF_BW_DQ_NT>(k_rs, k_rowb, 64 * ld_kt, k_tile(st), k_loff, j, wave);
+    ++ld_kt;
+  };
+  // does the wave have a score to keep in keys k .. k + 31 (lf_attn_bwd_dkdv has written those blocks)?
+  auto need = [&](int k) {
+    bool n = rows && k < p.Sk;
+#if LF_MASK >= 1
+    n = n && k <= wq0;
+#endif
+#if LF_MASK == 2
+    n = n && min(k + 32, p.Sk) - 1 >= wq0 - p.window + 1;
+#endif
+    return n;
+  };
+
+  lf_f32x16 dq[LF_NDB];
+#pragma unroll
+  for (int db = 0; db < LF_NDB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dq[db][i] = 0.0f;
+  const unsigned tr_off = lf_bw_tr_off(lane);
+  // dS^T[key][query] fragments: lane % 32 the query, keys 16 * kk + 8 * half + 4 * g + 0 .. 3
+  const int j16 = lane & 15, hq = (lane >> 4) & 1, u = 2 * hq + (j16 & 1);
+  const unsigned ds_off = (unsigned)(512 * u + 64 * (g ^ u) + 16 * (j16 >> 2) + 8 * ((j16 >> 1) & 1));
+  if (kt_begin < kt_end) {
+#pragma unroll
+    for (int s = 0; s < kS - 1; ++s) issue(s);
+    int st = 0;
+    for (int kt = kt_begin; kt < kt_end; ++kt) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt((kLoads * (kS - 2)) | 0x70);          // the tile has landed (the next one's loads are in flight) ...
+      __builtin_amdgcn_s_barrier();                       // ... for every wave, and every wave is done with the one before
+      asm volatile("" ::: "memory");
+      issue(st == 0 ? kS - 1 : st - 1);
+      const unsigned kb0 = k_tile(st) + tr_off, sb0 = ds_tile(st) + ds_off;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        if (!need(64 * kt + 32 * kb)) continue;
+#pragma unroll
+        for (int kk = 2 * kb; kk < 2 * kb + 2; ++kk) {
+          lf_u32x4 sf;
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            const unsigned at = (half ? sb0 ^ 128u : sb0) + (unsigned)(2048 * kb + 256 * (kk & 1));
+            const lf_u32x2 t = __builtin_bit_cast(lf_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lf_bw_lds_s16x4)(size_t)at));
+            sf[2 * half] = t[0];
+            sf[2 * half + 1] = t[1];
+          }
+#pragma unroll
+          for (int db = 0; db < LF_NDB; ++db)
+            dq[db] = lf_mfma32(__builtin_bit_cast(lf_elem8, lf_bw_read_tr(kb0, 0, kk, db)), __builtin_bit_cast(lf_elem8, sf), dq[db]);
+        }
+      }
+      st = st == kS - 1 ? 0 : st + 1;
+    }
+    __builtin_amdgcn_s_waitcnt(0x0070);      // the last loads, against an empty range, before the LDS is given back
+  }
+#pragma unroll
+  for (int db = 0; db < LF_NDB; ++db) asm volatile(LF_BW_MFMA_DRAIN_LAST : "+a"(dq[db]));
+#pragma unroll
+  for (int db = 0; db < LF_NDB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dq[db][i] *= p.scale;
+  lf_bw_store_rows(dq, p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)qr * p.dq_ss, my_q < p.Sq, g);
+}
+#else
 // dQ of LF_BW_DQ_NT / 2 query rows of one (batch, head), 32 per wave.
 // A wave walks blocks of 32 keys, two per 64-key tile, as lf_attn_bwd_dkdv walks blocks of queries: fragments through one
 // read-ahead ring, three LDS stages, one barrier in the middle of a step.  Per block:
@@ -983,3 +1203,4 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
     for (int i = 0; i < 16; ++i) dq[db][i] *= p.scale;
   lf_bw_store_rows(dq, p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)qr * p.dq_ss, my_q < p.Sq, g);
 }
+#endif

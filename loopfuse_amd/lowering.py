@@ -1093,8 +1093,23 @@ class AttnBwdParams(ctypes.Structure):
         [(n, ctypes.c_void_p) for n in ("q", "k", "v", "o", "dout", "dq", "dk", "dv", "lse", "delta")]
         + [(f"{t}_{x}", ctypes.c_longlong) for t in ("q", "k", "v", "o", "do", "dq", "dk", "dv") for x in ("sb", "sh", "ss")]
         + [(n, ctypes.c_int) for n in ("B", "Hq", "Hkv", "Sq", "Sk", "window")]
-        + [("scale", ctypes.c_float), ("softcap", ctypes.c_float)]
+        + [("scale", ctypes.c_float), ("softcap", ctypes.c_float), ("ds", ctypes.c_void_p), ("ds_sh", ctypes.c_longlong)]
     )
+
+
+BWD_DS_BLOCK = 32 * 32      # elements of a block of dS (lf_bw_ds_row in csrc/kernels/lf_attn_bwd.hip)
+
+
+def bwd_ds_blocks(mask: int, window: int, Sq: int, Sk: int) -> int:
+    """Blocks of dS of one (batch, query head): ``lf_bw_ds_row`` of the row behind the last, and under a window the blocks in
+    front of the first key that the last row's start leaves out."""
+    nqb, nkb = -(-Sq // 32), -(-Sk // 32)
+    if mask == MASK_NONE:
+        return nqb * nkb
+    if mask == MASK_CAUSAL:
+        m = min(nqb, nkb)
+        return m * (m + 1) // 2 + (nqb - m) * nkb
+    return nqb * ((window + 30) // 32 + 1)
 
 
 def bwd_dq_threads(D: int, mask: int, softcap: bool, units: int, Sq: int, Sk: int) -> int:
@@ -1134,21 +1149,37 @@ def bwd_key_blocks(D: int, mask: int, softcap: bool, units: int, Sk: int) -> int
     return 2 if n >= 256 and n >= 0.85 * 256 * -(-n // 256) else 1
 
 
+def bwd_keep_ds(D: int, softcap: bool, units: int, group: int, Sk: int, blocks: int) -> bool:
+    """Does lf_attn_bwd_dkdv leave dS in memory, so that lf_attn_bwd_dq is one product that reads it instead of three that form
+    it again?  ``units`` = batch x query heads, ``blocks`` = of dS in all (2 KB each; up to 2 GiB).  Seven products instead of
+    nine against 2 bytes per visible score written and read, both by non-temporal accesses.  All launches, recomputed / kept, us:
+    head dimension 128, causal B4 H32 S2048 549 / 521 (545 MB), B2 32/8 S4096 953 / 909, B6 64/32 S769 369 / 307, with a softcap
+    B4 32/8 S2048 644 / 561, window 256 252 / 204, unmasked H2 S7033 392 / 311; of 30 drawn shapes one was slower, short with
+    eight heads per group (B6 16/2 S135 62 / 65).  Head dimension 64 has half the matrix work per score: with a softcap B4 H32
+    S2048 424 / 379, without B4 H32 S2048 304 / 333, B8 16/4 S1000 140 / 143, and kept where few heads leave CUs to the
+    recomputation's longest workgroups: H8 S4520 181 / 158, H2 S1038 52 / 47, B4 H16 S535 50 / 47."""
+    size = 2 * BWD_DS_BLOCK * blocks
+    if size > 2 << 30 or (Sk < 192 and group > 4):
+        return False
+    return D == 128 or softcap or (units <= 64 and Sk >= 512 and size <= 256 << 20)
+
+
 def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False, key_blocks: int = 1,
-             dq_threads: int = 512) -> KernelSpec:
+             dq_threads: int = 512, keep_ds: bool = False) -> KernelSpec:
     return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap,
-                      extra=(f"-DLF_BW_DQ_NT={dq_threads}", f"-DLF_BW_W={key_blocks}"))
+                      extra=(f"-DLF_BW_DQ_NT={dq_threads}", f"-DLF_BW_W={key_blocks}") + (("-DLF_BW_DS=1",) if keep_ds else ()))
 
 
 def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
                        dout: torch.Tensor, plan: AttnPlan, *, key_blocks: Optional[int] = None,
-                       dq_threads: Optional[int] = None):
+                       dq_threads: Optional[int] = None, keep_ds: Optional[bool] = None):
     """Gradients of ``attention(q, k, v, plan)`` for dense K/V (mask none / causal / sliding, scale,
     softcap; no bias or paging): returns ``(dq, dk, dv)`` in the operands' dtype.  ``o`` and ``lse``
     are the forward's output and row log-sum-exp (``attention(..., lse=...)``).  Two or
     three launches (csrc/kernels/lf_attn_bwd.hip): delta = rowsum(dO * O), together with dQ where that has small
-    workgroups; dK and dV, one workgroup per 128 or 256 keys of a (batch, kv head); dQ, one workgroup per 128
-    or 256 query rows.  No atomics: results are reproducible bit for bit."""
+    workgroups and forms dS itself; dK and dV, one workgroup per 128 or 256 keys of a (batch, kv head); dQ, one workgroup per 128
+    or 256 query rows, from dS left in a scratch tensor where ``bwd_keep_ds`` says so (``keep_ds`` overrides it).  No
+    atomics: results are reproducible bit for bit."""
     dtype = q.dtype
     if dtype not in _DTYPE_CODE:
         raise UnsupportedPlan(f"dtype {dtype} not supported by the MFMA kernels (bf16/fp16 only)")
@@ -1206,13 +1237,22 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     P.softcap = softcap if softcap is not None else 0.0
     keys = key_blocks or bwd_key_blocks(D, mask, cap, B * Hkv, Sk)
     nt = dq_threads or bwd_dq_threads(D, mask, cap, B * Hq, Sq, Sk)
-    spec = bwd_spec(dtype, D, mask, cap, keys, nt)
-    keep = (q, k, v, o, dout, lse, delta, dq, dk, dv)  # noqa: F841  (tensors stay alive until the launches are queued)
+    ds_blocks = bwd_ds_blocks(mask, window, Sq, Sk)
+    ds = None
+    if keep_ds if keep_ds is not None else bwd_keep_ds(D, cap, B * Hq, Hq // Hkv, Sk, B * Hq * ds_blocks):
+        try:
+            ds = torch.empty((B * Hq, ds_blocks, BWD_DS_BLOCK), dtype=dtype, device=q.device)
+            P.ds, P.ds_sh = ds.data_ptr(), ds.stride(0)
+        except torch.OutOfMemoryError:
+            if keep_ds:
+                raise                    # without it the gradients need no such room
+    spec = bwd_spec(dtype, D, mask, cap, keys, nt, ds is not None)
+    keep = (q, k, v, o, dout, lse, delta, dq, dk, dv, ds)  # noqa: F841  (tensors stay alive until the launches are queued)
     steps = {"lf_attn_bwd_delta": (-(-B * Hq * Sq // 16), 256),
              "lf_attn_bwd_dkdv": (xcd_slots(B * Hkv, -(-Sk // (128 * keys))), 256),
              "lf_attn_bwd_dq": (xcd_slots(B * Hkv, (Hq // Hkv) * -(-Sq // (nt // 2))), nt)}
-    # with 256 threads lf_attn_bwd_dq forms delta itself, and lf_attn_bwd_dkdv reads it
-    names = ["lf_attn_bwd_dq", "lf_attn_bwd_dkdv"] if nt == 256 else list(steps)
+    # without dS of lf_attn_bwd_dkdv, lf_attn_bwd_dq with 256 threads forms delta itself, and lf_attn_bwd_dkdv reads it
+    names = ["lf_attn_bwd_dq", "lf_attn_bwd_dkdv"] if nt == 256 and ds is None else list(steps)
     for name in names:
         grid, block = steps[name]
         get_kernel(spec, name).launch((grid, 1, 1), (block, 1, 1), P)
