@@ -91,6 +91,17 @@ int lf_launch(void* fn, unsigned gx, unsigned gy, unsigned gz,
               unsigned lds_bytes, void* stream, void** args);
 
 /*
+ * `count` launches in order on one stream that take the same parameter block (`params`, one by-value argument, read by
+ * every launch before the call returns): the kernels of one step, as a host that has launched it before keeps them.
+ * Blocks are (bx, 1, 1), no dynamic LDS.  Stops at the first launch that fails and returns its error.
+ */
+typedef struct lf_launch_item {
+  void* fn;
+  unsigned gx, gy, gz, bx;
+} lf_launch_item;
+int lf_launch_list(const lf_launch_item* items, int count, void* params, void* stream);
+
+/*
  * No counterpart in the reference.  For callers that cannot allocate device memory
  * (a stream under HIP graph capture, a tight serving loop, a harness that forbids
  * hipMalloc): one split decode step -- `fn_decode` (lf_attn_decode) on a (gx, gy)

@@ -271,6 +271,17 @@ int lf_launch(void* fn, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsi
   return 0;
 }
 
+int lf_launch_list(const lf_launch_item* items, int count, void* params, void* stream) {
+  if (!items || count < 1 || !params) return fail(LF_EINVAL, "lf_launch_list: no launches or no parameters");
+  void* args[1] = {params};
+  for (int i = 0; i < count; ++i) {
+    const lf_launch_item& it = items[i];
+    int rc = lf_launch(it.fn, it.gx, it.gy, it.gz, it.bx, 1, 1, 0, stream, args);
+    if (rc) return rc;
+  }
+  return 0;
+}
+
 int lf_device_count(void) {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess) return 0;

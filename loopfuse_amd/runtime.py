@@ -36,6 +36,7 @@ ABI_SYMBOLS = (
     "lf_get_function",
     "lf_module_unload",
     "lf_launch",
+    "lf_launch_list",
     "lf_launch_decode_static",
     "lf_static_scratch_bytes",
     "lf_device_info",
@@ -95,6 +96,8 @@ def lib() -> ctypes.CDLL:
         L.lf_module_unload.argtypes = [ctypes.c_void_p]
         L.lf_launch.restype = ctypes.c_int
         L.lf_launch.argtypes = [ctypes.c_void_p] + [ctypes.c_uint] * 7 + [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+        L.lf_launch_list.restype = ctypes.c_int
+        L.lf_launch_list.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
         L.lf_launch_decode_static.restype = ctypes.c_int
         L.lf_launch_decode_static.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
                                               ctypes.c_size_t, ctypes.c_size_t] + [ctypes.c_uint] * 5 + [ctypes.c_void_p]
@@ -193,6 +196,28 @@ class Kernel:
                           lds_bytes, ctypes.c_void_p(stream), args)
         if rc:
             _check(f"lf_launch[{self.symbol}]", rc)
+
+
+class _LaunchItem(ctypes.Structure):
+    """Mirror of ``lf_launch_item`` in include/lf_shim.h."""
+
+    _fields_ = [("fn", ctypes.c_void_p)] + [(n, ctypes.c_uint) for n in ("gx", "gy", "gz", "bx")]
+
+
+class LaunchList:
+    """The launches of a step, ``(kernel, grid, threads)`` each, for parameter blocks to come: one call of the library
+    instead of one per kernel."""
+
+    def __init__(self, steps: Sequence[tuple]):
+        self.kernels = [k for k, _, _ in steps]          # keeps the modules alive
+        self._items = (_LaunchItem * len(steps))(*[_LaunchItem(k.handle, *grid, threads) for k, grid, threads in steps])
+        self._at, self._count = ctypes.addressof(self._items), len(steps)
+        self._launch = lib().lf_launch_list
+
+    def launch(self, params: ctypes.Structure) -> None:
+        rc = self._launch(self._at, self._count, ctypes.addressof(params), current_stream_handle())
+        if rc:
+            _check(f"lf_launch_list[{', '.join(k.symbol for k in self.kernels)}]", rc)
 
 
 def launch_decode_static(decode: Kernel, combine: Kernel, params: ctypes.Structure, part_acc_bytes: int,

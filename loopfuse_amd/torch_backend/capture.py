@@ -31,6 +31,7 @@ example, so it costs microseconds and is immune to duck-sized symbols
 from __future__ import annotations
 
 import dataclasses
+import functools
 import itertools
 import math
 import operator
@@ -279,13 +280,46 @@ class AttentionMatch:
                                  denom_add=sum(self._number(t, vals) for t in self.denom_add),
                                  zero_blind_rows=self.zero_blind_rows)
 
+    @functools.cached_property
+    def plain(self) -> bool:
+        """Neither biases nor a second score product."""
+        return self.bias is None and self.out_bias is None and self.q2 is None and self.k2 is None
+
+    def _plan_of(self, vals) -> lowering.AttnPlan:
+        """``plan_for``, formed once per set of sizes and numbers among the inputs (one that holds a number in a tensor: on
+        every call)."""
+        key = []
+        for x in vals:
+            if isinstance(x, torch.Tensor):
+                if x.numel() <= 1:
+                    return self.plan_for(vals)
+                x = x.shape
+            elif type(x) is not int and type(x) is not float:
+                return self.plan_for(vals)
+            key.append(x)
+        key = tuple(key)
+        plan = self._plans.get(key)
+        if plan is None:
+            plan = self.plan_for(vals)
+            if len(self._plans) >= 64:
+                self._plans.clear()
+            self._plans[key] = plan
+        return plan
+
+    @functools.cached_property
+    def _plans(self) -> dict:
+        return {}
+
     def _operand(self, op: Operand, vals):
         t = vals[op.index]
         if op.paged:
             return t, vals[op.table_index]
         if t.dim() == 3:
             t = t.unsqueeze(0)         # [B*H, S, D] given without a batch dim
-        t = t.permute(op.perm)
+        if tuple(op.perm) != (0, 1, 2, 3):
+            t = t.permute(op.perm)
+        elif t.is_contiguous() and t.shape[-1] % 8 == 0 and not (t.is_cuda and t.data_ptr() % 16):
+            return t, None
         # the kernels read rows of D contiguous elements with 16-byte loads: a view that
         # walks D with a stride (K given as [B, H, D, S], reference tests/test_attention.py:265-282)
         # or sits on odd strides is copied once, O(S D) beside the O(S^2 D) attention
@@ -362,8 +396,15 @@ class AttentionMatch:
             raise lowering.UnsupportedPlan("tensors are not on the GPU")
         k, kt = self._operand(self.k, vals)
         v, vt = self._operand(self.v, vals)
-        B, Hq, Sq, Sk, D = self._shapes(vals)
         run = lowering.tuned_attention if self.tune else lowering.attention
+        if self.plain:
+            # no bias, no second product: nothing else of the call depends on the shapes
+            given = {"out": self.empty_out(vals, q.dtype, q.device)} if self.out_order else {}
+            out = run(q, k, v, self._plan_of(vals), kt, vt, **given)
+            if self.out_rank == 3:
+                out = out.view(out.shape[0] * out.shape[1], out.shape[2], out.shape[3])
+            return out
+        B, Hq, Sq, Sk, D = self._shapes(vals)
         given = {"out": self.empty_out(vals, q.dtype, q.device)} if self.out_order else {}
         added = self._bias_view(self.bias, vals, (B, Hq, Sq, Sk), as_mask=True)
         if added is not None and self.bias.keep:

@@ -242,8 +242,11 @@ def _training_graph(gm: torch.fx.GraphModule, sample_inputs):
 
 def _training_compiler(gm: torch.fx.GraphModule, sample_inputs) -> Callable:
     """fw_compiler / bw_compiler of a fused training graph: the graphs hold the custom ops
-    (``loopfuse_amd::attention_fwd`` / ``attention_bwd``) and run as they are."""
+    (``loopfuse_amd::attention_fwd`` / ``attention_bwd``), which are called without the dispatcher, and run as they are."""
+    from . import training
+
     stats["compiled_graphs"] += 1
+    gm = training.direct_calls(gm)
 
     def run(*args):
         stats["fused_training"] += 1

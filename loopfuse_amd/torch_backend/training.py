@@ -10,6 +10,7 @@ log-sum-exp -- ``B*H*S`` floats instead of the ``B*H*S*S`` probabilities the unf
 """
 from __future__ import annotations
 
+import functools
 import logging
 
 import torch
@@ -30,14 +31,16 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
     return t
 
 
-@torch.library.custom_op("loopfuse_amd::attention_fwd", mutates_args=())
-def attention_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: int, window: int,
-                  scale: float, softcap: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """O [B, Hq, Sq, D] and the rows' log-sum-exp [B, Hq, Sq] (float32, log2 units)."""
+@functools.lru_cache(maxsize=256)
+def _plan(mask: int, window: int, scale: float, softcap: float) -> lowering.AttnPlan:
+    return lowering.AttnPlan(mask=_MASK_NAME[mask], window=int(window), scale=float(scale),
+                             softcap=float(softcap) if softcap else None)       # 0: no cap
+
+
+def _attention_fwd(q, k, v, mask, window, scale, softcap):
     if not q.is_cuda:
         raise RuntimeError("loopfuse_amd: attention_fwd needs tensors on the GPU; the HIP path has no CPU fallback")
-    plan = lowering.AttnPlan(mask=_MASK_NAME[mask], window=int(window), scale=float(scale),
-                             softcap=float(softcap) if softcap else None)       # 0: no cap
+    plan = _plan(mask, window, scale, softcap)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
     counters["fwd"] += 1
     # the log-sum-exp is written by the direct-to-LDS kernel only: ask for it whatever LOOPFUSE_PREFILL says
@@ -50,19 +53,22 @@ def attention_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: int, 
                                   choice={"prefill": "swp"}), lse
 
 
+@torch.library.custom_op("loopfuse_amd::attention_fwd", mutates_args=())
+def attention_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: int, window: int,
+                  scale: float, softcap: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """O [B, Hq, Sq, D] and the rows' log-sum-exp [B, Hq, Sq] (float32, log2 units)."""
+    return _attention_fwd(q, k, v, mask, window, scale, softcap)
+
+
 @attention_fwd.register_fake
 def _(q, k, v, mask, window, scale, softcap):
     return q.new_empty(q.shape), q.new_empty(q.shape[:-1], dtype=torch.float32)
 
 
-@torch.library.custom_op("loopfuse_amd::attention_bwd", mutates_args=())
-def attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
-                  dout: torch.Tensor, mask: int, window: int, scale: float,
-                  softcap: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+def _attention_bwd(q, k, v, o, lse, dout, mask, window, scale, softcap):
     if not q.is_cuda:
         raise RuntimeError("loopfuse_amd: attention_bwd needs tensors on the GPU; the HIP path has no CPU fallback")
-    plan = lowering.AttnPlan(mask=_MASK_NAME[mask], window=int(window), scale=float(scale),
-                             softcap=float(softcap) if softcap else None)
+    plan = _plan(mask, window, scale, softcap)
     counters["bwd"] += 1
     try:
         return lowering.attention_backward(_rows(q), _rows(k), _rows(v), _rows(o), lse.contiguous(), _rows(dout), plan)
@@ -70,6 +76,13 @@ def attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Te
         counters["repacked"] += 1
         return lowering.attention_backward(q.contiguous(), k.contiguous(), v.contiguous(), o.contiguous(),
                                            lse.contiguous(), dout.contiguous(), plan)
+
+
+@torch.library.custom_op("loopfuse_amd::attention_bwd", mutates_args=())
+def attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
+                  dout: torch.Tensor, mask: int, window: int, scale: float,
+                  softcap: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    return _attention_bwd(q, k, v, o, lse, dout, mask, window, scale, softcap)
 
 
 @attention_bwd.register_fake
@@ -92,6 +105,31 @@ def _backward(ctx, d_o, d_lse):
 
 
 attention_fwd.register_autograd(_backward, setup_context=_setup)
+
+
+def _direct(op, fn):
+    """``op``'s implementation for a graph that AOTAutograd has already differentiated: plain tensors go straight to it, past
+    the dispatcher's autograd wrapper and the custom op's own (40 us per step of a small attention).  Anything that has to see
+    the op -- a tensor subclass, a dispatch or function mode, a functorch transform -- still does."""
+    def call(q, *rest):
+        if type(q) in (torch.Tensor, torch.nn.Parameter) and not torch._C._len_torch_dispatch_stack() \
+                and not torch._C._len_torch_function_stack() and torch._C._functorch.peek_interpreter_stack() is None:
+            return fn(q, *rest)
+        return op(q, *rest)
+    return call
+
+
+_DIRECT = {torch.ops.loopfuse_amd.attention_fwd.default: _direct(torch.ops.loopfuse_amd.attention_fwd.default, _attention_fwd),
+           torch.ops.loopfuse_amd.attention_bwd.default: _direct(torch.ops.loopfuse_amd.attention_bwd.default, _attention_bwd)}
+
+
+def direct_calls(gm: torch.fx.GraphModule) -> torch.fx.GraphModule:
+    """The forward or backward graph of AOTAutograd with its attention ops called as ``_direct`` does."""
+    for node in gm.graph.nodes:
+        if node.op == "call_function" and node.target in _DIRECT:
+            node.target = _DIRECT[node.target]
+    gm.recompile()
+    return gm
 
 
 def trainable(match, dtype_of) -> str:

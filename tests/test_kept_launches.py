@@ -1,0 +1,178 @@
+"""Launches repeated from the record of a call with the same signature (``lowering._Kept``)."""
+import os
+
+import pytest
+import torch
+
+import loopfuse_amd  # noqa: F401
+from loopfuse_amd import lowering
+from loopfuse_amd.lowering import AttnPlan, attention, attention_backward
+
+BF = torch.bfloat16
+
+
+def _fresh(fn):
+    """``fn()`` through the general path, and what it recorded."""
+    lowering._kept.clear()
+    return fn(), dict(lowering._last_launch._get())
+
+
+def test_no_signature_for_what_is_not_plain(monkeypatch):
+    """Tensors that are not on the GPU, a plan that holds a tensor, options that are no plain values and an environment put in
+    the place of the imported one leave a call to the general path."""
+    q = torch.zeros((1, 1, 1, 64), dtype=BF)
+    assert lowering._signature("fwd", (q, None), AttnPlan(), None) is None
+    assert lowering._signature("fwd", (None,), AttnPlan(scale=torch.tensor(1.0)), None) is None
+    assert lowering._signature("fwd", (None,), AttnPlan(), {"bn": torch.tensor(32)}) is None
+    monkeypatch.setattr(os, "environ", dict(os.environ))
+    assert lowering._signature("fwd", (None,), AttnPlan(), None) is None
+
+
+def _r(shape, seed, dtype=BF):
+    return torch.randn(shape, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda").to(dtype)
+
+
+def _paged(seed, page, B=2, Hkv=8, S=512, D=128):
+    n = S // page
+    pool = (B * n, Hkv, D) if page == 1 else (B * n, page, Hkv, D)
+    table = torch.randperm(B * n, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda").view(B, n).to(torch.int32)
+    return _r(pool, seed), _r(pool, seed + 1), table
+
+
+FORMS = {
+    "prefill": lambda s: ((_r((2, 4, 300, 128), s), _r((2, 2, 300, 128), s + 1), _r((2, 2, 300, 128), s + 2), AttnPlan("causal", scale=0.1)), {}),
+    "prefill views": lambda s: ((_r((2, 300, 4, 64), s).transpose(1, 2), _r((2, 300, 4, 64), s + 1).transpose(1, 2),
+                                 _r((2, 300, 4, 64), s + 2).transpose(1, 2), AttnPlan("sliding", window=50, scale=0.1, softcap=20.0)), {}),
+    "prefill into a view": lambda s: ((_r((2, 4, 100, 64), s), _r((2, 4, 100, 64), s + 1), _r((2, 4, 100, 64), s + 2), AttnPlan(scale=0.1)),
+                                      {"out": torch.zeros((2, 100, 4, 64), dtype=BF, device="cuda").transpose(1, 2)}),
+    "prefill with lse": lambda s: ((_r((1, 4, 100, 64), s), _r((1, 4, 100, 64), s + 1), _r((1, 4, 100, 64), s + 2), AttnPlan("causal", scale=0.1)),
+                                   {"lse": torch.zeros((1, 4, 100), device="cuda"), "choice": {"prefill": "swp"}}),
+    "decode": lambda s: ((_r((3, 8, 1, 64), s), _r((3, 2, 700, 64), s + 1), _r((3, 2, 700, 64), s + 2), AttnPlan(scale=0.1)), {}),
+    "decode paged": lambda s: ((_r((2, 16, 1, 128), s), *_paged(s, 16)[:2], AttnPlan(scale=0.1, k_paged=True, v_paged=True), *[_paged(s, 16)[2]] * 2), {}),
+    "decode one-token pages, whole": lambda s: ((_r((2, 8, 1, 128), s), *_paged(s, 1)[:2], AttnPlan(scale=0.1, k_paged=True, v_paged=True),
+                                                 *[_paged(s, 1)[2]] * 2), {"choice": {"splits": 1}}),
+    "padded head dim": lambda s: ((_r((2, 2, 60, 40), s), _r((2, 2, 60, 40), s + 1), _r((2, 2, 60, 40), s + 2), AttnPlan(scale=0.1)), {}),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", list(FORMS), ids=lambda f: f.replace(" ", "_"))
+def test_a_repeated_call_is_the_general_path_on_its_own_tensors(form):
+    """Every form of call: the bits and the record of launches of the general path, for tensors that were not there when the launches
+    were recorded, whose results and log-sum-exps are written and no earlier call's; replayed from a graph as well."""
+    args, kw = FORMS[form](1)
+    attention(*args, **kw)                                    # recorded
+    for seed in (11, 12):
+        args, kw = FORMS[form](seed)
+        before = len(lowering._kept)
+        got, lse = attention(*args, **kw), kw.get("lse")
+        assert len(lowering._kept) == before and before       # repeated
+        record = dict(lowering._last_launch._get())
+        lse = None if lse is None else lse.clone()
+        mine = got.clone()
+        want, full = _fresh(lambda: attention(*args, **kw))
+        assert torch.equal(mine, want) and record == full
+        assert lse is None or torch.equal(lse, kw["lse"])
+        assert "out" not in kw or got is kw["out"]
+    graph, out = torch.cuda.CUDAGraph(), None
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = attention(*args, **kw)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        attention(*FORMS[form](21)[0], **kw if "choice" in kw and "lse" not in kw else {})
+        torch.cuda.synchronize()
+        assert "out" in kw or torch.equal(out, mine)
+
+
+@pytest.mark.gpu
+def test_what_changes_the_launches_changes_the_signature(monkeypatch):
+    """A switch set after the launches were recorded, another option, other strides, another length: each takes the route it would
+    take in a new process; a refusal is not recorded, and a call that is refused is refused again."""
+    def call(S=512, view=False, **kw):
+        q, k, v = (_r((1, 4, S, 64), i) for i in range(3))
+        if view:
+            k = _r((1, S, 4, 64), 1).transpose(1, 2)
+        return attention(q, k, v, AttnPlan("causal", scale=0.1), **kw)
+
+    lowering._kept.clear()
+    base = call()
+    assert lowering._last_launch["kernels"] == ["lf_attn_prefill_swp"] and len(lowering._kept) == 1
+    call(choice={"prefill": "w32"})
+    assert lowering._last_launch["kernels"] == ["lf_attn_prefill"]
+    monkeypatch.setenv("LOOPFUSE_PREFILL", "w32")
+    call()
+    assert lowering._last_launch["kernels"] == ["lf_attn_prefill"]
+    monkeypatch.delenv("LOOPFUSE_PREFILL")
+    assert torch.equal(call(), base) and lowering._last_launch["kernels"] == ["lf_attn_prefill_swp"]
+    call(S=500)
+    call(view=True)
+    assert len(lowering._kept) == 5
+    q, k = _r((1, 4, 64, 64), 1), _r((1, 4, 64, 64), 2)
+    for _ in range(2):
+        with pytest.raises(lowering.UnsupportedPlan):
+            attention(q, k, k.float(), AttnPlan(scale=0.1))
+        with pytest.raises(lowering.UnsupportedPlan):
+            attention(q, k, k, AttnPlan(scale=float("nan")))
+    assert len(lowering._kept) == 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,mask,keep", [(128, "causal", None), (64, None, False), (128, "sliding", True)])
+def test_a_repeated_backward_is_the_general_path(D, mask, keep):
+    def operands(seed):
+        q, k, v, dout = _r((2, 4, 200, D), seed), _r((2, 2, 200, D), seed + 1), _r((2, 2, 200, D), seed + 2), _r((2, 4, 200, D), seed + 3)
+        lse = torch.empty((2, 4, 200), device="cuda")
+        o = attention(q, k, v, plan, lse=lse, choice={"prefill": "swp"})
+        return q, k, v, o, lse, dout, plan
+
+    plan = AttnPlan(mask, window=70 if mask == "sliding" else 0, scale=0.1)
+    attention_backward(*operands(1), keep_ds=keep)
+    args = operands(31)
+    before = len(lowering._kept)
+    got = attention_backward(*args, keep_ds=keep)
+    record = dict(lowering._last_launch._get())
+    assert len(lowering._kept) == before
+    want, full = _fresh(lambda: attention_backward(*args, keep_ds=keep))
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and record == full
+
+
+@pytest.mark.gpu
+def test_a_dispatch_mode_still_sees_the_training_ops():
+    """A training graph calls its attention past the dispatcher, except where something is there that has to see the ops."""
+    import functools
+
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from loopfuse_amd import loopfuse_backend
+    from loopfuse_amd.torch_backend import training
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    def attn(q, k, v):
+        s = torch.ops.loopfuse.causal_mask(q @ k.transpose(-2, -1) * 0.125)
+        return torch.softmax(s, dim=-1) @ v
+
+    fn = torch.compile(attn, backend=functools.partial(loopfuse_backend, mode=None), dynamic=False)
+    q, k, v = (_r((1, 2, 100, 64), i).requires_grad_(True) for i in range(3))
+    dout = _r((1, 2, 100, 64), 9)
+    out = fn(q, k, v)
+    want = torch.autograd.grad(out, (q, k, v), dout)
+    before = dict(training.counters)
+    inner = fn(q, k, v)
+    got = torch.autograd.grad(inner, (q, k, v), dout)
+    assert training.counters["fwd"] == before["fwd"] + 1 and training.counters["bwd"] == before["bwd"] + 1
+    assert torch.equal(inner, out) and all(torch.equal(a, b) for a, b in zip(got, want))
+    mode = Seen()
+    call = training._DIRECT[torch.ops.loopfuse_amd.attention_fwd.default]
+    with torch.no_grad(), mode:
+        call(q.detach(), k.detach(), v.detach(), 1, 0, 0.125, 0.0)
+    assert any("attention_fwd" in n for n in mode.names)
