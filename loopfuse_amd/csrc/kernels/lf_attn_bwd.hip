@@ -12,8 +12,8 @@
 //   lf_attn_bwd_dq    : a workgroup owns 128 or 256 query rows of one (batch, head) -- 4 or 8 waves x
 //                       32 rows, Q^T and dO^T in registers -- and walks the kv tiles (64 keys); with LF_BW_DS it
 //                       reads the dS that lf_attn_bwd_dkdv has left instead of forming it, and runs behind it
-//   lf_attn_bwd_dkdv  : a workgroup owns 128 or 256 keys of one (batch, kv head) -- 4 waves x 32 or 64
-//                       keys, K^T and V^T of its keys in registers as MFMA B operands -- and walks the
+//   lf_attn_bwd_dkdv  : a workgroup owns 64, 128 or 256 keys of one (batch, kv head) -- 4 waves x 32 or 64
+//                       keys (64: two waves of keys, twice over), K^T and V^T of its keys in registers as MFMA B operands -- and walks the
 //                       q tiles (64 rows) of the query heads of the group that can see them
 // The tiles that are walked are kept in LDS once and read both ways: along their rows (ds_read_b128,
 // rows of the tile = MFMA rows) and transposed (rows of the tile = MFMA k).  As in the forward, the accumulator of the first product is, as
@@ -281,6 +281,15 @@ __device__ __forceinline__ void lf_bw_mfma_hidden(const lf_f32x16& c, const lf_u
 #ifndef LF_BW_W
 #define LF_BW_W 1        /* 32-key blocks per wave of lf_attn_bwd_dkdv: every fragment read from LDS feeds so many MFMAs */
 #endif
+#ifndef LF_BW_QSPLIT
+#define LF_BW_QSPLIT 0   /* 1: two waves of keys instead of four, twice over: one pair takes the first 32 queries of a tile, one the others */
+#endif
+// s_waitcnt vmcnt: all but the newest kMost (and kMore beyond them, if there are that many)
+template <int kMost, int kMore> __device__ __forceinline__ void lf_bw_wait(int more) {
+  constexpr int kBoth = kMost + kMore;
+  if (kMore > 0 && more == kMore) __builtin_amdgcn_s_waitcnt((kBoth & 15) | 0x70 | ((kBoth >> 4) << 14));
+  else __builtin_amdgcn_s_waitcnt((kMost & 15) | 0x70 | ((kMost >> 4) << 14));
+}
 #ifndef LF_BW_PF
 #define LF_BW_PF (LF_BW_W == 2 && LF_HEAD_DIM == 128 ? 3 : 4)   /* fragments read ahead of the MFMAs that take them (there, a fourth spills) */
 #endif
@@ -308,13 +317,18 @@ __device__ __forceinline__ void lf_bw_mfma_hidden(const lf_f32x16& c, const lf_u
 // 129 / 127, unmasked B2 32/8 S4096 1627 / 1618, softcap B4 32/8 S2048 631 / 628).
 // Three LDS stages: a tile's loads are issued in the second half of the step two before its own, and the one barrier per
 // step, in its middle, says both that the next tile has landed and that the tile before this one is free.
+// With LF_BW_QSPLIT a workgroup owns 64 keys, 32 per wave, every key held by two waves: one pair walks the first 32 queries of each
+// tile, the other the last, and their sums meet in LDS at the end.  A tile is then one block per wave: its barrier stands in
+// front of the block and waits for loads issued two blocks before, which takes a fourth stage.  For launches of few
+// workgroups (lowering.bwd_q_split): causal D64 B8 16/4 S1000, 256 workgroups of 128 keys whose longest walks twice the mean,
+// 89 -> 60 us.
 // With LF_BW_DS the B operands dS also leave for memory, two stores per 32 x 32 block between the MFMAs that take them, and the
 // barrier does not wait for them: 297 -> 340 us of the above for 545 MB (352 with plain stores, which take L2 from Q and dO).
 extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const LfAttnBwdParams p) {
-  constexpr int KB = LF_BW_W;
-  constexpr int kKeys = 128 * KB;
-  __shared__ __attribute__((aligned(256))) lf_elem tiles[3][2][64 * LF_D];        // Q, dO
-  __shared__ __attribute__((aligned(16))) float stats[3][2][64];                  // of the 64 rows: L, start of dP
+  constexpr int KB = LF_BW_W, kKeyWaves = LF_BW_QSPLIT ? 2 : 4, kStages = LF_BW_QSPLIT ? 4 : 3;
+  constexpr int kKeys = 32 * KB * kKeyWaves;
+  __shared__ __attribute__((aligned(256))) lf_elem tiles[kStages][2][64 * LF_D];        // Q, dO
+  __shared__ __attribute__((aligned(16))) float stats[kStages][2][64];                  // of the 64 rows: L, start of dP
 #if LF_BW_VL
   __shared__ lf_u32x4 v_lds[LF_BW_VL][KB][LF_BW_NT];                               // V^T operands that the registers have no room for
 #endif
@@ -333,7 +347,8 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   const int hkv = bhkv % p.Hkv;
   const int b = bhkv / p.Hkv;
   const int group = p.Hq / p.Hkv;
-  const int key0 = kKeys * kt + 32 * KB * wave;    // first key of this wave
+  const int key0 = kKeys * kt + 32 * KB * (wave % kKeyWaves);    // first key of this wave
+  const int my_qb = wave / kKeyWaves;                            // LF_BW_QSPLIT: the wave's 32 queries of a tile
   const int klast = min(key0 + 32 * KB, p.Sk) - 1;
   const int nqt = (p.Sq + 63) / 64;
 
@@ -431,8 +446,9 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
       lf_dma_dword_to_lds_at(stat_rs, (unsigned)(ld_q0 + lane) * 4u, stat0 + (unsigned)((2 * st + wave) * 256));
   };
   // statistic `which` of the queries of block qb in accumulator order: element 4*i4 + e is query 32*qb + 8*i4 + 4*g + e
+  const int stat_at = 4 * g + 32 * my_qb;
   auto read_stat4 = [&](int st, int which, int qb, int i4) {
-    return *reinterpret_cast<const lf_f32x4*>(&stats[st][which][32 * qb + 8 * i4 + 4 * g]);
+    return *reinterpret_cast<const lf_f32x4*>(&stats[st][which][32 * qb + 8 * i4 + stat_at]);
   };
   auto read_stats = [&](int st, int which, int qb) {
     lf_f32x16 r;
@@ -445,7 +461,7 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     return r;
   };
 
-  unsigned rm_off = lf_bw_rm_off(l32, g), tr_off = lf_bw_tr_off(lane);
+  unsigned rm_off = lf_bw_rm_off(l32, g) + (unsigned)(32 * my_qb * LF_BW_ROWB), tr_off = lf_bw_tr_off(lane) + (unsigned)(32 * my_qb * LF_BW_ROWB);
   asm volatile("" : "+v"(rm_off), "+v"(tr_off));
   constexpr int NS = LF_NKS, NT = 2 * LF_NDB, NF = 2 * NS + 2 * NT;     // fragments of a block
   static_assert(kLoads <= NS, "a block's loads go out during its first two phases");
@@ -465,10 +481,10 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     for (int f = 0; f < LF_BW_PF; ++f) pre[f] = frag(st, qb, f);
   };
 
+  int ds_young = 0;                // LF_BW_DS: stores of this wave behind its last direct loads
 #if LF_BW_DS
   const int nkb = (p.Sk + 31) / 32;
   lf_elem* ds_head = p.ds + ((long long)b * p.Hq + hkv * group) * p.ds_sh;      // of the query head that is walked
-  int ds_young = 0;                // stores of this wave behind its last direct loads
   unsigned ds_off = lf_bw_ds_chunk(l32, g);
   asm volatile("" : "+v"(ds_off));
 #endif
@@ -666,6 +682,47 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
     aim();
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) issue(1, j);
+#if LF_BW_QSPLIT
+    aim();
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) issue(2, j);
+    LF_BW_BARRIER();
+    read_ahead(0, 0);
+    int st = 0, q0 = 64 * qt_begin + 32 * my_qb, left = ntq;
+    // this wave's loads but the newest tile's, and stores of dS behind those, are done (the counter retires in order; waves
+    // 0 and 1 have a load of statistics more); then every wave's
+    auto stage = [&]() {
+      asm volatile("" ::: "memory");
+      if (wave < 2) lf_bw_wait<kLoads + 1, LF_BW_DS ? 2 * KB : 0>(ds_young);
+      else lf_bw_wait<kLoads, LF_BW_DS ? 2 * KB : 0>(ds_young);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      ds_young = 0;
+    };
+    for (int it = 0; it < nsteps; ++it) {
+      const int st1 = (st + 1) & 3, st3 = (st + 3) & 3;
+      stage();                    // the next tile has landed; every wave is done with the one before this
+      aim();
+      if (!need(q0)) {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) issue(st3, j);
+        read_ahead(st1, 0);
+      } else if (full(q0)) {
+        block(0, st, q0, false, true, st3, st1, 0);
+      } else {
+        block(0, st, q0, true, true, st3, st1, 0);
+      }
+      st = st1;
+      q0 += 64;
+      if (--left == 0) {
+        left = ntq;
+        q0 = 64 * qt_begin + 32 * my_qb;
+#if LF_BW_DS
+        ds_head += p.ds_sh;
+#endif
+      }
+    }
+#else
     LF_BW_BARRIER();
     read_ahead(0, 0);
     int st = 0, q0 = 64 * qt_begin, left = ntq;
@@ -708,12 +765,50 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
 #endif
       }
     }
+#endif
     __builtin_amdgcn_s_waitcnt(0x0070);      // the last loads, against an empty range, before the LDS is given back
   }
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
     for (int db = 0; db < LF_NDB; ++db) asm volatile(LF_BW_MFMA_DRAIN_LAST : "+a"(dk[kb][db]), "+a"(dv[kb][db]));
+#if LF_BW_QSPLIT
+  // the sums of the waves that held the same keys, through LDS (nobody reads its tiles any more), lane by lane
+  {
+    lf_f32x4* sums = reinterpret_cast<lf_f32x4*>(&tiles[0][0][0]);
+    static_assert(KB * LF_NDB * 8 * 128 * 16 <= (int)sizeof(tiles), "the sums fit the tiles");
+    auto at = [&](int j, int i4) -> lf_f32x4& { return sums[(j * 4 + i4) * 128 + (tid & 127)]; };
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int db = 0; db < LF_NDB; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int j = 2 * (kb * LF_NDB + db);
+          if (my_qb == 1) {
+            at(j, i4) = lf_f32x4{dk[kb][db][4 * i4], dk[kb][db][4 * i4 + 1], dk[kb][db][4 * i4 + 2], dk[kb][db][4 * i4 + 3]};
+            at(j + 1, i4) = lf_f32x4{dv[kb][db][4 * i4], dv[kb][db][4 * i4 + 1], dv[kb][db][4 * i4 + 2], dv[kb][db][4 * i4 + 3]};
+          }
+        }
+    __syncthreads();
+    if (my_qb == 1) return;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int db = 0; db < LF_NDB; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int j = 2 * (kb * LF_NDB + db);
+          const lf_f32x4 x = at(j, i4), y = at(j + 1, i4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            dk[kb][db][4 * i4 + e] += x[e];
+            dv[kb][db][4 * i4 + e] += y[e];
+          }
+        }
+  }
+#endif
   // the parameters of the output are read only now: held over the loop they cost scalar registers it needs
   auto ep = (const LfAttnBwdParams __attribute__((address_space(4)))*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(ep));

@@ -1199,6 +1199,21 @@ class AttnBwdParams(ctypes.Structure):
 BWD_DS_BLOCK = 32 * 32      # elements of a block of dS (lf_bw_ds_row in csrc/kernels/lf_attn_bwd.hip)
 
 
+def bwd_q_split(D: int, mask: int, units: int, Sk: int) -> bool:
+    """Is lf_attn_bwd_dkdv launched with workgroups of 64 keys, whose waves hold each 32 of them twice, one for the first and one
+    for the last 32 queries of a tile?  Twice the workgroups and half as long a chain of tiles in each, against twice the Q / dO
+    loads: it pays where the workgroups of 128 keys leave CUs idle, or alone with the longest of them.  ``units`` = batch x
+    kv heads.  All launches, whole / split, us, over 70 shapes: causal D 64 B8 16/4 S1000 (256 workgroups of 128 keys) 140 / 110,
+    B10 64/8 S445 (320) 170 / 126, B5 16/4 S3539 (560) 607 / 614; causal D 128 B1 32/8 S2048 (128) 307 / 209, B6 H8 S500 (192)
+    44.6 / 44.6, B10 8/2 S1748 (280) 328 / 367; window D 64 B3 8/4 S2183 (216) 91 / 76, B15 64/8 S383 (360) 148 / 136, B6 16/2
+    S5110 (480) 267 / 277, D 128 B2 64/8 S524 (80) 97 / 66, B3 32/8 S1055 (216) 106 / 113; unmasked D 64 B1 16/8 S2120 (136)
+    155 / 135, B1 H8 S5043 (320) 279 / 280, D 128 B6 H4 S1784 (336) 177 / 170, B10 H4 S1879 (600) 320 / 326."""
+    n = units * -(-Sk // 128)
+    if mask == MASK_NONE:
+        return n <= (192 if D == 64 else 352)
+    return n <= (384 if D == 64 else 192)
+
+
 def bwd_ds_blocks(mask: int, window: int, Sq: int, Sk: int) -> int:
     """Blocks of dS of one (batch, query head): ``lf_bw_ds_row`` of the row behind the last, and under a window the blocks in
     front of the first key that the last row's start leaves out."""
@@ -1253,33 +1268,35 @@ def bwd_keep_ds(D: int, softcap: bool, units: int, group: int, Sk: int, blocks: 
     it again?  ``units`` = batch x query heads, ``blocks`` = of dS in all (2 KB each; up to 2 GiB).  Seven products instead of
     nine against 2 bytes per visible score written and read, both by non-temporal accesses.  All launches, recomputed / kept, us:
     head dimension 128, causal B4 H32 S2048 549 / 521 (545 MB), B2 32/8 S4096 953 / 909, B6 64/32 S769 369 / 307, with a softcap
-    B4 32/8 S2048 644 / 561, window 256 252 / 204, unmasked H2 S7033 392 / 311; of 30 drawn shapes one was slower, short with
-    eight heads per group (B6 16/2 S135 62 / 65).  Head dimension 64 has half the matrix work per score: with a softcap B4 H32
-    S2048 424 / 379, without B4 H32 S2048 304 / 333, B8 16/4 S1000 140 / 143, and kept where few heads leave CUs to the
-    recomputation's longest workgroups: H8 S4520 181 / 158, H2 S1038 52 / 47, B4 H16 S535 50 / 47."""
+    B4 32/8 S2048 644 / 561, window 256 252 / 204, unmasked H2 S7033 392 / 311; of 60 drawn shapes three were slower by more than
+    2 %, short ones with eight heads per group (B6 16/2 S135 62 / 65).  Head dimension 64 has half the matrix work per score:
+    with a softcap B4 H32 S2048 424 / 379, without B4 H32 S2048 304 / 333, B8 16/4 S1000 140 / 143, and kept where few heads leave
+    CUs to the recomputation's longest workgroups: H8 S4520 181 / 158, H2 S1038 52 / 47, B4 H16 S535 50 / 47."""
     size = 2 * BWD_DS_BLOCK * blocks
     if size > 2 << 30 or (Sk < 192 and group > 4):
         return False
-    return D == 128 or softcap or (units <= 64 and Sk >= 512 and size <= 256 << 20)
+    return D == 128 or softcap or (units <= 64 and group <= 4 and Sk >= 512 and size <= 176 << 20)
 
 
 def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False, key_blocks: int = 1,
-             dq_threads: int = 512, keep_ds: bool = False) -> KernelSpec:
+             dq_threads: int = 512, keep_ds: bool = False, q_split: bool = False) -> KernelSpec:
     return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap,
-                      extra=(f"-DLF_BW_DQ_NT={dq_threads}", f"-DLF_BW_W={key_blocks}") + (("-DLF_BW_DS=1",) if keep_ds else ()))
+                      extra=(f"-DLF_BW_DQ_NT={dq_threads}", f"-DLF_BW_W={key_blocks}") + (("-DLF_BW_DS=1",) if keep_ds else ())
+                      + (("-DLF_BW_QSPLIT=1",) if q_split else ()))
 
 
 def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
                        dout: torch.Tensor, plan: AttnPlan, *, key_blocks: Optional[int] = None,
-                       dq_threads: Optional[int] = None, keep_ds: Optional[bool] = None):
+                       dq_threads: Optional[int] = None, keep_ds: Optional[bool] = None, q_split: Optional[bool] = None):
     """Gradients of ``attention(q, k, v, plan)`` for dense K/V (mask none / causal / sliding, scale,
     softcap; no bias or paging): returns ``(dq, dk, dv)`` in the operands' dtype.  ``o`` and ``lse``
     are the forward's output and row log-sum-exp (``attention(..., lse=...)``).  Two or
     three launches (csrc/kernels/lf_attn_bwd.hip): delta = rowsum(dO * O), together with dQ where that has small
     workgroups and forms dS itself; dK and dV, one workgroup per 128 or 256 keys of a (batch, kv head); dQ, one workgroup per 128
     or 256 query rows, from dS left in a scratch tensor where ``bwd_keep_ds`` says so (``keep_ds`` overrides it).  No
-    atomics: results are reproducible bit for bit."""
-    key = _signature("bwd", (q, k, v, o, lse, dout), plan, {"key_blocks": key_blocks, "dq_threads": dq_threads, "keep_ds": keep_ds})
+    atomics: results are reproducible bit for bit.  ``key_blocks``, ``dq_threads`` and ``q_split`` override the rules of the work
+    splits (``bwd_key_blocks``, ``bwd_dq_threads``, ``bwd_q_split``)."""
+    key = _signature("bwd", (q, k, v, o, lse, dout), plan, {"key_blocks": key_blocks, "dq_threads": dq_threads, "keep_ds": keep_ds, "q_split": q_split})
     kept = _kept.get(key)
     if kept is not None:
         res = _backward_again(kept, q, k, v, o, lse, dout)
@@ -1316,6 +1333,8 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     cap = softcap is not None
     if key_blocks and key_blocks != 1 and (key_blocks != 2 or not bwd_two_key_blocks(D, mask, cap)):
         raise UnsupportedPlan(f"key_blocks {key_blocks!r}: 1, or 2 at head dim 128 without a window and a softcap")
+    if q_split and key_blocks and key_blocks != 1:
+        raise UnsupportedPlan("q_split: with one key block per wave")
     if dq_threads and dq_threads not in (256, 512):
         raise UnsupportedPlan(f"dq_threads {dq_threads!r}: 256 or 512")
     for name, t in (("Q", q), ("K", k), ("V", v), ("O", o), ("dO", dout)):
@@ -1352,10 +1371,14 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
             if keep_ds:
                 raise
             key = None                   # the gradients need no such room; the next call may find it
-    spec = bwd_spec(dtype, D, mask, cap, keys, nt, ds is not None)
+    if q_split is None:
+        q_split = not (key_blocks and key_blocks != 1) and bwd_q_split(D, mask, B * Hkv, Sk)
+    if q_split:
+        keys = 1
+    spec = bwd_spec(dtype, D, mask, cap, keys, nt, ds is not None, q_split)
     keep = (q, k, v, o, dout, lse, delta, dq, dk, dv, ds)  # noqa: F841  (tensors stay alive until the launches are queued)
     steps = {"lf_attn_bwd_delta": (-(-B * Hq * Sq // 16), 256),
-             "lf_attn_bwd_dkdv": (xcd_slots(B * Hkv, -(-Sk // (128 * keys))), 256),
+             "lf_attn_bwd_dkdv": (xcd_slots(B * Hkv, -(-Sk // (128 * keys // (2 if q_split else 1)))), 256),
              "lf_attn_bwd_dq": (xcd_slots(B * Hkv, (Hq // Hkv) * -(-Sq // (nt // 2))), nt)}
     # without dS of lf_attn_bwd_dkdv, lf_attn_bwd_dq with 256 threads forms delta itself, and lf_attn_bwd_dkdv reads it
     names = ["lf_attn_bwd_dq", "lf_attn_bwd_dkdv"] if nt == 256 and ds is None else list(steps)
