@@ -810,13 +810,18 @@ extern "C" __global__ void __launch_bounds__(LF_DT, 8 / LF_DW) lf_attn_decode(co
 
 #endif  // LF_COOP
 
-// Merge nsplit partial results per query row.  A thread owns 4 consecutive d of one row;
-// block = 256 threads = 1024 / LF_HEAD_DIM rows, grid = ceil(B*Hkv*rows / rows per block).
+// Merge nsplit partial results per query row.  A thread owns 4 consecutive d of one row; block = 256 threads = 1024 /
+// LF_HEAD_DIM rows, grid = ceil(B*Hkv*rows / rows per block), or one row per block, its splits shared by the block's groups of
+// threads and their results merged through LDS.  Bound by its chain of loads, a round trip per four splits: with one group
+// per row 16 splits were four in a row, and finer splits of the step cost here what they gained there.
 extern "C" __global__ void __launch_bounds__(256) lf_attn_decode_combine(const LfAttnParams p) {
   constexpr int kTPR = LF_HEAD_DIM / 4;              // threads per row
   constexpr int kRPB = 256 / kTPR;                   // rows per block
-  const long long rowid = (long long)blockIdx.x * kRPB + threadIdx.x / kTPR;   // (bh * rows + qr)
   const long long nrows = (long long)p.B * p.Hkv * p.rows;
+  // a grid of one block per row: kRPB groups of threads share the row's splits, four at a time each
+  const bool row_per_block = (long long)gridDim.x >= nrows;
+  const int part = threadIdx.x / kTPR;
+  const long long rowid = row_per_block ? blockIdx.x : (long long)blockIdx.x * kRPB + part;   // (bh * rows + qr)
   if (rowid >= nrows) return;
   const int d0 = 4 * (threadIdx.x % kTPR);
   const int qr = (int)(rowid % p.rows);
@@ -828,7 +833,8 @@ extern "C" __global__ void __launch_bounds__(256) lf_attn_decode_combine(const L
   float m = LF_NEG_INF;
   float l = 0.0f;
   lf_f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int z0 = 0; z0 < p.nsplit; z0 += 4) {
+  const int step = row_per_block ? 4 * kRPB : 4;
+  for (int z0 = row_per_block ? 4 * part : 0; z0 < p.nsplit; z0 += step) {
     lf_f32x2 ml[4];
     lf_f32x4 ac[4];
 #pragma unroll
@@ -853,6 +859,27 @@ extern "C" __global__ void __launch_bounds__(256) lf_attn_decode_combine(const L
         a += ac[u] * f;
       }
     m = mc;
+  }
+  if (row_per_block) {
+    __shared__ lf_f32x4 acc[kRPB][kTPR];
+    __shared__ lf_f32x2 ml[kRPB];
+    acc[part][d0 / 4] = a;
+    if (d0 == 0) ml[part] = lf_f32x2{m, l};
+    __syncthreads();
+    if (part) return;
+    float mc = m;
+#pragma unroll
+    for (int u = 1; u < kRPB; ++u) mc = fmaxf(mc, ml[u][0]);
+    const float m_sub = (mc == LF_NEG_INF) ? 0.0f : mc;
+    const float r = (m == LF_NEG_INF) ? 0.0f : lf_exp2(m - m_sub);
+    l *= r;
+    a *= r;
+#pragma unroll
+    for (int u = 1; u < kRPB; ++u) {
+      const float f = (ml[u][0] == LF_NEG_INF) ? 0.0f : lf_exp2(ml[u][0] - m_sub);     // a group without a split: 0 * 0
+      l += ml[u][1] * f;
+      a += acc[u][d0 / 4] * f;
+    }
   }
   lf_elem* orow = p.o + (long long)b * p.o_sb + (long long)hkv * p.o_sh + (long long)qr * p.o_ss;
   const float inv = lf_inv_sum(l);

@@ -352,6 +352,25 @@ def decode_split(units: int, Sk: int, cus: int = 256, per_cu: int = 2) -> int:
     return max(1, min(want, most))
 
 
+@functools.lru_cache(maxsize=1024)
+def decode_even_split(units: int, Sk: int, D: int, cus: int = 256) -> int:
+    """KV splits of a step whose four waves share a head (``units`` workgroups per split): the count with the least cost in a
+    model of CUs that stream a split's keys and 64 more at the head of it, per round of one workgroup per CU -- a first round that
+    is not full costs nineteen twentieths of one, a later one six tenths --, of the merge launch (230 keys of 128) and of its partials.  Splits are
+    as short as 48 keys, down to where the merge reads as much as it saves.  Fitted on every count for 234 steps of 2 ... 512
+    units, 208 ... 20 000 keys, head dimensions 64 and 128: 0.8 % from the best in the mean (11 % at worst), where the rule before
+    (splits of 512 keys and more, two workgroups per CU, rounded up) was 8.5 %.  Before / now, us: 8 units (one sequence of 8 kv
+    heads, D 128) of 600 keys 13.9 / 8.8, 2048 14.7 / 9.4, 8208 18.0 / 15.7; 24 of 10 432 39 / 31; 80 of 20 000 172 / 134; 192 of
+    2048, which it split, 47.5 / 40.7."""
+    def cost(n: int) -> float:
+        splits, size = _split_lengths(n, Sk)
+        full, rest = divmod(units * splits, cus)
+        rounds = full + (max(0.6 if full else 0.95, rest / cus) if rest else 0.0)
+        return (size + 64) * rounds * D / 128 + (230 if splits > 1 else 0) + (0.84 * splits if splits > 4 else 0)
+
+    return min((cost(n), n) for n in range(1, max(1, min(64, Sk // 48)) + 1))[1]
+
+
 def _coop_cost(n: int, units: int, Sk: int, rows: int, cus: int = 256) -> float:
     """Time of a decode step with cooperative loads in ``n`` KV splits (``units`` workgroups each), in tokens streamed by
     one workgroup per CU: rounds of one workgroup per CU, a last one that is not full costing nine tenths of one (fewer
@@ -405,6 +424,13 @@ def _split_lengths(n: int, Sk: int) -> tuple:
     """(splits, keys per split) of a decode step asked to make ``n``: whole pairs of 16-token steps."""
     size = (-(-Sk // n) + 31) // 32 * 32
     return -(-Sk // size), size
+
+
+def decode_combine_grid(rows: int, nsplit: int, D: int) -> int:
+    """Blocks of lf_attn_decode_combine: 256 threads, 4 consecutive d each; several rows to a block, or one row whose splits the
+    block's groups of threads share, where there are more than they fetch at a time (4) and few rows."""
+    per_block = 1024 // D
+    return rows if nsplit > 4 and rows <= 4096 else -(-rows // per_block)
 
 
 def static_split_runs(n: int, Sk: int, rows: int, D: int, room: int) -> bool:
@@ -1135,8 +1161,10 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                 _decode_headwave(paged, page_size, Hkv, D, P, B * ((Hkv + 7) // 8) * chunks, Sk)
             plain = decode_split(B * ((Hkv + 7) // 8 if eight else Hkv) * chunks, Sk, per_cu=1 if eight else 2)
             num_splits = decode_static_split(num_splits, plain, Sk, B * Hkv * rows, D, runtime.static_scratch_bytes())
-    elif not num_splits:
+    elif not num_splits and (headwave or static_scratch or _env("LOOPFUSE_DECODE_SPLITS")):
         num_splits = decode_split(units, Sk, per_cu=1 if headwave else 2)
+    elif not num_splits:
+        num_splits = decode_even_split(units, Sk, D)
     nsplit, split_len = _split_lengths(num_splits, Sk)
     P.rows, P.nsplit, P.split_len = rows, nsplit, split_len
     spec = KernelSpec("decode", _DTYPE_CODE[dtype], D, MASK_NONE, plan.softcap is not None, paged,
@@ -1145,8 +1173,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                       rowload=not coop and _decode_rowload(paged, page_size, page_size_v, bias_bits),
                       bias=bias_bits, safe=plan.zero_blind_rows and bool(bias_bits),
                       extra=tuple(_env("LOOPFUSE_KOPTS", "").split()))
-    rows_per_block = 1024 // D       # combine kernel: 256 threads, 4 consecutive d each
-    combine_grid = (B * Hkv * rows + rows_per_block - 1) // rows_per_block
+    combine_grid = decode_combine_grid(B * Hkv * rows, nsplit, D)
     if static_scratch:
         if nsplit <= 1 or not merge_splits:
             raise UnsupportedPlan("static_scratch serves split decode steps (this call does not split the keys)")
