@@ -107,20 +107,27 @@ def _backward(ctx, d_o, d_lse):
 attention_fwd.register_autograd(_backward, setup_context=_setup)
 
 
-def _direct(op, fn):
-    """``op``'s implementation for a graph that AOTAutograd has already differentiated: plain tensors go straight to it, past
-    the dispatcher's autograd wrapper and the custom op's own (40 us per step of a small attention).  Anything that has to see
-    the op -- a tensor subclass, a dispatch or function mode, a functorch transform -- still does."""
-    def call(q, *rest):
-        if type(q) in (torch.Tensor, torch.nn.Parameter) and not torch._C._len_torch_dispatch_stack() \
-                and not torch._C._len_torch_function_stack() and torch._C._functorch.peek_interpreter_stack() is None:
-            return fn(q, *rest)
-        return op(q, *rest)
+def _plain(tensors) -> bool:
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.is_neg() or (grad and t.requires_grad):
+            return False
+    return not torch._C._len_torch_dispatch_stack() and not torch._C._len_torch_function_stack() \
+        and torch._C._functorch.peek_interpreter_stack() is None
+
+
+def _direct(op, fn, tensors):
+    """``op``'s implementation for a graph that AOTAutograd has already differentiated: plain tensors (its first ``tensors``
+    arguments) go straight to it, past the dispatcher's autograd wrapper and the custom op's own (40 us per step of a small
+    attention).  Anything that has to see the op -- a tensor subclass, a view whose negation is still to be applied, a tensor
+    whose gradient is recorded, a dispatch or function mode, a functorch transform -- still does."""
+    def call(*args):
+        return fn(*args) if _plain(args[:tensors]) else op(*args)
     return call
 
 
-_DIRECT = {torch.ops.loopfuse_amd.attention_fwd.default: _direct(torch.ops.loopfuse_amd.attention_fwd.default, _attention_fwd),
-           torch.ops.loopfuse_amd.attention_bwd.default: _direct(torch.ops.loopfuse_amd.attention_bwd.default, _attention_bwd)}
+_DIRECT = {torch.ops.loopfuse_amd.attention_fwd.default: _direct(torch.ops.loopfuse_amd.attention_fwd.default, _attention_fwd, 3),
+           torch.ops.loopfuse_amd.attention_bwd.default: _direct(torch.ops.loopfuse_amd.attention_bwd.default, _attention_bwd, 6)}
 
 
 def direct_calls(gm: torch.fx.GraphModule) -> torch.fx.GraphModule:

@@ -176,3 +176,23 @@ def test_a_dispatch_mode_still_sees_the_training_ops():
     with torch.no_grad(), mode:
         call(q.detach(), k.detach(), v.detach(), 1, 0, 0.125, 0.0)
     assert any("attention_fwd" in n for n in mode.names)
+
+
+def test_only_plain_tensors_pass_the_dispatcher():
+    """A view whose negation is still to be applied, a tensor whose gradient is recorded and a subclass, in the place of any
+    operand, go through the op."""
+    from loopfuse_amd.torch_backend import training
+
+    class Sub(torch.Tensor):
+        pass
+
+    call = training._direct(lambda *a: "op", lambda *a: "direct", 3)
+    a = torch.zeros(2, 4)
+    assert call(a, a, a, 1) == "direct" and call(a, torch.nn.Parameter(a, requires_grad=False), a, 1) == "direct"
+    neg = torch.zeros(2, 4, dtype=torch.complex64).conj().imag
+    grad = torch.zeros(2, 4, requires_grad=True)
+    for odd in (neg, grad, a.as_subclass(Sub)):
+        for at in range(3):
+            assert call(*[odd if i == at else a for i in range(3)], 1) == "op"
+    with torch.no_grad():
+        assert call(grad, grad, grad, 1) == "direct"
