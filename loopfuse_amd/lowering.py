@@ -352,7 +352,6 @@ def decode_split(units: int, Sk: int, cus: int = 256, per_cu: int = 2) -> int:
     return max(1, min(want, most))
 
 
-@functools.lru_cache(maxsize=1024)
 def decode_even_split(units: int, Sk: int, D: int, cus: int = 256) -> int:
     """KV splits of a step whose four waves share a head (``units`` workgroups per split): the count with the least cost in a
     model of CUs that stream a split's keys and 64 more at the head of it, per round of one workgroup per CU -- a first round that
@@ -362,13 +361,20 @@ def decode_even_split(units: int, Sk: int, D: int, cus: int = 256) -> int:
     (splits of 512 keys and more, two workgroups per CU, rounded up) was 8.5 %.  Before / now, us: 8 units (one sequence of 8 kv
     heads, D 128) of 600 keys 13.9 / 8.8, 2048 14.7 / 9.4, 8208 18.0 / 15.7; 24 of 10 432 39 / 31; 80 of 20 000 172 / 134; 192 of
     2048, which it split, 47.5 / 40.7."""
+    return _even_best(units, Sk, D, cus)[0]
+
+
+@functools.lru_cache(maxsize=1024)
+def _even_best(units: int, Sk: int, D: int, cus: int = 256) -> tuple:
+    """(splits, cost) of the cheapest count of a step whose four waves share a head."""
     def cost(n: int) -> float:
         splits, size = _split_lengths(n, Sk)
         full, rest = divmod(units * splits, cus)
         rounds = full + (max(0.6 if full else 0.95, rest / cus) if rest else 0.0)
         return (size + 64) * rounds * D / 128 + (230 if splits > 1 else 0) + (0.84 * splits if splits > 4 else 0)
 
-    return min((cost(n), n) for n in range(1, max(1, min(64, Sk // 48)) + 1))[1]
+    best, n = min((cost(n), n) for n in range(1, max(1, min(64, Sk // 48)) + 1))
+    return n, best
 
 
 def _coop_cost(n: int, units: int, Sk: int, rows: int, cus: int = 256) -> float:
@@ -407,7 +413,8 @@ def decode_coop_fills(units: int, Sk: int, page_size: int) -> bool:
 
 
 def decode_coop_pays(units: int, Sk: int, rows: int, page_size: int, cus: int = 256) -> bool:
-    """Does a step with ``units`` workgroups per split pay with cooperative loads, against four waves per head?
+    """Does a step with ``units`` workgroups per split pay with cooperative loads, against four waves per head in the splits of
+    ``decode_split``, which steps in the library's static array and steps of a given number of splits make?
     First, there must be about as many workgroups as CUs.  Pages of 16 tokens and more, where the other form reads whole
     pages too: at up to 8 splits of 512 tokens (28 sequences of 4096 tokens, 8 heads, D 128: 79 against 84 us; 16 of 2048 32
     against 29).  Shorter pages: at up to 32 splits of 160 tokens (16 of 8192: 90 against 111 us).
@@ -418,6 +425,22 @@ def decode_coop_pays(units: int, Sk: int, rows: int, page_size: int, cus: int = 
     the lines, 24 are more than 4 % slower than the other form without this, by up to 41 %, and 15 with it, by up to 12 %."""
     even = (1.8 if page_size % 16 == 0 else 2.4) * units * Sk
     return decode_coop_fills(units, Sk, page_size) and _coop_best(units, Sk, rows, cus)[1] * cus < even
+
+
+def decode_coop_beats(units: int, waves: int, units_wave: int, Sk: int, rows: int, page_size: int, D: int) -> bool:
+    """Is a step, its splits chosen by either form's own rule, faster with cooperative loads (``units`` workgroups of ``waves``
+    heads per split) than with four waves per head (``units_wave`` workgroups)?  The costs of the two split rules, in tokens of
+    one head, against each other, a token of the cooperative form at 0.6 of the other's time with pages of 16 tokens and more, at
+    0.4 with shorter ones, which the other form reads in quarter rows.  Fitted on 470 steps and checked on 420 others of 64 ...
+    32 768 keys: 0.46 and 0.42 % (short, long pages) off the faster form in the mean there, where ``decode_coop_pays`` was 2.4 %.
+    Of the 107 steps that go the other way now, 0.90 of their time in the mean, three are 3 ... 4 % slower.  Before / now, us: 2
+    sequences of 8930, 16 heads of 64, one-token pages 24.0 / 18.8; 9 of 5120, 24 heads of 64, pages of 16 60 / 48; 60 of 64, 32
+    heads of 128, pages of 8 23.0 / 15.4.  A few workgroups more than CUs that are not split keep the older rule (264 of 611
+    keys, pages of 1: 156 against 137 us)."""
+    if 256 < units < 288:
+        return decode_coop_pays(units, Sk, rows, page_size)
+    rate, fixed = (0.6, 50) if page_size % 16 == 0 else (0.4, 75)
+    return rate * waves * D / 128 * _coop_best(units, Sk, rows)[1] + fixed < _even_best(units_wave, Sk, D)[1]
 
 
 def _split_lengths(n: int, Sk: int) -> tuple:
@@ -1145,10 +1168,15 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         headwave = _decode_headwave(paged, page_size, Hkv, D, P, B * ((Hkv + 7) // 8) * chunks, Sk) and not page_size_v
     else:
         units_coop = B * (Hkv // coop) * chunks
-        headwave = decode_coop_pays(units_coop, Sk, min(rows, DECODE_QROWS), page_size)
-        if static_scratch and not (headwave or num_splits or choice.get("splits")) and decode_coop_fills(units_coop, Sk, page_size):
-            # more splits of fewer workgroups: a step that does not run in the static array with the other loads may with these
-            headwave = not static_split_runs(decode_split(units, Sk), Sk, B * Hkv * rows, D, runtime.static_scratch_bytes())
+        if static_scratch:
+            headwave = decode_coop_pays(units_coop, Sk, min(rows, DECODE_QROWS), page_size)
+            if not (headwave or num_splits or choice.get("splits")) and decode_coop_fills(units_coop, Sk, page_size):
+                # more splits of fewer workgroups: a step that does not run in the static array with the other loads may with these
+                headwave = not static_split_runs(decode_split(units, Sk), Sk, B * Hkv * rows, D, runtime.static_scratch_bytes())
+        elif _env("LOOPFUSE_DECODE_SPLITS") or num_splits or choice.get("splits"):
+            headwave = decode_coop_pays(units_coop, Sk, min(rows, DECODE_QROWS), page_size)      # (a given count: neither rule's)
+        else:
+            headwave = decode_coop_beats(units_coop, coop, units, Sk, min(rows, DECODE_QROWS), page_size, D)
     coop = coop if headwave else 0
     if headwave:
         waves = coop or 8

@@ -46,3 +46,37 @@ def test_merge_of_any_number_of_splits(splits, D):
         whole = attention(q, k, v, plan, num_splits=1, **kw)
         err, err_whole = ((x.double() - want).norm() / want.norm() for x in (out, whole))
         assert err <= 1.5 * err_whole + 2.0 ** -9       # either rounds once to bf16 and P to bf16 on the way
+
+
+@pytest.mark.parametrize("B,Hkv,D,Sk,group,page,beats", [
+    (2, 16, 64, 8930, 1, 1, True), (9, 24, 64, 5120, 1, 16, True), (60, 32, 128, 64, 1, 8, True),      # measured on both sides
+    (64, 8, 128, 2048, 4, 16, True), (64, 4, 128, 2048, 8, 1, True),
+    (66, 32, 128, 611, 2, 1, False), (1, 8, 128, 8208, 4, 16, False), (1, 16, 128, 108, 1, 1, False)])
+def test_cooperative_decode_is_chosen_where_it_is_faster(B, Hkv, D, Sk, group, page, beats):
+    waves = 8 if Hkv % 8 == 0 else 4
+    assert lowering.decode_coop_beats(B * Hkv // waves, waves, B * Hkv, Sk, group, page, D) == beats
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hkv,D,Sk,group,page", [(2, 16, 64, 8931, 1, 1), (9, 24, 64, 2064, 2, 16), (60, 32, 128, 64, 1, 8),
+                                                   (1, 8, 128, 20000, 1, 4), (3, 32, 128, 33, 3, 1)])
+def test_steps_at_the_edges_of_the_rule(B, Hkv, D, Sk, group, page):
+    """Few workgroups in many splits, a sequence of a few steps: both forms against float64 (P and the result are rounded to
+    bf16, 2^-9 each), the rule's choice the bits of the form that it names."""
+    n = Sk // page
+    g = torch.Generator(device="cuda").manual_seed(Sk)
+    q = torch.randn((B, Hkv * group, 1, D), generator=g, device="cuda").bfloat16()
+    pool = (B * n, Hkv, D) if page == 1 else (B * n, page, Hkv, D)
+    k, v = (torch.randn(pool, generator=g, device="cuda").bfloat16() for _ in range(2))
+    table = torch.randperm(B * n, generator=g, device="cuda").view(B, n).to(torch.int32)
+    kk, vv = (x[table.long()].reshape(B, n * page, Hkv, D).transpose(1, 2).double().repeat_interleave(group, 1) for x in (k, v))
+    plan = AttnPlan(scale=D ** -0.5, k_paged=True, v_paged=True)
+    want = torch.matmul(torch.softmax(torch.matmul(q.double(), kk.transpose(-1, -2).contiguous()) * plan.scale, dim=-1), vv)
+    got = attention(q, k, v, plan, table, table)
+    coop = bool(lowering.attention.last_launch["cooperative_loads"])
+    assert coop == lowering.decode_coop_beats(B * Hkv // 8, 8, B * Hkv, Sk, group, page, D)
+    for form in (True, False):
+        out = attention(q, k, v, plan, table, table, choice={"head_per_wave": form})
+        assert (out.double() - want).norm() / want.norm() <= 2.0 ** -8
+        if form == coop:
+            assert torch.equal(out, got)
