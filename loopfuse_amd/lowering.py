@@ -1451,14 +1451,15 @@ def _backward_again(kept: _Kept, q, k, v, o, lse, dout):
     dtype, ds_shape = kept.results
     P = AttnBwdParams.from_buffer_copy(kept.params)
     dev = q.device
+    dq, dk, dv = torch.empty(q.shape, dtype=dtype, device=dev), torch.empty(k.shape, dtype=dtype, device=dev), torch.empty(k.shape, dtype=dtype, device=dev)
+    delta = torch.empty(lse.shape, dtype=torch.float32, device=dev)
     if ds_shape is not None:
+        # last: it may take what room is left, which the results need and it does not
         try:
             ds = torch.empty(ds_shape, dtype=dtype, device=dev)
         except torch.OutOfMemoryError:
             return None
         P.ds = ds.data_ptr()
-    dq, dk, dv = torch.empty(q.shape, dtype=dtype, device=dev), torch.empty(k.shape, dtype=dtype, device=dev), torch.empty(k.shape, dtype=dtype, device=dev)
-    delta = torch.empty(lse.shape, dtype=torch.float32, device=dev)
     P.q, P.k, P.v, P.o, P.dout = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr()
     P.dq, P.dk, P.dv, P.lse, P.delta = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), lse.data_ptr(), delta.data_ptr()
     kept.launches.launch(P)

@@ -196,3 +196,45 @@ def test_only_plain_tensors_pass_the_dispatcher():
             assert call(*[odd if i == at else a for i in range(3)], 1) == "op"
     with torch.no_grad():
         assert call(grad, grad, grad, 1) == "direct"
+
+
+def _record_of_a_backward(ds_shape):
+    """A record of ``attention_backward`` whose launches only count, and operands on the CPU for it."""
+    class Launches:
+        count = 0
+
+        def launch(self, params):
+            self.count += 1
+
+    kept = lowering._Kept.__new__(lowering._Kept)
+    kept.params, kept.launches = bytes(lowering.AttnBwdParams()), Launches()
+    kept.results, kept.scratch, kept.record = (BF, ds_shape), None, {"kernels": []}
+    q, k = torch.zeros((1, 4, 40, 64), dtype=BF), torch.zeros((1, 2, 40, 64), dtype=BF)
+    return kept, (q, k, k, q, torch.zeros((1, 4, 40)), q)
+
+
+def _no_room_for(monkeypatch, shape):
+    """``torch.empty`` finds no room for tensors of ``shape``; returns the list of the shapes that it is asked for."""
+    asked, empty = [], torch.empty
+
+    def limited(size, *args, **kw):
+        asked.append(tuple(size))
+        if tuple(size) == shape:
+            raise torch.OutOfMemoryError("no room")
+        return empty(size, *args, **kw)
+
+    monkeypatch.setattr(torch, "empty", limited)
+    return asked
+
+
+def test_a_repeated_backward_takes_its_results_before_ds(monkeypatch):
+    """The results and delta are what a call needs, dS is what it can do without: allocated last, so that it cannot take their
+    room, and where it finds none nothing is launched and the caller is told."""
+    shape = (4, 3, lowering.BWD_DS_BLOCK)
+    kept, args = _record_of_a_backward(shape)
+    asked = _no_room_for(monkeypatch, shape)
+    assert lowering._backward_again(kept, *args) is None and kept.launches.count == 0
+    assert asked == [(1, 4, 40, 64), (1, 2, 40, 64), (1, 2, 40, 64), (1, 4, 40), shape]
+    monkeypatch.undo()
+    dq, dk, dv = lowering._backward_again(kept, *args)
+    assert kept.launches.count == 1 and dq.shape == args[0].shape and dk.shape == dv.shape == args[1].shape
