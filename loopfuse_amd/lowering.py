@@ -657,6 +657,7 @@ _SWITCHES = tuple(n.encode() for n in (
     "LOOPFUSE_DECODE_ROWLOAD", "LOOPFUSE_DECODE_SPLITS", "LOOPFUSE_DECODE_WAVES", "LOOPFUSE_GQAPACK", "LOOPFUSE_KOPTS",
     "LOOPFUSE_PAGED_SWP", "LOOPFUSE_PREFILL", "LOOPFUSE_RECORD_SPECS", "USE_HARDCODE_KERNEL"))
 _MAX_KEPT = 512
+_NO_ROOM_CALLS = 1000      # calls of a backward that found no room for dS until it looks for it again
 _kept: dict = {}
 _PLAIN = (int, float, str, bool, type(None))
 
@@ -687,13 +688,14 @@ def _signature(kind: str, tensors, plan: AttnPlan, options: Optional[dict]):
 
 class _Kept:
     """The launches of one signature.  ``params``: the parameter block, its pointers still to be set; ``results``: shape and
-    dtype of what a call allocates; ``scratch``: floats of split-K partials and where their second array starts."""
+    dtype of what a call allocates; ``scratch``: floats of split-K partials and where their second array starts; ``calls``: how
+    often the record serves (None: as long as it is kept)."""
 
-    __slots__ = ("params", "launches", "results", "scratch", "record")
+    __slots__ = ("params", "launches", "results", "scratch", "record", "calls")
 
-    def __init__(self, params, steps, results, record, scratch=None):
+    def __init__(self, params, steps, results, record, scratch=None, calls=None):
         self.params, self.launches, self.results = bytes(params), runtime.LaunchList(steps), results
-        self.scratch, self.record = scratch, record
+        self.scratch, self.record, self.calls = scratch, record, calls
 
     def attention(self, q, k, v, k_table, v_table, out, lse):
         P = AttnParams.from_buffer_copy(self.params)
@@ -1353,10 +1355,16 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     splits (``bwd_key_blocks``, ``bwd_dq_threads``, ``bwd_q_split``)."""
     key = _signature("bwd", (q, k, v, o, lse, dout), plan, {"key_blocks": key_blocks, "dq_threads": dq_threads, "keep_ds": keep_ds, "q_split": q_split})
     kept = _kept.get(key)
+    if kept is not None and kept.calls is not None:
+        kept.calls -= 1
+        if kept.calls < 0:
+            kept = None
+    room = True
     if kept is not None:
         res = _backward_again(kept, q, k, v, o, lse, dout)
         if res is not None:
             return res
+        room = False                     # (dS asked for by the caller is tried again below, and its error raised)
     dtype = q.dtype
     if dtype not in _DTYPE_CODE:
         raise UnsupportedPlan(f"dtype {dtype} not supported by the MFMA kernels (bf16/fp16 only)")
@@ -1418,14 +1426,14 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     nt = dq_threads or bwd_dq_threads(D, mask, cap, B * Hq, Sq, Sk)
     ds_blocks = bwd_ds_blocks(mask, window, Sq, Sk)
     ds = None
-    if keep_ds if keep_ds is not None else bwd_keep_ds(D, cap, B * Hq, Hq // Hkv, Sk, B * Hq * ds_blocks):
+    if keep_ds or (keep_ds is None and room and bwd_keep_ds(D, cap, B * Hq, Hq // Hkv, Sk, B * Hq * ds_blocks)):
         try:
             ds = torch.empty((B * Hq, ds_blocks, BWD_DS_BLOCK), dtype=dtype, device=q.device)
             P.ds, P.ds_sh = ds.data_ptr(), ds.stride(0)
         except torch.OutOfMemoryError:
             if keep_ds:
                 raise
-            key = None                   # the gradients need no such room; the next call may find it
+            room = False                 # the gradients need no such room
     if q_split is None:
         q_split = not (key_blocks and key_blocks != 1) and bwd_q_split(D, mask, B * Hkv, Sk)
     if q_split:
@@ -1442,7 +1450,9 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
         fn.launch(grid, (block, 1, 1), P)
     _last_launch.set({"kernels": names})
     if key is not None and delta.data_ptr() % 16 == 0:
-        _keep(key, _Kept(P, launches, (dtype, None if ds is None else tuple(ds.shape)), {"kernels": list(names)}))
+        # An allocation that fails makes the allocator give back what it holds and wait for the device: the form without dS is
+        # kept, and room for dS looked for again once in many calls
+        _keep(key, _Kept(P, launches, (dtype, None if ds is None else tuple(ds.shape)), {"kernels": list(names)}, calls=None if room else _NO_ROOM_CALLS))
     return dq, dk, dv
 
 

@@ -208,7 +208,7 @@ def _record_of_a_backward(ds_shape):
 
     kept = lowering._Kept.__new__(lowering._Kept)
     kept.params, kept.launches = bytes(lowering.AttnBwdParams()), Launches()
-    kept.results, kept.scratch, kept.record = (BF, ds_shape), None, {"kernels": []}
+    kept.results, kept.scratch, kept.record, kept.calls = (BF, ds_shape), None, {"kernels": []}, None
     q, k = torch.zeros((1, 4, 40, 64), dtype=BF), torch.zeros((1, 2, 40, 64), dtype=BF)
     return kept, (q, k, k, q, torch.zeros((1, 4, 40)), q)
 
@@ -238,3 +238,32 @@ def test_a_repeated_backward_takes_its_results_before_ds(monkeypatch):
     monkeypatch.undo()
     dq, dk, dv = lowering._backward_again(kept, *args)
     assert kept.launches.count == 1 and dq.shape == args[0].shape and dk.shape == dv.shape == args[1].shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("recorded", [False, True])
+def test_a_backward_without_room_for_ds_looks_for_it_once(recorded, monkeypatch):
+    """No room on the first call of a signature, or on a repeated one that had it: the gradients of the form without dS, which is
+    what the following calls repeat without another attempt, until many calls later there is room again."""
+    q, k, v, dout = (_r((2, h, 300, 128), i) for i, h in enumerate((4, 2, 2, 4)))
+    plan, lse = AttnPlan("causal", scale=0.1), torch.empty((2, 4, 300), device="cuda")
+    args = (q, k, v, attention(q, k, v, plan, lse=lse, choice={"prefill": "swp"}), lse, dout, plan)
+    shape = (8, lowering.bwd_ds_blocks(lowering.MASK_CAUSAL, 0, 300, 300), lowering.BWD_DS_BLOCK)
+    assert lowering.bwd_keep_ds(128, False, 8, 2, 300, 8 * shape[1])
+    want = attention_backward(*args, keep_ds=False)
+    lowering._kept.clear()
+    monkeypatch.setattr(lowering, "_NO_ROOM_CALLS", 3)
+    with_ds = None
+    for _ in range(3 if recorded else 0):
+        with_ds = attention_backward(*args)
+    asked = _no_room_for(monkeypatch, shape)
+    for attempts in (1, 1, 1, 1, 2):
+        got = attention_backward(*args)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)) and asked.count(shape) == attempts
+    with pytest.raises(torch.OutOfMemoryError):
+        attention_backward(*args, keep_ds=True)
+    monkeypatch.undo()
+    lowering._kept.clear()
+    got = attention_backward(*args)
+    assert lowering._last_launch["kernels"] == ["lf_attn_bwd_delta", "lf_attn_bwd_dkdv", "lf_attn_bwd_dq"]
+    assert with_ds is None or all(torch.equal(a, b) for a, b in zip(got, with_ds))
