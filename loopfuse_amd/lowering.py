@@ -352,29 +352,48 @@ def decode_split(units: int, Sk: int, cus: int = 256, per_cu: int = 2) -> int:
     return max(1, min(want, most))
 
 
-def decode_even_split(units: int, Sk: int, D: int, cus: int = 256) -> int:
-    """KV splits of a step whose four waves share a head (``units`` workgroups per split): the count with the least cost in a
-    model of CUs that stream a split's keys and 64 more at the head of it, per round of one workgroup per CU -- a first round that
-    is not full costs nineteen twentieths of one, a later one six tenths --, of the merge launch (230 keys of 128) and of its partials.  Splits are
-    as short as 48 keys, down to where the merge reads as much as it saves.  Fitted on every count for 234 steps of 2 ... 512
-    units, 208 ... 20 000 keys, head dimensions 64 and 128: 0.8 % from the best in the mean (11 % at worst), where the rule before
-    (splits of 512 keys and more, two workgroups per CU, rounded up) was 8.5 %.  Before / now, us: 8 units (one sequence of 8 kv
-    heads, D 128) of 600 keys 13.9 / 8.8, 2048 14.7 / 9.4, 8208 18.0 / 15.7; 24 of 10 432 39 / 31; 80 of 20 000 172 / 134; 192 of
-    2048, which it split, 47.5 / 40.7."""
-    return _even_best(units, Sk, D, cus)[0]
+def decode_even_split(units: int, Sk: int, D: int, cus: int = 256, rows: Optional[int] = None) -> int:
+    """KV splits of a step whose four waves share a head (``units`` workgroups per split, ``rows`` output rows in all, one per
+    unit unless given): the count with the least cost in a model, in keys of 128 streamed by a workgroup per CU, of
+    - rounds of one workgroup per CU, each of a split's keys and 53 more at the head of it; a first round that is not full costs
+      0.89 of one at least, a later one 0.78;
+    - the merge launch, 235, and past four splits, where it takes one row per block, 44 and 34 per round of one row per CU;
+    - the partials, 5.2 per split and round of one row per CU, and 0.9 per split past four.
+    Up to one split per 48 keys, whose lengths are then rounded up to whole multiples of 32 (64 and more, the last what is left).
+    Fitted on every count for 801 steps of 1 ... 512 units, 1 ... 64 rows each, 256 ... 30 000 keys, head dimensions 64 and 128: 0.9 %
+    from the best measured count in the mean.  On 3446 other steps 0.870 of the time of splits of 512 keys, two workgroups per CU, in
+    the mean, and slower than those by more than 3 % on 29 (12 % at worst); a model without the rows 0.883, 238 (25 %).  Splits of 512 keys /
+    without rows / with them, us: D 64, 32 units of 16 rows 2511 keys 9.6 / 11.2 / 9.6, 96 of 16 1188 keys 10.2 / 12.8 / 10.1, 2 of 16 576
+    keys 5.6 / 6.6 / 5.6; D 128, 8 units of 16 rows 2987 keys 13.2 / 9.9 / 9.3, of one row 1730 keys 12.1 / 7.2 / 7.2, of 4 rows 8208 keys
+    13.4 / 12.3 / 12.3; 48 units of 16 rows, D 64, 25 814 keys 68.7 / 54.3 / 54.3."""
+    return _even_best(units, Sk, D, units if rows is None else rows, cus)
 
 
 @functools.lru_cache(maxsize=1024)
-def _even_best(units: int, Sk: int, D: int, cus: int = 256) -> tuple:
-    """(splits, cost) of the cheapest count of a step whose four waves share a head."""
+def _even_best(units: int, Sk: int, D: int, rows: int, cus: int = 256) -> int:
+    per_cu = rows / cus
+
     def cost(n: int) -> float:
         splits, size = _split_lengths(n, Sk)
         full, rest = divmod(units * splits, cus)
-        rounds = full + (max(0.6 if full else 0.95, rest / cus) if rest else 0.0)
-        return (size + 64) * rounds * D / 128 + (230 if splits > 1 else 0) + (0.84 * splits if splits > 4 else 0)
+        t = (size + 53) * (full + (max(0.78 if full else 0.89, rest / cus) if rest else 0.0)) * D / 128
+        if splits > 1:
+            t += 235 + 5.2 * splits * per_cu * D / 128
+        if splits > 4:
+            t += 44 + 0.9 * splits + 34 * per_cu
+        return t
 
-    best, n = min((cost(n), n) for n in range(1, max(1, min(64, Sk // 48)) + 1))
-    return n, best
+    return min((cost(n), n) for n in range(1, max(1, min(64, Sk // 48)) + 1))[1]
+
+
+def _even_time(units: int, Sk: int, D: int, rows: int, cus: int = 256) -> float:
+    """Time of a step in the splits of ``decode_even_split`` as ``decode_coop_beats`` compares it, by the model that its
+    constants were fitted to: CUs that stream a split's keys and 64 more at the head of it, a first round that is not full at
+    nineteen twentieths, a later one at six tenths of a full one, the merge launch and its partials."""
+    splits, size = _split_lengths(_even_best(units, Sk, D, rows, cus), Sk)
+    full, rest = divmod(units * splits, cus)
+    rounds = full + (max(0.6 if full else 0.95, rest / cus) if rest else 0.0)
+    return (size + 64) * rounds * D / 128 + (230 if splits > 1 else 0) + (0.84 * splits if splits > 4 else 0)
 
 
 def _coop_cost(n: int, units: int, Sk: int, rows: int, cus: int = 256) -> float:
@@ -440,7 +459,7 @@ def decode_coop_beats(units: int, waves: int, units_wave: int, Sk: int, rows: in
     if 256 < units < 288:
         return decode_coop_pays(units, Sk, rows, page_size)
     rate, fixed = (0.6, 50) if page_size % 16 == 0 else (0.4, 75)
-    return rate * waves * D / 128 * _coop_best(units, Sk, rows)[1] + fixed < _even_best(units_wave, Sk, D)[1]
+    return rate * waves * D / 128 * _coop_best(units, Sk, rows)[1] + fixed < _even_time(units_wave, Sk, D, units_wave * rows)
 
 
 def _split_lengths(n: int, Sk: int) -> tuple:
@@ -1194,7 +1213,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     elif not num_splits and (headwave or static_scratch or _env("LOOPFUSE_DECODE_SPLITS")):
         num_splits = decode_split(units, Sk, per_cu=1 if headwave else 2)
     elif not num_splits:
-        num_splits = decode_even_split(units, Sk, D)
+        num_splits = decode_even_split(units, Sk, D, rows=B * Hkv * rows)
     nsplit, split_len = _split_lengths(num_splits, Sk)
     P.rows, P.nsplit, P.split_len = rows, nsplit, split_len
     spec = KernelSpec("decode", _DTYPE_CODE[dtype], D, MASK_NONE, plan.softcap is not None, paged,

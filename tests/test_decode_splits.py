@@ -23,6 +23,15 @@ def test_even_splits_stay_within_their_limits():
             assert grid == rows or grid * (1024 // D) >= rows
 
 
+@pytest.mark.parametrize("units,rows,Sk,D,splits", [
+    # all counts measured: more splits cost the partials and the merge of many rows more than their shorter chains gain
+    (32, 512, 2511, 64, 4), (96, 1536, 1188, 64, 2), (2, 32, 576, 64, 1), (64, 1024, 384, 128, 1), (48, 384, 733, 64, 1),
+    # ... and of few rows they do not
+    (8, 8, 1730, 128, 28), (8, 8, 2048, 128, 32), (8, 32, 8208, 128, 29), (2, 2, 640, 128, 10)])
+def test_the_rows_of_a_step_weigh_in_its_splits(units, rows, Sk, D, splits):
+    assert lowering._split_lengths(lowering.decode_even_split(units, Sk, D, rows=rows), Sk)[0] == splits
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("splits", [2, 4, 5, 8, 9, 17, 33, 64])
