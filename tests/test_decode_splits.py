@@ -32,6 +32,20 @@ def test_the_rows_of_a_step_weigh_in_its_splits(units, rows, Sk, D, splits):
     assert lowering._split_lengths(lowering.decode_even_split(units, Sk, D, rows=rows), Sk)[0] == splits
 
 
+def test_few_counts_find_the_cheapest():
+    """A call at a length not seen before evaluates at most ten counts, and the cheapest of all 64 is at most 4 % cheaper (0.2 %
+    in the mean)."""
+    excess = []
+    for units in (1, 2, 8, 12, 32, 48, 64, 96, 128, 200, 256, 257, 512, 1040):
+        for Sk in (1, 47, 95, 96, 200, 576, 1037, 2048, 5003, 16384, 65537):
+            for rows, weight in ((1, 0.5), (1, 1.0), (4, 1.0), (16, 0.5), (16, 1.0)):
+                counts = lowering._even_counts(units, Sk, weight, rows * units / 256)
+                costs = [lowering._even_cost(n, units, Sk, weight, rows * units / 256) for n in range(1, max(1, min(64, Sk // 48)) + 1)]
+                assert len(counts) <= 10 and min(counts) >= 1 and max(counts) <= len(costs)
+                excess.append(min(costs[n - 1] for n in counts) / min(costs) - 1)
+    assert max(excess) <= 0.04 and sum(excess) / len(excess) <= 0.002
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("splits", [2, 4, 5, 8, 9, 17, 33, 64])
