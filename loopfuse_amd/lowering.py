@@ -95,6 +95,16 @@ class KernelSpec:
     bn: int = 0            # prefill_swp: keys per LDS tile, 32 (three workgroups per CU) or 0 / 64 (two)
     extra: tuple = ()      # further -D options (tuning experiments)
 
+    def __hash__(self):    # formed once: a call looks its kernels up by it, several times
+        h = self.__dict__.get("_hash")
+        if h is None:
+            h = hash(tuple(getattr(self, f) for f in self.__dataclass_fields__))
+            object.__setattr__(self, "_hash", h)
+        return h
+
+    def __getstate__(self):    # (strings hash otherwise in another process)
+        return {k: v for k, v in self.__dict__.items() if k != "_hash"}
+
     def options(self) -> list[str]:
         o = list(COMMON_OPTS) + [
             f"-DLF_DTYPE={self.dtype}",
@@ -155,6 +165,9 @@ class KernelSpec:
 
     def source(self) -> str:
         return runtime.read_kernel_source(*self.files())
+
+
+_spec = functools.lru_cache(maxsize=1024)(KernelSpec)      # (half the cost of making one)
 
 
 @dataclasses.dataclass
@@ -366,7 +379,8 @@ def decode_even_split(units: int, Sk: int, D: int, cus: int = 256, rows: Optiona
     without rows / with them, us: D 64, 32 units of 16 rows 2511 keys 9.6 / 11.2 / 9.6, 96 of 16 1188 keys 10.2 / 12.8 / 10.1, 2 of 16 576
     keys 5.6 / 6.6 / 5.6; D 128, 8 units of 16 rows 2987 keys 13.2 / 9.9 / 9.3, of one row 1730 keys 12.1 / 7.2 / 7.2, of 4 rows 8208 keys
     13.4 / 12.3 / 12.3; 48 units of 16 rows, D 64, 25 814 keys 68.7 / 54.3 / 54.3."""
-    return _even_best(units, Sk, D, units if rows is None else rows, cus)
+    # one evaluation for 32 lengths: a cache grows by a token per step, and a length that has not been seen costs 7 us
+    return min(_even_best(units, (Sk + 31) // 32 * 32, D, units if rows is None else rows, cus), max(1, Sk // 48))
 
 
 def _even_cost(n: int, units: int, Sk: int, weight: float, per_cu: float, cus: int = 256) -> float:
@@ -402,7 +416,7 @@ def _even_time(units: int, Sk: int, D: int, rows: int, cus: int = 256) -> float:
     """Time of a step in the splits of ``decode_even_split`` as ``decode_coop_beats`` compares it, by the model that its
     constants were fitted to: CUs that stream a split's keys and 64 more at the head of it, a first round that is not full at
     nineteen twentieths, a later one at six tenths of a full one, the merge launch and its partials."""
-    splits, size = _split_lengths(_even_best(units, Sk, D, rows, cus), Sk)
+    splits, size = _split_lengths(decode_even_split(units, Sk, D, cus, rows), Sk)
     full, rest = divmod(units * splits, cus)
     rounds = full + (max(0.6 if full else 0.95, rest / cus) if rest else 0.0)
     return (size + 64) * rounds * D / 128 + (230 if splits > 1 else 0) + (0.84 * splits if splits > 4 else 0)
@@ -1113,13 +1127,13 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             family = "prefill"                          # swp was refused above (spans): the register-staged kernel
         if family != "prefill_swp" or (mask_own is not None and mask_own.stride(3) != 1):
             write_mask_bias()
-        spec = KernelSpec(family, _DTYPE_CODE[dtype], D, mask, plan.softcap is not None, paged,
-                          page_size, table_i64, v_tr=v_tr if family == "prefill" else True, bias=bias_bits,
-                          denom=plan.denom_add != 0.0, d2=d2, page_size_v=page_size_v, pack=pack, extra=extra,
-                          safe=plan.zero_blind_rows and bool(bias_bits & 1),
-                          bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
-                                             min(Sk, P.window) if mask == MASK_SLIDING else Sk)
-                          if family == "prefill_swp" else 0)
+        spec = _spec(family, _DTYPE_CODE[dtype], D, mask, plan.softcap is not None, paged,
+                     page_size, table_i64, v_tr=v_tr if family == "prefill" else True, bias=bias_bits,
+                     denom=plan.denom_add != 0.0, d2=d2, page_size_v=page_size_v, pack=pack, extra=extra,
+                     safe=plan.zero_blind_rows and bool(bias_bits & 1),
+                     bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
+                                        min(Sk, P.window) if mask == MASK_SLIDING else Sk)
+                     if family == "prefill_swp" else 0)
         bm, bn = TILE_SHAPES[family]
         nw = 4
         for e in spec.extra:                    # tuning: -DLF_NW=8 doubles the q tile
@@ -1161,12 +1175,15 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             get_kernel(spec, classify).launch((nqt, nb_ * nh_, (nkt + 3) // 4), (256, 1, 1), P)
             names.insert(0, classify)
         fn = get_kernel(spec, spec.entry())
-        fn.launch((grid, 1, 1), (64 * nw, 1, 1), P)
         record = {"kernels": names, "grid": grid, "block": 64 * nw, "q_tile_rows": bm, "kv_tile_rows": bn,
                   "heads_per_workgroup": spec.pack or 1}
-        _last_launch.set(record)
         if keeps:
-            _keep(key, _Kept(P, [(fn, (grid, 1, 1), 64 * nw)], (tuple(out.shape), dtype), dict(record)))
+            kept = _Kept(P, [(fn, (grid, 1, 1), 64 * nw)], ((B, Hq, Sq, D), dtype), record)
+            kept.launches.launch(P)
+            _keep(key, kept)
+        else:
+            fn.launch((grid, 1, 1), (64 * nw, 1, 1), P)
+        _last_launch.set(dict(record))
         return (out, visits) if record_visits else out
 
     if family != "decode":
@@ -1228,12 +1245,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         num_splits = decode_even_split(units, Sk, D, rows=B * Hkv * rows)
     nsplit, split_len = _split_lengths(num_splits, Sk)
     P.rows, P.nsplit, P.split_len = rows, nsplit, split_len
-    spec = KernelSpec("decode", _DTYPE_CODE[dtype], D, MASK_NONE, plan.softcap is not None, paged,
-                      page_size, table_i64, rows=DECODE_QROWS, waves=waves, headwave=headwave, page_size_v=page_size_v,
-                      coop=coop > 0,
-                      rowload=not coop and _decode_rowload(paged, page_size, page_size_v, bias_bits),
-                      bias=bias_bits, safe=plan.zero_blind_rows and bool(bias_bits),
-                      extra=tuple(_env("LOOPFUSE_KOPTS", "").split()))
+    spec = _spec("decode", _DTYPE_CODE[dtype], D, MASK_NONE, plan.softcap is not None, paged,
+                 page_size, table_i64, rows=DECODE_QROWS, waves=waves, headwave=headwave, page_size_v=page_size_v,
+                 coop=coop > 0,
+                 rowload=not coop and _decode_rowload(paged, page_size, page_size_v, bias_bits),
+                 bias=bias_bits, safe=plan.zero_blind_rows and bool(bias_bits),
+                 extra=tuple(_env("LOOPFUSE_KOPTS", "").split()))
     combine_grid = decode_combine_grid(B * Hkv * rows, nsplit, D)
     if static_scratch:
         if nsplit <= 1 or not merge_splits:
@@ -1248,25 +1265,30 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
     named = _kernels_of(spec)
     step, combine = get_kernel(spec, "lf_attn_decode", named), get_kernel(spec, "lf_attn_decode_combine", named)
     steps = [(step, (units, nsplit, 1), 64 * spec.waves)] + ([(combine, (combine_grid, 1, 1), 256)] if nsplit > 1 else [])
-    scratch_size = None
+    record = {"kernels": ["lf_attn_decode"] + (["lf_attn_decode_combine"] if nsplit > 1 and merge_splits else []),
+              "grid": (units, nsplit), "block": 64 * spec.waves, "head_per_wave": headwave,
+              "cooperative_loads": spec.coop}
+    nrow = B * Hkv * rows * nsplit
+    if keeps:
+        kept = _Kept(P, steps, ((B, Hq, Sq, D), dtype), record, (nrow * (D + 2), 4 * nrow * D) if nsplit > 1 else None)
     if nsplit > 1:
-        nrow = B * Hkv * rows * nsplit
-        scratch_size = (nrow * (D + 2), 4 * nrow * D)
         with _scratch_lock:        # no other thread's step on this stream between the two launches
             scratch = _get_scratch(q.device, nrow * (D + 2))
             P.part_acc = scratch.data_ptr()
             P.part_ml = scratch.data_ptr() + 4 * nrow * D
-            step.launch((units, nsplit, 1), (64 * spec.waves, 1, 1), P)
-            if merge_splits:
-                combine.launch((combine_grid, 1, 1), (256, 1, 1), P)
+            if keeps:
+                kept.launches.launch(P)
+            else:
+                step.launch((units, nsplit, 1), (64 * spec.waves, 1, 1), P)
+                if merge_splits:
+                    combine.launch((combine_grid, 1, 1), (256, 1, 1), P)
+    elif keeps:
+        kept.launches.launch(P)
     else:
         step.launch((units, nsplit, 1), (64 * spec.waves, 1, 1), P)
-    record = {"kernels": ["lf_attn_decode"] + (["lf_attn_decode_combine"] if nsplit > 1 and merge_splits else []),
-              "grid": (units, nsplit), "block": 64 * spec.waves, "head_per_wave": headwave,
-              "cooperative_loads": spec.coop}
-    _last_launch.set(record)
     if keeps:
-        _keep(key, _Kept(P, steps, (tuple(out.shape), dtype), dict(record), scratch_size))
+        _keep(key, kept)
+    _last_launch.set(dict(record))
     return out
 
 
@@ -1366,6 +1388,7 @@ def bwd_keep_ds(D: int, softcap: bool, units: int, group: int, Sk: int, blocks: 
     return D == 128 or softcap or (units <= 64 and group <= 4 and Sk >= 512 and size <= 176 << 20)
 
 
+@functools.lru_cache(maxsize=256)
 def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False, key_blocks: int = 1,
              dq_threads: int = 512, keep_ds: bool = False, q_split: bool = False) -> KernelSpec:
     return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap,
@@ -1446,10 +1469,14 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     for name, t in (("q", q), ("k", k), ("v", v), ("o", o), ("dout", dout), ("dq", dq), ("dk", dk), ("dv", dv),
                     ("lse", lse), ("delta", delta)):
         setattr(P, name, t.data_ptr())
-    for pre, t in (("q", q), ("k", k), ("v", v), ("o", o), ("do", dout), ("dq", dq), ("dk", dk), ("dv", dv)):
-        setattr(P, pre + "_sb", t.stride(0))
-        setattr(P, pre + "_sh", t.stride(1))
-        setattr(P, pre + "_ss", t.stride(2))
+    P.q_sb, P.q_sh, P.q_ss = q.stride()[:3]
+    P.k_sb, P.k_sh, P.k_ss = k.stride()[:3]
+    P.v_sb, P.v_sh, P.v_ss = v.stride()[:3]
+    P.o_sb, P.o_sh, P.o_ss = o.stride()[:3]
+    P.do_sb, P.do_sh, P.do_ss = dout.stride()[:3]
+    P.dq_sb, P.dq_sh, P.dq_ss = dq.stride()[:3]
+    P.dk_sb, P.dk_sh, P.dk_ss = dk.stride()[:3]
+    P.dv_sb, P.dv_sh, P.dv_ss = dv.stride()[:3]
     P.B, P.Hq, P.Hkv, P.Sq, P.Sk, P.window = B, Hq, Hkv, Sq, Sk, window
     P.scale = float(plan.scale)
     P.softcap = softcap if softcap is not None else 0.0
@@ -1476,14 +1503,18 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
              "lf_attn_bwd_dq": (xcd_slots(B * Hkv, (Hq // Hkv) * -(-Sq // (nt // 2))), nt)}
     # without dS of lf_attn_bwd_dkdv, lf_attn_bwd_dq with 256 threads forms delta itself, and lf_attn_bwd_dkdv reads it
     names = ["lf_attn_bwd_dq", "lf_attn_bwd_dkdv"] if nt == 256 and ds is None else list(steps)
-    launches = [(get_kernel(spec, name), (steps[name][0], 1, 1), steps[name][1]) for name in names]
-    for fn, grid, block in launches:
-        fn.launch(grid, (block, 1, 1), P)
-    _last_launch.set({"kernels": names})
-    if key is not None and delta.data_ptr() % 16 == 0:
+    named = _kernels_of(spec)
+    launches = [(get_kernel(spec, name, named), (steps[name][0], 1, 1), steps[name][1]) for name in names]
+    if key is not None:
         # An allocation that fails makes the allocator give back what it holds and wait for the device: the form without dS is
         # kept, and room for dS looked for again once in many calls
-        _keep(key, _Kept(P, launches, (dtype, None if ds is None else tuple(ds.shape)), {"kernels": list(names)}, calls=None if room else _NO_ROOM_CALLS))
+        kept = _Kept(P, launches, (dtype, None if ds is None else tuple(ds.shape)), {"kernels": names}, calls=None if room else _NO_ROOM_CALLS)
+        kept.launches.launch(P)
+        _keep(key, kept)
+    else:
+        for fn, grid, block in launches:
+            fn.launch(grid, (block, 1, 1), P)
+    _last_launch.set({"kernels": names})
     return dq, dk, dv
 
 

@@ -210,7 +210,7 @@ class LaunchList:
 
     def __init__(self, steps: Sequence[tuple]):
         self.kernels = [k for k, _, _ in steps]          # keeps the modules alive
-        self._items = (_LaunchItem * len(steps))(*[_LaunchItem(k.handle, *grid, threads) for k, grid, threads in steps])
+        self._items = (_LaunchItem * len(steps))(*[(k.handle, *grid, threads) for k, grid, threads in steps])
         self._at, self._count = ctypes.addressof(self._items), len(steps)
         self._launch = lib().lf_launch_list
 

@@ -46,6 +46,14 @@ def test_few_counts_find_the_cheapest():
     assert max(excess) <= 0.04 and sum(excess) / len(excess) <= 0.002
 
 
+def test_a_growing_cache_evaluates_its_splits_once_in_32_steps():
+    lowering._even_best.cache_clear()
+    for Sk in range(1, 1025):
+        n = lowering.decode_even_split(8, Sk, 128, rows=32)
+        assert n == 1 or Sk // n >= 48
+    assert lowering._even_best.cache_info().misses <= 1024 // 32 + 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("splits", [2, 4, 5, 8, 9, 17, 33, 64])

@@ -267,3 +267,32 @@ def test_a_backward_without_room_for_ds_looks_for_it_once(recorded, monkeypatch)
     got = attention_backward(*args)
     assert lowering._last_launch["kernels"] == ["lf_attn_bwd_delta", "lf_attn_bwd_dkdv", "lf_attn_bwd_dq"]
     assert with_ds is None or all(torch.equal(a, b) for a, b in zip(got, with_ds))
+
+
+@pytest.mark.gpu
+def test_a_recorded_call_launches_through_its_record(monkeypatch):
+    """The first call of a signature too: one call of the library for all its kernels."""
+    from loopfuse_amd import runtime
+
+    calls = []
+    one, many = runtime.Kernel.launch, runtime.LaunchList.launch
+    monkeypatch.setattr(runtime.Kernel, "launch", lambda self, *a, **kw: (calls.append("one"), one(self, *a, **kw))[1])
+    monkeypatch.setattr(runtime.LaunchList, "launch", lambda self, *a: (calls.append("list"), many(self, *a))[1])
+    for form in ("prefill", "decode", "decode paged"):
+        args, kw = FORMS[form](41)
+        lowering._kept.clear()
+        calls.clear()
+        first, second = attention(*args, **kw), attention(*args, **kw)
+        assert calls == ["list", "list"] and torch.equal(first, second)
+
+
+def test_a_specialisation_hashes_anew_in_another_process():
+    """The hash is formed once per object, and is not what a copy in another process, whose strings hash otherwise, may keep."""
+    import dataclasses
+    import pickle
+
+    spec = lowering.bwd_spec(BF, 64, lowering.MASK_CAUSAL)
+    assert hash(spec) == hash(dataclasses.replace(spec)) and spec.__dict__["_hash"] == hash(spec)
+    again = pickle.loads(pickle.dumps(spec))
+    assert "_hash" not in again.__dict__ and again == spec and {spec: 1}[again] == 1
+    assert dataclasses.replace(spec, head_dim=128) != spec and hash(dataclasses.replace(spec, head_dim=128)) != hash(spec)
