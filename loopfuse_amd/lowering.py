@@ -604,6 +604,19 @@ _tuned: dict = {}
 _TUNE_FILE = os.path.join(runtime.CACHE_DIR, "autotune.json")
 
 
+@functools.lru_cache(maxsize=None)
+def _rules_version() -> str:
+    """Digest of the kernels' sources and of the rules in this file: a choice measured before either changed was measured among
+    other candidates, against another default, and is not taken from the file any more."""
+    import hashlib
+    h = hashlib.sha256()
+    for path in [os.path.join(runtime.KERNEL_DIR, f) for f in sorted(os.listdir(runtime.KERNEL_DIR))] + [__file__]:
+        if os.path.isfile(path):
+            with open(path, "rb") as fh:
+                h.update(fh.read())
+    return h.hexdigest()[:12]
+
+
 def _tune_key(q, k, plan: AttnPlan, k_table, bias_bits: int) -> str:
     B, Hq, Sq, D = q.shape
     if plan.k_paged:
@@ -614,7 +627,7 @@ def _tune_key(q, k, plan: AttnPlan, k_table, bias_bits: int) -> str:
         Hkv, Sk, ps = k.shape[1], k.shape[2], 0
     bucket = lambda n: 1 << max(0, (int(n) - 1)).bit_length()       # next power of two
     return (f"{q.dtype}|D{D}|m{plan.mask}|c{int(plan.softcap is not None)}|p{int(plan.k_paged)}{int(plan.v_paged)}x{ps}"
-            f"|B{bucket(B * Hkv)}|g{Hq // Hkv}|q{bucket(Sq)}|k{bucket(Sk)}|b{bias_bits}")
+            f"|B{bucket(B * Hkv)}|g{Hq // Hkv}|q{bucket(Sq)}|k{bucket(Sk)}|b{bias_bits}|r{_rules_version()}")
 
 
 def _load_tuned() -> None:
@@ -622,16 +635,16 @@ def _load_tuned() -> None:
         try:
             import json
             with open(_TUNE_FILE) as fh:
-                _tuned.update(json.load(fh))
-        except (OSError, ValueError):
+                _tuned.update({key: choice for key, choice in json.load(fh).items() if key.endswith(f"|r{_rules_version()}")})
+        except (OSError, ValueError, AttributeError):
             pass
 
 
 def tuned_attention(q, k, v, plan: AttnPlan, k_table=None, v_table=None, **kw):
     """``attention`` with the launch heuristics chosen by measurement: on the first call
     of a shape class each candidate is timed on the call's own tensors (HIP events, a few
-    launches), the winner is remembered in the process and in ``autotune.json`` beside
-    the code-object cache.  Used by the backend under ``mode="max-autotune"``."""
+    launches), the winner is remembered in the process and, until a kernel or a rule changes, in
+    ``autotune.json`` beside the code-object cache.  Used by the backend under ``mode="max-autotune"``."""
     if kw.get("score_bias") is not None or kw.get("score_mask") is not None or kw.get("out_bias") is not None or kw.get("record_visits") \
             or kw.get("force_family") or kw.get("num_splits") or kw.get("choice") or plan.denom_add != 0.0 or kw.get("q2") is not None:
         return attention(q, k, v, plan, k_table, v_table, **kw)

@@ -296,3 +296,22 @@ def test_a_specialisation_hashes_anew_in_another_process():
     again = pickle.loads(pickle.dumps(spec))
     assert "_hash" not in again.__dict__ and again == spec and {spec: 1}[again] == 1
     assert dataclasses.replace(spec, head_dim=128) != spec and hash(dataclasses.replace(spec, head_dim=128)) != hash(spec)
+
+
+def test_a_tuned_choice_is_not_taken_from_before_the_kernels_changed(monkeypatch, tmp_path):
+    """The file of measured choices holds those of other kernels and rules too: they are neither found nor written again."""
+    import json
+
+    q, k = torch.zeros((1, 8, 1, 64), dtype=BF), torch.zeros((1, 8, 500, 64), dtype=BF)
+    key = lowering._tune_key(q, k, AttnPlan(scale=0.1), None, 0)
+    path = tmp_path / "autotune.json"
+    monkeypatch.setattr(lowering, "_TUNE_FILE", str(path))
+    monkeypatch.setattr(lowering, "_tuned", {})
+    path.write_text(json.dumps({key: {"splits": 4}, key.rsplit("|r", 1)[0]: {"splits": 2}, key[:-1] + "x": {"splits": 8}}))
+    lowering._load_tuned()
+    assert lowering._tuned == {key: {"splits": 4}}
+    monkeypatch.setattr(lowering, "_rules_version", lambda: "later")
+    assert lowering._tune_key(q, k, AttnPlan(scale=0.1), None, 0) != key
+    lowering._tuned.clear()
+    lowering._load_tuned()
+    assert lowering._tuned == {}
