@@ -107,7 +107,7 @@ __device__ __forceinline__ lfg_u32x4 lfg_make_buffer(const void* base, unsigned 
   return rs;
 }
 // One wave-level direct-to-LDS load (not tracked by the compiler's wait counters: callers wait with s_waitcnt vmcnt);
-// kNt: non-temporal, for an operand that one workgroup alone reads
+// kNt: non-temporal, for an operand that is not read again
 template <bool kNt>
 __device__ __forceinline__ void lfg_dma(const lfg_u32x4& rs, unsigned voff, unsigned lds_addr) {
   unsigned m0_written;
@@ -172,6 +172,7 @@ class GemmInfo:
     b_dims: tuple               # (dim of B indexed by n, dim indexed by k)
     a_batch_dims: list          # dims of A indexed by a batch atom
     b_batch_dims: list
+    b_batch: list               # the batch atoms that index them
     flags_at: int = 0           # n[flags_at]: the output's rows are contiguous and aligned for 8- / 16-byte stores;
                                 # n[flags_at + 1], n[flags_at + 2]: bytes of A / B reachable from a batch element's base;
                                 # n[flags_at + 3], n[flags_at + 4]: parts that k is split into, steps of 64 k per part
@@ -231,7 +232,15 @@ def match(nest: ir.Nest, dtypes: dict) -> Optional[GemmInfo]:
     pos = lambda lst, a: next(i for i, x in enumerate(lst) if x is a)      # noqa: E731
     return GemmInfo(m, n, k, batch, d.a.buf, d.b.buf, (pos(ia, m), pos(ia, k)), (pos(ib, n), pos(ib, k)),
                     [i for i, x in enumerate(ia) if x is not None and has(batch, x)],
-                    [i for i, x in enumerate(ib) if x is not None and has(batch, x)])
+                    [i for i, x in enumerate(ib) if x is not None and has(batch, x)],
+                    [x for x in ib if x is not None and has(batch, x)])
+
+
+def b_batches(info: GemmInfo, ext: dict, stride) -> tuple:
+    """(matrices B that the batch holds, batch elements that share each): an atom shares B where it does not index it or, in an
+    expanded tensor, does not move along it (``stride(d)`` of its dimension d)."""
+    own = [a for d, a in zip(info.b_batch_dims, info.b_batch) if stride(d)]
+    return math.prod(ext[a.id] for a in own), math.prod(ext[a.id] for a in info.batch if not any(a is x for x in own))
 
 
 class GemmEmitter(Emitter):
@@ -608,8 +617,18 @@ def choose(M: int, N: int, K: int, batch: int) -> tuple:
     return best
 
 
-def stream_b(M: int) -> bool:
-    """B by non-temporal loads: where at most four tile rows, resident at the same time, read it, so that it need not stay in an
-    L2 it would push A out of.  us, plain / non-temporal, M x N x K: 16 x 4096 x 4096 14.1 / 13.3, 64 x 16384 x 4096 33.7 /
-    30.4, 256 x 16384 x 4096 48.3 / 46.2; 512 x 4096 x 4096 32.6 / 33.1, 400 x 2048 x 8192 30.0 / 31.3."""
-    return M <= 256
+def stream_b(M: int, N: int, K: int, own: int, shared: int) -> bool:
+    """B by non-temporal loads (16-bit elements; ``own``, ``shared`` of ``b_batches``): they leave an L2 to A, and cost where several
+    tiles read B at different times, or where it would have stayed in a cache.
+    Non-temporal over plain, weights from HBM, 204 drawn products of one matrix B and 72 chosen ones: up to 32 rows 0.98 in the mean
+    (100 MB and more 0.95); 33 ... 64 rows 0.99 below 18 MB, 1.01 up to 100 MB; 65 ... 256 rows 1.01 below 18 MB, 1.06 (up to 1.2) up to
+    100 MB, 1.01 up to 150, 0.97 beyond.  us, M x N x K, plain / non-temporal: 32 x 16384 x 4096 30.9 / 29.0, 64 x 1024 x 4096 11.3 / 10.6,
+    64 x 28672 x 8192 83.5 / 74.2, 128 x 4096 x 4096 16.2 / 18.4, 256 x 4096 x 4096 22.4 / 27.2, 256 x 2048 x 8192 22.3 / 26.1; linear -> gelu
+    -> linear of 256 rows, 2048 / 8192 wide 45.2 / 48.6, 4096 / 16384 103.7 / 99.0.  A B that is still in a cache from the call before: 256
+    x 4096 x 4096 21.6 / 27.2, 256 x 16384 x 4096 46.5 / 48.3.
+    Batches, B x M x N x K: shared weights 2 x 128 x 4096 x 4096 25.4 / 28.7, 4 x 16 x 16384 x 4096 76 / 87, 16 x 128 x 16384 x 4096 319 / 407;
+    a B for each 64 x 64 x 512 x 512 11.4 / 10.7, 32 x 100 x 2048 x 2048 77 / 66, 16 x 256 x 1024 x 1024 19.1 / 19.2."""
+    if shared > 1 or M > 256:
+        return False
+    size = 2 * N * K
+    return own > 1 or M <= (64 if size < 16 << 20 else 32) or size >= 96 << 20

@@ -251,7 +251,10 @@ class GenericProgram:
                     layouts = None
                 if layouts is not None and all(ext.get(a.id, 0) > 0 for a in self.gemm[ni][0].atoms):
                     shape, parts = self._gemm_shape(self.gemm[ni][1], ext)
-                    fns = self._gemm_kernel(ni, layouts, shape, parts > 1, emit_gemm.stream_b(ext[self.gemm[ni][1].m.id]))
+                    info = self.gemm[ni][1]
+                    streams = emit_gemm.stream_b(ext[info.m.id], ext[info.n.id], ext[info.k.id],
+                                                 *emit_gemm.b_batches(info, ext, bufs[info.b_buf.name].stride))
+                    fns = self._gemm_kernel(ni, layouts, shape, parts > 1, streams)
                     steps += self._launch_gemm(fns, shape, parts, *self.gemm[ni],
                                                bufs, ext, args, lambda name, n: allocs.append((len(steps), name, (n,), torch.float32)))
                     counters["mfma"] += 1

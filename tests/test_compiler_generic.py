@@ -341,6 +341,26 @@ def test_contractions_of_half_precision_operands_get_an_mfma_kernel():
     assert len(sm32.nests) == 3 and not sm32.gemm
 
 
+@pytest.mark.parametrize("a,b,expanded,batches,streams", [
+    ((32, 4096), (4096, 4096), False, (1, 1), True), ((33, 4096), (4096, 4096), False, (1, 1), False), ((256, 4096), (4096, 4096), False, (1, 1), False),
+    ((64, 1024), (1024, 4096), False, (1, 1), True), ((65, 1024), (1024, 4096), False, (1, 1), False),
+    ((256, 4096), (4096, 16384), False, (1, 1), True), ((257, 4096), (4096, 16384), False, (1, 1), False),
+    ((2, 16, 512), (512, 64), False, (1, 2), False), ((2, 3, 16, 512), (512, 64), False, (1, 6), False),       # shared by the batch
+    ((16, 128, 512), (16, 512, 64), False, (16, 1), True), ((16, 128, 512), (16, 512, 64), True, (1, 16), False),
+    ((16, 257, 512), (16, 512, 64), False, (16, 1), False)])
+def test_which_operands_are_streamed(a, b, expanded, batches, streams):
+    """By the rows and the bytes that meet B; never a B that the elements of a batch share, also as a matrix expanded over them."""
+    from loopfuse_amd.compiler import emit_gemm
+
+    prog = generic.GenericProgram(_bf16_graph(lambda x, y: torch.nn.functional.gelu(x @ y), [a, b]))
+    (_, info), = prog.gemm.values()
+    x, y = torch.empty(a, dtype=torch.bfloat16), torch.empty(b[-2:] if expanded else b, dtype=torch.bfloat16).expand(b)
+    bufs, ext = {t.name: arg for t, arg in zip((info.a_buf, info.b_buf), (x, y))}, {}
+    prog._solve(prog.nests[0], bufs, ext, {})
+    assert emit_gemm.b_batches(info, ext, y.stride) == batches
+    assert emit_gemm.stream_b(a[-2], b[-1], b[-2], *batches) == streams
+
+
 @pytest.mark.parametrize("shape", ["s", "l"])
 @pytest.mark.parametrize("layouts", [(1, 1), (1, 0), (0, 1), (0, 0)])
 def test_mfma_kernel_compiles_for_every_operand_layout(shim_built, layouts, shape):
