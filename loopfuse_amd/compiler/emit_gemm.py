@@ -594,13 +594,15 @@ def choose(M: int, N: int, K: int, batch: int) -> tuple:
     s 90.3 us) and 11 % off (100 x 1024, K 4096: n in 16 parts 12.8, in 8 11.5).  What it is for: a product whose tiles leave
     most CUs idle, or alone with the latency of their loads.  M 256, us: N 4096 K 16384 218 (64 tiles s) -> 49 (d, 4 parts);
     N 16384 K 4096 66 -> 46 (d); M 64, N 4096 K 16384 214 -> 29 (n, 8 parts); M 1024, N 4096 K 16384 218 -> 130 (l, 4 parts);
-    M 2000, N 1024 K 512 17 -> 11 (n)."""
+    M 2000, N 1024 K 512 17 -> 11 (n).  n serves the fewest rows too: its tile pads least.  M up to 32, d or
+    s / n, us: 16 x 4096, K 4096 13.5 / 12.7; 32 x 1024, K 4096 11.0 / 10.0; 8 x 4096, K 16384 29.4 / 26.3; 3 x 21888, K 3456 35.2 / 29.5; of
+    99 drawn products, batches of 1 ... 16, 0.93 of the time in the mean, two are 4 % slower."""
     steps = -(-K // BK)
     best, best_t = ("s", 1), math.inf
     for shape, ((step_1, step_2), fixed, slots) in _COST.items():
         bm, bn = tile_extent(shape)
-        if shape in "mln" and M <= bm // 2 or shape == "l" and N <= bn // 2:
-            continue                         # half of the tile would be padding
+        if shape in "ml" and M <= bm // 2 or shape == "l" and N <= bn // 2:
+            continue                         # half of the tile would be padding, and a smaller one has less (s, d, n)
         tiles = -(-M // bm) * -(-N // bn) * batch
         for parts in range(1, max(1, min(32, steps // 4)) + 1):
             if parts > 1 and tiles * parts > slots:      # one round, whose partials are 2^24 floats at most

@@ -425,7 +425,7 @@ def test_every_tile_of_a_product_fits_its_registers_and_lds(shim_built, shape, s
 def test_tile_and_parts_of_a_product_stay_within_their_limits():
     """``emit_gemm.choose`` over sizes from 1 on: every part holds at least four steps, a split launch is one round of
     resident workgroups of its tile (which bounds its partials, 2^24 floats at most), and tiles that are half padding are
-    not taken."""
+    not taken where a smaller one has less."""
     from loopfuse_amd.compiler import emit_gemm
 
     sizes = [1, 17, 64, 129, 257, 700, 2048, 8191, 65536]
@@ -440,4 +440,12 @@ def test_tile_and_parts_of_a_product_stay_within_their_limits():
                     assert 1 <= parts <= 32 and (parts == 1 or steps // parts >= 4)
                     if parts > 1:
                         assert tiles * parts <= emit_gemm._COST[shape][2] and parts * tiles * bm * bn <= 1 << 24
-                    assert shape in "sd" or M > bm // 2
+                    assert shape in "sdn" or M > bm // 2
+
+
+@pytest.mark.parametrize("N,K", [(4096, 4096), (1024, 4096), (4096, 16384), (1024, 1024), (640, 2880), (2880, 640), (4096, 512)])
+def test_few_rows_take_the_tile_that_pads_least(N, K):
+    """... as more rows do that its 64 hold: at 33 and 64 rows the tile of 64, so at 1 ... 32 of them."""
+    from loopfuse_amd.compiler import emit_gemm
+
+    assert {emit_gemm.choose(M, N, K, 1)[0] for M in (1, 8, 16, 32, 33, 64)} == {"n"}
