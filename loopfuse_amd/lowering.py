@@ -480,10 +480,14 @@ def decode_coop_beats(units: int, waves: int, units_wave: int, Sk: int, rows: in
     32 768 keys: 0.46 and 0.42 % (short, long pages) off the faster form in the mean there, where ``decode_coop_pays`` was 2.4 %.
     Of the 107 steps that go the other way now, 0.90 of their time in the mean, three are 3 ... 4 % slower.  Before / now, us: 2
     sequences of 8930, 16 heads of 64, one-token pages 24.0 / 18.8; 9 of 5120, 24 heads of 64, pages of 16 60 / 48; 60 of 64, 32
-    heads of 128, pages of 8 23.0 / 15.4.  A few workgroups more than CUs that are not split keep the older rule (264 of 611
-    keys, pages of 1: 156 against 137 us)."""
-    if 256 < units < 288:
-        return decode_coop_pays(units, Sk, rows, page_size)
+    heads of 128, pages of 8 23.0 / 15.4.  A few workgroups more than CUs that are not split, pages shorter than 16: 8 heads of 128
+    leave the second round to the other form, at any length (257 ... 287 workgroups, 305 ... 5602 keys: 1.04 ... 1.17 of its time; 264 of 611 keys
+    156 against 137 us), half as many bytes per token do not (0.84 ... 1.04 from 128 keys on, 285 of 144 24.6 against 29.5).  Over 404 steps of
+    257 ... 530 workgroups that is 0.6 % off the faster form in the mean there (by the costs 6.1, by ``decode_coop_pays`` 5.6); the costs
+    are 0.5 % off with short pages from 288 workgroups on, with pages of 16 1.1 % up to there and 6 % beyond (7.6 by ``decode_coop_pays``).
+    """
+    if 256 < units < 288 and page_size % 16:
+        return waves * D < 1024
     rate, fixed = (0.6, 50) if page_size % 16 == 0 else (0.4, 75)
     return rate * waves * D / 128 * _coop_best(units, Sk, rows)[1] + fixed < _even_time(units_wave, Sk, D, units_wave * rows)
 

@@ -82,7 +82,8 @@ def test_merge_of_any_number_of_splits(splits, D):
 @pytest.mark.parametrize("B,Hkv,D,Sk,group,page,beats", [
     (2, 16, 64, 8930, 1, 1, True), (9, 24, 64, 5120, 1, 16, True), (60, 32, 128, 64, 1, 8, True),      # measured on both sides
     (64, 8, 128, 2048, 4, 16, True), (64, 4, 128, 2048, 8, 1, True),
-    (66, 32, 128, 611, 2, 1, False), (1, 8, 128, 8208, 4, 16, False), (1, 16, 128, 108, 1, 1, False)])
+    (66, 32, 128, 611, 2, 1, False), (281, 8, 128, 305, 4, 1, False), (269, 8, 128, 5602, 2, 1, False), (272, 8, 64, 129, 2, 1, True),
+    (285, 4, 128, 144, 8, 1, True), (264, 8, 128, 496, 4, 16, False), (1, 8, 128, 8208, 4, 16, False), (1, 16, 128, 108, 1, 1, False)])
 def test_cooperative_decode_is_chosen_where_it_is_faster(B, Hkv, D, Sk, group, page, beats):
     waves = 8 if Hkv % 8 == 0 else 4
     assert lowering.decode_coop_beats(B * Hkv // waves, waves, B * Hkv, Sk, group, page, D) == beats
