@@ -390,9 +390,9 @@ def test_mfma_kernel_compiles_for_every_operand_layout(shim_built, layouts, shap
 
 
 @pytest.mark.parametrize("split", [False, True])
-@pytest.mark.parametrize("shape", ["s", "d", "m", "l"])
+@pytest.mark.parametrize("shape", ["s", "d", "m", "l", "n"])
 def test_every_tile_of_a_product_fits_its_registers_and_lds(shim_built, shape, split):
-    """All four tiles, whole and split with the kernel that adds up the parts: no scratch memory, two waves per SIMD, LDS as
+    """All tiles, whole and split with the kernel that adds up the parts: no scratch memory, two waves per SIMD, LDS as
     the stages of the tile say."""
     import re
     import subprocess

@@ -7,14 +7,14 @@ from loopfuse_amd.lowering import AttnPlan, attention
 
 
 def test_even_splits_stay_within_their_limits():
-    """Splits of 48 keys at least and 64 of them at most; the sequence is covered; a short sequence and a launch that fills the
+    """64 splits at most, all but the last of the same length, 64 keys at least, the last what is left; the sequence is covered; a short sequence and a launch that fills the
     CUs by itself are left whole; a long one of few units is split over all CUs."""
     for D in (64, 128):
         for units in (1, 2, 8, 24, 96, 255, 256, 257, 700):
             for Sk in (16, 47, 96, 208, 1000, 8208, 65536):
                 n = lowering.decode_even_split(units, Sk, D)
                 splits, size = lowering._split_lengths(n, Sk)
-                assert 1 <= n <= 64 and (n == 1 or Sk // n >= 48) and splits * size >= Sk > (splits - 1) * size
+                assert 1 <= splits <= n <= 64 and (splits == 1 or size >= 64) and 1 <= Sk - (splits - 1) * size <= size
         assert lowering.decode_even_split(256, 4000, D) == 1 and lowering.decode_even_split(4, 90, D) == 1
         assert lowering._split_lengths(lowering.decode_even_split(8, 20000, D), 20000)[0] >= 29
     for rows, nsplit in ((1, 1), (7, 4), (8, 5), (4097, 64)):
@@ -50,18 +50,19 @@ def test_a_growing_cache_evaluates_its_splits_once_in_32_steps():
     lowering._even_best.cache_clear()
     for Sk in range(1, 1025):
         n = lowering.decode_even_split(8, Sk, 128, rows=32)
-        assert n == 1 or Sk // n >= 48
+        splits, size = lowering._split_lengths(n, Sk)
+        assert splits == 1 or size >= 64
     assert lowering._even_best.cache_info().misses <= 1024 // 32 + 1
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("splits", [2, 4, 5, 8, 9, 17, 33, 64])
+@pytest.mark.parametrize("splits", [2, 4, 5, 8, 9, 17, 33, 37, 64, 70])
 def test_merge_of_any_number_of_splits(splits, D):
-    """Fewer splits than a block's groups of threads take at a time, as many, more than one round of them, and a last group that
-    has none; against float64 with the error of the unsplit step (fp32 sums: the order of the merge does not show in bf16),
+    """Fewer splits than a block's groups of threads take at a time, as many, a second round of some of the groups (from 33 splits at
+    head dimension 128, 65 at 64), and a last group that has none; against float64 with the error of the unsplit step (fp32 sums: the order of the merge does not show in bf16),
     also where whole splits hold nothing but keys of probability 0 (a bias of -inf) and where a row sees a single key."""
-    B, Hq, Hkv, S = 2, 6, 2, 64 * 64
+    B, Hq, Hkv, S = 2, 6, 2, 64 * splits - 16
     g = torch.Generator(device="cuda").manual_seed(splits)
     q, k, v = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((B, Hq, 1, D), (B, Hkv, S, D), (B, Hkv, S, D)))
     plan = AttnPlan(scale=D ** -0.5)
@@ -73,6 +74,7 @@ def test_merge_of_any_number_of_splits(splits, D):
         kw = {} if live == slice(0, S) else {"score_bias": bias}
         out = attention(q, k, v, plan, num_splits=splits, **kw)
         assert lowering.attention.last_launch["kernels"] == ["lf_attn_decode", "lf_attn_decode_combine"]
+        assert lowering.attention.last_launch["grid"][1] == splits
         want = torch.matmul(torch.softmax(scores + bias.double(), dim=-1), vv)
         whole = attention(q, k, v, plan, num_splits=1, **kw)
         err, err_whole = ((x.double() - want).norm() / want.norm() for x in (out, whole))

@@ -216,17 +216,23 @@ def test_every_backward_build_keeps_its_accumulators(shim_built, spec):
 
 
 def test_every_split_the_rules_choose_is_built():
-    """The rules for the work split never leave the set of builds that the test above covers."""
-    built = set(_backward_builds())
+    """The rules for the work split -- key blocks, threads, queries split over the waves, dS kept where the rule says so and not
+    where there is no room for it -- never leave the set of builds that the test above covers."""
+    built, chosen = set(_backward_builds()), set()
     for dtype in (torch.bfloat16, torch.float16):
         for D in (64, 128):
             for mask in (lowering.MASK_NONE, lowering.MASK_CAUSAL, lowering.MASK_SLIDING):
                 for cap in (False, True):
-                    for units in (1, 31, 100, 256, 4096):
+                    for units, group in ((1, 1), (1, 8), (31, 1), (50, 2), (100, 8), (256, 1), (4096, 4)):
                         for S in (1, 300, 1024, 2048, 8192):
-                            spec = lowering.bwd_spec(dtype, D, mask, cap, lowering.bwd_key_blocks(D, mask, cap, units, S),
-                                                     lowering.bwd_dq_threads(D, mask, cap, units, S, S))
-                            assert spec in built, spec
+                            q_split = lowering.bwd_q_split(D, mask, units, S)
+                            blocks = units * group * lowering.bwd_ds_blocks(mask, 256, S, S)
+                            for keep in {False, lowering.bwd_keep_ds(D, cap, units * group, group, S, blocks)}:
+                                spec = lowering.bwd_spec(dtype, D, mask, cap, 1 if q_split else lowering.bwd_key_blocks(D, mask, cap, units, S),
+                                                         lowering.bwd_dq_threads(D, mask, cap, units * group, S, S), keep, q_split)
+                                assert spec in built, spec
+                                chosen.add(spec)
+    assert {("-DLF_BW_DS=1" in s.extra, "-DLF_BW_QSPLIT=1" in s.extra) for s in chosen} == {(a, b) for a in (False, True) for b in (False, True)}
 
 
 def test_the_check_sees_an_unsettled_operand():
