@@ -591,7 +591,7 @@ def choose(M: int, N: int, K: int, batch: int) -> tuple:
     resident workgroups, plus, for a split product, the sum's launch and the traffic of its partials.  The model's constants
     are fitted to every candidate on 42 shapes (M 16 ... 8192, N 640 ... 16384, K 512 ... 16384, weights from HBM); there the
     choice is within 3 % of the best on 39, the others are 5 % (777 x 3000, K 5000), 10 % (6388 x 2880, K 1472, with gelu: m 98.9,
-    s 90.3 us) and 11 % off (100 x 1024, K 4096: n in 16 parts 12.8, in 8 11.5).  What it is for: a product whose tiles leave
+    s 90.3 us) and 7 % off (100 x 1024, K 4096: n in 13 parts 12.6, in 8 11.8).  What it is for: a product whose tiles leave
     most CUs idle, or alone with the latency of their loads.  M 256, us: N 4096 K 16384 218 (64 tiles s) -> 49 (d, 4 parts);
     N 16384 K 4096 66 -> 46 (d); M 64, N 4096 K 16384 214 -> 29 (n, 8 parts); M 1024, N 4096 K 16384 218 -> 130 (l, 4 parts);
     M 2000, N 1024 K 512 17 -> 11 (n).  n serves the fewest rows too: its tile pads least.  M up to 32, d or
