@@ -622,15 +622,14 @@ def choose(M: int, N: int, K: int, batch: int) -> tuple:
 def stream_b(M: int, N: int, K: int, own: int, shared: int) -> bool:
     """B by non-temporal loads (16-bit elements; ``own``, ``shared`` of ``b_batches``): they leave an L2 to A, and cost where several
     tiles read B at different times, or where it would have stayed in a cache.
-    Non-temporal over plain, weights from HBM, 204 drawn products of one matrix B and 72 chosen ones: up to 32 rows 0.98 in the mean
-    (100 MB and more 0.95); 33 ... 64 rows 0.99 below 18 MB, 1.01 up to 100 MB; 65 ... 256 rows 1.01 below 18 MB, 1.06 (up to 1.2) up to
-    100 MB, 1.01 up to 150, 0.97 beyond.  us, M x N x K, plain / non-temporal: 32 x 16384 x 4096 30.9 / 29.0, 64 x 1024 x 4096 11.3 / 10.6,
-    64 x 28672 x 8192 83.5 / 74.2, 128 x 4096 x 4096 16.2 / 18.4, 256 x 4096 x 4096 22.4 / 27.2, 256 x 2048 x 8192 22.3 / 26.1; linear -> gelu
-    -> linear of 256 rows, 2048 / 8192 wide 45.2 / 48.6, 4096 / 16384 103.7 / 99.0.  A B that is still in a cache from the call before: 256
-    x 4096 x 4096 21.6 / 27.2, 256 x 16384 x 4096 46.5 / 48.3.
+    Non-temporal over plain, 160 drawn steps linear -> gelu -> linear, weights of other layers in between: 17 ... 128 rows 1.00 ... 1.10 (mean 1.04)
+    below 50 MB, 0.98 from there to 100, 0.94 beyond; 129 ... 256 rows 1.06 below 50 MB, 1.03 up to 100, 0.97 beyond.  204 drawn single products:
+    up to 16 rows 0.98 (0.95 from 50 MB on); 17 ... 64 rows 1.00 below 100 MB, 0.95 beyond; 65 ... 256 rows 1.04 below 100 MB, 1.01 beyond.  us,
+    M x N x K, plain / non-temporal: 8 x 16384 x 4096 31.0 / 28.9, 64 x 28672 x 8192 83.5 / 74.2, 128 x 4096 x 4096 16.2 / 18.4, 256 x 4096 x 4096 22.4 /
+    27.2, 256 x 2048 x 8192 22.3 / 26.1; linear -> gelu -> linear of 256 rows, 2048 / 8192 wide 45.2 / 48.6, 4096 / 16384 103.7 / 99.0.  A B that is
+    still in a cache from the call before: 256 x 4096 x 4096 21.6 / 27.2, 256 x 16384 x 4096 46.5 / 48.3.
     Batches, B x M x N x K: shared weights 2 x 128 x 4096 x 4096 25.4 / 28.7, 4 x 16 x 16384 x 4096 76 / 87, 16 x 128 x 16384 x 4096 319 / 407;
     a B for each 64 x 64 x 512 x 512 11.4 / 10.7, 32 x 100 x 2048 x 2048 77 / 66, 16 x 256 x 1024 x 1024 19.1 / 19.2."""
     if shared > 1 or M > 256:
         return False
-    size = 2 * N * K
-    return own > 1 or M <= (64 if size < 16 << 20 else 32) or size >= 96 << 20
+    return own > 1 or M <= 16 or 2 * N * K >= (48 << 20 if M <= 128 else 96 << 20)

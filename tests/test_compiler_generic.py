@@ -342,8 +342,8 @@ def test_contractions_of_half_precision_operands_get_an_mfma_kernel():
 
 
 @pytest.mark.parametrize("a,b,expanded,batches,streams", [
-    ((32, 4096), (4096, 4096), False, (1, 1), True), ((33, 4096), (4096, 4096), False, (1, 1), False), ((256, 4096), (4096, 4096), False, (1, 1), False),
-    ((64, 1024), (1024, 4096), False, (1, 1), True), ((65, 1024), (1024, 4096), False, (1, 1), False),
+    ((16, 4096), (4096, 4096), False, (1, 1), True), ((17, 4096), (4096, 4096), False, (1, 1), False), ((256, 4096), (4096, 4096), False, (1, 1), False),
+    ((128, 4096), (4096, 6144), False, (1, 1), True), ((129, 4096), (4096, 6144), False, (1, 1), False), ((128, 4096), (4096, 6136), False, (1, 1), False),
     ((256, 4096), (4096, 16384), False, (1, 1), True), ((257, 4096), (4096, 16384), False, (1, 1), False),
     ((2, 16, 512), (512, 64), False, (1, 2), False), ((2, 3, 16, 512), (512, 64), False, (1, 6), False),       # shared by the batch
     ((16, 128, 512), (16, 512, 64), False, (16, 1), True), ((16, 128, 512), (16, 512, 64), True, (1, 16), False),
