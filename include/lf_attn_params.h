@@ -31,13 +31,15 @@ typedef struct LfAttnParamsHost {
   const void* v_table;
   float* part_acc;      /* decode split-K scratch: [units, nsplit, rows, D] floats; lf_attn_prefill_swp -DLF_BIAS=1 and
                            lf_bias_classify: int32 [units', kv tiles of 64] tile classes of the score bias (written by
-                           lf_bias_classify or lf_mask_tiles, launched first with the same block; units' = distinct
-                           (batch, head) of the bias x q tiles of the attention kernel) */
+                           lf_bias_classify, launched first with the same block; units' = distinct (batch, head) of the bias x
+                           q tiles of the attention kernel); -DLF_BIAS=2 and lf_mask_tiles: uint32 [units'', rows / 32,
+                           keys / 1024, 2] (both rounded up; units'' = distinct (batch, head) of the mask) */
   float* part_ml;       /* decode split-K scratch: [units, nsplit, rows, 2] floats; lf_attn_prefill_swp: optional
                            output [B, Hq, Sq] floats, the rows' log-sum-exp in log2 units (NULL: not written) */
   unsigned char* visits;/* optional [B*Hq*q_tiles, kv_tiles] visited-tile record, else NULL */
   const void* bias;     /* LF_BIAS & 1: additive score bias [B, Hq, Sq, Sk]; lf_attn_decode -DLF_BIAS=1: [B, Hkv, rows, Sk].
-                           lf_mask_tiles writes it (0 / -inf, mixed blocks only; rows of a multiple of 8 elements) */
+                           lf_attn_prefill_swp -DLF_BIAS=2: uint64 [units'', rows / 32, keys / 32, 16], written by
+                           lf_mask_tiles; of bias_sb / bias_sh / bias_sq only which are 0 counts */
   const void* obias;    /* LF_BIAS & 2: additive output bias [B, Hq, Sq, D]; lf_mask_tiles: the bytes of a boolean mask,
                            ob_sb / ob_sh / ob_sq their strides in bytes, key stride 1 */
   const void* q2;       /* LF_D2: second score product Q2 [B, Hq, Sq, D2] ... */

@@ -70,7 +70,12 @@
 #ifndef LF_BIAS
 #define LF_BIAS 0        /* 1: additive score bias [B, Hq, Sq, Sk] (a mask given as a tensor) with the tile classes
                             that lf_bias_classify wrote into p.part_acc: dead tiles at either end of a q tile's
-                            range are not walked, all-zero tiles cost nothing, the others add their values */
+                            range are not walked, all-zero tiles cost nothing, the others add their values;
+                            2: a boolean mask as lf_mask_tiles leaves it (lf_mask_bits.hip): classes per 32 rows x 32 keys in
+                            p.part_acc, so that a wave computes only what its own rows see, and in p.bias a 64-bit word per
+                            accumulator element of a mixed block, which is the lane select as it is: 32 scalar registers and
+                            no vector load in the loop, so that 32-key tiles fit three workgroups per CU as without a mask.
+                            B4 H32 S1536 D128, causal and padding: 99 -> 85 us against the 16-bit bias of form 1 */
 #endif
 #define LF_BARRIER_VM0() asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory")
 
@@ -274,7 +279,43 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
       if (lo > 0) kt_begin = lo / LF_BN;
     }
 #endif
-#if LF_BIAS
+#if LF_BIAS == 2
+    // The mask's words for this (batch, head): one per 32 rows and 1024 keys; broadcast dims of the mask collapse
+    constexpr int kRb = LF_BM / 32, kPer = LF_BN / 32;         // blocks of 32 rows per q tile, of 32 keys per tile
+    const int mnh = p.bias_sh ? p.Hq : 1;
+    const int nrb = p.bias_sq ? (p.Sq + 31) / 32 : 1, nwords = (p.Sk + 1023) / 1024;
+    const long long mrow = (long long)((p.bias_sb ? b : 0) * mnh + (p.bias_sh ? h : 0)) * nrb;
+    {
+      // the q tile's range shrinks to its first .. last tile of which something is seen (every wave for itself: lane =
+      // (word, block of rows), 64 / kRb words per step)
+      const lf_u32x2* words = reinterpret_cast<const lf_u32x2*>(p.part_acc);
+      const int rb = min(p.bias_sq ? q0 / 32 + lane % kRb : 0, nrb - 1);
+      int lo = kt_end, hi = kt_begin;
+      for (int c0 = kPer * kt_begin / 32; c0 < nwords; c0 += 64 / kRb) {
+        const int c = c0 + lane / kRb;
+        unsigned w = c < nwords ? words[(mrow + rb) * nwords + c][0] : 0u;
+#if LF_MASK >= 1
+        const int from = kPer * kt_begin - 32 * c, to = kPer * kt_end - 32 * c;
+        if (from > 0) w = from < 32 ? w & (~0u << from) : 0u;
+        if (to < 32) w = to > 0 ? w & ((1u << to) - 1u) : 0u;
+#endif
+        const unsigned long long live = __builtin_amdgcn_ballot_w64(w != 0u);
+        if (live != 0ull) {
+          const int first = (int)__builtin_ctzll(live) / kRb, last = (63 - (int)__builtin_clzll(live)) / kRb;
+          unsigned wf = 0u, wl = 0u;
+#pragma unroll
+          for (int r = 0; r < kRb; ++r) {
+            wf |= __builtin_amdgcn_readlane(w, first * kRb + r);
+            wl |= __builtin_amdgcn_readlane(w, last * kRb + r);
+          }
+          lo = min(lo, (32 * (c0 + first) + (int)__builtin_ctz(wf)) / kPer);
+          hi = (32 * (c0 + last) + 31 - (int)__builtin_clz(wl)) / kPer + 1;
+        }
+      }
+      kt_begin = __builtin_amdgcn_readfirstlane(min(lo, kt_end));
+      kt_end = __builtin_amdgcn_readfirstlane(max(hi, kt_begin));
+    }
+#elif LF_BIAS
     // tile classes of the bias for this (batch, head, q tile): broadcast dims of the bias collapse
     const int nhh = p.bias_sh ? p.Hq : 1;
     const int cunit = ((p.bias_sb ? b : 0) * nhh + (p.bias_sh ? h : 0)) * nqt + qt;
@@ -363,8 +404,65 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
 #pragma unroll
     for (int f = 0; f < LF_KPF; ++f) kpre[f] = k_frag(k_row_addr(0, 0) + kb_off0, f);
 
+#if LF_BIAS == 2
+    // this wave's 32 rows: {seen, hidden} of the 1024 keys around the tile, and the selects of its blocks
+    const long long mblock = mrow + (p.bias_sq ? min(wq0 / 32, nrb - 1) : 0);
+    const lf_cu32* mwords = reinterpret_cast<const lf_cu32*>(reinterpret_cast<unsigned long long>(p.part_acc)) + 2 * mblock * nwords;
+    const lf_cu64* mbits = reinterpret_cast<const lf_cu64*>(reinterpret_cast<unsigned long long>(p.bias)) +
+                           16 * mblock * ((p.Sk + 31) / 32);
+    const int mfirst = min(kPer * kt_begin / 32, nwords - 1);
+    unsigned mseen = mwords[2 * mfirst], mhidden = mwords[2 * mfirst + 1];
+#endif
     int ks_cur = 0;   // K slot of tile kt
+#if LF_BIAS == 2
+    auto mask_next = [&](int kt) {       // behind tile kt
+      const int t = kPer * (kt + 1);
+      if (t % 32 == 0) {
+        const int next = min(t / 32, nwords - 1);
+        mseen = mwords[2 * next];
+        mhidden = mwords[2 * next + 1];
+      }
+    };
+    constexpr unsigned kBlocks = (1u << kPer) - 1u;
+    auto mask_need = [&](int kt) {
+      bool n = wave_has_rows && (mseen >> (kPer * kt % 32) & kBlocks) != 0u;
+#if LF_MASK >= 1
+      n = n && kt * LF_BN <= wqlast;
+#endif
+#if LF_MASK == 2
+      n = n && min(kt * LF_BN + LF_BN, p.Sk) - 1 >= wq0 - p.window + 1;
+#endif
+      return n;
+    };
+    auto stage_only = [&](int kt) {
+      const int ks_nxt = (ks_cur == LF_KSLOTS - 1) ? 0 : ks_cur + 1, ks_ld = (ks_nxt == LF_KSLOTS - 1) ? 0 : ks_nxt + 1;
+      lf_u32x4 k_cur = k_rsq, v_cur = v_rsq;
+      if (kt + 2 >= kt_end) k_cur[2] = 0u;
+      if (kt + 1 >= kt_end) v_cur[2] = 0u;
+#pragma unroll
+      for (int ps = 0; ps < LF_NPASS; ++ps) {
+        dma_k_pass(k_cur, kt + 2, ks_ld, ps, kpg[ps]);
+        dma_v_pass(v_cur, kt + 1, (kt - kt_begin + 1) & 1, ps, vpg[ps]);
+        kpg[ps] = kPagedK ? page_off(0, kt + 3, ps) : 0u;
+        vpg[ps] = kPagedV ? page_off(1, kt + 2, ps) : 0u;
+      }
+#pragma unroll
+      for (int f = 0; f < LF_KPF; ++f) kpre[f] = k_frag(k_row_addr(ks_nxt, 0) + kb_off0, f);
+      mask_next(kt);
+      LF_BARRIER_VM0();
+      ks_cur = ks_nxt;
+    };
+#endif
     for (int kt = kt_begin; kt < kt_end; ++kt) {
+#if LF_BIAS == 2
+      // Tiles of which this wave's rows see nothing are staged, not computed: in a loop of their own, because with a branch
+      // around the products the compiler keeps O^T twice and copies it every tile (47 registers spilled at three waves per SIMD)
+      while (!mask_need(kt)) {
+        stage_only(kt);
+        if (++kt == kt_end) break;
+      }
+      if (kt == kt_end) break;
+#endif
       const int rel = kt - kt_begin;
       const int ks_nxt = (ks_cur == LF_KSLOTS - 1) ? 0 : ks_cur + 1;   // slot of K(kt+1)
       const int ks_ld = (ks_nxt == LF_KSLOTS - 1) ? 0 : ks_nxt + 1;    // slot K(kt+2) is loaded into
@@ -402,7 +500,11 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
       full = full && (wq0 + 31 - k0 < p.window);
 #endif
 
-#if LF_BIAS
+#if LF_BIAS == 2
+      const int mt = kPer * kt;                                  // the tile's (first) block of 32 keys
+      need = true;
+      const unsigned biased = mhidden >> (mt % 32) & kBlocks;
+#elif LF_BIAS
       // class 2: the tile's bias values are requested before the S^T products.  Element i of block kb is
       // key j = k0 + 32*kb + 8*(i/4) + 4*g + i%4 of row my_q: four consecutive keys per 8-byte load
       // class 0 inside the range (a dead tile between live ones): staged like any tile, not computed
@@ -501,7 +603,17 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
 #pragma unroll
           for (int i = 0; i < 16; ++i) s[kb][i] = __builtin_amdgcn_rcpf(-1.0f - lf_exp2(s[kb][i] * sc_exp));   // -r
 #endif
-#if LF_BIAS
+#if LF_BIAS == 2
+        // hidden elements: -inf (a sum, as a score bias of -inf gives it: a NaN stays one)
+#pragma unroll
+        for (int kb = 0; kb < LF_NKB; ++kb)
+          if (biased >> kb & 1u) {
+            __builtin_amdgcn_sched_barrier(0);       // one block's 16 words at a time: 32 scalar registers
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              s[kb][i] += lf_lane_bit(mbits[16 * (mt + kb) + i]) ? 0.0f : LF_NEG_INF;
+          }
+#elif LF_BIAS
         if (biased) {
           // x = scale * s + bias: the scores stay in units of 1 / scale, so the bias is divided by it; capped
           // scores are held as -r with c * tanh = c - 2 c r: there the unit is 2 c
@@ -629,6 +741,9 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
 #pragma unroll
         for (int f = 0; f < LF_KPF; ++f) kpre[f] = k_frag(knext, f);
       }
+#if LF_BIAS == 2
+      mask_next(kt);
+#endif
       LF_BARRIER_VM0();
       ks_cur = ks_nxt;
 #pragma unroll

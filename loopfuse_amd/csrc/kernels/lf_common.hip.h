@@ -69,6 +69,8 @@ typedef float lf_f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int lf_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int lf_u32x2 __attribute__((ext_vector_type(2)));
 typedef const int __attribute__((address_space(4))) lf_cint;   /* read-only table entries fetched with scalar loads */
+typedef const unsigned __attribute__((address_space(4))) lf_cu32;
+typedef const unsigned long long __attribute__((address_space(4))) lf_cu64;
 
 #if LF_TABLE_I64
 typedef long long lf_table_t;
@@ -133,12 +135,12 @@ struct LfAttnParams {
   lf_elem* o;
   const void* k_table;       // [B, pages_per_seq] page ids (lf_table_t) when paged
   const void* v_table;
-  float* part_acc;           // split-K scratch: [units, nsplit, rows, D]; prefill_swp with LF_BIAS: the bias tile classes (int32)
+  float* part_acc;           // split-K scratch: [units, nsplit, rows, D]; prefill_swp with LF_BIAS: the tile classes
   float* part_ml;            // split-K scratch: [units, nsplit, rows, 2] (max, sum); lf_attn_prefill_swp: optional
                              // output [B, Hq, Sq], the rows' log-sum-exp in log2 units (null: not written)
   unsigned char* visits;     // optional [B*Hq*nqt, nkt] visited-tile record
   const lf_elem* bias;       // LF_BIAS & 1: additive score bias [B, Hq, Sq, Sk] (key stride 1),
-                             // added after scale / softcap and before the mask
+                             // added after scale / softcap and before the mask; prefill_swp with LF_BIAS 2: a mask's bits
   const lf_elem* obias;      // LF_BIAS & 2: additive output bias [B, Hq, Sq, D] (d stride 1)
   const lf_elem* q2;         // LF_D2: second score product, scores = Q K^T + Q2 K2^T (the two-part
   const lf_elem* k2;         // scores of reference tests/test_attention.py:126-151); dense, depth LF_D2
@@ -210,6 +212,10 @@ __device__ __forceinline__ float lf_max_halves(float x) {
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
   return fmaxf(a, b);
 }
+
+// This lane's bit of a wave-uniform word, as a condition (the word itself is the select's operand).  The intrinsic by its
+// name: hipRTC's compiler knows no builtin for it yet.
+extern "C" __device__ bool lf_lane_bit(unsigned long long word) __asm("llvm.amdgcn.inverse.ballot.i64");
 
 __device__ __forceinline__ float lf_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 

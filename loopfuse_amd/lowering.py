@@ -30,6 +30,7 @@ from . import runtime
 from .skip import TILE_SHAPES
 
 MASK_NONE, MASK_CAUSAL, MASK_SLIDING = 0, 1, 2
+MASK_BITS = 8        # KernelSpec.bias of a call whose boolean mask the kernel reads as bits (lf_mask_bits.hip)
 DECODE_QROWS = 16    # query rows one decode unit holds (the MFMA N dimension)
 _MASK_NAMES = {"none": MASK_NONE, None: MASK_NONE, "causal": MASK_CAUSAL, "sliding": MASK_SLIDING}
 _DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1}
@@ -87,7 +88,8 @@ class KernelSpec:
     coop: bool = False     # decode, headwave: the workgroup loads whole 16-token blocks, rows reach the waves through LDS
     rowload: bool = False  # decode, register-staged path: whole-row non-temporal loads, K through a wave-private LDS tile
     denom: bool = False    # prefill: softmax denominator sum + c (c a run-time parameter)
-    bias: int = 0          # prefill: bit 0 additive score bias tensor, bit 1 additive output bias tensor, bit 2 unaligned rows
+    bias: int = 0          # prefill: bit 0 additive score bias tensor, bit 1 additive output bias tensor, bit 2 unaligned rows;
+                           # prefill_swp: MASK_BITS a boolean mask as bits instead
     pack: int = 0          # prefill_swp, grouped-query attention: a workgroup's waves take 2 or 4 heads of one group
     page_size_v: int = 0   # tokens per page of the V pool when it differs from K's (0 = same)
     d2: int = 0            # prefill: depth of a second score product Q2 K2^T (0, 16, 32, 64)
@@ -136,7 +138,7 @@ class KernelSpec:
             if self.pack:
                 o += [f"-DLF_GQAPACK={int(self.pack)}"]
             if self.bias:
-                o += ["-DLF_BIAS=1"]
+                o += ["-DLF_BIAS=2" if self.bias == MASK_BITS else "-DLF_BIAS=1"]
         if self.safe:
             o += ["-DLF_SAFE=1"]
         return o + list(self.extra)
@@ -148,8 +150,9 @@ class KernelSpec:
             return ("lf_common.hip.h", kernel)
         # the two prefill kernels: their own tuning macros come first (the shared blocks use LF_BN)
         if self.family == "prefill_swp" and self.bias:
-            # one code object holds the attention kernel and the kernel that classifies the bias tiles for it
-            return ("lf_common.hip.h", "lf_prefill_blocks.hip.h", kernel, "lf_bias_classify.hip")
+            # one code object holds the attention kernel and the kernel that reads the mask or the bias ahead of it
+            return ("lf_common.hip.h", "lf_prefill_blocks.hip.h", kernel,
+                    "lf_mask_bits.hip" if self.bias == MASK_BITS else "lf_bias_classify.hip")
         return ("lf_common.hip.h", "lf_prefill_blocks.hip.h", kernel)
 
     def entry(self) -> str:
@@ -578,9 +581,12 @@ def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, w
     workgroups of 6211 keys; one 6001-token prompt, 1504 workgroups, 328 against 312 us); from 2048 workgroups on 0.95
     (0.79 ... 1.05); 500 ... 767 either way (0.72 ... 1.15).  At head
     dimension 64 it does not pay.  The bias tile
-    classes are per 64 keys, so biased calls keep 64.  ``choice["bn"]`` (the tuner) or
+    classes of a score bias are per 64 keys, so biased calls keep 64.  A boolean mask has classes per 32 keys and follows the rule
+    without one: times with 32 over 64, 90 launches of causal, padding, window and random masks, 768 ... 2047 workgroups of up to
+    2047 keys 0.94 (0.83 ... 1.04), of more 1.03 (0.97 ... 1.07), from 2048 workgroups on 0.95 (0.87 ... 1.01), 400 ... 767 1.01 (0.84 ...
+    1.19); beside a softcap, whose scores such a kernel holds in another form, it keeps 64 too (B4 H32 S1536 104 / 111 us).  ``choice["bn"]`` (the tuner) or
     ``LOOPFUSE_BN`` override the default."""
-    if bias_bits:
+    if bias_bits & 7:
         return 0
     want = (choice or {}).get("bn", _env("LOOPFUSE_BN"))
     if want is not None:
@@ -1033,7 +1039,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         P.bias = score_bias.data_ptr()
         P.bias_sb, P.bias_sh, P.bias_sq = score_bias.stride(0), score_bias.stride(1), score_bias.stride(2)
         bias_bits |= 1
-    mask_own = None        # the mask without the dims it is shared over, while its bias buffer is not written yet
+    mask_own = None        # the mask without the dims it is shared over, while nothing of it is written yet
     if score_mask is not None:
         if score_bias is not None:
             raise UnsupportedPlan("a score mask and a score bias")
@@ -1044,18 +1050,19 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
         except RuntimeError:
             raise UnsupportedPlan(f"score mask does not broadcast to [{B}, {Hq}, {Sq}, {Sk}]")
         mask_own = score_mask[tuple(slice(0, 1) if st == 0 else slice(None) for st in score_mask.stride()[:3])]
-        mask_buf = torch.empty((*mask_own.shape[:3], (Sk + 7) // 8 * 8), dtype=dtype, device=q.device)[..., :Sk]
-        score_bias = mask_buf.expand(B, Hq, Sq, Sk)
-        P.bias = mask_buf.data_ptr()
-        P.bias_sb, P.bias_sh, P.bias_sq = score_bias.stride(0), score_bias.stride(1), score_bias.stride(2)
+        P.bias_sb, P.bias_sh, P.bias_sq = (int(st != 0) for st in score_mask.stride()[:3])      # what it is shared over; strides below
         bias_bits |= 1
 
     def write_mask_bias():
         """The whole bias of a boolean mask, for the kernels that read every element of it."""
-        nonlocal mask_own
+        nonlocal mask_own, score_bias
         if mask_own is not None:
             shown, hidden = 0.0, float("-inf")
+            mask_buf = torch.empty((*mask_own.shape[:3], (Sk + 7) // 8 * 8), dtype=dtype, device=q.device)[..., :Sk]
             mask_buf.fill_(hidden if mask_keep else shown).masked_fill_(mask_own, shown if mask_keep else hidden)
+            score_bias = mask_buf.expand(B, Hq, Sq, Sk)
+            P.bias = mask_buf.data_ptr()
+            P.bias_sb, P.bias_sh, P.bias_sq = score_bias.stride(0), score_bias.stride(1), score_bias.stride(2)
             mask_own = None
 
     if out_bias is not None:
@@ -1144,11 +1151,14 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             family = "prefill"                          # swp was refused above (spans): the register-staged kernel
         if family != "prefill_swp" or (mask_own is not None and mask_own.stride(3) != 1):
             write_mask_bias()
+            keep += (score_bias,)
+        if mask_own is not None:
+            bias_bits = MASK_BITS
         spec = _spec(family, _DTYPE_CODE[dtype], D, mask, plan.softcap is not None, paged,
                      page_size, table_i64, v_tr=v_tr if family == "prefill" else True, bias=bias_bits,
                      denom=plan.denom_add != 0.0, d2=d2, page_size_v=page_size_v, pack=pack, extra=extra,
-                     safe=plan.zero_blind_rows and bool(bias_bits & 1),
-                     bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
+                     safe=plan.zero_blind_rows and bool(bias_bits & (1 | MASK_BITS)),
+                     bn=prefill_kv_tile(D, bias_bits | int(bias_bits == MASK_BITS and plan.softcap is not None), choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
                                         min(Sk, P.window) if mask == MASK_SLIDING else Sk)
                      if family == "prefill_swp" else 0)
         bm, bn = TILE_SHAPES[family]
@@ -1178,18 +1188,23 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
             P.part_ml = lse.data_ptr()
         names = [spec.entry()]
         if family == "prefill_swp" and bias_bits:
-            # tile classes of the bias, once per distinct (batch, head) it holds: int32 [units][kv tiles]
             nb_, nh_ = (B if P.bias_sb else 1), (Hq if P.bias_sh else 1)
-            table = torch.empty((nb_ * nh_ * nqt * nkt,), dtype=torch.int32, device=q.device)
-            keep += (table,)
-            P.part_acc = table.data_ptr()
-            classify = "lf_bias_classify"
             if mask_own is not None:
-                # classes straight from the mask's bytes, the bias only where the attention kernel reads it
-                classify = "lf_mask_tiles"
+                # the mask's bits and the words of its 32 x 32 blocks, once per distinct (batch, head) it holds
+                classify, nrb, chunks = "lf_mask_tiles", (-(-Sq // 32) if P.bias_sq else 1), -(-Sk // 1024)
+                words = nb_ * nh_ * nrb * chunks
+                table = torch.empty((words + nb_ * nh_ * nrb * -(-Sk // 32) * 16,), dtype=torch.int64, device=q.device)
+                P.part_acc, P.bias = table.data_ptr(), table.data_ptr() + 8 * words
                 P.obias, P.rows = mask_own.data_ptr(), int(mask_keep)
                 P.ob_sb, P.ob_sh, P.ob_sq = (st if n > 1 else 0 for n, st in zip(mask_own.shape, mask_own.stride()[:3]))
-            get_kernel(spec, classify).launch((nqt, nb_ * nh_, (nkt + 3) // 4), (256, 1, 1), P)
+                ahead = (nrb, nb_ * nh_, chunks)
+            else:
+                # tile classes of the bias, once per distinct (batch, head) it holds: int32 [units][kv tiles]
+                classify, ahead = "lf_bias_classify", (nqt, nb_ * nh_, (nkt + 3) // 4)
+                table = torch.empty((nb_ * nh_ * nqt * nkt,), dtype=torch.int32, device=q.device)
+                P.part_acc = table.data_ptr()
+            keep += (table,)
+            get_kernel(spec, classify).launch(ahead, (256, 1, 1), P)
             names.insert(0, classify)
         fn = get_kernel(spec, spec.entry())
         record = {"kernels": names, "grid": grid, "block": 64 * nw, "q_tile_rows": bm, "kv_tile_rows": bn,

@@ -1165,6 +1165,42 @@ def test_boolean_masks_equal_the_bias_they_stand_for(Sq, Sk, mshape, group, keep
     assert torch.equal(walked, want_walked) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("Sq,Sk,group,flag,dt", [
+    (130, 1024, 1, None, 0),       # one word of 32 blocks, exactly
+    (130, 1025, 1, None, 1),       # ... and one key: byte loads, a second word of a single key
+    (300, 2112, 4, None, 0),       # three words, packed heads
+    (300, 2111, 2, "causal", 0),   # the flag clips the words
+    (515, 1600, 1, "sliding", 1),
+    (33, 4, 1, None, 0),
+])
+def test_mask_bits_with_both_key_tiles(Sq, Sk, group, flag, dt):
+    """Words and selects of lf_mask_tiles under 32- and 64-key tiles at head dim 128: 64 keys give the bits that the 0 / -inf bias
+    gives, 32 keys the oracle's values (TOL, as for the flag kernels)."""
+    g = torch.Generator().manual_seed(Sq * Sk)
+    B, H, D, dtype = 2, 4, 128, (torch.bfloat16, torch.float16)[dt]
+    q, k, v = (rand((B, h, n, D), dtype, s) for h, n, s in ((H, Sq, 1), (H // group, Sk, 2), (H // group, Sk, 3)))
+    i, j = torch.arange(Sq)[:, None], torch.arange(Sk)[None, :]
+    shown = (j <= i + Sk // 2).expand(B, 1, Sq, Sk).clone()
+    shown[0, :, :, Sk // 3:Sk // 3 + 40] &= torch.rand((1, Sq, 1), generator=g) < 0.5       # mixed blocks
+    shown[1, :, :, Sk // 4:Sk // 2] = False                                                 # dead ones between live ones
+    shown[1, :, 32:64] = shown[1, :, 32:64] & (torch.rand((1, 1, Sk), generator=g) < 0.1)
+    shown[..., 0] = True
+    plan = lowering.AttnPlan(mask=flag, window=700 if flag == "sliding" else 0, scale=D ** -0.5)
+    bias = torch.zeros(shown.shape).masked_fill(~shown, float("-inf")).to(dtype)
+    on = [t.to(dev()) for t in (q, k, v)]
+    want = O.attention_reference(q, k, v, mask=flag, window=plan.window, score_bias=bias.float())
+    blind = torch.isnan(want).any(-1)
+    same = lowering.attention(*on, plan, score_bias=bias.to(dev()))
+    for bn in (64, 32):
+        got, walked = lowering.attention(*on, plan, score_mask=shown.to(dev()), choice={"bn": bn}, record_visits=True)
+        assert lowering.attention.last_launch["kernels"] == ["lf_mask_tiles", "lf_attn_prefill_swp"]
+        assert lowering.attention.last_launch["kv_tile_rows"] == bn and walked.shape[1] == -(-Sk // bn)
+        if bn == 64:
+            assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(same))
+        got = got.float().cpu()
+        assert torch.isnan(got[blind]).all() and (got[~blind] - want[~blind]).abs().max().item() <= TOL[dtype]
+
+
 @pytest.mark.parametrize("case", ["decode", "key_stride", "register_staged"])
 def test_boolean_masks_where_the_whole_bias_is_read(case, monkeypatch):
     B, H, Sq, Sk, D = 2, 3, 1 if case == "decode" else 130, 700, 64
