@@ -728,6 +728,7 @@ _MAX_KEPT = 512
 _NO_ROOM_CALLS = 1000      # calls of a backward that found no room for dS until it looks for it again
 _kept: dict = {}
 _PLAIN = (int, float, str, bool, type(None))
+_PLAIN_TYPES = frozenset(_PLAIN)
 
 
 
@@ -739,19 +740,18 @@ def _signature(kind: str, tensors, plan: AttnPlan, options: Optional[dict]):
     for t in tensors:
         if t is None:
             operands.append(None)
+        elif not t.is_cuda or t.data_ptr() % 16:
+            return None
         else:
-            if not t.is_cuda or t.data_ptr() % 16:
-                return None
             operands.append((t.shape, t.stride(), t.dtype, t.get_device()))
     fields = (plan.mask, plan.window, plan.scale, plan.softcap, plan.k_paged, plan.v_paged, plan.denom_add, plan.zero_blind_rows)
     choice = tuple(options.items()) if options else ()
-    for x in fields:
-        if not isinstance(x, _PLAIN):
-            return None
+    if not _PLAIN_TYPES.issuperset(map(type, fields)) and not all(isinstance(x, _PLAIN) for x in fields):
+        return None
     for _, x in choice:
         if not isinstance(x, _PLAIN):
             return None
-    return (kind, fields, choice, torch.cuda.current_device(), tuple(map(_VARIABLES.get, _SWITCHES)), tuple(operands))
+    return (kind, fields, choice, runtime.current_device(), tuple(map(_VARIABLES.get, _SWITCHES)), tuple(operands))
 
 
 class _Kept:
@@ -783,7 +783,7 @@ class _Kept:
         else:
             P.part_ml = None if lse is None else lse.data_ptr()
             self.launches.launch(P)
-        _last_launch.set(dict(self.record))
+        _last_launch.set(self.record)
         return out
 
 
@@ -824,7 +824,7 @@ def _on_device_of_first_argument(fn):
     device: make the device of Q current for the duration of the call when it is not."""
     @functools.wraps(fn)
     def guarded(q, *args, **kw):
-        if isinstance(q, torch.Tensor) and q.is_cuda and q.device.index != torch.cuda.current_device():
+        if isinstance(q, torch.Tensor) and q.is_cuda and q.get_device() != runtime.current_device():
             with torch.cuda.device(q.device):
                 return fn(q, *args, **kw)
         return fn(q, *args, **kw)
@@ -1439,7 +1439,9 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     or 256 query rows, from dS left in a scratch tensor where ``bwd_keep_ds`` says so (``keep_ds`` overrides it).  No
     atomics: results are reproducible bit for bit.  ``key_blocks``, ``dq_threads`` and ``q_split`` override the rules of the work
     splits (``bwd_key_blocks``, ``bwd_dq_threads``, ``bwd_q_split``)."""
-    key = _signature("bwd", (q, k, v, o, lse, dout), plan, {"key_blocks": key_blocks, "dq_threads": dq_threads, "keep_ds": keep_ds, "q_split": q_split})
+    given = key_blocks is not None or dq_threads is not None or keep_ds is not None or q_split is not None
+    key = _signature("bwd", (q, k, v, o, lse, dout), plan,
+                     {"key_blocks": key_blocks, "dq_threads": dq_threads, "keep_ds": keep_ds, "q_split": q_split} if given else None)
     kept = _kept.get(key)
     if kept is not None and kept.calls is not None:
         kept.calls -= 1
@@ -1567,5 +1569,5 @@ def _backward_again(kept: _Kept, q, k, v, o, lse, dout):
     P.q, P.k, P.v, P.o, P.dout = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr()
     P.dq, P.dk, P.dv, P.lse, P.delta = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), lse.data_ptr(), delta.data_ptr()
     kept.launches.launch(P)
-    _last_launch.set(dict(kept.record))
+    _last_launch.set(kept.record)
     return dq, dk, dv

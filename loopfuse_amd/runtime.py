@@ -167,11 +167,19 @@ def private_segment_bytes(code: bytes) -> dict:
     return out
 
 
+def current_device() -> int:
+    """Index of torch's current device: the raw accessor, a third of the time, once torch has set the GPU up."""
+    return _get_device() if torch.cuda.is_initialized() else torch.cuda.current_device()
+
+
+_get_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def current_stream_handle() -> int:
     """hipStream_t of torch's current stream on the current device, as an integer
     (the raw accessor: the launch path is called once per kernel)."""
     try:
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        return torch._C._cuda_getCurrentRawStream(current_device())
     except AttributeError:            # older / newer torch without the raw accessor
         return torch.cuda.current_stream().cuda_stream
 

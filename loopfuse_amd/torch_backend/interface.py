@@ -183,8 +183,41 @@ def loopfuse_backend(gm: torch.fx.GraphModule, sample_inputs, mode="max-autotune
                         "is not one the backward kernels serve, so this graph runs unfused.  Wrap inference in "
                         "torch.no_grad().")
         return aot_module_simplified(gm, sample_inputs, fw_compiler=_unfused_compiler)
-    compiler = partial(loopfuse_compiler, input_names=get_input_names(gm), **kwargs)
-    return aot_module_simplified(gm, sample_inputs, fw_compiler=compiler)
+    found: list = []
+    compiler = partial(loopfuse_compiler, input_names=get_input_names(gm), alone=found, **kwargs)
+    general = aot_module_simplified(gm, sample_inputs, fw_compiler=compiler)
+    return _one_attention(gm, found, general)
+
+
+def _one_attention(gm: torch.fx.GraphModule, found: list, general: Callable) -> Callable:
+    """``general``, AOTAutograd's callable for an inference graph, with a shorter way for calls over plain tensors where the graph
+    is nothing but one attention over its inputs (``found``, from ``loopfuse_compiler``): the fused call itself, without
+    the wrappers that find out on every call what this graph does not have (aliases, mutations, subclasses).  B2 H8 S512
+    D64: 34.5 -> 28.6 us a call.  Calls with anything else than plain tensors, and graphs of which a call was refused, go
+    through ``general``."""
+    from . import training
+
+    if len(found) != 1 or any(True for _ in gm.parameters()) or any(True for _ in gm.buffers()):
+        return general
+    match, at, count, refused, refuse = found[0]
+    if count != len(get_input_names(gm)):
+        return general
+
+    def call(*args):
+        if refused or len(args) != count:
+            return general(*args)
+        vals = [args[i] for i in at]
+        if not training._plain([x for x in vals if isinstance(x, torch.Tensor)]):
+            return general(*args)
+        try:
+            out = match.run(vals)
+        except lowering.UnsupportedPlan as e:
+            return refuse(args, e)
+        stats["fused"] += 1
+        return (out,)
+
+    call.__dict__.update(general.__dict__)
+    return call
 
 
 _warned_training = False
@@ -237,7 +270,9 @@ def _training_graph(gm: torch.fx.GraphModule, sample_inputs):
         for m in matches:
             print(m.describe())
         print(rewritten.code)
-    return aot_module_simplified(rewritten, sample_inputs, fw_compiler=_training_compiler, bw_compiler=_training_compiler)
+    training.stats = stats
+    general = aot_module_simplified(rewritten, sample_inputs, fw_compiler=_training_compiler, bw_compiler=_training_compiler)
+    return training.one_attention(rewritten, sample_inputs, general)
 
 
 def _training_compiler(gm: torch.fx.GraphModule, sample_inputs) -> Callable:
@@ -390,8 +425,10 @@ def _generic_program(gm: torch.fx.GraphModule, tune: bool = False):
 
 
 def loopfuse_compiler(gm: torch.fx.GraphModule, sample_inputs, input_names: list[str] | None = None,
-                      symint_names: dict[str, str] | None = None, mode: str | None = None) -> Callable:
-    """fw_compiler: ATen graph -> callable over the flat placeholder list."""
+                      symint_names: dict[str, str] | None = None, mode: str | None = None, alone: list | None = None) -> Callable:
+    """fw_compiler: ATen graph -> callable over the flat placeholder list.  ``alone`` receives, of a graph that is nothing but one
+    attention over its inputs, its match, the positions of its inputs, the number of placeholders, the signatures refused
+    so far and what runs a call that the kernels refuse."""
     global _codegen_sink
     stats["compiled_graphs"] += 1
     if DEBUG:
@@ -509,6 +546,25 @@ def loopfuse_compiler(gm: torch.fx.GraphModule, sample_inputs, input_names: list
         stats["eager_runtime"] += 1
         return gm(*args)
 
+    def refuse(args, why):
+        if _strict():
+            raise why
+        if len(refused) >= 64:      # bounded: forget old refusals rather than grow
+            refused.clear()
+        refused.add(signature(args))
+        stats["refused_signatures"] += 1
+        log.warning("fused path not applicable to this call (%s); calls with these argument layouts run "
+                    "the graph unfused", why)
+        return run_unfused(args)
+
+    if alone is not None and len(matches) == 1:
+        nodes = list(fused_gm.graph.nodes)
+        calls = [n for n in nodes if n.op == "call_function"]
+        placeholders = [n for n in nodes if n.op == "placeholder"]
+        out = next(n for n in nodes if n.op == "output").args[0]
+        if len(calls) == 1 and isinstance(out, (tuple, list)) and list(out) == calls and all(n in placeholders for n in calls[0].args[1:]):
+            alone.append((matches[0], [placeholders.index(n) for n in calls[0].args[1:]], len(placeholders), refused, refuse))
+
     def optimized_fn(*args):
         sig = signature(args) if refused else None
         if sig is not None and sig in refused:
@@ -516,15 +572,7 @@ def loopfuse_compiler(gm: torch.fx.GraphModule, sample_inputs, input_names: list
         try:
             out = fused_gm(*args)
         except lowering.UnsupportedPlan as e:
-            if _strict():
-                raise
-            if len(refused) >= 64:      # bounded: forget old refusals rather than grow
-                refused.clear()
-            refused.add(signature(args))
-            stats["refused_signatures"] += 1
-            log.warning("fused path not applicable to this call (%s); calls with these argument layouts run "
-                        "the graph unfused", e)
-            return run_unfused(args)
+            return refuse(args, e)
         stats["fused"] += 1
         return out
 

@@ -1,0 +1,104 @@
+"""Graphs that are one attention over their inputs: calls over plain tensors go past AOTAutograd's wrappers
+(``training.one_attention``, ``interface._one_attention``), with their results and what they refuse."""
+import functools
+
+import pytest
+import torch
+
+from loopfuse_amd import loopfuse_backend
+from loopfuse_amd.torch_backend import capture, interface, training
+
+
+def _graph(second_output=False, extra=False, twice=False, perm=(0, 1, 2, 3)):
+    graph = torch.fx.Graph()
+    ins = [graph.placeholder(n) for n in "qkv"]
+    attr = graph.get_attr("_m")
+    out = graph.call_function(training.fused_call_train, (attr, *((ins[0], ins[0], ins[2]) if twice else ins)))
+    if extra:
+        out = graph.call_function(torch.neg, (out,))
+    graph.output((out, ins[0]) if second_output else (out,))
+    ops = [capture.Operand(i, perm) for i in range(3)]
+    root = torch.nn.Module()
+    root._m = capture.AttentionMatch(out_node=None, inputs=ins, q=ops[0], k=ops[1], v=ops[2], factors=[0.125], post_factors=[],
+                                     has_tanh=False, mask="causal", window=0, out_rank=4)
+    return torch.fx.GraphModule(root, graph)
+
+
+def test_only_graphs_of_one_attention_take_the_short_way():
+    def general(*args):
+        return "general"
+
+    x = [torch.zeros(1, 2, 8, 64, dtype=torch.bfloat16) for _ in range(3)]
+    assert training.one_attention(_graph(), x, general) is not general
+    for other in (_graph(second_output=True), _graph(extra=True), _graph(twice=True), _graph(perm=(0, 2, 1, 3))):
+        assert training.one_attention(other, x, general) is general
+    assert training.one_attention(_graph(), [x[0], x[1], 7], general) is general
+    assert training.one_attention(_graph(), [x[0][0], x[1][0], x[2][0]], general) is general
+    # what is not plain is sent on, call by call
+    call = training.one_attention(_graph(), x, general)
+    assert call(*x) == "general"                     # the first one
+    assert call(x[0], x[1], torch._neg_view(x[2])) == "general" and call(x[0], x[1]) == "general"
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert call(x[0].as_subclass(Sub), x[1], x[2]) == "general"
+
+
+def _attn(q, k, v):
+    s = torch.ops.loopfuse.causal_mask(q @ k.transpose(-2, -1) * (q.shape[-1] ** -0.5))
+    return torch.softmax(s, dim=-1) @ v
+
+
+def _compiled():
+    torch._dynamo.reset()
+    return torch.compile(_attn, backend=functools.partial(loopfuse_backend, mode=None), dynamic=False)
+
+
+def _tensors(S=130):
+    g = torch.Generator(device="cuda").manual_seed(S)
+    return [torch.empty((2, 4, S, 64), dtype=torch.bfloat16, device="cuda").normal_(generator=g) for _ in range(4)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dout", ["dense", "strided", "expanded"])
+def test_the_short_way_gives_the_bits_of_the_general_one(dout, monkeypatch):
+    *x, d = _tensors()
+    x = [t.requires_grad_() for t in x]
+    d = {"dense": d, "strided": d.transpose(1, 2).contiguous().transpose(1, 2), "expanded": d[..., :1].expand_as(d)}[dout]
+
+    def step(fn):
+        out = fn(*x)
+        return (out.detach(), *torch.autograd.grad(out, x, d))
+
+    fn = _compiled()
+    step(fn)
+    before = dict(interface.stats)
+    short = step(fn)
+    assert interface.stats["fused_training"] == before["fused_training"] + 2
+    assert torch.autograd.grad(fn(*x), x[1], d)[0].equal(short[2])
+    with torch.no_grad():
+        alone = fn(*x)
+    assert interface.stats["fused"] == before["fused"] + 1
+    monkeypatch.setattr(training, "one_attention", lambda gm, inputs, general: general)
+    monkeypatch.setattr(interface, "_one_attention", lambda gm, found, general: general)
+    fn = _compiled()
+    assert all(a.equal(b) for a, b in zip(short, step(fn)))
+    with torch.no_grad():
+        assert fn(*x).equal(alone)
+
+
+@pytest.mark.gpu
+def test_hooks_and_second_derivatives_of_the_short_way():
+    *x, d = _tensors(100)
+    x = [t.requires_grad_() for t in x]
+    fn = _compiled()
+    want = [torch.autograd.grad(fn(*x), x, d) for _ in range(2)][1]
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(1), t.cpu())[1], lambda t: t.cuda()):
+        out = fn(*x)
+    assert len(packed) == 5 and all(a.equal(b) for a, b in zip(want, torch.autograd.grad(out, x, d)))
+    first = torch.autograd.grad(fn(*x), x, d, create_graph=True)
+    assert all(a.equal(b) for a, b in zip(want, first))
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(first[0].float().sum(), x[1])
