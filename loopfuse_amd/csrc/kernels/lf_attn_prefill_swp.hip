@@ -411,7 +411,9 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
     const lf_cu64* mbits = reinterpret_cast<const lf_cu64*>(reinterpret_cast<unsigned long long>(p.bias)) +
                            16 * mblock * ((p.Sk + 31) / 32);
     const int mfirst = min(kPer * kt_begin / 32, nwords - 1);
-    unsigned mseen = mwords[2 * mfirst], mhidden = mwords[2 * mfirst + 1];
+    // (scalar registers, said explicitly: what the loop decides with them reaches the direct loads' addresses)
+    auto mword = [&](int i) { return (unsigned)__builtin_amdgcn_readfirstlane((int)mwords[i]); };
+    unsigned mseen = mword(2 * mfirst), mhidden = mword(2 * mfirst + 1);
 #endif
     int ks_cur = 0;   // K slot of tile kt
 #if LF_BIAS == 2
@@ -419,8 +421,8 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
       const int t = kPer * (kt + 1);
       if (t % 32 == 0) {
         const int next = min(t / 32, nwords - 1);
-        mseen = mwords[2 * next];
-        mhidden = mwords[2 * next + 1];
+        mseen = mword(2 * next);
+        mhidden = mword(2 * next + 1);
       }
     };
     constexpr unsigned kBlocks = (1u << kPer) - 1u;
@@ -462,6 +464,8 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
         if (++kt == kt_end) break;
       }
       if (kt == kt_end) break;
+      kt = __builtin_amdgcn_readfirstlane(kt);
+      ks_cur = __builtin_amdgcn_readfirstlane(ks_cur);
 #endif
       const int rel = kt - kt_begin;
       const int ks_nxt = (ks_cur == LF_KSLOTS - 1) ? 0 : ks_cur + 1;   // slot of K(kt+1)
