@@ -151,27 +151,32 @@ __device__ __forceinline__ void lf_bw_mfma_vva(lf_f32x16& c, const lf_u32x4& a, 
   asm volatile(LF_BW_MFMA " %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(b));
 }
 // accumulators X^T[d][n] (lane n = lane % 32; element i of block db is d = 32*db + 8*(i/4) + 4*g + i%4)
-// -> rows n of a [rows, D] matrix, 16 bytes per store (the exchange of the forward's epilogue)
-__device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, lf_elem* row_ptr, bool valid, int g) {
+// -> rows 0 .. 31 of a [.., D] matrix, those below `valid`.  They meet in the wave's part of the LDS (`rows_lds`, LF_BW_ROWS_LDS
+// bytes that nobody reads any more) and leave whole, neighbouring lanes with the pieces of one row, by non-temporal stores:
+// 32-byte pieces of every lane's own row took the L2 from what the launch reads.  All backward launches, us: causal B4 H32 S2048 D128
+// 580 -> 567, unmasked 901 -> 853, window 256 B4 32/8 S2048 216 -> 204, unmasked B10 H32 S739 396 -> 380; launches of 25 us pay 0.5 for
+// the way through LDS.
+#define LF_BW_OUT_STRIDE (LF_D * 2 + 16)
+#define LF_BW_ROWS_LDS (32 * LF_BW_OUT_STRIDE)
+__device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, unsigned rows_lds, lf_elem* rows, long long stride, int valid, int lane) {
+  typedef __attribute__((address_space(3))) lf_u32x2* lds_write_t;
+  typedef __attribute__((address_space(3))) const lf_u32x4* lds_read_t;
+  const int l32 = lane & 31, g = lane >> 5;
 #pragma unroll
-  for (int db = 0; db < LF_NDB; ++db) {
-    unsigned ch[4][2];
+  for (int db = 0; db < LF_NDB; ++db)
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       lf_elem4 w;
 #pragma unroll
       for (int e = 0; e < 4; ++e) w[e] = lf_from_float(acc[db][4 * i4 + e]);
-      const lf_u32x2 wu = __builtin_bit_cast(lf_u32x2, w);
-      ch[i4][0] = wu[0];
-      ch[i4][1] = wu[1];
+      *(lds_write_t)(size_t)(rows_lds + (unsigned)(l32 * LF_BW_OUT_STRIDE + 64 * db + 16 * i4 + 8 * g)) = __builtin_bit_cast(lf_u32x2, w);
     }
+  constexpr int kRows = 64 / LF_CPR;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      auto r0 = __builtin_amdgcn_permlane32_swap(ch[2 * j][0], ch[2 * j + 1][0], false, false);
-      auto r1 = __builtin_amdgcn_permlane32_swap(ch[2 * j][1], ch[2 * j + 1][1], false, false);
-      const lf_u32x4 out = {r0[0], r1[0], r0[1], r1[1]};
-      if (valid) *reinterpret_cast<lf_u32x4*>(row_ptr + 32 * db + 16 * j + 8 * g) = out;
-    }
+  for (int i = 0; i < 32 / kRows; ++i) {
+    const int r = kRows * i + lane / LF_CPR, c = lane % LF_CPR;
+    const lf_u32x4 x = *(lds_read_t)(size_t)(rows_lds + (unsigned)(r * LF_BW_OUT_STRIDE + 16 * c));
+    if (r < valid) __builtin_nontemporal_store(x, reinterpret_cast<lf_u32x4*>(rows + r * stride + 8 * c));
   }
 }
 
@@ -813,17 +818,25 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
   auto ep = (const LfAttnBwdParams __attribute__((address_space(4)))*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(ep));
   const float scale = ep->scale;
+#if LF_BW_QSPLIT
+  const unsigned rows_lds = lds0 + (unsigned)(KB * LF_NDB * 8 * 128 * 16 + wave * LF_BW_ROWS_LDS);      // behind the sums
+  static_assert(KB * LF_NDB * 8 * 128 * 16 + kKeyWaves * LF_BW_ROWS_LDS <= (int)sizeof(tiles), "sums and rows fit the tiles");
+#else
+  static_assert(4 * LF_BW_ROWS_LDS <= (int)sizeof(tiles), "the rows fit the tiles");
+  const unsigned rows_lds = lds0 + (unsigned)(wave * LF_BW_ROWS_LDS);
+  __syncthreads();               // nobody reads the tiles any more
+#endif
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
-    const int my_key = key0 + 32 * kb + l32;
-    const bool valid = my_key < p.Sk;
-    const int kr = min(my_key, p.Sk - 1);
+    const int first = key0 + 32 * kb;
 #pragma unroll
     for (int db = 0; db < LF_NDB; ++db)
 #pragma unroll
       for (int i = 0; i < 16; ++i) dk[kb][db][i] *= scale;
-    lf_bw_store_rows(dk[kb], ep->dk + (long long)b * ep->dk_sb + (long long)hkv * ep->dk_sh + (long long)kr * ep->dk_ss, valid, g);
-    lf_bw_store_rows(dv[kb], ep->dv + (long long)b * ep->dv_sb + (long long)hkv * ep->dv_sh + (long long)kr * ep->dv_ss, valid, g);
+    lf_bw_store_rows(dk[kb], rows_lds, ep->dk + (long long)b * ep->dk_sb + (long long)hkv * ep->dk_sh + (long long)first * ep->dk_ss, ep->dk_ss,
+                     p.Sk - first, lane);
+    lf_bw_store_rows(dv[kb], rows_lds, ep->dv + (long long)b * ep->dv_sb + (long long)hkv * ep->dv_sh + (long long)first * ep->dv_ss, ep->dv_ss,
+                     p.Sk - first, lane);
   }
 }
 
@@ -860,7 +873,6 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
   const int h = hkv * group + row % group;
   const int q0 = kBM * qt;
   const int wq0 = q0 + 32 * wave;                    // first row of this wave
-  const int my_q = wq0 + l32, qr = min(my_q, p.Sq - 1);
 
   int kt_begin = 0, kt_end = (p.Sk + 63) / 64;
   {
@@ -970,7 +982,10 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
   for (int db = 0; db < LF_NDB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[db][i] *= p.scale;
-  lf_bw_store_rows(dq, p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)qr * p.dq_ss, my_q < p.Sq, g);
+  static_assert(kWaves * LF_BW_ROWS_LDS <= (int)sizeof(ds_tiles), "the rows fit the tiles");
+  __syncthreads();               // nobody reads the tiles any more
+  lf_bw_store_rows(dq, ds0_lds + (unsigned)(wave * LF_BW_ROWS_LDS), p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)wq0 * p.dq_ss,
+                   p.dq_ss, p.Sq - wq0, lane);
 }
 #else
 // dQ of LF_BW_DQ_NT / 2 query rows of one (batch, head), 32 per wave.
@@ -1296,6 +1311,9 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
   for (int db = 0; db < LF_NDB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[db][i] *= p.scale;
-  lf_bw_store_rows(dq, p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)qr * p.dq_ss, my_q < p.Sq, g);
+  static_assert(LF_BW_DQ_NT / 64 * LF_BW_ROWS_LDS <= (int)sizeof(tiles), "the rows fit the tiles");
+  __syncthreads();               // nobody reads the tiles any more
+  lf_bw_store_rows(dq, lds0 + (unsigned)(wave * LF_BW_ROWS_LDS), p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)wq0 * p.dq_ss,
+                   p.dq_ss, p.Sq - wq0, lane);
 }
 #endif
