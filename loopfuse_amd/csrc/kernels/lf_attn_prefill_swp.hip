@@ -416,6 +416,7 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
     unsigned mseen = mword(2 * mfirst), mhidden = mword(2 * mfirst + 1);
 #endif
     int ks_cur = 0;   // K slot of tile kt
+#if LF_BIAS
 #if LF_BIAS == 2
     auto mask_next = [&](int kt) {       // behind tile kt
       const int t = kPer * (kt + 1);
@@ -426,15 +427,24 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
       }
     };
     constexpr unsigned kBlocks = (1u << kPer) - 1u;
+#else
+    // (the class in a scalar register, said explicitly: it reaches the direct loads' addresses)
+    auto tile_class = [&](int kt) { return __builtin_amdgcn_readfirstlane((int)ccls[kt]); };
+    auto mask_next = [](int) {};
+#endif
     auto mask_need = [&](int kt) {
+#if LF_BIAS == 2
       bool n = wave_has_rows && (mseen >> (kPer * kt % 32) & kBlocks) != 0u;
+#else
+      bool n = wave_has_rows && tile_class(kt) != 0;
+#endif
 #if LF_MASK >= 1
       n = n && kt * LF_BN <= wqlast;
 #endif
 #if LF_MASK == 2
       n = n && min(kt * LF_BN + LF_BN, p.Sk) - 1 >= wq0 - p.window + 1;
 #endif
-      return n;
+      return __builtin_amdgcn_readfirstlane((int)n) != 0;
     };
     auto stage_only = [&](int kt) {
       const int ks_nxt = (ks_cur == LF_KSLOTS - 1) ? 0 : ks_cur + 1, ks_ld = (ks_nxt == LF_KSLOTS - 1) ? 0 : ks_nxt + 1;
@@ -456,9 +466,11 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
     };
 #endif
     for (int kt = kt_begin; kt < kt_end; ++kt) {
-#if LF_BIAS == 2
+#if LF_BIAS
       // Tiles of which this wave's rows see nothing are staged, not computed: in a loop of their own, because with a branch
-      // around the products the compiler keeps O^T twice and copies it every tile (47 registers spilled at three waves per SIMD)
+      // around the products the compiler keeps O^T twice and copies it every tile (47 registers spilled at three waves per SIMD;
+      // with a bias tensor and four packed heads 26..71 at two, and B 8 x 2048, 32/8 heads, cap, window 256 as a bias takes
+      // 335 us instead of 152)
       while (!mask_need(kt)) {
         stage_only(kt);
         if (++kt == kt_end) break;
@@ -517,10 +529,8 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
 #elif LF_BIAS
       // class 2: the tile's bias values are requested before the S^T products.  Element i of block kb is
       // key j = k0 + 32*kb + 8*(i/4) + 4*g + i%4 of row my_q: four consecutive keys per 8-byte load
-      // class 0 inside the range (a dead tile between live ones): staged like any tile, not computed
-      const int tile_class = (int)ccls[kt];
-      need = need && tile_class != 0;
-      const bool biased = need && tile_class == 2;
+      need = true;                     // class 0 inside the range, a dead tile between live ones, was only staged above
+      const bool biased = tile_class(kt) == 2;
       lf_u32x2 bias_v[LF_NKB][4];
       if (biased) {
         const lf_elem* brow = p.bias + (long long)b * p.bias_sb + (long long)h * p.bias_sh +
@@ -751,7 +761,7 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
 #pragma unroll
         for (int f = 0; f < LF_KPF; ++f) kpre[f] = k_frag(knext, f);
       }
-#if LF_BIAS == 2
+#if LF_BIAS
       mask_next(kt);
 #endif
       LF_BARRIER_VM0();

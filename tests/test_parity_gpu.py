@@ -230,6 +230,25 @@ def test_biased_attention_paged_kv():
     check(q, kp, vp, mask="causal", k_table=table, v_table=table, score_bias=sb)
 
 
+@pytest.mark.parametrize("flag,bn", [("causal", 64), ("causal", 32), ("sliding", 64), ("sliding", 32)])
+def test_boolean_mask_with_paged_kv_and_a_flag(flag, bn):
+    B, H, S, D, P = 2, 2, 256, 128, 16
+    n = B * S // P
+    kp, vp = rand((n, P, H, D), torch.bfloat16, 1), rand((n, P, H, D), torch.bfloat16, 2)
+    table = torch.randperm(n, generator=torch.Generator().manual_seed(9)).view(B, S // P).to(torch.int32)
+    q = rand((B, H, S, D), torch.bfloat16, 3)
+    shown = torch.rand((B, 1, S, S), generator=torch.Generator().manual_seed(4)) < 0.6
+    shown[:, :, :, 64:128] = False
+    shown |= torch.eye(S, dtype=torch.bool)
+    on = [t.to(dev()) for t in (q, kp, vp, table, shown)]
+    plan = lowering.AttnPlan(mask=flag, window=100 if flag == "sliding" else 0, scale=D ** -0.5, k_paged=True, v_paged=True)
+    got = lowering.attention(*on[:3], plan, k_table=on[3], v_table=on[3], score_mask=on[4], choice={"bn": bn})
+    assert lowering.attention.last_launch["kernels"] == ["lf_mask_tiles", "lf_attn_prefill_swp"]
+    want = O.attention_reference(q, kp, vp, mask=flag, window=plan.window, k_table=table, v_table=table,
+                                 score_bias=torch.zeros(shown.shape).masked_fill(~shown, float("-inf")))
+    assert (got.float().cpu() - want).abs().max().item() <= TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("copy", ["1", "0"])
 def test_unaligned_bias_rows(copy, monkeypatch):
     # contiguous [.., 333, 333] bias: rows start at odd element offsets -> a copy with padded
@@ -1199,6 +1218,22 @@ def test_mask_bits_with_both_key_tiles(Sq, Sk, group, flag, dt):
             assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(same))
         got = got.float().cpu()
         assert torch.isnan(got[blind]).all() and (got[~blind] - want[~blind]).abs().max().item() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("Sq", [1, 31, 33, 127, 129])
+@pytest.mark.parametrize("D,group,bn", [(64, 1, 64), (128, 1, 64), (128, 1, 32), (128, 2, 32), (128, 4, 32)])
+def test_output_rows_end_where_the_queries_end(Sq, D, group, bn):
+    """The output leaves in whole rows from LDS: into a view with guard rows and columns around it, nothing beyond a head's rows."""
+    B, H = 2, 4
+    q, k, v = (rand((B, h, n, D), torch.bfloat16, s) for h, n, s in ((H, Sq, 1), (H // group, 200, 2), (H // group, 200, 3)))
+    buf = torch.full((B, H, Sq + 3, D + 8), 123.0, dtype=torch.bfloat16, device=dev())
+    out = buf[:, :, 1:Sq + 1, :D]
+    lowering.attention(q.to(dev()), k.to(dev()), v.to(dev()), lowering.AttnPlan(scale=D ** -0.5), out=out, choice={"bn": bn},
+                       force_family="prefill_swp")
+    assert lowering.attention.last_launch["kernels"] == ["lf_attn_prefill_swp"]
+    assert (out.float().cpu() - O.attention_reference(q, k, v)).abs().max().item() <= TOL[torch.bfloat16]
+    out.fill_(123.0)
+    assert (buf == 123.0).all()
 
 
 @pytest.mark.parametrize("case", ["decode", "key_stride", "register_staged"])
