@@ -74,8 +74,8 @@
                             2: a boolean mask as lf_mask_tiles leaves it (lf_mask_bits.hip): classes per 32 rows x 32 keys in
                             p.part_acc, so that a wave computes only what its own rows see, and in p.bias a 64-bit word per
                             accumulator element of a mixed block, which is the lane select as it is: 32 scalar registers and
-                            no vector load in the loop, so that 32-key tiles fit three workgroups per CU as without a mask.
-                            B4 H32 S1536 D128, causal and padding: 99 -> 85 us against the 16-bit bias of form 1 */
+                            no vector load in the loop.  B4 H32 S1536 D128, causal and padding, both launches: 110 us with the
+                            16-bit bias of form 1 for mixed blocks, 101 with the bits */
 #endif
 #define LF_BARRIER_VM0() asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory")
 
@@ -468,8 +468,8 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
     for (int kt = kt_begin; kt < kt_end; ++kt) {
 #if LF_BIAS
       // Tiles of which this wave's rows see nothing are staged, not computed: in a loop of their own, because with a branch
-      // around the products the compiler keeps O^T twice and copies it every tile (47 registers spilled at three waves per SIMD;
-      // with a bias tensor and four packed heads 26..71 at two, and B 8 x 2048, 32/8 heads, cap, window 256 as a bias takes
+      // around the products the compiler keeps O^T twice and copies it every tile (with a bias
+      // tensor and four packed heads 26..71 registers spilled, and B 8 x 2048, 32/8 heads, cap, window 256 as a bias takes
       // 335 us instead of 152)
       while (!mask_need(kt)) {
         stage_only(kt);

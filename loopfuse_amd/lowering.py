@@ -580,13 +580,12 @@ def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, w
     768 ... 2047 workgroups, up to 700 keys 0.90 (0.80 ... 1.10), 700 ... 2047 0.97 (0.90 ... 1.04), 2048 and more 1.02 (0.94 ... 1.13: 784
     workgroups of 6211 keys; one 6001-token prompt, 1504 workgroups, 328 against 312 us); from 2048 workgroups on 0.95
     (0.79 ... 1.05); 500 ... 767 either way (0.72 ... 1.15).  At head
-    dimension 64 it does not pay.  The bias tile
-    classes of a score bias are per 64 keys, so biased calls keep 64.  A boolean mask has classes per 32 keys and follows the rule
-    without one: times with 32 over 64, 90 launches of causal, padding, window and random masks, 768 ... 2047 workgroups of up to
-    2047 keys 0.94 (0.83 ... 1.04), of more 1.03 (0.97 ... 1.07), from 2048 workgroups on 0.95 (0.87 ... 1.01), 400 ... 767 1.01 (0.84 ...
-    1.19); beside a softcap, whose scores such a kernel holds in another form, it keeps 64 too (B4 H32 S1536 104 / 111 us).  ``choice["bn"]`` (the tuner) or
-    ``LOOPFUSE_BN`` override the default."""
-    if bias_bits & 7:
+    dimension 64 it does not pay.  The bias tile classes of a score bias are per 64 keys, so biased calls keep 64.  So does a
+    boolean mask, for its error: the exponents' first offset is the maximum of the first tile, and over 32 keys the largest weight
+    is less often exactly 1 (relative 2-norm against float64, 64 / 32 keys: bf16 1024 keys 2.338e-3 / 2.346e-3, 300 keys with
+    inputs of 6 1.821e-3 / 1.901e-3); a padding mask of 4 x 32 heads x 1536 takes 101 and 92 us, 110 before its bits.
+    ``choice["bn"]`` (the tuner) or ``LOOPFUSE_BN`` override the default without a bias or mask."""
+    if bias_bits:
         return 0
     want = (choice or {}).get("bn", _env("LOOPFUSE_BN"))
     if want is not None:
@@ -1158,7 +1157,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                      page_size, table_i64, v_tr=v_tr if family == "prefill" else True, bias=bias_bits,
                      denom=plan.denom_add != 0.0, d2=d2, page_size_v=page_size_v, pack=pack, extra=extra,
                      safe=plan.zero_blind_rows and bool(bias_bits & (1 | MASK_BITS)),
-                     bn=prefill_kv_tile(D, bias_bits | int(bias_bits == MASK_BITS and plan.softcap is not None), choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
+                     bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
                                         min(Sk, P.window) if mask == MASK_SLIDING else Sk)
                      if family == "prefill_swp" else 0)
         bm, bn = TILE_SHAPES[family]

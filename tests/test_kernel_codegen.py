@@ -270,11 +270,10 @@ def test_backward_code_that_spills_is_refused(shim_built):
         runtime.private_segment_bytes(b"no code object")
 
 
-@pytest.mark.parametrize("bias,mask,softcap,paged,pack,bn", [
-    (b, m, c, pg, pk, bn) for b, bn in ((1, 0), (lowering.MASK_BITS, 0), (lowering.MASK_BITS, 32))
-    for m, c, pg, pk in ((1, False, 3, 0), (2, False, 3, 0), (0, False, 0, 4), (2, True, 0, 4), (1, False, 3, 4))])
-def test_masked_prefill_builds_and_does_not_spill(shim_built, bias, mask, softcap, paged, pack, bn):
+@pytest.mark.parametrize("bias,mask,softcap,paged,pack", [
+    (b, m, c, pg, pk) for b in (1, lowering.MASK_BITS) for m, c, pg, pk in ((1, False, 3, 0), (2, False, 3, 0), (0, False, 0, 4), (2, True, 0, 4), (1, False, 3, 4))])
+def test_masked_prefill_builds_and_does_not_spill(shim_built, bias, mask, softcap, paged, pack):
     """What the loop over dead tiles decides reaches the scalar operand of the direct loads (a decision left in a vector register
     does not assemble), and a branch around the products instead of that loop costs a second copy of O^T (spills)."""
-    spec = lowering.KernelSpec("prefill_swp", 0, 128, mask, softcap, paged, 16 if paged else 1, bias=bias, pack=pack, bn=bn)
+    spec = lowering.KernelSpec("prefill_swp", 0, 128, mask, softcap, paged, 16 if paged else 1, bias=bias, pack=pack)
     assert not any("scratch_" in ln for ln in _kernels(spec)["lf_attn_prefill_swp"])

@@ -230,8 +230,8 @@ def test_biased_attention_paged_kv():
     check(q, kp, vp, mask="causal", k_table=table, v_table=table, score_bias=sb)
 
 
-@pytest.mark.parametrize("flag,bn", [("causal", 64), ("causal", 32), ("sliding", 64), ("sliding", 32)])
-def test_boolean_mask_with_paged_kv_and_a_flag(flag, bn):
+@pytest.mark.parametrize("flag", ["causal", "sliding"])
+def test_boolean_mask_with_paged_kv_and_a_flag(flag):
     B, H, S, D, P = 2, 2, 256, 128, 16
     n = B * S // P
     kp, vp = rand((n, P, H, D), torch.bfloat16, 1), rand((n, P, H, D), torch.bfloat16, 2)
@@ -242,7 +242,7 @@ def test_boolean_mask_with_paged_kv_and_a_flag(flag, bn):
     shown |= torch.eye(S, dtype=torch.bool)
     on = [t.to(dev()) for t in (q, kp, vp, table, shown)]
     plan = lowering.AttnPlan(mask=flag, window=100 if flag == "sliding" else 0, scale=D ** -0.5, k_paged=True, v_paged=True)
-    got = lowering.attention(*on[:3], plan, k_table=on[3], v_table=on[3], score_mask=on[4], choice={"bn": bn})
+    got = lowering.attention(*on[:3], plan, k_table=on[3], v_table=on[3], score_mask=on[4])
     assert lowering.attention.last_launch["kernels"] == ["lf_mask_tiles", "lf_attn_prefill_swp"]
     want = O.attention_reference(q, kp, vp, mask=flag, window=plan.window, k_table=table, v_table=table,
                                  score_bias=torch.zeros(shown.shape).masked_fill(~shown, float("-inf")))
@@ -1192,9 +1192,9 @@ def test_boolean_masks_equal_the_bias_they_stand_for(Sq, Sk, mshape, group, keep
     (515, 1600, 1, "sliding", 1),
     (33, 4, 1, None, 0),
 ])
-def test_mask_bits_with_both_key_tiles(Sq, Sk, group, flag, dt):
-    """Words and selects of lf_mask_tiles under 32- and 64-key tiles at head dim 128: 64 keys give the bits that the 0 / -inf bias
-    gives, 32 keys the oracle's values (TOL, as for the flag kernels)."""
+def test_mask_bits(Sq, Sk, group, flag, dt):
+    """Words and selects of lf_mask_tiles at head dim 128: the oracle's values (TOL, as for the flag kernels) and the bits that the
+    0 / -inf bias gives, which is also what a call that asks for 32-key tiles gets."""
     g = torch.Generator().manual_seed(Sq * Sk)
     B, H, D, dtype = 2, 4, 128, (torch.bfloat16, torch.float16)[dt]
     q, k, v = (rand((B, h, n, D), dtype, s) for h, n, s in ((H, Sq, 1), (H // group, Sk, 2), (H // group, Sk, 3)))
@@ -1213,9 +1213,8 @@ def test_mask_bits_with_both_key_tiles(Sq, Sk, group, flag, dt):
     for bn in (64, 32):
         got, walked = lowering.attention(*on, plan, score_mask=shown.to(dev()), choice={"bn": bn}, record_visits=True)
         assert lowering.attention.last_launch["kernels"] == ["lf_mask_tiles", "lf_attn_prefill_swp"]
-        assert lowering.attention.last_launch["kv_tile_rows"] == bn and walked.shape[1] == -(-Sk // bn)
-        if bn == 64:
-            assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(same))
+        assert lowering.attention.last_launch["kv_tile_rows"] == 64 and walked.shape[1] == -(-Sk // 64)
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(same))
         got = got.float().cpu()
         assert torch.isnan(got[blind]).all() and (got[~blind] - want[~blind]).abs().max().item() <= TOL[dtype]
 
