@@ -193,13 +193,13 @@ def _one_attention(gm: torch.fx.GraphModule, found: list, general: Callable) -> 
     """``general``, AOTAutograd's callable for an inference graph, with a shorter way for calls over plain tensors where the graph
     is nothing but one attention over its inputs (``found``, from ``loopfuse_compiler``): the fused call itself, without
     the wrappers that find out on every call what this graph does not have (aliases, mutations, subclasses).  B2 H8 S512
-    D64: 34.5 -> 28.6 us a call.  Calls with anything else than plain tensors, and graphs of which a call was refused, go
-    through ``general``."""
+    D64: 34.5 -> 28.6 us a call.  Graphs whose one output is not the caller's as it is (``_result_as_it_is``), calls with
+    anything else than plain tensors, and those that the kernels refuse go through ``general``."""
     from . import training
 
     if len(found) != 1 or any(True for _ in gm.parameters()) or any(True for _ in gm.buffers()):
         return general
-    match, at, count, refused, refuse = found[0]
+    match, at, count, refused, note = found[0]
     if count != len(get_input_names(gm)):
         return general
 
@@ -212,12 +212,23 @@ def _one_attention(gm: torch.fx.GraphModule, found: list, general: Callable) -> 
         try:
             out = match.run(vals)
         except lowering.UnsupportedPlan as e:
-            return refuse(args, e)
+            note(args, e)
+            return general(*args)
         stats["fused"] += 1
         return (out,)
 
     call.__dict__.update(general.__dict__)
     return call
+
+
+def _result_as_it_is() -> bool:
+    """Does the graph that AOTAutograd is compiling return one tensor, which its callable hands on untouched?  Not where
+    an input is written to (``out=`` and in-place operations become results that the callable copies back; a function
+    that returns nothing else leaves a graph of one output, too) or where the output is a view of an input."""
+    context = torch._guards.TracingContext.try_get()
+    meta = getattr(context, "fw_metadata", None)
+    return meta is not None and not any(i.mutates_data or i.mutates_metadata for i in meta.input_info) \
+        and [o.output_type.name for o in meta.output_info] == ["non_alias"]
 
 
 _warned_training = False
@@ -428,7 +439,7 @@ def loopfuse_compiler(gm: torch.fx.GraphModule, sample_inputs, input_names: list
                       symint_names: dict[str, str] | None = None, mode: str | None = None, alone: list | None = None) -> Callable:
     """fw_compiler: ATen graph -> callable over the flat placeholder list.  ``alone`` receives, of a graph that is nothing but one
     attention over its inputs, its match, the positions of its inputs, the number of placeholders, the signatures refused
-    so far and what runs a call that the kernels refuse."""
+    so far and what notes one more."""
     global _codegen_sink
     stats["compiled_graphs"] += 1
     if DEBUG:
@@ -546,7 +557,7 @@ def loopfuse_compiler(gm: torch.fx.GraphModule, sample_inputs, input_names: list
         stats["eager_runtime"] += 1
         return gm(*args)
 
-    def refuse(args, why):
+    def note(args, why):
         if _strict():
             raise why
         if len(refused) >= 64:      # bounded: forget old refusals rather than grow
@@ -555,15 +566,14 @@ def loopfuse_compiler(gm: torch.fx.GraphModule, sample_inputs, input_names: list
         stats["refused_signatures"] += 1
         log.warning("fused path not applicable to this call (%s); calls with these argument layouts run "
                     "the graph unfused", why)
-        return run_unfused(args)
 
-    if alone is not None and len(matches) == 1:
+    if alone is not None and len(matches) == 1 and _result_as_it_is():
         nodes = list(fused_gm.graph.nodes)
         calls = [n for n in nodes if n.op == "call_function"]
         placeholders = [n for n in nodes if n.op == "placeholder"]
         out = next(n for n in nodes if n.op == "output").args[0]
         if len(calls) == 1 and isinstance(out, (tuple, list)) and list(out) == calls and all(n in placeholders for n in calls[0].args[1:]):
-            alone.append((matches[0], [placeholders.index(n) for n in calls[0].args[1:]], len(placeholders), refused, refuse))
+            alone.append((matches[0], [placeholders.index(n) for n in calls[0].args[1:]], len(placeholders), refused, note))
 
     def optimized_fn(*args):
         sig = signature(args) if refused else None
@@ -572,7 +582,8 @@ def loopfuse_compiler(gm: torch.fx.GraphModule, sample_inputs, input_names: list
         try:
             out = fused_gm(*args)
         except lowering.UnsupportedPlan as e:
-            return refuse(args, e)
+            note(args, e)
+            return run_unfused(args)
         stats["fused"] += 1
         return out
 

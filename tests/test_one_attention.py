@@ -45,6 +45,75 @@ def test_only_graphs_of_one_attention_take_the_short_way():
     assert call(x[0].as_subclass(Sub), x[1], x[2]) == "general"
 
 
+def _probabilities(q, k):
+    return torch.softmax(torch.ops.loopfuse.causal_mask(q @ k.transpose(-2, -1) * (q.shape[-1] ** -0.5)), dim=-1)
+
+
+def _alone(q, k, v, d):
+    return torch.bmm(_probabilities(q, k), v)
+
+
+def _out(q, k, v, d):
+    torch.bmm(_probabilities(q, k), v, out=d)
+
+
+def _out_returned(q, k, v, d):
+    return torch.bmm(_probabilities(q, k), v, out=d)
+
+
+def _copied(q, k, v, d):
+    d.copy_(torch.bmm(_probabilities(q, k), v))
+
+
+def _scaled_in_place(q, k, v, d):
+    d.mul_(2.0)
+    return torch.bmm(_probabilities(q, k), v)
+
+
+def _input_returned(q, k, v, d):
+    return torch.bmm(_probabilities(q, k), v), q
+
+
+def _input_reshaped(q, k, v, d):
+    d.unsqueeze_(0)
+    return torch.bmm(_probabilities(q, k), v)
+
+
+@pytest.mark.parametrize("refused", [False, True])
+@pytest.mark.parametrize("fn", [_alone, _out, _out_returned, _copied, _scaled_in_place, _input_returned, _input_reshaped])
+def test_what_the_short_way_leaves_in_outputs_and_inputs(fn, refused, monkeypatch):
+    """Outputs and inputs after the first and the second call are those of the function itself, also where the kernels refuse the
+    call (CPU tensors).  The graph that is nothing but an attention skips the general callable, one whose only result is
+    written into an input does not, though it too is one attention with one output.  torch takes the kernel's place here."""
+    short = []
+
+    def run(self, vals):
+        q, k, v = (self._operand(o, vals)[0] for o in (self.q, self.k, self.v))
+        return (_probabilities(q, k) @ v)[0]
+
+    real = interface._one_attention
+
+    def seen(gm, found, general):
+        short.append(real(gm, found, general) is not general)
+        return real(gm, found, general)
+
+    if not refused:
+        monkeypatch.setattr(capture.AttentionMatch, "run", run)
+    monkeypatch.setattr(interface, "_one_attention", seen)
+    torch._dynamo.reset()
+    compiled = torch.compile(fn, backend=functools.partial(loopfuse_backend, mode=None), dynamic=False)
+    g = torch.Generator().manual_seed(1)
+    for _ in range(2):
+        want_in = [torch.randn(4, 40, 64, generator=g) for _ in range(4)]
+        got_in = [t.clone() for t in want_in]
+        with torch.no_grad():
+            want, got = fn(*want_in), compiled(*got_in)
+        torch.testing.assert_close(got, want)
+        torch.testing.assert_close(got_in, want_in)
+    if fn in (_alone, _out):
+        assert short == [fn is _alone]
+
+
 def _attn(q, k, v):
     s = torch.ops.loopfuse.causal_mask(q @ k.transpose(-2, -1) * (q.shape[-1] ** -0.5))
     return torch.softmax(s, dim=-1) @ v
