@@ -167,8 +167,8 @@ def one_attention(gm: torch.fx.GraphModule, sample_inputs, general):
     where the graph is nothing but one attention over its inputs as they are: ``_Attention``, without the wrappers that
     find out on every call what this graph does not have (aliases, mutations, subclasses, tangents of another layout).
     B8 16/4 S1000 D64 fp16, forward and backward (139 us of kernels): 251 -> 151 us a step.  Everything else -- what ``_plain``
-    sends away, dynamic sizes, operands that are views, one tensor in two places, several outputs -- goes through
-    ``general``, and so does the first call: its graphs, the backward's too, are then there for whoever needs them."""
+    sends away, dynamic sizes, operands that are views or held by the graph, one tensor in two places, several outputs -- goes
+    through ``general``, and so does the first call: its graphs, the backward's too, are then there for whoever needs them."""
     nodes = list(gm.graph.nodes)
     calls = [n for n in nodes if n.op == "call_function"]
     placeholders = [n for n in nodes if n.op == "placeholder"]
@@ -178,6 +178,8 @@ def one_attention(gm: torch.fx.GraphModule, sample_inputs, general):
         return general
     match = getattr(gm, calls[0].args[0].target)
     operands = calls[0].args[1:]
+    if not all(n in placeholders for n in operands):
+        return general                           # a parameter or buffer that the graph holds itself
     if match.out_order or match.out_rank != 4 or any(o.paged or tuple(o.perm) != (0, 1, 2, 3) for o in (match.q, match.k, match.v)):
         return general
     at = [placeholders.index(operands[o.index]) for o in (match.q, match.k, match.v)]

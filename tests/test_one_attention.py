@@ -9,9 +9,9 @@ from loopfuse_amd import loopfuse_backend
 from loopfuse_amd.torch_backend import capture, interface, training
 
 
-def _graph(second_output=False, extra=False, twice=False, perm=(0, 1, 2, 3)):
+def _graph(second_output=False, extra=False, twice=False, perm=(0, 1, 2, 3), held=""):
     graph = torch.fx.Graph()
-    ins = [graph.placeholder(n) for n in "qkv"]
+    ins = [graph.get_attr("_" + n) if n in held else graph.placeholder(n) for n in "qkv"]
     attr = graph.get_attr("_m")
     out = graph.call_function(training.fused_call_train, (attr, *((ins[0], ins[0], ins[2]) if twice else ins)))
     if extra:
@@ -19,6 +19,8 @@ def _graph(second_output=False, extra=False, twice=False, perm=(0, 1, 2, 3)):
     graph.output((out, ins[0]) if second_output else (out,))
     ops = [capture.Operand(i, perm) for i in range(3)]
     root = torch.nn.Module()
+    for n in held:
+        setattr(root, "_" + n, torch.nn.Parameter(torch.zeros(1, 2, 8, 64, dtype=torch.bfloat16)))
     root._m = capture.AttentionMatch(out_node=None, inputs=ins, q=ops[0], k=ops[1], v=ops[2], factors=[0.125], post_factors=[],
                                      has_tanh=False, mask="causal", window=0, out_rank=4)
     return torch.fx.GraphModule(root, graph)
@@ -32,6 +34,9 @@ def test_only_graphs_of_one_attention_take_the_short_way():
     assert training.one_attention(_graph(), x, general) is not general
     for other in (_graph(second_output=True), _graph(extra=True), _graph(twice=True), _graph(perm=(0, 2, 1, 3))):
         assert training.one_attention(other, x, general) is general
+    # parameters and buffers that the graph holds itself (torch._dynamo.config.inline_inbuilt_nn_modules off)
+    for held in ("k", "kv", "q"):
+        assert training.one_attention(_graph(held=held), x[len(held):], general) is general
     assert training.one_attention(_graph(), [x[0], x[1], 7], general) is general
     assert training.one_attention(_graph(), [x[0][0], x[1][0], x[2][0]], general) is general
     # what is not plain is sent on, call by call
@@ -155,6 +160,38 @@ def test_the_short_way_gives_the_bits_of_the_general_one(dout, monkeypatch):
     assert all(a.equal(b) for a, b in zip(short, step(fn)))
     with torch.no_grad():
         assert fn(*x).equal(alone)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("buffer", [False, True])
+def test_training_with_keys_that_the_graph_holds(buffer, monkeypatch):
+    """Learnable keys and values of a module whose parameters are not inputs of its graph."""
+    monkeypatch.setattr(torch._dynamo.config, "inline_inbuilt_nn_modules", False)
+    q, k, v, d = _tensors(90)
+    q.requires_grad_()
+
+    class Memory(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.v = torch.nn.Parameter(v)
+            if buffer:
+                self.register_buffer("k", k)
+            else:
+                self.k = torch.nn.Parameter(k)
+
+        def forward(self, q):
+            return _attn(q, self.k, self.v)
+
+    memory = Memory()
+    torch._dynamo.reset()
+    compiled = torch.compile(memory, backend=functools.partial(loopfuse_backend, mode=None), dynamic=False)
+    given = [q, *memory.parameters()]
+    want = torch.autograd.grad(_compiled()(q, memory.k, memory.v), given, d)
+    before = interface.stats["fused_training"]
+    for _ in range(2):
+        got = torch.autograd.grad(compiled(q), given, d)
+        assert all(a.equal(b) for a, b in zip(got, want))
+    assert interface.stats["fused_training"] > before
 
 
 @pytest.mark.gpu
