@@ -269,16 +269,8 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
     const int q0 = qt * LF_BM;
     const int qlast = min(q0 + LF_BM, p.Sq) - 1;
     // ---- block skip: KV tiles [kt_begin, kt_end) hold an unmasked (i, j) for rows q0..qlast
-    int kt_begin = 0, kt_end = nkt;
-#if LF_MASK >= 1
-    kt_end = min(nkt, qlast / LF_BN + 1);
-#endif
-#if LF_MASK == 2
-    {
-      int lo = q0 - p.window + 1;
-      if (lo > 0) kt_begin = lo / LF_BN;
-    }
-#endif
+    int kt_begin, kt_end;
+    lf_tile_range(q0, qlast, nkt, p.window, kt_begin, kt_end);
 #if LF_BIAS == 2
     // The mask's words for this (batch, head): one per 32 rows and 1024 keys; broadcast dims of the mask collapse
     constexpr int kRb = LF_BM / 32, kPer = LF_BN / 32;         // blocks of 32 rows per q tile, of 32 keys per tile

@@ -137,6 +137,23 @@ __device__ __forceinline__ bool lf_slot_of_block(unsigned block, int units, int 
   return unit < units && tile < tiles;
 }
 
+// The key tiles [begin, end), begin <= end <= nkt, that rows q0 .. qlast reach under the flag mask alone.  Rows whose window
+// lies behind the last key reach none: the range is then empty, [nkt, nkt), so that what narrows it further (the classes of a
+// mask or a bias) or stages from its first tile stays within the keys.
+__device__ __forceinline__ void lf_tile_range(int q0, int qlast, int nkt, int window, int& begin, int& end) {
+  begin = 0;
+  end = nkt;
+#if LF_MASK >= 1
+  end = min(nkt, qlast / LF_BN + 1);
+#endif
+#if LF_MASK == 2
+  begin = min(max(q0 - window + 1, 0) / LF_BN, end);
+#endif
+  (void)q0;
+  (void)qlast;
+  (void)window;
+}
+
 // Is score (query row q, key j) kept?  Top-left aligned masks of the reference
 // (loopfuse/torch_backend/ops.py:675-751) plus the bound of the key sequence.
 __device__ __forceinline__ bool lf_mask_keep(int q, int j, int Sk, int window) {

@@ -1219,6 +1219,30 @@ def test_mask_bits(Sq, Sk, group, flag, dt):
         assert torch.isnan(got[blind]).all() and (got[~blind] - want[~blind]).abs().max().item() <= TOL[dtype]
 
 
+@pytest.mark.parametrize("given", ["mask", "bias", None])
+@pytest.mark.parametrize("Sq,Sk,D,group", [(1100, 64, 128, 1), (1100, 100, 64, 4), (700, 130, 128, 2)])
+def test_window_that_ends_behind_the_last_key(given, Sq, Sk, D, group):
+    """Queries beyond the last key by more than the window see nothing: no tile is walked for them, with a mask or a bias too."""
+    B, H, window = 2, 4, 64
+    q, k, v = (rand((B, h, n, D), torch.bfloat16, s) for h, n, s in ((H, Sq, 1), (H // group, Sk, 2), (H // group, Sk, 3)))
+    shown = torch.rand((B, 1, Sq, Sk), generator=torch.Generator().manual_seed(Sq)) < 0.7
+    shown |= torch.eye(Sq, Sk, dtype=torch.bool)
+    bias = torch.zeros(shown.shape).masked_fill(~shown, float("-inf"))
+    extra = {"mask": {"score_mask": shown.to(dev())}, "bias": {"score_bias": bias.bfloat16().to(dev())}}.get(given, {})
+    plan = lowering.AttnPlan(mask="sliding", window=window, scale=D ** -0.5)
+    got, walked = lowering.attention(*(t.to(dev()) for t in (q, k, v)), plan, record_visits=True, **extra)
+    launch = lowering.attention.last_launch
+    assert launch["kernels"][-1] == "lf_attn_prefill_swp"
+    walked = walked.cpu().view(B, H // launch["heads_per_workgroup"], -1, walked.shape[1]).bool()
+    dense = O.visited_tiles_dense("sliding", Sq, Sk, window, launch["q_tile_rows"], launch["kv_tile_rows"])
+    assert walked[0, 0, 0].any() and not (walked & ~dense).any()
+    want = O.attention_reference(q, k, v, mask="sliding", window=window, score_bias=bias if given else None)
+    blind = torch.isnan(want).any(-1)
+    got = got.float().cpu()
+    assert blind[:, :, Sk + window:].all() and torch.isnan(got[blind]).all()
+    assert (got[~blind] - want[~blind]).abs().max().item() <= TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("Sq", [1, 31, 33, 127, 129])
 @pytest.mark.parametrize("D,group,bn", [(64, 1, 64), (128, 1, 64), (128, 1, 32), (128, 2, 32), (128, 4, 32)])
 def test_output_rows_end_where_the_queries_end(Sq, D, group, bn):

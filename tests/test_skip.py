@@ -1,10 +1,13 @@
 """Block-skip set: closed-form tile ranges == brute force over the dense mask, bit-exact."""
+import ctypes
 import dataclasses
+import os
+import subprocess
 
 import pytest
 import torch
 
-from loopfuse_amd import skip
+from loopfuse_amd import runtime, skip
 from oracle import attention_oracle as O
 
 
@@ -30,6 +33,29 @@ def test_other_tile_shapes(bm, bn):
         for qt, (b, e) in enumerate(skip.visited_tiles(mask, 101, 97, w, bm, bn)):
             got[qt, b:e] = True
         assert torch.equal(got, dense)
+
+
+@pytest.mark.parametrize("mask,code", [(None, 0), ("causal", 1), ("sliding", 2)])
+@pytest.mark.parametrize("bm,bn", [(128, 64), (32, 32), (64, 32), (32, 64)])
+def test_device_range_stays_within_the_keys(mask, code, bm, bn, tmp_path):
+    """``lf_tile_range`` itself, compiled as host C++: the tiles of ``skip.tile_range``, and an empty range inside [0, nkt] where the
+    queries outnumber the keys by more than the window."""
+    text = open(os.path.join(runtime.KERNEL_DIR, "lf_prefill_blocks.hip.h")).read()
+    a = text.index("__device__ __forceinline__ void lf_tile_range")
+    src, out = tmp_path / "range.cpp", tmp_path / "range.so"
+    src.write_text("#include <algorithm>\nusing std::max; using std::min;\n" +
+                   text[a:text.index("\n}\n", a) + 3].replace("__device__ __forceinline__", "static") +
+                   'extern "C" void range(int q0, int qlast, int nkt, int w, int* b, int* e) { lf_tile_range(q0, qlast, nkt, w, *b, *e); }\n')
+    subprocess.run(["g++", "-std=c++17", f"-DLF_MASK={code}", f"-DLF_BN={bn}", "-shared", "-fPIC", str(src), "-o", str(out)], check=True)
+    fn, b, e = ctypes.CDLL(str(out)).range, ctypes.c_int(), ctypes.c_int()
+    for Sq, Sk in ((1, 1), (129, 129), (1100, 64), (2000, 100), (515, 700), (3000, 1000)):
+        for window in (1, 64, 65, 200, 2 ** 31 - 1) if code == 2 else (0,):
+            nkt = skip.cdiv(Sk, bn)
+            for qt in range(skip.cdiv(Sq, bm)):
+                fn(qt * bm, min(qt * bm + bm, Sq) - 1, nkt, window, ctypes.byref(b), ctypes.byref(e))
+                assert 0 <= b.value <= e.value <= nkt
+                want = skip.tile_range(mask, qt, Sq, Sk, window, bm, bn)
+                assert range(b.value, e.value) == range(*want)      # (two empty ranges are equal)
 
 
 def test_baseline_counts():
