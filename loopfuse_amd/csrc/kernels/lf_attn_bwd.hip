@@ -162,6 +162,7 @@ __device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, unsigned 
   typedef __attribute__((address_space(3))) lf_u32x2* lds_write_t;
   typedef __attribute__((address_space(3))) const lf_u32x4* lds_read_t;
   const int l32 = lane & 31, g = lane >> 5;
+  lf_wave_exchange();              // the rows before these have been read
 #pragma unroll
   for (int db = 0; db < LF_NDB; ++db)
 #pragma unroll
@@ -171,6 +172,7 @@ __device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, unsigned 
       for (int e = 0; e < 4; ++e) w[e] = lf_from_float(acc[db][4 * i4 + e]);
       *(lds_write_t)(size_t)(rows_lds + (unsigned)(l32 * LF_BW_OUT_STRIDE + 64 * db + 16 * i4 + 8 * g)) = __builtin_bit_cast(lf_u32x2, w);
     }
+  lf_wave_exchange();
   constexpr int kRows = 64 / LF_CPR;
 #pragma unroll
   for (int i = 0; i < 32 / kRows; ++i) {

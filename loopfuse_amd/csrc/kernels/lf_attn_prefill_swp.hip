@@ -796,6 +796,7 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
       lf_elem* ohead = p.o + (long long)b * p.o_sb + (long long)h * p.o_sh;
 #pragma unroll
       for (int turn = 0; turn < kTurns; ++turn) {
+        if (turn) lf_wave_exchange();
         if (kTurns == 1 || l32 / kTurnRows == turn) {
 #pragma unroll
           for (int db = 0; db < LF_NDB; ++db)
@@ -808,6 +809,7 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
                   __builtin_bit_cast(lf_u32x2, w);
             }
         }
+        lf_wave_exchange();
 #pragma unroll
         for (int i = 0; i < kTurnRows / kRows; ++i) {
           const int r = kRows * i + lane / LF_CPR, c = lane % LF_CPR, q = wq0 + kTurnRows * turn + r;

@@ -213,6 +213,14 @@ __device__ __forceinline__ float lf_max_halves(float x) {
   return fmaxf(a, b);
 }
 
+// Between LDS accesses by which the lanes of one wave hand values to each other: the hardware keeps a wave's LDS operations
+// in order, and this tells the compiler, which reasons lane by lane, to keep them so.  No instruction.
+__device__ __forceinline__ void lf_wave_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // This lane's bit of a wave-uniform word, as a condition (the word itself is the select's operand).  The intrinsic by its
 // name: hipRTC's compiler knows no builtin for it yet.
 extern "C" __device__ bool lf_lane_bit(unsigned long long word) __asm("llvm.amdgcn.inverse.ballot.i64");

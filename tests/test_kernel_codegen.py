@@ -277,3 +277,29 @@ def test_masked_prefill_builds_and_does_not_spill(shim_built, bias, mask, softca
     does not assemble), and a branch around the products instead of that loop costs a second copy of O^T (spills)."""
     spec = lowering.KernelSpec("prefill_swp", 0, 128, mask, softcap, paged, 16 if paged else 1, bias=bias, pack=pack)
     assert not any("scratch_" in ln for ln in _kernels(spec)["lf_attn_prefill_swp"])
+
+
+@pytest.mark.parametrize("spec,kernels", [
+    (lowering.KernelSpec("prefill_swp", 0, 128, 1, False, bn=32), ["lf_attn_prefill_swp"]),
+    (lowering.KernelSpec("prefill_swp", 1, 64, 0, False), ["lf_attn_prefill_swp"]),
+    # (8 waves over 32-key tiles: the rows of a wave leave in two turns)
+    (lowering.KernelSpec("prefill_swp", 0, 128, 0, False, bn=32, extra=("-DLF_NW=8", "-DLF_WPE=1")), ["lf_attn_prefill_swp"]),
+    (lowering.bwd_spec(torch.bfloat16, 128, lowering.MASK_CAUSAL), ["lf_attn_bwd_dkdv", "lf_attn_bwd_dq"]),
+    (lowering.bwd_spec(torch.float16, 64, lowering.MASK_SLIDING), ["lf_attn_bwd_dkdv", "lf_attn_bwd_dq"]),
+], ids=["swp_bn32", "swp_d64", "swp_two_turns", "bwd_d128", "bwd_d64"])
+def test_rows_that_meet_in_lds_are_written_before_they_are_read(spec, kernels, tmp_path):
+    """The results' rows go from lane to lane through LDS without a barrier, a wave at a time.  Behind a kernel's last MFMA,
+    writes and the reads on either side of them are kept apart by a wave barrier (a note to the compiler) or a workgroup's."""
+    src, out = tmp_path / "kernel.hip", tmp_path / "kernel.s"
+    src.write_text(spec.source())
+    subprocess.run(["hipcc", "-x", "hip", "--offload-arch=gfx950", "--cuda-device-only", "-std=c++17", "-S", *spec.options(),
+                    str(src), "-o", str(out)], check=True, capture_output=True)
+    text = out.read_text()
+    for name in kernels:
+        body = text[text.index(f"\n{name}:"):text.index(f".size\t{name},")]
+        tail = body[body.rindex("v_mfma"):]
+        events = re.findall(r"ds_write|ds_read|wave barrier|s_barrier", tail)
+        steps = [e for i, e in enumerate(events) if i == 0 or e != events[i - 1]]
+        assert "ds_write" in steps and steps[-1] == "ds_read"
+        for a, b in zip(steps, steps[1:]):
+            assert {a, b} != {"ds_write", "ds_read"}, f"{name}: {steps}"
