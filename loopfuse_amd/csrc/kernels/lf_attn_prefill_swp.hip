@@ -90,6 +90,15 @@
 #define LF_CAP2_X0 0.4f
 #define LF_CAP2_B1 (-0.33269722f)
 #define LF_CAP2_B2 0.12145087f
+#ifndef LF_STAY
+#define LF_STAY 0        /* 1: O leaves in 32-byte pieces of every lane's own row by plain stores, 0: in whole rows by non-temporal ones.
+                            Whole rows save what partial lines take of the L2 from Q, K and V, but whoever reads O next fetches
+                            it from further away.  Times whole over pieces, 40 launches, the kernel alone / with an
+                            element-wise kernel or a product behind it: O of 6 ... 70 MB 0.88 ... 1.02 / 0.91 ... 1.03 (9 MB, B3 64/8
+                            S185 11.1 -> 9.8 us, with the product 58.0 -> 55.8; 67 MB, window 256 B4 32/8 S2048 56.4 -> 53.2), of 0.2 ... 5 MB
+                            0.97 ... 1.03 / 0.98 ... 1.12 (0.8 MB, B6 H4 S131 8.0 -> 8.1, with the product 16.7 -> 18.3).  Whole rows by
+                            plain stores: 1 % slower than pieces (lowering.prefill_out_stays) */
+#endif
 #ifndef LF_QGROUP
 #define LF_QGROUP 8      /* (batch, head) pairs per group of slots */
 #endif
@@ -778,22 +787,41 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
       p.part_ml[((long long)b * p.Hq + h) * p.Sq + my_q] = mc_ref + __builtin_log2f(l_tot);
 #endif
     {
-      // Rows leave whole, by non-temporal stores: a row's values meet in the tiles' LDS (behind the last tile's barrier nobody
-      // reads it any more; each wave has a part of its own), and neighbouring lanes write the 16-byte pieces of one row, 1 KB
-      // of consecutive bytes per store at head dim 128.  The lines then pass the L2 without taking it from Q, K and V:
-      // causal B8 32/8 S2048 278 -> 267 us, window 256 112 -> 98, window 256 with a cap 119 -> 108, causal B8 H32 with a cap 334 ->
-      // 325, without 299 -> 296, B8 16/4 S1000 D64 fp16 30.5 -> 28.5.  Whole rows alone, or 32-byte pieces without them: 1 %.
 #if LF_SAFE
       const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;      // a row that saw no key gives zeros
 #else
       const float inv = 1.0f / l_tot;
 #endif
+      lf_elem* ohead = p.o + (long long)b * p.o_sb + (long long)h * p.o_sh;
+      auto chunk = [&](int db, int i4) {       // d = 32*db + 8*i4 + 4*g + 0..3 of row my_q
+        lf_elem4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = lf_from_float(o[db][4 * i4 + e] * inv);
+        return __builtin_bit_cast(lf_u32x2, w);
+      };
+#if LF_STAY
+      // one v_permlane32_swap per register pair trades chunks with the lane that holds the other half of the same row, so that each
+      // lane owns 8 consecutive d's: 32 contiguous bytes per row and store
+      lf_elem* orow = ohead + (long long)min(my_q, p.Sq - 1) * p.o_ss;
+#pragma unroll
+      for (int db = 0; db < LF_NDB; ++db)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const lf_u32x2 c0 = chunk(db, 2 * j), c1 = chunk(db, 2 * j + 1);
+          auto r0 = __builtin_amdgcn_permlane32_swap(c0[0], c1[0], false, false);
+          auto r1 = __builtin_amdgcn_permlane32_swap(c0[1], c1[1], false, false);
+          const lf_u32x4 out = {r0[0], r1[0], r0[1], r1[1]};
+          if (my_q < p.Sq) *reinterpret_cast<lf_u32x4*>(orow + 32 * db + 16 * j + 8 * g) = out;
+        }
+#else
+      // Rows leave whole, by non-temporal stores: a row's values meet in the tiles' LDS (behind the last tile's barrier nobody
+      // reads it any more; each wave has a part of its own), and neighbouring lanes write the 16-byte pieces of one row, 1 KB
+      // of consecutive bytes per store at head dim 128.  The lines then pass the L2 without taking it from Q, K and V.
       constexpr int kStride = LF_D * 2 + 16, kSpace = (LF_KSLOTS + LF_VSLOTS) * LF_BN * LF_D * 2 / LF_NW;      // bytes per wave
       constexpr int kTurns = 32 * kStride <= kSpace ? 1 : 2, kTurnRows = 32 / kTurns, kRows = 64 / LF_CPR;      // rows per turn, per store
       static_assert(kTurnRows * kStride <= kSpace && kTurnRows % kRows == 0, "the rows of a turn fit a wave's part of the LDS");
       typedef __attribute__((address_space(3))) lf_u32x2* lf_lds_u32x2_out;
       const unsigned mine = lds0 + (unsigned)(wave * kTurnRows * kStride);
-      lf_elem* ohead = p.o + (long long)b * p.o_sb + (long long)h * p.o_sh;
 #pragma unroll
       for (int turn = 0; turn < kTurns; ++turn) {
         if (turn) lf_wave_exchange();
@@ -801,13 +829,8 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
 #pragma unroll
           for (int db = 0; db < LF_NDB; ++db)
 #pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-              lf_elem4 w;
-#pragma unroll
-              for (int e = 0; e < 4; ++e) w[e] = lf_from_float(o[db][4 * i4 + e] * inv);
-              *(lf_lds_u32x2_out)(size_t)(mine + (unsigned)(l32 % kTurnRows * kStride + 64 * db + 16 * i4 + 8 * g)) =
-                  __builtin_bit_cast(lf_u32x2, w);
-            }
+            for (int i4 = 0; i4 < 4; ++i4)
+              *(lf_lds_u32x2_out)(size_t)(mine + (unsigned)(l32 % kTurnRows * kStride + 64 * db + 16 * i4 + 8 * g)) = chunk(db, i4);
         }
         lf_wave_exchange();
 #pragma unroll
@@ -817,6 +840,7 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
           if (q < p.Sq) __builtin_nontemporal_store(x, reinterpret_cast<lf_u32x4*>(ohead + (long long)q * p.o_ss + 8 * c));
         }
       }
+#endif
     }
   };
 

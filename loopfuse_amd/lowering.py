@@ -96,6 +96,7 @@ class KernelSpec:
     safe: bool = False     # rows that saw no key come out as zeros instead of NaN
     bn: int = 0            # prefill_swp: keys per LDS tile, 32 (three workgroups per CU) or 0 / 64 (two)
     extra: tuple = ()      # further -D options (tuning experiments)
+    stay: bool = False     # prefill_swp: O by plain stores (prefill_out_stays)
 
     def __hash__(self):    # formed once: a call looks its kernels up by it, several times
         h = self.__dict__.get("_hash")
@@ -139,6 +140,8 @@ class KernelSpec:
                 o += [f"-DLF_GQAPACK={int(self.pack)}"]
             if self.bias:
                 o += ["-DLF_BIAS=2" if self.bias == MASK_BITS else "-DLF_BIAS=1"]
+            if self.stay:
+                o += ["-DLF_STAY=1"]
         if self.safe:
             o += ["-DLF_SAFE=1"]
         return o + list(self.extra)
@@ -163,7 +166,7 @@ class KernelSpec:
         return (f"lf_{self.family}_t{self.dtype}_d{self.head_dim}_m{self.mask}_c{int(self.softcap)}"
                 f"_p{self.paged}x{self.page_size}i{int(self.table_i64)}_r{self.rows}w{self.waves}v{int(self.v_tr)}h{int(self.headwave)}b{self.bias}n{int(self.denom)}"
                 + (f"_q{self.d2}" if self.d2 else "") + (f"_gp{int(self.pack)}" if self.pack else "") + (f"_pv{self.page_size_v}" if self.page_size_v else "")
-                + ("_z" if self.safe else "") + (f"_bn{self.bn}" if self.bn else "") + ("_co" if self.coop else "") + ("_rl" if self.rowload else "")
+                + ("_z" if self.safe else "") + (f"_bn{self.bn}" if self.bn else "") + ("_co" if self.coop else "") + ("_rl" if self.rowload else "") + ("_st" if self.stay else "")
                 + "".join("_" + e.replace("-D", "").replace("=", "") for e in self.extra))
 
     def source(self) -> str:
@@ -591,6 +594,14 @@ def prefill_kv_tile(D: int, bias_bits: int = 0, choice: Optional[dict] = None, w
     if want is not None:
         return 32 if int(want) == 32 else 0
     return 32 if D == 128 and workgroups >= (3 * 256 if keys < 2048 else 8 * 256) else 0
+
+
+def prefill_out_stays(nbytes: int) -> bool:
+    """Does lf_attn_prefill_swp write an output of so many bytes by plain stores (``-DLF_STAY=1``), which leave it near whoever reads
+    it next, and not in whole rows past the caches?  Whole over plain, the kernel with an element-wise kernel or a product
+    behind it, over 40 launches: below 5 MB 0.98 ... 1.12, 5 ... 6 MB 0.96 ... 1.05, 6 ... 10 MB 0.91 ... 1.01, above 0.94 ... 1.03; the
+    kernel alone 0.97 ... 1.03, 0.97 ... 1.00, 0.88 ... 1.00 and 0.91 ... 1.03."""
+    return nbytes < 6_000_000
 
 
 def prefill_variant(Sq: int, v_tr: bool = True) -> str:
@@ -1159,7 +1170,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPlan,
                      safe=plan.zero_blind_rows and bool(bias_bits & (1 | MASK_BITS)),
                      bn=prefill_kv_tile(D, bias_bits, choice, B * (Hq // (pack or 1)) * (-(-Sq // (128 // (pack or 1)))),
                                         min(Sk, P.window) if mask == MASK_SLIDING else Sk)
-                     if family == "prefill_swp" else 0)
+                     if family == "prefill_swp" else 0,
+                     stay=family == "prefill_swp" and prefill_out_stays(2 * B * Hq * Sq * D))
         bm, bn = TILE_SHAPES[family]
         nw = 4
         for e in spec.extra:                    # tuning: -DLF_NW=8 doubles the q tile

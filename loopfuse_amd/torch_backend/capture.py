@@ -473,6 +473,7 @@ class AttentionMatch:
                                           min(Sk, plan.window) if plan.mask == "sliding" else Sk)
         return [lowering.KernelSpec(family, dt, D, mask, plan.softcap is not None, paged, ps, i64, bias=bias, d2=d2,
                                     page_size_v=psv, pack=pack, extra=extra, bn=bn,
+                                    stay=family == "prefill_swp" and lowering.prefill_out_stays(2 * B * Hq * Sq * D),
                                     safe=plan.zero_blind_rows and bool(bias & 1) and family == "prefill")]
 
 

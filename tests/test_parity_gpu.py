@@ -1246,17 +1246,25 @@ def test_window_that_ends_behind_the_last_key(given, Sq, Sk, D, group):
 @pytest.mark.parametrize("Sq", [1, 31, 33, 127, 129])
 @pytest.mark.parametrize("D,group,bn", [(64, 1, 64), (128, 1, 64), (128, 1, 32), (128, 2, 32), (128, 4, 32)])
 def test_output_rows_end_where_the_queries_end(Sq, D, group, bn):
-    """The output leaves in whole rows from LDS: into a view with guard rows and columns around it, nothing beyond a head's rows."""
-    B, H = 2, 4
-    q, k, v = (rand((B, h, n, D), torch.bfloat16, s) for h, n, s in ((H, Sq, 1), (H // group, 200, 2), (H // group, 200, 3)))
-    buf = torch.full((B, H, Sq + 3, D + 8), 123.0, dtype=torch.bfloat16, device=dev())
-    out = buf[:, :, 1:Sq + 1, :D]
-    lowering.attention(q.to(dev()), k.to(dev()), v.to(dev()), lowering.AttnPlan(scale=D ** -0.5), out=out, choice={"bn": bn},
-                       force_family="prefill_swp")
-    assert lowering.attention.last_launch["kernels"] == ["lf_attn_prefill_swp"]
-    assert (out.float().cpu() - O.attention_reference(q, k, v)).abs().max().item() <= TOL[torch.bfloat16]
-    out.fill_(123.0)
-    assert (buf == 123.0).all()
+    """Into a view with guard rows and columns around it, nothing beyond a head's rows: where the output is small enough for
+    32-byte pieces, and where, of the same inputs again and again, it leaves in whole rows from LDS (6 MB and more): the same bits."""
+    B, H, Sk = 2, 4, 40 if Sq == 1 else 200
+    q, k, v = (rand((B, h, n, D), torch.bfloat16, s) for h, n, s in ((H, Sq, 1), (H // group, Sk, 2), (H // group, Sk, 3)))
+    want = O.attention_reference(q, k, v)
+    small = None
+    for copies in (1, -(-6000000 // (2 * B * H * Sq * D))):
+        buf = torch.full((copies * B, H, Sq + 3, D + 8), 123.0, dtype=torch.bfloat16, device=dev())
+        out = buf[:, :, 1:Sq + 1, :D]
+        lowering.attention(*(t.to(dev()).repeat(copies, 1, 1, 1) for t in (q, k, v)), lowering.AttnPlan(scale=D ** -0.5), out=out,
+                           choice={"bn": bn}, force_family="prefill_swp")
+        assert lowering.attention.last_launch["kernels"] == ["lf_attn_prefill_swp"]
+        assert lowering.prefill_out_stays(2 * out.numel()) == (copies == 1)
+        if small is None:
+            small = out.clone()
+            assert (small.float().cpu() - want).abs().max().item() <= TOL[torch.bfloat16]
+        assert torch.equal(out, small.repeat(copies, 1, 1, 1))
+        out.fill_(123.0)
+        assert (buf == 123.0).all()
 
 
 @pytest.mark.parametrize("case", ["decode", "key_stride", "register_staged"])
