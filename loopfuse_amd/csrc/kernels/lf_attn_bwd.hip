@@ -153,15 +153,45 @@ __device__ __forceinline__ void lf_bw_mfma_vva(lf_f32x16& c, const lf_u32x4& a, 
 // accumulators X^T[d][n] (lane n = lane % 32; element i of block db is d = 32*db + 8*(i/4) + 4*g + i%4)
 // -> rows 0 .. 31 of a [.., D] matrix, those below `valid`.  They meet in the wave's part of the LDS (`rows_lds`, LF_BW_ROWS_LDS
 // bytes that nobody reads any more) and leave whole, neighbouring lanes with the pieces of one row, by non-temporal stores:
-// 32-byte pieces of every lane's own row took the L2 from what the launch reads.  All backward launches, us: causal B4 H32 S2048 D128
-// 580 -> 567, unmasked 901 -> 853, window 256 B4 32/8 S2048 216 -> 204, unmasked B10 H32 S739 396 -> 380; launches of 25 us pay 0.5 for
-// the way through LDS.
+// 32-byte pieces of every lane's own row take the L2 from what the launch reads.
+#ifndef LF_STAY
+#define LF_STAY 0        /* 1: 32-byte pieces by plain stores all the same, which save the way through LDS and leave the gradients
+                            nearer to whoever reads them next.  All backward launches, times whole over pieces, 57 shapes, alone / with an
+                            element-wise kernel behind them that reads the gradients: dQ of 0.2 ... 10 MB 0.98 ... 1.04 / 0.99 ... 1.13 (0.4
+                            MB, unmasked B5 H4 S163 D64 16.6 -> 16.8 and 27.1 -> 30.5 us), 10 ... 30 MB 0.95 ... 1.00 / 0.99 ... 1.03, above
+                            0.90 ... 1.00 / 0.95 ... 1.01 (67 MB, causal B4 H32 S2048 D128 556 -> 535 and 618 -> 613, unmasked 885 -> 855
+                            and 953 -> 906) (lowering.bwd_grads_stay) */
+#endif
 #define LF_BW_OUT_STRIDE (LF_D * 2 + 16)
 #define LF_BW_ROWS_LDS (32 * LF_BW_OUT_STRIDE)
 __device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, unsigned rows_lds, lf_elem* rows, long long stride, int valid, int lane) {
   typedef __attribute__((address_space(3))) lf_u32x2* lds_write_t;
   typedef __attribute__((address_space(3))) const lf_u32x4* lds_read_t;
   const int l32 = lane & 31, g = lane >> 5;
+#if LF_STAY
+  (void)rows_lds;
+  lf_elem* row = rows + l32 * stride + 8 * g;
+#pragma unroll
+  for (int db = 0; db < LF_NDB; ++db) {
+    unsigned ch[4][2];
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      lf_elem4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = lf_from_float(acc[db][4 * i4 + e]);
+      const lf_u32x2 wu = __builtin_bit_cast(lf_u32x2, w);
+      ch[i4][0] = wu[0];
+      ch[i4][1] = wu[1];
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {      // halves of a row change lanes: 8 consecutive d's each, 32 contiguous bytes per row and store
+      auto r0 = __builtin_amdgcn_permlane32_swap(ch[2 * j][0], ch[2 * j + 1][0], false, false);
+      auto r1 = __builtin_amdgcn_permlane32_swap(ch[2 * j][1], ch[2 * j + 1][1], false, false);
+      const lf_u32x4 out = {r0[0], r1[0], r0[1], r1[1]};
+      if (l32 < valid) *reinterpret_cast<lf_u32x4*>(row + 32 * db + 16 * j) = out;
+    }
+  }
+#else
   lf_wave_exchange();              // the rows before these have been read
 #pragma unroll
   for (int db = 0; db < LF_NDB; ++db)
@@ -180,6 +210,7 @@ __device__ __forceinline__ void lf_bw_store_rows(const lf_f32x16* acc, unsigned 
     const lf_u32x4 x = *(lds_read_t)(size_t)(rows_lds + (unsigned)(r * LF_BW_OUT_STRIDE + 16 * c));
     if (r < valid) __builtin_nontemporal_store(x, reinterpret_cast<lf_u32x4*>(rows + r * stride + 8 * c));
   }
+#endif
 }
 
 // ---- tiles that are kept in LDS once and read both ways.  A 64-row tile is row-major and unpadded; the 16-byte
@@ -826,7 +857,9 @@ extern "C" __global__ void __launch_bounds__(LF_BW_NT, 1) lf_attn_bwd_dkdv(const
 #else
   static_assert(4 * LF_BW_ROWS_LDS <= (int)sizeof(tiles), "the rows fit the tiles");
   const unsigned rows_lds = lds0 + (unsigned)(wave * LF_BW_ROWS_LDS);
+#if !LF_STAY
   __syncthreads();               // nobody reads the tiles any more
+#endif
 #endif
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
@@ -985,7 +1018,9 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[db][i] *= p.scale;
   static_assert(kWaves * LF_BW_ROWS_LDS <= (int)sizeof(ds_tiles), "the rows fit the tiles");
+#if !LF_STAY
   __syncthreads();               // nobody reads the tiles any more
+#endif
   lf_bw_store_rows(dq, ds0_lds + (unsigned)(wave * LF_BW_ROWS_LDS), p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)wq0 * p.dq_ss,
                    p.dq_ss, p.Sq - wq0, lane);
 }
@@ -1314,7 +1349,9 @@ extern "C" __global__ void __launch_bounds__(LF_BW_DQ_NT, LF_BW_DQ_NT / 256) lf_
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[db][i] *= p.scale;
   static_assert(LF_BW_DQ_NT / 64 * LF_BW_ROWS_LDS <= (int)sizeof(tiles), "the rows fit the tiles");
+#if !LF_STAY
   __syncthreads();               // nobody reads the tiles any more
+#endif
   lf_bw_store_rows(dq, lds0 + (unsigned)(wave * LF_BW_ROWS_LDS), p.dq + (long long)b * p.dq_sb + (long long)h * p.dq_sh + (long long)wq0 * p.dq_ss,
                    p.dq_ss, p.Sq - wq0, lane);
 }

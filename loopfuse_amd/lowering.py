@@ -96,7 +96,7 @@ class KernelSpec:
     safe: bool = False     # rows that saw no key come out as zeros instead of NaN
     bn: int = 0            # prefill_swp: keys per LDS tile, 32 (three workgroups per CU) or 0 / 64 (two)
     extra: tuple = ()      # further -D options (tuning experiments)
-    stay: bool = False     # prefill_swp: O by plain stores (prefill_out_stays)
+    stay: bool = False     # prefill_swp, bwd: results by plain stores (prefill_out_stays, bwd_grads_stay)
 
     def __hash__(self):    # formed once: a call looks its kernels up by it, several times
         h = self.__dict__.get("_hash")
@@ -140,8 +140,8 @@ class KernelSpec:
                 o += [f"-DLF_GQAPACK={int(self.pack)}"]
             if self.bias:
                 o += ["-DLF_BIAS=2" if self.bias == MASK_BITS else "-DLF_BIAS=1"]
-            if self.stay:
-                o += ["-DLF_STAY=1"]
+        if self.stay:
+            o += ["-DLF_STAY=1"]
         if self.safe:
             o += ["-DLF_SAFE=1"]
         return o + list(self.extra)
@@ -1431,10 +1431,18 @@ def bwd_keep_ds(D: int, softcap: bool, units: int, group: int, Sk: int, blocks: 
     return D == 128 or softcap or (units <= 64 and group <= 4 and Sk >= 512 and size <= 176 << 20)
 
 
-@functools.lru_cache(maxsize=256)
+def bwd_grads_stay(nbytes: int) -> bool:
+    """Are the gradients written by plain stores (``-DLF_STAY=1``), which leave them near whoever reads them next, and not in
+    whole rows past the caches?  ``nbytes`` = size of dQ.  Whole over plain, 57 shapes, all launches alone / with an element-wise kernel
+    behind them that reads the gradients: below 10 MB 0.98 ... 1.04 / 0.99 ... 1.13, 10 ... 30 MB 0.95 ... 1.00 / 0.99 ... 1.03,
+    above 0.90 ... 1.00 / 0.95 ... 1.01."""
+    return nbytes < 10_000_000
+
+
+@functools.lru_cache(maxsize=512)
 def bwd_spec(dtype: torch.dtype, D: int, mask: int, softcap: bool = False, key_blocks: int = 1,
-             dq_threads: int = 512, keep_ds: bool = False, q_split: bool = False) -> KernelSpec:
-    return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap,
+             dq_threads: int = 512, keep_ds: bool = False, q_split: bool = False, stay: bool = False) -> KernelSpec:
+    return KernelSpec("bwd", _DTYPE_CODE[dtype], D, mask, softcap, stay=stay,
                       extra=(f"-DLF_BW_DQ_NT={dq_threads}", f"-DLF_BW_W={key_blocks}") + (("-DLF_BW_DS=1",) if keep_ds else ())
                       + (("-DLF_BW_QSPLIT=1",) if q_split else ()))
 
@@ -1541,7 +1549,7 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
         q_split = not (key_blocks and key_blocks != 1) and bwd_q_split(D, mask, B * Hkv, Sk)
     if q_split:
         keys = 1
-    spec = bwd_spec(dtype, D, mask, cap, keys, nt, ds is not None, q_split)
+    spec = bwd_spec(dtype, D, mask, cap, keys, nt, ds is not None, q_split, bwd_grads_stay(2 * B * Hq * Sq * D))
     keep = (q, k, v, o, dout, lse, delta, dq, dk, dv, ds)  # noqa: F841  (tensors stay alive until the launches are queued)
     steps = {"lf_attn_bwd_delta": (-(-B * Hq * Sq // 16), 256),
              "lf_attn_bwd_dkdv": (xcd_slots(B * Hkv, -(-Sk // (128 * keys // (2 if q_split else 1)))), 256),

@@ -388,6 +388,34 @@ def test_dq_workgroup_size_rule(units, Sq, want):
     assert lowering.bwd_dq_threads(64, lowering.MASK_SLIDING, False, units, Sq, Sq) == 256
 
 
+@pytest.mark.parametrize("Hq,Hkv,Sq,Sk,D,mask,key_blocks,dq_threads,keep_ds,q_split", [
+    (4, 4, 333, 333, 128, "causal", 1, 512, True, False),
+    (4, 2, 333, 333, 128, None, 2, 256, False, False),
+    (4, 4, 129, 250, 128, None, 2, 512, True, False),
+    (4, 4, 300, 300, 64, "sliding", 1, 256, False, True),
+    (4, 1, 161, 161, 64, "causal", 1, 512, True, True),
+])
+def test_both_forms_of_the_gradients_stores(Hq, Hkv, Sq, Sk, D, mask, key_blocks, dq_threads, keep_ds, q_split):
+    """A batch of one, whose gradients are small enough for plain stores, and the same inputs so often that they leave in whole rows
+    past the caches (dQ of 10 MB and more): the same bits, rows that end inside a tile included."""
+    g = torch.Generator().manual_seed(Sq + D)
+    q, k, v, dout = (torch.randn((1, h, n, D), generator=g).bfloat16().to(DEV) for h, n in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk), (Hq, Sq)))
+    plan = lowering.AttnPlan(mask=mask, window=70 if mask == "sliding" else 0, scale=D ** -0.5)
+    lse = torch.empty((1, Hq, Sq), dtype=torch.float32, device=DEV)
+    o = lowering.attention(q, k, v, plan, lse=lse)
+    want = _ref(q, k, v, dout, mask, plan.window, plan.scale)[2:]
+    first = None
+    for copies in (1, -(-10_000_000 // (2 * Hq * Sq * D))):
+        assert lowering.bwd_grads_stay(2 * copies * Hq * Sq * D) == (copies == 1)
+        got = lowering.attention_backward(*(t.repeat(copies, *[1] * (t.dim() - 1)) for t in (q, k, v, o, lse, dout)), plan,
+                                          key_blocks=key_blocks, dq_threads=dq_threads, keep_ds=keep_ds, q_split=q_split)
+        if first is None:
+            first = got
+            for a, w in zip(got, want):
+                assert ((a.double() - w).norm() / w.norm()).item() <= 1e-2      # (2^-9 per rounded operand and result, a few of them)
+        assert all(torch.equal(a, b.expand_as(a)) for a, b in zip(got, first))
+
+
 @pytest.mark.parametrize("scale", [64.0, 0.0])
 @pytest.mark.parametrize("Hkv,D,mask,key_blocks", [(2, 128, "causal", 1), (2, 128, "causal", 2), (1, 64, None, 1)])
 def test_dv_rounds_a_large_exponent_once(Hkv, D, mask, key_blocks, scale):

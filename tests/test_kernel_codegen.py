@@ -229,7 +229,8 @@ def test_every_split_the_rules_choose_is_built():
                             blocks = units * group * lowering.bwd_ds_blocks(mask, 256, S, S)
                             for keep in {False, lowering.bwd_keep_ds(D, cap, units * group, group, S, blocks)}:
                                 spec = lowering.bwd_spec(dtype, D, mask, cap, 1 if q_split else lowering.bwd_key_blocks(D, mask, cap, units, S),
-                                                         lowering.bwd_dq_threads(D, mask, cap, units * group, S, S), keep, q_split)
+                                                         lowering.bwd_dq_threads(D, mask, cap, units * group, S, S), keep, q_split,
+                                                         lowering.bwd_grads_stay(2 * units * group * S * D))
                                 assert spec in built, spec
                                 chosen.add(spec)
     assert {("-DLF_BW_DS=1" in s.extra, "-DLF_BW_QSPLIT=1" in s.extra) for s in chosen} == {(a, b) for a in (False, True) for b in (False, True)}
