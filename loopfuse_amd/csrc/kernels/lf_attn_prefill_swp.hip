@@ -77,6 +77,9 @@
                             no vector load in the loop.  B4 H32 S1536 D128, causal and padding, both launches: 110 us with the
                             16-bit bias of form 1 for mixed blocks, 101 with the bits */
 #endif
+#if LF_BIAS == 2 && LF_BN != 64
+#error "a boolean mask goes with 64-key tiles: under 32 keys its results are less exact (lowering.prefill_kv_tile)"
+#endif
 #define LF_BARRIER_VM0() asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory")
 
 #define LF_CAPPOLY (LF_SOFTCAP && !LF_BIAS)   /* polynomial fast path of the softcap (below) */
@@ -509,7 +512,8 @@ extern "C" __global__ void __launch_bounds__(LF_NT, LF_WPE) lf_attn_prefill_swp(
       bool need = wave_has_rows;
       bool full = (k0 + LF_BN <= p.Sk);
 #if LF_BM == 32
-      need = true;               // every tile of the range holds something for the 32 rows that all waves share
+      need = true;               // all waves share the 32 rows that the range is formed for (behind the last key it may hold a tile that
+                                 // a window hides as a whole: its scores are masked one by one)
 #elif LF_MASK >= 1
       need = need && (k0 <= wqlast);
 #if LF_MASK == 2

@@ -166,7 +166,7 @@ def one_attention(gm: torch.fx.GraphModule, sample_inputs, general):
     """``general``, AOTAutograd's callable for the rewritten training graph ``gm``, with a shorter way for calls over plain tensors
     where the graph is nothing but one attention over its inputs as they are: ``_Attention``, without the wrappers that
     find out on every call what this graph does not have (aliases, mutations, subclasses, tangents of another layout).
-    B8 16/4 S1000 D64 fp16, forward and backward (139 us of kernels): 251 -> 151 us a step.  Everything else -- what ``_plain``
+    B8 16/4 S1000 D64 fp16, forward and backward (143 us of kernels): 252 -> 162 us a step.  Everything else -- what ``_plain``
     sends away, dynamic sizes, operands that are views or held by the graph, one tensor in two places, several outputs -- goes
     through ``general``, and so does the first call: its graphs, the backward's too, are then there for whoever needs them."""
     nodes = list(gm.graph.nodes)

@@ -280,6 +280,11 @@ def test_masked_prefill_builds_and_does_not_spill(shim_built, bias, mask, softca
     assert not any("scratch_" in ln for ln in _kernels(spec)["lf_attn_prefill_swp"])
 
 
+def test_boolean_masks_build_with_64_key_tiles_only(shim_built):
+    with pytest.raises(RuntimeError, match="64-key tiles"):
+        lowering.compile_spec(lowering.KernelSpec("prefill_swp", 0, 128, 0, False, bias=lowering.MASK_BITS, bn=32))
+
+
 @pytest.mark.parametrize("spec,kernels", [
     (lowering.KernelSpec("prefill_swp", 0, 128, 1, False, bn=32), ["lf_attn_prefill_swp"]),
     (lowering.KernelSpec("prefill_swp", 1, 64, 0, False), ["lf_attn_prefill_swp"]),
