@@ -26,6 +26,7 @@ there, ``interface.py:157-161``).  Set ``LOOPFUSE_STRICT=1`` to raise instead;
 """
 from __future__ import annotations
 
+import functools
 import logging
 import os
 from functools import partial
@@ -249,6 +250,9 @@ def _training_graph(gm: torch.fx.GraphModule, sample_inputs):
         return None
     if not all(t.is_cuda for t in sample_inputs if isinstance(t, torch.Tensor)):
         return None                                          # the kernels run on the GPU only: CPU graphs stay unfused
+    if _cuts_gradients(gm, sample_inputs):
+        log.info("training graph: detach or a change of grad mode inside; running unfused")
+        return None
     try:
         with torch.no_grad():
             aten_gm = make_fx(gm, tracing_mode="real", _allow_non_fake_inputs=True)(*sample_inputs)
@@ -284,6 +288,44 @@ def _training_graph(gm: torch.fx.GraphModule, sample_inputs):
     training.stats = stats
     general = aot_module_simplified(rewritten, sample_inputs, fw_compiler=_training_compiler, bw_compiler=_training_compiler)
     return training.one_attention(rewritten, sample_inputs, general)
+
+
+def _cuts_gradients(gm: torch.fx.GraphModule, sample_inputs) -> bool:
+    """Does the graph stop a gradient that would flow otherwise (``detach`` or ``.data`` of something that has one, a region under
+    ``no_grad`` that reads it)?  The forward that is traced for the matcher, without gradients, does not show where, and what
+    AOTAutograd differentiates is made from it."""
+    def name(n):
+        return getattr(n.target, "__name__", str(n.target))
+
+    def calls(module):
+        return [n for n in module.graph.nodes if n.op in ("call_function", "call_method", "call_module")]
+
+    stops = ("detach", "get_data_attr")
+    bodies = [m for m in gm.modules() if isinstance(m, torch.fx.GraphModule) and m is not gm]
+    inside = any(w in name(n) for m in bodies for n in calls(m) for w in (*stops, "set_grad_enabled", "inference_mode"))
+    given = iter(sample_inputs)
+    graded, recording = set(), [True]
+    for n in gm.graph.nodes:
+        if n.op == "placeholder":
+            has = getattr(next(given, None), "requires_grad", False)
+        elif n.op == "get_attr":
+            has = getattr(functools.reduce(getattr, n.target.split("."), gm), "requires_grad", False) is True
+        elif n.op == "output":
+            continue
+        elif "set_grad_enabled" in name(n):
+            recording[-1] = bool(n.args[0])
+            continue
+        elif "inference_mode" in name(n):
+            recording.append(False) if "enter" in name(n) else recording.pop()
+            continue
+        else:
+            has = any(x in graded for x in n.all_input_nodes) or \
+                (n.op == "call_module" and any(p.requires_grad for p in gm.get_submodule(n.target).parameters()))
+            if has and (not recording[-1] or inside or any(w in name(n) for w in stops)):
+                return True
+        if has:
+            graded.add(n)
+    return False
 
 
 def _training_compiler(gm: torch.fx.GraphModule, sample_inputs) -> Callable:

@@ -162,6 +162,49 @@ def test_the_short_way_gives_the_bits_of_the_general_one(dout, monkeypatch):
         assert fn(*x).equal(alone)
 
 
+def _no_grad_values(q, k, v):
+    with torch.no_grad():
+        v = v * 0.5
+    return _attn(q, k, v)
+
+
+def _no_grad_angles(q, k, v):
+    with torch.no_grad():      # (as rotary embeddings form theirs: nothing with a gradient is read)
+        turn = torch.arange(q.shape[2], device=q.device).to(q.dtype)[:, None].cos()
+    return _attn(q * turn, k, v)
+
+
+_CUT = {"queries": lambda q, k, v: _attn(q.detach(), k, v), "data": lambda q, k, v: _attn(q, k.data, v), "values": _no_grad_values,
+        "none": lambda q, k, v: _attn(q * 0.5, k, v), "nothing": _no_grad_angles}
+
+
+@pytest.mark.parametrize("cut", sorted(_CUT))
+def test_cut_gradients_are_seen(cut):
+    seen = []
+    torch._dynamo.reset()
+    torch.compile(_CUT[cut], backend=lambda gm, inputs: (seen.append(interface._cuts_gradients(gm, inputs)), gm)[1])(
+        *(torch.randn(1, 2, 8, 64, requires_grad=True) for _ in range(3)))
+    assert seen == [cut in ("queries", "data", "values")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cut", sorted(_CUT))
+def test_gradients_stop_where_the_function_stops_them(cut):
+    *x, d = _tensors(70)
+    x = [t.requires_grad_() for t in x]
+    torch._dynamo.reset()
+    fn = torch.compile(_CUT[cut], backend=functools.partial(loopfuse_backend, mode=None), dynamic=False)
+    want = torch.autograd.grad(_CUT[cut](*x), x, d, allow_unused=True)
+    graphs = interface.stats["training_graphs"]
+    for _ in range(2):
+        got = torch.autograd.grad(fn(*x), x, d, allow_unused=True)
+        for a, w in zip(got, want):
+            assert (a is None) == (w is None)
+            # bf16 operands, probabilities and results on either side: 2^-9 each, a few of them per value
+            assert a is None or ((a.double() - w.double()).norm() / w.double().norm()).item() <= 2e-2
+    assert interface.stats["training_graphs"] == graphs + (cut in ("none", "nothing"))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("buffer", [False, True])
 def test_training_with_keys_that_the_graph_holds(buffer, monkeypatch):
