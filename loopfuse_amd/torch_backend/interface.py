@@ -255,7 +255,7 @@ def _training_graph(gm: torch.fx.GraphModule, sample_inputs):
         return None
     try:
         with torch.no_grad():
-            aten_gm = make_fx(gm, tracing_mode="real", _allow_non_fake_inputs=True)(*sample_inputs)
+            aten_gm = make_fx(gm, tracing_mode="real", _allow_non_fake_inputs=True)(*_to_trace_on(gm, sample_inputs))
         matches = capture.match_attention(aten_gm)
     except capture.NoMatch as e:
         log.info("training graph: no attention found (%s)", e)
@@ -288,6 +288,24 @@ def _training_graph(gm: torch.fx.GraphModule, sample_inputs):
     training.stats = stats
     general = aot_module_simplified(rewritten, sample_inputs, fw_compiler=_training_compiler, bw_compiler=_training_compiler)
     return training.one_attention(rewritten, sample_inputs, general)
+
+
+def _to_trace_on(gm: torch.fx.GraphModule, sample_inputs) -> list:
+    """``sample_inputs`` for a trace that computes with them: copies of those that the graph may write to, so that the first
+    call's own run is the one that counts.  These are what a run without data writes to, and whatever has no
+    gradient (the running statistics of a normalisation change unseen there); weights are never copied for nothing."""
+    from torch._subclasses import FakeTensorMode
+
+    try:
+        with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+            fakes = [mode.from_tensor(t) if isinstance(t, torch.Tensor) else t for t in sample_inputs]
+            before = [t._version if isinstance(t, torch.Tensor) else 0 for t in fakes]
+            gm(*fakes)
+            written = [isinstance(t, torch.Tensor) and t._version != v for t, v in zip(fakes, before)]
+    except Exception as e:
+        log.info("training graph: run without data failed (%s: %s); traced on copies", type(e).__name__, e)
+        written = [True] * len(sample_inputs)
+    return [t.clone() if isinstance(t, torch.Tensor) and (w or not t.requires_grad) else t for t, w in zip(sample_inputs, written)]
 
 
 def _cuts_gradients(gm: torch.fx.GraphModule, sample_inputs) -> bool:

@@ -205,6 +205,38 @@ def test_gradients_stop_where_the_function_stops_them(cut):
     assert interface.stats["training_graphs"] == graphs + (cut in ("none", "nothing"))
 
 
+def _counts(q, k, v, d, n):
+    d.mul_(2.0)
+    n += 1
+    return _attn(q, k, v)
+
+
+def test_a_trace_writes_to_copies():
+    seen = []
+
+    def backend(gm, inputs):
+        names = [n.name for n in gm.graph.nodes if n.op == "placeholder"]
+        seen.append({name.strip("l_"): a is not b for name, a, b in zip(names, inputs, interface._to_trace_on(gm, inputs))})
+        return gm
+
+    torch._dynamo.reset()
+    leaf = [torch.randn(1, 2, 8, 64, requires_grad=True) for _ in range(4)]
+    torch.compile(_counts, backend=backend)(*leaf[:3], leaf[3] * 1.0, torch.zeros(()))
+    assert seen == [{"q": False, "k": False, "v": False, "d": True, "n": True}]
+
+
+@pytest.mark.gpu
+def test_the_first_call_writes_once():
+    q, k, v, d = _tensors(60)
+    q.requires_grad_()
+    n, once = torch.zeros((), device="cuda"), 2.0 * d
+    torch._dynamo.reset()
+    fn = torch.compile(_counts, backend=functools.partial(loopfuse_backend, mode=None), dynamic=False)
+    for calls in (1, 2):
+        fn(q, k, v, d, n).sum().backward()
+        assert n.item() == calls and torch.equal(d, once * 2.0 ** (calls - 1))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("buffer", [False, True])
 def test_training_with_keys_that_the_graph_holds(buffer, monkeypatch):
